@@ -140,7 +140,7 @@ def _case_mesh(case):
 
 
 def _params(case, dt):
-    p = W.spark_params(t_final=1e9, states_interval=20 * dt)
+    p = W.spark_params(t_final=1e9, states_interval=0.01)
     p.setr(T_STEP=dt, INIT_RYR_HOLD=dt)
     p.seti(INIT_RYR=0)
     if case.get("physics") == "extended":
