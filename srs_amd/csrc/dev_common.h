@@ -368,7 +368,7 @@ struct HostMesh {
   std::vector<uint16_t> cls;
   std::vector<double> tab;
   int32_t n_class = 0;
-  int32_t *d_nbr = nullptr;
+  int32_t *d_nbr = nullptr, *d_inv = nullptr;
   double *d_coef = nullptr, *d_V0 = nullptr, *d_tt = nullptr, *d_br = nullptr, *d_tab = nullptr;
   uint8_t* d_flags = nullptr;
   int16_t *d_off = nullptr, *d_dq = nullptr;
@@ -452,7 +452,7 @@ struct srs_ctx {
   bool tiles_compacted = false;
   int32_t* d_groups = nullptr;  // [n_groups][group] realization ids, -1 pads
   std::vector<int32_t> groups;
-  double* stage = nullptr;       // staging buffer for state transfers of grouped realizations
+  double* stage = nullptr;       // staging buffer of state transfers (state_xfer)
   size_t stage_len = 0;
   double last_total_ms = 0, last_sweep_ms = 0;
   // captured step blocks, keyed by (steps, gate mode)
@@ -510,7 +510,7 @@ int tiles_compact(srs_ctx* c);
 int plan_subsets(srs_ctx* c);
 void launch_subset_block(srs_ctx* c, int64_t m, uint32_t gmode);
 int live_rw(srs_ctx* c, int32_t r, RealLive* lv, bool write);
-int slot_copy(srs_ctx* c, const RealDesc& d, double* dev, double* host, bool to_dev);
+int state_xfer(srs_ctx* c, int32_t r, double* host, bool to_dev);
 
 // The line-scan kernels (linescan.hip), also launched by the adjoint.
 __global__ void k_scan_blur(const RealDesc* __restrict__ D, const RealLive* __restrict__ L, int r,
