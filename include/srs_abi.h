@@ -276,26 +276,26 @@ int srs_ctx_create(int device, srs_ctx** out);
 /* Kernel and layout tunables (no reference counterpart; the reference fixes
  * 256-thread blocks, gpu/RunSimulation.cu:784).  They change speed only,
  * never results.  Layout keys must be set before the first mesh is added,
- * the tile before srs_ctx_finalize; the rest at any time.  The defaults are
- * the fastest setting measured on the 3M-element dyad mesh in either element
- * order, short of the register budget (which helps in the block order only). */
-#define SRS_TUNE_TILE 1          /* elements per sweep workgroup: 128, 256, 512; by default srs_ctx_finalize
-                                    takes 512 when a realization's mesh has 2^20 elements or more, else 256 */
+ * the tile before srs_ctx_finalize; the rest at any time. */
+#define SRS_TUNE_TILE 1          /* elements per sweep workgroup: 128, 256 or 512 (default) */
 #define SRS_TUNE_NT_GEOMETRY 2   /* 1 (default): non-temporal loads of operator rows and flags */
 #define SRS_TUNE_NT_STATE 3      /* 1: non-temporal stores of the new state */
 #define SRS_TUNE_PLANE_PAD 4     /* extra elements (multiple of 64) between SoA planes */
-#define SRS_TUNE_COMPACT 5       /* 1 (default): store operator rows as class + int16 ulp deltas and
-                                    neighbours as int16 offsets where that reproduces them exactly */
-#define SRS_TUNE_OCCUPANCY 6     /* sweep register budget: 0 compiler's choice; 6 or 8: at most 80 or 64
-                                    VGPRs, so that six or eight wavefronts share each SIMD */
+#define SRS_TUNE_COMPACT 5       /* 1 (default): store operator rows as class + int16 deltas of the
+                                    bit patterns where that reproduces them exactly */
+#define SRS_TUNE_OCCUPANCY 6     /* register budget of the single-realization step with the gating folded
+                                    in (SRS_TUNE_GATED_SWEEP): 0 compiler's choice; 6: at most 80 VGPRs,
+                                    so that six wavefronts share each SIMD; 8: separate gating launches.
+                                    The sweep itself fits 64 VGPRs and has no budget */
 #define SRS_TUNE_GROUP 7         /* 1 (default), 2 or 4: realizations of one mesh whose states are interleaved
-                                    per element so that each sweep tile loads the operator rows once for all
-                                    of them (set before srs_ctx_finalize) */
-#define SRS_TUNE_LDS 8           /* 1 (default): stage each sweep tile's diffusing species in LDS and read
-                                    neighbours inside the tile from there (groups of 1) */
+                                    per 64 elements and whose tiles are swept side by side, so that the
+                                    operator rows come from cache for all but the first (set before
+                                    srs_ctx_finalize) */
+#define SRS_TUNE_LDS 8           /* accepted and ignored: each sweep tile's diffusing species, and those
+                                    of the elements its own neighbour, are always staged in LDS */
 #define SRS_TUNE_DROP_FINISHED 9 /* 1 (default): srs_explicit_step leaves the tiles of groups whose
                                     realizations have all finished out of the sweep; 0: sweep them all */
-#define SRS_TUNE_GATED_SWEEP 10  /* 1 (default): a single-realization context with the LDS sweep runs each
+#define SRS_TUNE_GATED_SWEEP 10  /* 1 (default): a single-realization context runs each
                                     step's gating (and, with SRS_STEP_PROTOCOL, the loop body) inside the
                                     next step's sweep launch (register budget 0 or 6; 0 with the loop
                                     body); 0: a gating launch after every sweep */

@@ -32,34 +32,59 @@ constexpr int MAX_LCC = 1024;
 constexpr int NXCD = 8;        // MI355X: 8 XCDs, workgroups dispatched round-robin
 
 enum : uint8_t { F_JSR = 1, F_TROPC = 2, F_SL = 4, F_BR = 8, F_CHAN = 16 };
+// What holds for every element of a 64-element block (the elements of one
+// wavefront of a sweep), read with one scalar load per wavefront.
+enum : uint32_t {
+  BLK_PLAIN = 1,  // every element is plain cytosol with troponin (F_TROPC and nothing else)
+};
 
 // State layout of one realization (6*np doubles): the four diffusing species
-// interleaved per element, (Ca, ATP, CaM, Fluo) in 32 bytes, so that one
-// neighbour gather fetches all four with one contiguous access; then the TnC
-// and CSQ planes, which are never gathered.
-constexpr int MOB_SLOT[6] = {0, 1, 2, -1, -1, 3};  // species -> slot in the interleaved quad
-// A realization group holds K realizations of one mesh in blocks of 64
-// elements: block b holds the 64 quads of slot 0, then slot 1, ..., so a
-// wavefront's loads of one realization stay contiguous.  Element e of slot
-// `slot` is entry ((e/64)*K + slot)*64 + e%64 of the quad array, and of the
-// TnC and CSQ planes (K*np entries each) that follow the 4*K*np quad doubles.
+// of 64 elements form a block of two halves, 64 pairs (Ca, ATP) and then 64
+// pairs (CaM, Fluo), so that each of a wavefront's 16-byte loads and stores of
+// consecutive elements covers 1 KB without gaps and a neighbour costs two
+// such loads; then the TnC and CSQ planes, which are never gathered.  With
+// the four species side by side (32 B per element) every access covered half
+// of each cache line it touched: a plain copy in that form ran at 5.7 TB/s
+// against 6.3, and the write requests to L2 were 72 per wavefront instead of
+// 40 (48-member ensemble: 175.7 -> 171.8 us per step; with non-temporal
+// stores, which that form had made slower, 154 us).
+// A realization group holds K realizations of one mesh block by block: the
+// block of slot 0, then slot 1, ...  Element e of slot `slot` is pair
+// qidx(e, K, slot) of the array, its second pair 64 pairs on; in the TnC and
+// CSQ planes (K*np entries each) that follow the 4*K*np doubles it is entry
+// ((e/64)*K + slot)*64 + e%64.
+constexpr int QHALF = 64;              // pairs from an element's first pair to its second
+constexpr int FLUO_OFF = 2 * QHALF + 1;  // doubles from an element's Ca to its Fluo
 __host__ __device__ inline size_t gidx(size_t e, int K, int slot) {
   return ((e >> 6) * (size_t)K + (size_t)slot) * 64 + (e & 63);
 }
-__host__ __device__ inline size_t xoff(int s, size_t e, size_t np, int K = 1, int slot = 0) {
-  const size_t q = gidx(e, K, slot);
-  return s == srs::TRPN ? 4 * (size_t)K * np + q : s == srs::CSQN ? 5 * (size_t)K * np + q : 4 * q + MOB_SLOT[s];
+__host__ __device__ inline size_t qidx(size_t e, int K, int slot) {
+  return ((e >> 6) * (size_t)K + (size_t)slot) * (2 * QHALF) + (e & 63);
 }
+// Groups of one: pairs of 2^31 elements still count in 32 bits.
+__host__ __device__ inline uint32_t qidx1(uint32_t e) { return e + (e & ~63u); }
+__host__ __device__ inline size_t xoff(int s, size_t e, size_t np, int K = 1, int slot = 0) {
+  if (s == srs::TRPN) return 4 * (size_t)K * np + gidx(e, K, slot);
+  if (s == srs::CSQN) return 5 * (size_t)K * np + gidx(e, K, slot);
+  const size_t q = 2 * qidx(e, K, slot);
+  return s == srs::CA ? q : s == srs::ATP ? q + 1 : s == srs::CMDN ? q + FLUO_OFF - 1 : q + FLUO_OFF;
+}
+typedef double d2 __attribute__((ext_vector_type(2)));
 typedef double d4 __attribute__((ext_vector_type(4)));
 
 // Immutable per-realization descriptor (read with scalar loads).
 struct RealDesc {
-  const int32_t* nbr;     // [4][np]
-  const double* coef;     // [5][np] (plain layout)
-  const int16_t* off;     // compact layout: [4][np] neighbour offsets j' - j
-  const uint16_t* cls;    // compact layout: [np] operator-row class
-  const int16_t* dq;      // compact layout: [5][np] coefficient deltas in ulps of the class row
-  const double* tab;      // compact layout: [n_class][10] class row (5 values) and its ulps (5 values)
+  const int32_t* nbr;     // [np][4] neighbour indices
+  // tile map of the sweep (TileMap): where each element's neighbours are among
+  // its tile's staged quads
+  const uint16_t* loc;    // [np][4]
+  const int32_t* hal;     // halo elements, tile by tile
+  const int32_t* hoff;    // [tiles + 1] the tiles' runs in hal
+  int32_t qcap;           // quads a tile stages at most
+  const double* coef;     // [5][np] (plain rows)
+  const uint32_t* row;    // class rows: [np][3] words, the row's class and five deltas (int16 each)
+  const double* tab;      // class rows: [n_class][5] class values
+  const uint32_t* blk;    // [np / 64] flags of each 64-element block (BLK_*)
   int32_t n_class;
   const uint8_t* flags;   // [np]
   const double* V0;       // [np]
@@ -108,9 +133,8 @@ __host__ __device__ inline double br_scaled(double v, double D, double D_b) {
 // The D-free part Face_C b / V0 of a boundary rate (its derivative in D).
 __host__ __device__ inline double br_unit(double v, double D_b) { return D_b == 0.0 ? 0.0 : v / D_b; }
 
-// Offset of element e's Ca in a realization's state buffer (its quad's first
-// double); Fluo is at +3.
-__device__ __forceinline__ size_t cq(const RealDesc& d, int e) { return 4 * gidx((size_t)e, d.kst, d.slot); }
+// Offset of element e's Ca in a realization's state buffer; Fluo is at +FLUO_OFF.
+__device__ __forceinline__ size_t cq(const RealDesc& d, int e) { return 2 * qidx((size_t)e, d.kst, d.slot); }
 
 // Mutable per-realization loop state.
 struct RealLive {
@@ -185,47 +209,119 @@ __device__ __forceinline__ void stg(SRS_GLOBAL T* p, T v) {
   else *p = v;
 }
 
-// Operator row of one element: coefficients (diagonal first), neighbour
-// indices and flags.  Mesh-level data, shared by every realization of a
-// realization group.
+// The diffusing species (Ca, ATP, CaM, Fluo) at pair index q of a state or
+// adjoint buffer.
+__device__ __forceinline__ d4 ld_quad(const SRS_GLOBAL double* X, size_t q) {
+  const SRS_GLOBAL d2* p = (const SRS_GLOBAL d2*)X + q;
+  const d2 a = p[0], b = p[QHALF];
+  return d4{a.x, a.y, b.x, b.y};
+}
+template <bool NT>
+__device__ __forceinline__ void st_quad(SRS_GLOBAL double* X, size_t q, const d4 m) {
+  SRS_GLOBAL d2* p = (SRS_GLOBAL d2*)X + q;
+  stg<NT>(p, d2{m.x, m.y});
+  stg<NT>(p + QHALF, d2{m.z, m.w});
+}
+typedef int i2 __attribute__((ext_vector_type(2)));
+typedef int i4 __attribute__((ext_vector_type(4)));
+typedef int i3 __attribute__((ext_vector_type(3), aligned(4)));
+
+// A tile's quads in LDS: its own elements' first, then its halo's (the
+// elements outside the tile that its elements neighbour, each once), as two
+// arrays of pairs (consecutive lanes read consecutive 16 B).
+struct QuadTile {
+  d2 *a, *b;
+  __device__ __forceinline__ QuadTile(void* lds, int cap) : a((d2*)lds), b((d2*)lds + cap) {}
+  __device__ __forceinline__ void put(int k, const d4 m) const {
+    a[k] = d2{m.x, m.y};
+    b[k] = d2{m.z, m.w};
+  }
+  __device__ __forceinline__ d4 get(int k) const { return d4{a[k].x, a[k].y, b[k].x, b[k].y}; }
+};
+
+// Read-only data at a wavefront-uniform address: a scalar load.
+template <class T>
+__device__ __forceinline__ T sld(const T* p) { return *(const __attribute__((address_space(4))) T*)p; }
+
+// A tile's run of the halo list, and the halo elements of a thread: the first
+// HPRE of them are loaded ahead of everything that does not depend on them.
+constexpr int HPRE = 2;
+struct Halo {
+  int s, n, e[HPRE];
+};
+template <int BS, bool NTG>
+__device__ __forceinline__ Halo load_halo(const int32_t* hal, const int32_t* hoff, const int t) {
+  Halo h;
+  h.s = sld(hoff + t);
+  h.n = sld(hoff + t + 1) - h.s;
+#pragma unroll
+  for (int q = 0; q < HPRE; ++q) {
+    const int k = (int)threadIdx.x + q * BS;
+    h.e[q] = k < h.n ? ldg<NTG>(gp(hal) + h.s + k) : -1;
+  }
+  return h;
+}
+
+// Operator row of one element: coefficients (diagonal first), its neighbours'
+// places among the tile's staged quads, and flags.  Mesh-level data, shared
+// by every realization of a realization group.
 struct Geo {
   double a0, a1, a2, a3, a4;
-  int n1, n2, n3, n4;
+  int l1, l2, l3, l4;
   uint8_t f;
 };
 
-// FK >= 0: the caller knows the element's flags (a wavefront whose lanes are
-// all alike), so none are loaded.
-template <bool NTG, bool COMPACT, int FK>
-__device__ __forceinline__ Geo load_geo(const RealDesc& d, const int j) {
-  Geo g;
-  const int np = d.np;
-  g.f = FK >= 0 ? (uint8_t)FK : ldg<NTG>(gp(d.flags) + j);
-  if constexpr (COMPACT) {
-    // Operator row = class row + small integer multiples of its ulps, which
+// A class row's coefficient: the class value with its bit pattern moved by
+// the element's delta.
+__device__ __forceinline__ double ulps_from(const double t, const int delta) {
+  return __longlong_as_double(__double_as_longlong(t) + (long long)delta);
+}
+template <bool NTG, bool CLASS>
+__device__ __forceinline__ void load_coef(const RealDesc& d, const int j, Geo& g) {
+  if constexpr (CLASS) {
     // reproduces the assembled FP64 values exactly (every row was checked
-    // when the mesh was added).
-    const SRS_GLOBAL int16_t* off = gp(d.off);
-    g.n1 = j + ldg<NTG>(off + j);
-    g.n2 = j + ldg<NTG>(off + np + j);
-    g.n3 = j + ldg<NTG>(off + 2 * np + j);
-    g.n4 = j + ldg<NTG>(off + 3 * np + j);
-    const SRS_GLOBAL double* t = gp(d.tab) + 10 * (int)ldg<NTG>(gp(d.cls) + j);
-    const SRS_GLOBAL int16_t* dq = gp(d.dq);
-    g.a0 = t[0] + (double)ldg<NTG>(dq + j) * t[5];
-    g.a1 = t[1] + (double)ldg<NTG>(dq + np + j) * t[6];
-    g.a2 = t[2] + (double)ldg<NTG>(dq + 2 * np + j) * t[7];
-    g.a3 = t[3] + (double)ldg<NTG>(dq + 3 * np + j) * t[8];
-    g.a4 = t[4] + (double)ldg<NTG>(dq + 4 * np + j) * t[9];
+    // when the mesh was added)
+    const i3 r = ldg<NTG>((const SRS_GLOBAL i3*)((const SRS_GLOBAL uint32_t*)d.row + 3 * (size_t)j));
+    const SRS_GLOBAL double* t = gp(d.tab) + 5 * (r.x & 0xffff);
+    g.a0 = ulps_from(t[0], r.x >> 16);
+    g.a1 = ulps_from(t[1], (int16_t)r.y);
+    g.a2 = ulps_from(t[2], r.y >> 16);
+    g.a3 = ulps_from(t[3], (int16_t)r.z);
+    g.a4 = ulps_from(t[4], r.z >> 16);
   } else {
+    const int np = d.np;
     const SRS_GLOBAL double* cf = gp(d.coef);
-    const SRS_GLOBAL int32_t* nb = gp(d.nbr);
     g.a0 = ldg<NTG>(cf + j); g.a1 = ldg<NTG>(cf + np + j); g.a2 = ldg<NTG>(cf + 2 * np + j);
     g.a3 = ldg<NTG>(cf + 3 * np + j); g.a4 = ldg<NTG>(cf + 4 * np + j);
-    g.n1 = ldg<NTG>(nb + j); g.n2 = ldg<NTG>(nb + np + j); g.n3 = ldg<NTG>(nb + 2 * np + j);
-    g.n4 = ldg<NTG>(nb + 3 * np + j);
   }
+}
+// The row of an element of the workgroup's tile.  b: the flags of the
+// element's block; in a plain block no element flags are loaded.  A row is two
+// wide loads (places 8 B, class row 12 B).
+template <bool NTG, bool CLASS>
+__device__ __forceinline__ Geo load_geo(const RealDesc& d, const uint16_t* loc, const int j, const uint32_t b) {
+  Geo g;
+  g.f = (b & BLK_PLAIN) ? (uint8_t)F_TROPC : ldg<NTG>(gp(d.flags) + j);
+  const i2 q = ldg<NTG>((const SRS_GLOBAL i2*)loc + j);
+  g.l1 = q.x & 0xffff; g.l2 = (uint32_t)q.x >> 16;
+  g.l3 = q.y & 0xffff; g.l4 = (uint32_t)q.y >> 16;
+  load_coef<NTG, CLASS>(d, j, g);
   return g;
+}
+// The row of any element, with neighbour indices in place of tile places.
+template <bool NTG, bool CLASS>
+__device__ __forceinline__ Geo load_geo_nbr(const RealDesc& d, const int j) {
+  Geo g;
+  g.f = ldg<NTG>(gp(d.flags) + j);
+  const i4 q = ldg<NTG>((const SRS_GLOBAL i4*)d.nbr + j);
+  g.l1 = q.x; g.l2 = q.y; g.l3 = q.z; g.l4 = q.w;
+  load_coef<NTG, CLASS>(d, j, g);
+  return g;
+}
+// The flags of the block of element j, j consecutive across the wavefront from
+// a multiple of 64.
+__device__ __forceinline__ uint32_t block_flags(const RealDesc& d, const int j) {
+  return sld(d.blk + (__builtin_amdgcn_readfirstlane(j) >> 6));
 }
 
 // --------------------------------------------- line-scan geometry and sizes
@@ -349,11 +445,20 @@ struct DevBuf {
   size_t bytes = 0;
 };
 
+// Where the neighbours of a tile's elements are once the tile is staged: place
+// k < tile is the tile's own element k, place tile + i the i-th of its halo.
+struct TileMap {
+  int tile = 0;       // elements per tile; 0: not built
+  int32_t qcap = 0;   // the most quads a tile stages (its elements and its halo)
+  uint16_t* d_loc = nullptr;
+  int32_t *d_hal = nullptr, *d_hoff = nullptr;
+};
+
 struct HostMesh {
   int32_t n = 0, np = 0;
   std::vector<int32_t> perm;  // dev -> ref
   std::vector<int32_t> inv;   // ref -> dev
-  std::vector<int32_t> nbr;   // [4][np] dev numbering
+  std::vector<int32_t> nbr;   // [np][4] dev numbering
   std::vector<double> coef;   // [5][np]
   std::vector<uint8_t> flags;
   std::vector<double> V0, tt, br;  // br [4][np] or empty
@@ -362,17 +467,16 @@ struct HostMesh {
   // realization added on the mesh, which every later one must share.
   double br_d[4] = {0, 0, 0, 0};
   bool br_d_set = false;
+  TileMap map, map_adj;             // of the sweep's tiles and of the reverse step's
   // compact operator layout
-  bool compact = false;
-  std::vector<int16_t> off, dq;
-  std::vector<uint16_t> cls;
+  bool class_rows = false;          // row and tab reproduce every coefficient
+  std::vector<uint32_t> row;        // [np][3]
   std::vector<double> tab;
   int32_t n_class = 0;
   int32_t *d_nbr = nullptr, *d_inv = nullptr;
   double *d_coef = nullptr, *d_V0 = nullptr, *d_tt = nullptr, *d_br = nullptr, *d_tab = nullptr;
   uint8_t* d_flags = nullptr;
-  int16_t *d_off = nullptr, *d_dq = nullptr;
-  uint16_t* d_cls = nullptr;
+  uint32_t *d_blk = nullptr, *d_row = nullptr;
 };
 
 struct HostReal {
@@ -406,13 +510,13 @@ using namespace srs_dev;
 struct srs_ctx {
   int device = 0;
   int tile = 0;          // elements per k_sweep workgroup; 0: chosen by srs_ctx_finalize
+  size_t sweep_lds = 0;  // LDS bytes of a sweep workgroup (staged quads)
   int nt_geometry = 1;   // non-temporal loads of operator rows and flags
   int nt_state = 0;      // non-temporal stores of the new state
   int plane_pad = 0;     // extra elements per SoA plane
   int compact = 1;       // compress operator rows when a mesh allows it
-  int occ = 0;           // sweep register budget: 0 compiler's choice, 6 or 8 wavefronts per SIMD
+  int occ = 0;           // gated sweep's register budget: 0 compiler's choice, 6 or 8 wavefronts per SIMD
   int group = 1;         // realizations per realization group (1, 2 or 4)
-  int lds = 1;           // stage each tile's quads in LDS for the neighbour gathers (groups of 1)
   int drop_finished = 1; // sweep without the tiles of groups that have all finished
   int gated = 1;         // fold each step's gating into the next step's sweep (k_sweep_gated) where it applies
   int alt_order = 0;      // single-realization gated sweep: tiles in reverse order on alternate steps
@@ -422,7 +526,7 @@ struct srs_ctx {
   int adj_w = 0;          // adjoint w: 0 by launch size, 1 written by each step, 2 formed in the kernel
   int adj_last_levels = 0, adj_last_batch = 0;  // the plan of the last loss/gradient call
   int64_t adj_last_strides[6] = {};
-  bool compact_all = false;
+  bool class_all = false;  // class rows on every mesh
   bool layout_fixed = false;
   hipStream_t stream = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -493,6 +597,7 @@ struct DevMem {
 };
 
 // Context helpers (device.hip).
+int build_map(srs_ctx* c, HostMesh& hm, int tile, TileMap* m);
 int check_real(srs_ctx* c, int32_t r);
 void launch_sweep(srs_ctx* c);
 int launch_step(srs_ctx* c, uint32_t gmode);

@@ -32,12 +32,20 @@
 
 namespace srs_dev {
 
-// The state of one element of one realization: its own and its neighbours'
-// diffusing quads, TnC and CSQ where they are live.
+// The state of one element of one realization: its own diffusing quad, the
+// operator row applied to each diffusing species, TnC and CSQ where they are
+// live.
 struct Loc {
-  d4 m0, m1, m2, m3, m4;
+  d4 m0, s;
   double c_tr, c_cs;
 };
+
+// The operator row applied to an element's own and its neighbours' quads, in
+// the reference's order (cpu/RunSimulation.cpp:61-71).
+__device__ __forceinline__ d4 row_sum(const Geo& g, const d4& m0, const d4& m1, const d4& m2, const d4& m3,
+                                      const d4& m4) {
+  return m0 * g.a0 + m1 * g.a1 + m2 * g.a2 + m3 * g.a3 + m4 * g.a4;
+}
 
 // A realization's state buffers for one step: read X[cur], write X[cur ^ 1].
 // Both pointers are loaded and one is selected, so that the live index and
@@ -65,76 +73,48 @@ __device__ __forceinline__ uint64_t fold(const T... v) {
 }
 __device__ __forceinline__ void scalars_here(const uint64_t folded) { __asm__ volatile("" ::"s"(folded)); }
 
-template <int FK>
-__device__ __forceinline__ Loc load_loc(const RealDesc& d, const SRS_GLOBAL double* __restrict__ Xo, const int j,
-                                        const Geo& g) {
-  // Realization-group layout: element e of the realization in slot s of a
-  // group of K is quad gidx(e, K, s); the TnC and CSQ planes follow the quads.
-  const int K = d.kst, s = d.slot;
-  const size_t np = d.np;
-  const SRS_GLOBAL d4* Mo = (const SRS_GLOBAL d4*)Xo;
-  Loc c;
-  c.m0 = Mo[gidx(j, K, s)];
-  // TnC has a nonzero rate only in cytosol elements with troponin, CSQ only
-  // in the jSR (cpu/RunSimulation.cpp:45-46 reset both rates to zero).  A
-  // zero rate leaves the value unchanged, and both state buffers hold the same
-  // value, so those planes are neither read nor written elsewhere.
-  const uint8_t f = FK >= 0 ? (uint8_t)FK : g.f;
-  const bool live_tr = (f & (F_JSR | F_TROPC)) == F_TROPC;
-  const bool live_cs = (f & F_JSR) != 0;
-  c.c_tr = live_tr ? Xo[4 * K * np + gidx(j, K, s)] : 0.0;
-  c.c_cs = live_cs ? Xo[5 * K * np + gidx(j, K, s)] : 0.0;
-  c.m1 = Mo[gidx(g.n1, K, s)];
-  c.m2 = Mo[gidx(g.n2, K, s)];
-  c.m3 = Mo[gidx(g.n3, K, s)];
-  c.m4 = Mo[gidx(g.n4, K, s)];
-  return c;
+// Pair index of an element; ONE: the realization is alone in its group.
+template <bool ONE>
+__device__ __forceinline__ size_t qat(const RealDesc& d, const int e) {
+  return ONE ? (size_t)qidx1((uint32_t)e) : qidx((size_t)e, d.kst, d.slot);
 }
 
-// As load_loc for a single-realization layout, with the neighbour quads that
-// lie in the workgroup's own tile read from the copy staged in LDS.
-template <int FK, int BS>
-__device__ __forceinline__ Loc load_loc_lds(const RealDesc& d, const SRS_GLOBAL double* __restrict__ Xo, const int j,
-                                            const Geo& g, const d4* tq, const int base, const d4& m0,
-                                            const double tr) {
+// TnC has a nonzero rate only in cytosol elements with troponin, CSQ only in
+// the jSR (cpu/RunSimulation.cpp:45-46 reset both rates to zero).  A zero rate
+// leaves the value unchanged, and both state buffers hold the same value, so
+// those planes are neither read nor written elsewhere.
+__device__ __forceinline__ bool lives_tr(const uint8_t f) { return (f & (F_JSR | F_TROPC)) == F_TROPC; }
+__device__ __forceinline__ bool lives_cs(const uint8_t f) { return (f & F_JSR) != 0; }
+
+// Element j alone in its group, its neighbours read one by one (g holds their
+// indices).
+__device__ __forceinline__ Loc load_loc(const RealDesc& d, const SRS_GLOBAL double* __restrict__ Xo, const int j,
+                                        const Geo& g) {
   const size_t np = d.np;
-  const SRS_GLOBAL d4* Mo = (const SRS_GLOBAL d4*)Xo;
   Loc c;
-  c.m0 = m0;
-  const uint8_t f = FK >= 0 ? (uint8_t)FK : g.f;
-  const bool live_tr = (f & (F_JSR | F_TROPC)) == F_TROPC;
-  const bool live_cs = (f & F_JSR) != 0;
-  c.c_tr = live_tr ? tr : 0.0;
-  c.c_cs = live_cs ? Xo[5 * np + j] : 0.0;
-  auto nq = [&](int nb) -> d4 {
-    const unsigned k = (unsigned)(nb - base);
-    return k < (unsigned)BS ? tq[k] : Mo[nb];
-  };
-  c.m1 = nq(g.n1);
-  c.m2 = nq(g.n2);
-  c.m3 = nq(g.n3);
-  c.m4 = nq(g.n4);
+  c.m0 = ld_quad(Xo, qidx1(j));
+  c.c_tr = lives_tr(g.f) ? Xo[4 * np + j] : 0.0;
+  c.c_cs = lives_cs(g.f) ? Xo[5 * np + j] : 0.0;
+  c.s = row_sum(g, c.m0, ld_quad(Xo, qidx1(g.l1)), ld_quad(Xo, qidx1(g.l2)), ld_quad(Xo, qidx1(g.l3)),
+                ld_quad(Xo, qidx1(g.l4)));
   return c;
 }
 
 // The fused step of one element of one realization, from its loaded row and
 // state, in the reference's operation order (cpu/RunSimulation.cpp:591-648).
-template <bool NTS, int FK>
+template <bool NTS, int FK, bool ONE>
 __device__ __forceinline__ void step_elem(const RealDesc& d, const RealLive& l, const Bufs bf, const int j,
                                           const Geo& g, const Loc& c) {
-  const int K = d.kst, s = d.slot;
+  const int K = ONE ? 1 : d.kst;
   const size_t np = d.np;
   const SRS_GLOBAL double* __restrict__ Xo = bf.xo;
   SRS_GLOBAL double* __restrict__ Xn = bf.xn;
   const double* P = d.P;
   const double dt = P[SRS_R_T_STEP];
   const uint8_t f = FK >= 0 ? (uint8_t)FK : g.f;
-  const double a0 = g.a0, a1 = g.a1, a2 = g.a2, a3 = g.a3, a4 = g.a4;
   const double c_ca = c.m0.x, c_at = c.m0.y, c_cm = c.m0.z, c_dy = c.m0.w;
   const double c_tr = c.c_tr, c_cs = c.c_cs;
-  const d4 m1 = c.m1, m2 = c.m2, m3 = c.m3, m4 = c.m4;
-  const bool live_tr = (f & (F_JSR | F_TROPC)) == F_TROPC;
-  const bool live_cs = (f & F_JSR) != 0;
+  const bool live_tr = lives_tr(f), live_cs = lives_cs(f);
 
   double br_ca = 0.0, br_dy = 0.0, br_at = 0.0, br_cm = 0.0;
   if (f & F_BR) {
@@ -147,10 +127,10 @@ __device__ __forceinline__ void step_elem(const RealDesc& d, const RealLive& l, 
   // cpu/RunSimulation.cpp:61-71 (Ca uses D_CA in both domains; with the jSR
   // diffusion extension, D_CAJSR in jSR elements)
   const double d_ca = (live_cs && d.jsr_diff) ? P[SRS_R_D_CA_JSR] : P[SRS_R_D_CA];
-  double rca = d_ca * (c_ca * a0 + m1.x * a1 + m2.x * a2 + m3.x * a3 + m4.x * a4) + br_ca;
-  double rdy = P[SRS_R_D_DYE] * (c_dy * a0 + m1.w * a1 + m2.w * a2 + m3.w * a3 + m4.w * a4) + br_dy;
-  double rat = P[SRS_R_D_ATP] * (c_at * a0 + m1.y * a1 + m2.y * a2 + m3.y * a3 + m4.y * a4) + br_at;
-  double rcm = P[SRS_R_D_CMDN] * (c_cm * a0 + m1.z * a1 + m2.z * a2 + m3.z * a3 + m4.z * a4) + br_cm;
+  double rca = d_ca * c.s.x + br_ca;
+  double rdy = P[SRS_R_D_DYE] * c.s.w + br_dy;
+  double rat = P[SRS_R_D_ATP] * c.s.y + br_at;
+  double rcm = P[SRS_R_D_CMDN] * c.s.z + br_cm;
   double rtr = 0, rcs = 0;
   const double nsr = l.ca_nsr;
 
@@ -195,8 +175,8 @@ __device__ __forceinline__ void step_elem(const RealDesc& d, const RealLive& l, 
         if (ch >= 0) {
           const int i = ch >> 1;
           if (d.ryr_state[i]) {
-            const double J = P[SRS_R_V_RYR] * (Xo[4 * gidx(d.ryr_jsr[i], K, s)] -
-                                               Xo[4 * gidx(d.ryr_ele[i], K, s)]) * P[SRS_R_V_CELL];
+            const double J = P[SRS_R_V_RYR] * (Xo[2 * qat<ONE>(d, d.ryr_jsr[i])] -
+                                               Xo[2 * qat<ONE>(d, d.ryr_ele[i])]) * P[SRS_R_V_CELL];
             if (ch & 1) rca -= J / v0; else rca += J / v0;
           }
         } else {
@@ -224,145 +204,100 @@ __device__ __forceinline__ void step_elem(const RealDesc& d, const RealLive& l, 
 
   // :640-644 forward Euler
   const d4 mn = {c_ca + rca * dt, c_at + rat * dt, c_cm + rcm * dt, c_dy + rdy * dt};
-  const size_t q = gidx(j, K, s);
-  stg<NTS>((SRS_GLOBAL d4*)Xn + q, mn);
+  const size_t q = ONE ? (size_t)j : gidx(j, K, d.slot);
+  st_quad<NTS>(Xn, qat<ONE>(d, j), mn);
   if (live_tr) stg<NTS>(Xn + 4 * K * np + q, c_tr + rtr * dt);
   if (live_cs) stg<NTS>(Xn + 5 * K * np + q, c_cs + rcs * dt);
 }
 
-// Flags shared by every lane of a wavefront-sized element group: the low byte
-// is the OR of the lanes' flags, the high byte the AND.  A wavefront of plain
-// cytosol elements with troponin takes the path with the flags known.
-constexpr uint8_t F_SPECIAL = F_JSR | F_SL | F_BR | F_CHAN;
-
-// One tile of one realization group: the operator rows are loaded once and
-// applied to the KG realizations of the group, one after another; -1 marks an
-// empty slot or a member that does not step.
-template <bool NTS, int KG, int FK>
-__device__ __forceinline__ void sweep_group(const RealDesc* __restrict__ D, const RealLive* __restrict__ L,
-                                            const int* mem, const int j, const Geo& g) {
-  for (int s = 0; s < KG; ++s)
-    if (KG == 1 || mem[s] >= 0) {
-      const RealDesc& d = D[mem[s]];
-      const Bufs bf = bufs(d.X[0], d.X[1], L[mem[s]].cur);
-      const Loc c = load_loc<FK>(d, bf.xo, j, g);
-      step_elem<NTS, FK>(d, L[mem[s]], bf, j, g, c);
-    }
-}
-
-// The sizes and operator-row pointers of a mesh, folded for scalars_here.
-template <bool COMPACT>
+// The sizes and mesh pointers of a tile's rows and halo, folded for scalars_here.
+template <bool CLASS>
 __device__ __forceinline__ uint64_t geo_fold(const RealDesc& d) {
-  if constexpr (COMPACT) return fold(d.n, d.np, d.flags, d.off, d.cls, d.dq, d.tab);
-  else return fold(d.n, d.np, d.flags, d.coef, d.nbr);
+  const uint64_t m = fold(d.n, d.np, d.flags, d.blk, d.loc, d.hal, d.hoff, d.qcap);
+  if constexpr (CLASS) return m ^ fold(d.row, d.tab);
+  else return m ^ fold(d.coef);
 }
 
-// Single-realization groups with LDS staging: the tile's own quads are
-// loaded coalesced into LDS, and neighbour quads inside the tile come from
-// there instead of through the L1 cache.
-template <int BS, bool NTG, bool NTS, bool COMPACT, bool SKIP_CHAN = false>
-__device__ __forceinline__ void sweep_tile_lds(const RealDesc& d, const RealLive& l, const Bufs bf, int t) {
-  __shared__ d4 tq[BS];
-  const int base = t * BS;
-  const int j = base + threadIdx.x;
-  const bool in = j < d.n;
-  Geo g{};
-  d4 m0 = {0.0, 0.0, 0.0, 0.0};
-  double tr = 0.0;
-  if (in) {
-    // the element's TnC is loaded with its row and quad, before its flags are
-    // known (it is live in all but jSR and troponin-free cytosol elements), so
-    // that the loads after the barrier are only the neighbour gathers
-    g = load_geo<NTG, COMPACT, -1>(d, j);
-    m0 = ((const SRS_GLOBAL d4*)bf.xo)[j];
-    tr = bf.xo[4 * (size_t)d.np + j];
-  }
-  tq[threadIdx.x] = m0;
-  __syncthreads();
-  if (!in) return;
-  if (SKIP_CHAN && (g.f & F_CHAN)) return;  // updated by the gating workgroup (sweep_gated)
-  const bool plain = (g.f & F_SPECIAL) == 0 && (g.f & F_TROPC);
-  if (__builtin_amdgcn_ballot_w64(!plain) == 0) {
-    const Loc c = load_loc_lds<F_TROPC, BS>(d, bf.xo, j, g, tq, base, m0, tr);
-    step_elem<NTS, F_TROPC>(d, l, bf, j, g, c);
-  } else {
-    const Loc c = load_loc_lds<-1, BS>(d, bf.xo, j, g, tq, base, m0, tr);
-    step_elem<NTS, -1>(d, l, bf, j, g, c);
-  }
-}
+extern __shared__ double dyn_lds[];
 
-// The element's flags are loaded with its operator row; a wavefront whose
-// active lanes are all plain cytosol with troponin (the bulk of a mesh) then
-// runs the specialisation with the flags known at compile time.
-template <int BS, bool NTG, bool NTS, bool COMPACT, int KG>
-__device__ __forceinline__ void sweep_tile(const RealDesc* __restrict__ D, const RealLive* __restrict__ L,
-                                           const int2* __restrict__ tiles, int n_tiles, const int* __restrict__ groups,
-                                           int single) {
-  const int b = xcd_tile(blockIdx.x, gridDim.x);
-  if (b >= n_tiles) return;
-  const int2 tl = single ? make_int2(0, b) : tiles[b];  // {group, tile}
-  // members that step: a finished member (done) or one in the gating-only
-  // ffwd phase keeps its fields, so its part of the tile is skipped
-  int mem[KG];
-  int first = -1;
+// One tile of one realization.  The tile's quads and its halo's are staged in
+// LDS (every lane's own by consecutive loads, the halo's by the tile's sorted
+// list, each element once) and each element reads its neighbours from there.
+// Bound by the memory system, not by arithmetic (with the reactions left out
+// the step takes as long): a 48-member ensemble (7.05M elements) moves 107 B
+// per element-step at 5.0 TB/s, a copy of the same shape runs at 5.5.  When each
+// element gathered its out-of-tile neighbours itself, a neighbour of several
+// elements was fetched for each of them, and every wavefront held four quads
+// in flight in registers: 84 VGPRs against 64, 175 us against 160 us per step of
+// that ensemble with 512-element tiles, 71.4 against 66.8 us (separate gating,
+// 3M-element dyad).
+// A wavefront whose elements are all plain cytosol with troponin (the bulk of
+// a mesh, known from its block's flags) runs the specialisation with the flags
+// known at compile time.  KG: the realization's group size, s its slot.
+template <int BS, bool NTG, bool NTS, bool CLASS, int KG, bool SKIP_CHAN>
+__device__ __forceinline__ void sweep_tile(const RealDesc& d, const RealLive& l, const Bufs bf, const int s,
+                                           const int t) {
+  const QuadTile tq(dyn_lds, d.qcap);
+  const Halo h = load_halo<BS, NTG>(d.hal, d.hoff, t);
+  const int j = t * BS + (int)threadIdx.x;
+  // rows and states are padded to whole tiles, so the last tile's lanes past
+  // the mesh load (and discard) zeros
+  const uint32_t b = block_flags(d, j);
+  const Geo g = load_geo<NTG, CLASS>(d, d.loc, j, b);
+  const SRS_GLOBAL double* Xo = bf.xo;
+  const size_t np = d.np, pl = 4 * KG * np + (KG > 1 ? gidx(j, KG, s) : (size_t)j);
+  auto quad = [&](int e) { return ld_quad(Xo, KG > 1 ? qidx(e, KG, s) : (size_t)qidx1(e)); };
+  Loc c;
+  c.m0 = quad(j);
+  // the element's TnC is loaded with its quad, before its flags are known (it
+  // is live in all but jSR and troponin-free cytosol elements)
+  c.c_tr = Xo[pl];
+  tq.put(threadIdx.x, c.m0);
 #pragma unroll
-  for (int s = 0; s < KG; ++s) {
-    const int r = single ? (s == 0 ? 0 : -1) : groups[KG * tl.x + s];
-    mem[s] = (r >= 0 && !(L[r].done | L[r].ffwd)) ? r : -1;
-    if (first < 0) first = mem[s];
+  for (int q = 0; q < HPRE; ++q)
+    if (h.e[q] >= 0) tq.put(BS + threadIdx.x + q * BS, quad(h.e[q]));
+  for (int k = threadIdx.x + HPRE * BS; k < h.n; k += BS) tq.put(BS + k, quad(gp(d.hal)[h.s + k]));
+  __syncthreads();
+  if (j >= d.n || (SKIP_CHAN && (g.f & F_CHAN))) return;
+  c.s = row_sum(g, c.m0, tq.get(g.l1), tq.get(g.l2), tq.get(g.l3), tq.get(g.l4));
+  if (b & BLK_PLAIN) {
+    step_elem<NTS, F_TROPC, KG == 1>(d, l, bf, j, g, c);
+  } else {
+    if (!lives_tr(g.f)) c.c_tr = 0.0;
+    c.c_cs = lives_cs(g.f) ? Xo[pl + KG * np] : 0.0;
+    step_elem<NTS, -1, KG == 1>(d, l, bf, j, g, c);
   }
-  if (first < 0) return;
-  const RealDesc& d = D[first];
-  const int j = tl.y * BS + threadIdx.x;
-  if (j >= d.n) return;
-  const Geo g = load_geo<NTG, COMPACT, -1>(d, j);
-  const bool plain = (g.f & F_SPECIAL) == 0 && (g.f & F_TROPC);
-  if (__builtin_amdgcn_ballot_w64(!plain) == 0) sweep_group<NTS, KG, F_TROPC>(D, L, mem, j, g);
-  else sweep_group<NTS, KG, -1>(D, L, mem, j, g);
 }
 
-template <int BS, bool NTG, bool NTS, bool COMPACT>
-__device__ __forceinline__ void sweep_lds(const RealDesc* __restrict__ D, const RealLive* __restrict__ L,
-                                          const int2* __restrict__ tiles, int n_tiles, const int* __restrict__ groups,
-                                          int single) {
+// Workgroup b of a context with groups of KG takes slot b % KG of tile b / KG,
+// so that the slots' workgroups, which read the same rows and halo lists, run
+// side by side on one XCD.
+template <int BS, bool NTG, bool NTS, bool CLASS, int KG>
+__device__ __forceinline__ void sweep(const RealDesc* __restrict__ D, const RealLive* __restrict__ L,
+                                      const int2* __restrict__ tiles, int n_tiles, const int* __restrict__ groups,
+                                      int single) {
   const int b = xcd_tile(blockIdx.x, gridDim.x);
-  if (b >= n_tiles) return;
-  const int2 tl = single ? make_int2(0, b) : tiles[b];
-  const int r = single ? 0 : groups[tl.x];
+  if (b >= n_tiles * KG) return;
+  const int2 tl = single ? make_int2(0, b / KG) : tiles[b / KG];  // {group, tile}
+  const int s = b % KG;
+  const int r = single ? (s == 0 ? 0 : -1) : groups[KG * tl.x + s];
+  if (KG > 1 && r < 0) return;
   const RealDesc& d = D[r];
   const RealLive& l = L[r];
+  // a finished realization (done) or one in the gating-only ffwd phase keeps
+  // its fields
   const int skip = l.done | l.ffwd;
   const Bufs bf = bufs(d.X[0], d.X[1], l.cur);
-  scalars_here(fold(skip, bf.xo, bf.xn) ^ geo_fold<COMPACT>(d));
+  scalars_here(fold(skip, bf.xo, bf.xn) ^ geo_fold<CLASS>(d));
   if (skip) return;
-  sweep_tile_lds<BS, NTG, NTS, COMPACT>(d, l, bf, tl.y);
+  sweep_tile<BS, NTG, NTS, CLASS, KG, false>(d, l, bf, s, tl.y);
 }
 
-// Register budgets: the compiler's choice, or the largest that lets W
-// wavefronts share each SIMD (64 VGPRs for eight, 80 for six).
-template <int BS, bool NTG, bool NTS, bool COMPACT, int KG>
+template <int BS, bool NTG, bool NTS, bool CLASS, int KG>
 __global__ __launch_bounds__(BS) void k_sweep(const RealDesc* __restrict__ D, const RealLive* __restrict__ L,
                                               const int2* __restrict__ tiles, int n_tiles,
                                               const int* __restrict__ groups, int single) {
-  sweep_tile<BS, NTG, NTS, COMPACT, KG>(D, L, tiles, n_tiles, groups, single);
-}
-template <int BS, bool NTG, bool NTS, bool COMPACT, int KG, int W>
-__global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W))) void k_sweep_w(
-    const RealDesc* __restrict__ D, const RealLive* __restrict__ L, const int2* __restrict__ tiles, int n_tiles,
-    const int* __restrict__ groups, int single) {
-  sweep_tile<BS, NTG, NTS, COMPACT, KG>(D, L, tiles, n_tiles, groups, single);
-}
-template <int BS, bool NTG, bool NTS, bool COMPACT>
-__global__ __launch_bounds__(BS) void k_sweep_lds(const RealDesc* __restrict__ D, const RealLive* __restrict__ L,
-                                                  const int2* __restrict__ tiles, int n_tiles,
-                                                  const int* __restrict__ groups, int single) {
-  sweep_lds<BS, NTG, NTS, COMPACT>(D, L, tiles, n_tiles, groups, single);
-}
-template <int BS, bool NTG, bool NTS, bool COMPACT, int W>
-__global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W))) void k_sweep_lds_w(
-    const RealDesc* __restrict__ D, const RealLive* __restrict__ L, const int2* __restrict__ tiles, int n_tiles,
-    const int* __restrict__ groups, int single) {
-  sweep_lds<BS, NTG, NTS, COMPACT>(D, L, tiles, n_tiles, groups, single);
+  sweep<BS, NTG, NTS, CLASS, KG>(D, L, tiles, n_tiles, groups, single);
 }
 
 __device__ void write_record(const RealDesc& d, RealLive& l, const double* Ca, double t) {
@@ -407,16 +342,16 @@ __device__ void write_record(const RealDesc& d, RealLive& l, const double* Ca, d
 // LEAN loads each LCC's inputs when it is updated rather than with the RyRs'
 // before the first barrier: one more memory round trip, fewer live registers.
 // PROTO = false leaves out the loop body (callers that never pass G_PROTOCOL).
+// smem: GATE_LDS bytes.
+constexpr size_t GATE_LDS = 3 * MAX_RYR * sizeof(int);
 template <int NT, bool LEAN = false, bool PROTO = true>
 __device__ __forceinline__ void gate_workgroup(const RealDesc* __restrict__ D, RealLive* __restrict__ L, const int r,
-                                               const uint32_t mode) {
+                                               const uint32_t mode, int* smem) {
   static_assert(MAX_RYR % NT == 0 && MAX_LCC % NT == 0, "channel slots per thread");
   const RealDesc& d = D[r];
   RealLive& l = L[r];
   if (l.done) return;
-  __shared__ int s_old[MAX_RYR];
-  __shared__ int s_a[MAX_RYR];
-  __shared__ int s_b[MAX_RYR];
+  int *s_old = smem, *s_a = smem + MAX_RYR, *s_b = smem + 2 * MAX_RYR;
   const int tid = threadIdx.x;
   const int cur = l.cur;
   // In the flag_ffwd phase the sweep skipped this realization: the fields are
@@ -663,12 +598,14 @@ __device__ __forceinline__ void gate_workgroup(const RealDesc* __restrict__ D, R
 #if SRS_UNIT == 0
 __global__ __launch_bounds__(GATE_THREADS) void k_gate(const RealDesc* __restrict__ D, RealLive* __restrict__ L,
                                                        uint32_t mode) {
-  gate_workgroup<GATE_THREADS>(D, L, blockIdx.x, mode);
+  __shared__ int smem[3 * MAX_RYR];
+  gate_workgroup<GATE_THREADS>(D, L, blockIdx.x, mode, smem);
 }
 // The gating of the realizations of a list (one subset of the context).
 __global__ __launch_bounds__(GATE_THREADS) void k_gate_list(const RealDesc* __restrict__ D, RealLive* __restrict__ L,
                                                             const int32_t* __restrict__ rids, uint32_t mode) {
-  gate_workgroup<GATE_THREADS>(D, L, rids[blockIdx.x], mode);
+  __shared__ int smem[3 * MAX_RYR];
+  gate_workgroup<GATE_THREADS>(D, L, rids[blockIdx.x], mode, smem);
 }
 #endif
 
@@ -690,7 +627,7 @@ __global__ __launch_bounds__(GATE_THREADS) void k_gate_list(const RealDesc* __re
 // reverse order when the index is 1 (alternate steps), so that a step first
 // reads the tiles the step before wrote last, while they may still be in the
 // last-level cache.  The order changes no result.
-template <int BS, bool NTG, bool NTS, bool COMPACT, bool LEAN, bool PROTO>
+template <int BS, bool NTG, bool NTS, bool CLASS, bool LEAN, bool PROTO>
 __device__ __forceinline__ void sweep_gated(const RealDesc* __restrict__ D, RealLive* __restrict__ L, int n_tiles,
                                             int curx, uint32_t gmode, const double* xo_at, double* xn_at) {
   const int cur = curx & 1;
@@ -703,44 +640,44 @@ __device__ __forceinline__ void sweep_gated(const RealDesc* __restrict__ D, Real
   // the state buffers: X[cur] -> X[cur ^ 1], or the caller's (xo_at, xn_at)
   // (a replayed segment whose steps each have a slot of their own)
   const Bufs bf = xo_at ? Bufs{gp(xo_at), gpw(xn_at)} : bufs(d.X[0], d.X[1], cur);
-  scalars_here(fold(skip, bf.xo, bf.xn) ^ geo_fold<COMPACT>(d));
+  scalars_here(fold(skip, bf.xo, bf.xn) ^ geo_fold<CLASS>(d));
   if (b == 0) {
-    if (gmode) gate_workgroup<BS, LEAN, PROTO>(D, L, 0, gmode);
+    if (gmode) gate_workgroup<BS, LEAN, PROTO>(D, L, 0, gmode, (int*)dyn_lds);
     __syncthreads();  // the new channel states, written by this workgroup, before the flux reads them
     if (skip) return;
     for (int k = threadIdx.x; k < d.n_celem; k += BS) {
       const int j = gp(d.celem)[k];
-      const Geo g = load_geo<NTG, COMPACT, -1>(d, j);
-      const Loc c = load_loc<-1>(d, bf.xo, j, g);
-      step_elem<NTS, -1>(d, l, bf, j, g, c);
+      const Geo g = load_geo_nbr<NTG, CLASS>(d, j);
+      const Loc c = load_loc(d, bf.xo, j, g);
+      step_elem<NTS, -1, true>(d, l, bf, j, g, c);
     }
     return;
   }
   if (skip) return;
-  sweep_tile_lds<BS, NTG, NTS, COMPACT, true>(d, l, bf, b - 1);
+  sweep_tile<BS, NTG, NTS, CLASS, 1, true>(d, l, bf, 0, b - 1);
 }
 // Register budgets as for the sweep.  The gating workgroup's latency is on
 // the critical path of a small mesh's step, so the compiler's budget keeps
 // all of its loads in one round trip; with a budget the LCC loads wait for
 // the RyR update (LEAN), which is what lets the kernel fit 80 VGPRs.
-template <int BS, bool NTG, bool NTS, bool COMPACT>
+template <int BS, bool NTG, bool NTS, bool CLASS>
 __global__ __launch_bounds__(BS) void k_sweep_gated(const RealDesc* __restrict__ D, RealLive* __restrict__ L,
                                                     int n_tiles, int cur, uint32_t gmode, const double* xo_at,
                                                     double* xn_at) {
-  sweep_gated<BS, NTG, NTS, COMPACT, false, false>(D, L, n_tiles, cur, gmode, xo_at, xn_at);
+  sweep_gated<BS, NTG, NTS, CLASS, false, false>(D, L, n_tiles, cur, gmode, xo_at, xn_at);
 }
-template <int BS, bool NTG, bool NTS, bool COMPACT, int W>
+template <int BS, bool NTG, bool NTS, bool CLASS, int W>
 __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W))) void k_sweep_gated_w(
     const RealDesc* __restrict__ D, RealLive* __restrict__ L, int n_tiles, int cur, uint32_t gmode,
     const double* xo_at, double* xn_at) {
-  sweep_gated<BS, NTG, NTS, COMPACT, true, false>(D, L, n_tiles, cur, gmode, xo_at, xn_at);
+  sweep_gated<BS, NTG, NTS, CLASS, true, false>(D, L, n_tiles, cur, gmode, xo_at, xn_at);
 }
 // with the loop body (SRS_STEP_PROTOCOL), compiler's register budget only
-template <int BS, bool NTG, bool NTS, bool COMPACT>
+template <int BS, bool NTG, bool NTS, bool CLASS>
 __global__ __launch_bounds__(BS) void k_sweep_gated_p(const RealDesc* __restrict__ D, RealLive* __restrict__ L,
                                                       int n_tiles, int cur, uint32_t gmode, const double* xo_at,
                                                       double* xn_at) {
-  sweep_gated<BS, NTG, NTS, COMPACT, false, true>(D, L, n_tiles, cur, gmode, xo_at, xn_at);
+  sweep_gated<BS, NTG, NTS, CLASS, false, true>(D, L, n_tiles, cur, gmode, xo_at, xn_at);
 }
 
 // ------------------------------------------------------------ kernel choice
@@ -756,48 +693,24 @@ template <int BS>
 GatedFn pick_gated_bs(const srs_ctx* c, bool proto);
 
 #if SRS_UNIT == 1
-// The sweep kernel for a tile size, cache hints, register budget (0, 6 or 8
-// wavefronts per SIMD) and LDS staging (single-realization groups only).
-template <int BS, bool CMP, int KG, int W>
-SweepFn pick_w(int ntg, int nts, int lds) {
-  if constexpr (KG == 1) {
-    if (lds) {
-      if constexpr (W == 0) {
-        if (ntg) return nts ? k_sweep_lds<BS, true, true, CMP> : k_sweep_lds<BS, true, false, CMP>;
-        return nts ? k_sweep_lds<BS, false, true, CMP> : k_sweep_lds<BS, false, false, CMP>;
-      } else {
-        if (ntg) return nts ? k_sweep_lds_w<BS, true, true, CMP, W> : k_sweep_lds_w<BS, true, false, CMP, W>;
-        return nts ? k_sweep_lds_w<BS, false, true, CMP, W> : k_sweep_lds_w<BS, false, false, CMP, W>;
-      }
-    }
-  }
-  if constexpr (W == 0) {
-    if (ntg) return nts ? k_sweep<BS, true, true, CMP, KG> : k_sweep<BS, true, false, CMP, KG>;
-    return nts ? k_sweep<BS, false, true, CMP, KG> : k_sweep<BS, false, false, CMP, KG>;
-  } else {
-    if (ntg) return nts ? k_sweep_w<BS, true, true, CMP, KG, W> : k_sweep_w<BS, true, false, CMP, KG, W>;
-    return nts ? k_sweep_w<BS, false, true, CMP, KG, W> : k_sweep_w<BS, false, false, CMP, KG, W>;
-  }
-}
-
+// The sweep kernel for a tile size and cache hints.
 template <int BS, bool CMP, int KG>
-SweepFn pick3(int ntg, int nts, int occ, int lds) {
-  if (occ == 8) return pick_w<BS, CMP, KG, 8>(ntg, nts, lds);
-  if (occ == 6) return pick_w<BS, CMP, KG, 6>(ntg, nts, lds);
-  return pick_w<BS, CMP, KG, 0>(ntg, nts, lds);
+SweepFn pick_nt(int ntg, int nts) {
+  if (ntg) return nts ? k_sweep<BS, true, true, CMP, KG> : k_sweep<BS, true, false, CMP, KG>;
+  return nts ? k_sweep<BS, false, true, CMP, KG> : k_sweep<BS, false, false, CMP, KG>;
 }
 
 template <bool CMP, int KG>
 SweepFn pick_tile(const srs_ctx* c) {
   switch (c->tile) {
-    case 128: return pick3<128, CMP, KG>(c->nt_geometry, c->nt_state, c->occ, c->lds);
-    case 512: return pick3<512, CMP, KG>(c->nt_geometry, c->nt_state, c->occ, c->lds);
-    default: return pick3<256, CMP, KG>(c->nt_geometry, c->nt_state, c->occ, c->lds);
+    case 128: return pick_nt<128, CMP, KG>(c->nt_geometry, c->nt_state);
+    case 256: return pick_nt<256, CMP, KG>(c->nt_geometry, c->nt_state);
+    default: return pick_nt<512, CMP, KG>(c->nt_geometry, c->nt_state);
   }
 }
 
 template <int KG>
-SweepFn pick_kg(const srs_ctx* c) { return c->compact_all ? pick_tile<true, KG>(c) : pick_tile<false, KG>(c); }
+SweepFn pick_kg(const srs_ctx* c) { return c->class_all ? pick_tile<true, KG>(c) : pick_tile<false, KG>(c); }
 
 SweepFn pick_sweep(const srs_ctx* c) {
   return c->group == 4 ? pick_kg<4>(c) : c->group == 2 ? pick_kg<2>(c) : pick_kg<1>(c);
@@ -831,7 +744,7 @@ GatedFn pick_gated_cmp(const srs_ctx* c, bool proto) {
 
 template <int BS>
 GatedFn pick_gated_bs(const srs_ctx* c, bool proto) {
-  return c->compact_all ? pick_gated_cmp<BS, true>(c, proto) : pick_gated_cmp<BS, false>(c, proto);
+  return c->class_all ? pick_gated_cmp<BS, true>(c, proto) : pick_gated_cmp<BS, false>(c, proto);
 }
 // one tile size per unit: 128 in unit 2, 256 in unit 3, 512 in unit 4
 template GatedFn pick_gated_bs<SRS_UNIT == 2 ? 128 : SRS_UNIT == 3 ? 256 : 512>(const srs_ctx*, bool);
@@ -884,65 +797,80 @@ double quantize(double a, int bits) {
   return std::ldexp(std::nearbyint(std::ldexp(m, bits)), e - bits);
 }
 
-// Builds the compact operator layout: neighbours as int16 offsets, and each
-// row as a class row plus int16 multiples of the class row's ulps.  Leaves
-// hm.compact false unless every row of the mesh reconstructs exactly.
-void build_compact(HostMesh& hm) {
+// Each coefficient row as a class row plus int16 deltas of the bit patterns.
+// class_rows stays false unless every row of the mesh is reproduced exactly.
+void build_class_rows(HostMesh& hm) {
   const int n = hm.n, np = hm.np;
-  for (int q = 0; q < 4; ++q)
-    for (int k = 0; k < n; ++k) {
-      const long o = (long)hm.nbr[(size_t)q * np + k] - k;
-      if (o < -32767 || o > 32767) return;
-    }
   std::map<std::array<double, 5>, int> classes;
-  std::vector<int> row_class(n);
+  std::vector<uint32_t> row(3 * (size_t)np + 1, 0);
   for (int k = 0; k < n; ++k) {
     std::array<double, 5> key;
-    for (int q = 0; q < 5; ++q) key[q] = quantize(hm.coef[(size_t)q * np + k], 40);
+    int64_t d[5];
+    for (int q = 0; q < 5; ++q) {
+      const double a = hm.coef[(size_t)q * np + k];
+      if (!std::isfinite(a) || (a == 0.0 && std::signbit(a))) return;  // the classes are keyed by value
+      key[q] = quantize(a, 40);
+      int64_t ka, kt;
+      memcpy(&ka, &a, 8);
+      memcpy(&kt, &key[q], 8);
+      d[q] = ka - kt;  // as the kernel adds it back, for any pair of patterns
+      if (d[q] < -32768 || d[q] > 32767) return;
+    }
     auto it = classes.find(key);
     if (it == classes.end()) {
       if (classes.size() >= 65535) return;
       it = classes.emplace(key, (int)classes.size()).first;
     }
-    row_class[k] = it->second;
+    auto u = [](int64_t v) { return (uint32_t)(uint16_t)v; };
+    row[3 * (size_t)k] = (uint32_t)it->second | u(d[0]) << 16;
+    row[3 * (size_t)k + 1] = u(d[1]) | u(d[2]) << 16;
+    row[3 * (size_t)k + 2] = u(d[3]) | u(d[4]) << 16;
   }
-  const int nc = (int)classes.size();
-  std::vector<double> tab(10 * (size_t)nc);
+  hm.n_class = (int)classes.size();
+  hm.tab.resize(5 * (size_t)hm.n_class);
   for (auto& kv : classes)
-    for (int q = 0; q < 5; ++q) {
-      const double b = kv.first[q];
-      tab[10 * (size_t)kv.second + q] = b;
-      int e;
-      std::frexp(b, &e);
-      tab[10 * (size_t)kv.second + 5 + q] = (b == 0.0) ? 0.0 : std::ldexp(1.0, e - 53);  // ulp of b
-    }
-  std::vector<int16_t> off(4 * (size_t)np, 0), dq(5 * (size_t)np, 0);
-  std::vector<uint16_t> cls(np, 0);
-  for (int k = 0; k < n; ++k) {
-    for (int q = 0; q < 4; ++q) off[(size_t)q * np + k] = (int16_t)(hm.nbr[(size_t)q * np + k] - k);
-    const double* t = &tab[10 * (size_t)row_class[k]];
-    int16_t d[5];
-    for (int q = 0; q < 5; ++q) {
-      const double a = hm.coef[(size_t)q * np + k];
-      if (t[5 + q] == 0.0) {
-        if (!(a == t[q] && !std::signbit(a))) return;
-        d[q] = 0;
-        continue;
+    for (int q = 0; q < 5; ++q) hm.tab[5 * (size_t)kv.second + q] = kv.first[q];
+  hm.row.swap(row);
+  hm.class_rows = true;
+}
+
+// The tile map of a mesh for `tile` elements per tile, uploaded.  Halos are
+// sorted, so that a wavefront's loads of them fall in runs.
+int build_map(srs_ctx* c, HostMesh& hm, int tile, TileMap* m) {
+  const int n = hm.n, np = hm.np, nt = (n + tile - 1) / tile;
+  std::vector<uint16_t> loc(4 * (size_t)np, 0);
+  std::vector<int32_t> hal, hoff(nt + 1, 0), place(n, -1), out;
+  int h_max = 0;
+  for (int t = 0; t < nt; ++t) {
+    const int j0 = t * tile, j1 = std::min(n, j0 + tile);
+    out.clear();
+    for (size_t k = 4 * (size_t)j0; k < 4 * (size_t)j1; ++k) {
+      const int e = hm.nbr[k];
+      if ((e < j0 || e >= j0 + tile) && place[e] < 0) {
+        place[e] = 0;
+        out.push_back(e);
       }
-      const double m = (a - t[q]) / t[5 + q];
-      if (!(std::fabs(m) <= 32767.0) || m != std::nearbyint(m)) return;
-      d[q] = (int16_t)m;
-      if ((t[q] + (double)d[q] * t[5 + q]) != a) return;  // exact, as the kernel computes it
     }
-    cls[k] = (uint16_t)row_class[k];
-    for (int q = 0; q < 5; ++q) dq[(size_t)q * np + k] = d[q];
+    std::sort(out.begin(), out.end());
+    for (size_t i = 0; i < out.size(); ++i) place[out[i]] = tile + (int)i;
+    for (size_t k = 4 * (size_t)j0; k < 4 * (size_t)j1; ++k) {
+      const int e = hm.nbr[k];
+      loc[k] = (uint16_t)(e >= j0 && e < j0 + tile ? e - j0 : place[e]);
+    }
+    for (int e : out) place[e] = -1;
+    hal.insert(hal.end(), out.begin(), out.end());
+    if (hal.size() > (size_t)INT32_MAX) return srs::fail(SRS_E_ARG, "mesh too large for its halo lists");
+    hoff[t + 1] = (int32_t)hal.size();
+    h_max = std::max(h_max, (int)out.size());
   }
-  hm.off.swap(off);
-  hm.dq.swap(dq);
-  hm.cls.swap(cls);
-  hm.tab.swap(tab);
-  hm.n_class = nc;
-  hm.compact = true;
+  if (hal.empty()) hal.push_back(0);
+  int rc;
+  if ((rc = dev_upload(c, &m->d_loc, loc)) || (rc = dev_upload(c, &m->d_hal, hal)) ||
+      (rc = dev_upload(c, &m->d_hoff, hoff)))
+    return rc;
+  m->tile = tile;
+  m->qcap = tile + h_max;
+  return SRS_OK;
 }
 
 // cpu/RunSimulation.cpp:85-88, the parts that depend on CaNSR only.
@@ -967,7 +895,7 @@ void launch_sweep(srs_ctx* c) {
   if (c->grid_sweep == 0) return;  // every realization has finished
   // one realization: tile b is tile b of realization 0, no table lookups
   const int single = c->reals.size() == 1 ? 1 : 0;
-  hipLaunchKernelGGL(pick_sweep(c), dim3(c->grid_sweep), dim3(c->tile), 0, c->stream, c->d_desc, c->d_live,
+  hipLaunchKernelGGL(pick_sweep(c), dim3(c->grid_sweep), dim3(c->tile), c->sweep_lds, c->stream, c->d_desc, c->d_live,
                      c->d_tiles, c->n_tiles, (const int*)c->d_groups, single);
 }
 
@@ -979,7 +907,7 @@ void launch_subset_block(srs_ctx* c, int64_t m, uint32_t gmode) {
   for (const srs_ctx::Subset& sb : c->subsets)
     for (int64_t k = 0; k < m; ++k) {
       if (sb.nt > 0)
-        hipLaunchKernelGGL(pick_sweep(c), dim3((sb.nt + NXCD - 1) / NXCD * NXCD), dim3(c->tile), 0, c->stream,
+        hipLaunchKernelGGL(pick_sweep(c), dim3((sb.nt * c->group + NXCD - 1) / NXCD * NXCD), dim3(c->tile), c->sweep_lds, c->stream,
                            c->d_desc, c->d_live, c->d_tiles + sb.t0, sb.nt, (const int*)c->d_groups, 0);
       hipLaunchKernelGGL(k_gate_list, dim3((unsigned)sb.nr), dim3(GATE_THREADS), 0, c->stream, c->d_desc, c->d_live,
                          (const int32_t*)c->d_sub_rids + sb.r0, gmode);
@@ -1055,7 +983,7 @@ void launch_gated(srs_ctx* c, int cur, uint32_t gmode, bool proto, const double*
   const GatedFn f = c->tile == 128 ? pick_gated_bs<128>(c, proto)
                     : c->tile == 512 ? pick_gated_bs<512>(c, proto) : pick_gated_bs<256>(c, proto);
   const int grid = (c->n_tiles + 1 + NXCD - 1) / NXCD * NXCD;
-  hipLaunchKernelGGL(f, dim3(grid), dim3(c->tile), 0, c->stream, c->d_desc, c->d_live, c->n_tiles,
+  hipLaunchKernelGGL(f, dim3(grid), dim3(c->tile), std::max(c->sweep_lds, GATE_LDS), c->stream, c->d_desc, c->d_live, c->n_tiles,
                      cur | (c->alt_order ? 2 : 0), gmode, xo_at, xn_at);
 }
 
@@ -1087,7 +1015,7 @@ int drop_graphs(srs_ctx* c) {
 void set_tiles(srs_ctx* c, int2* d, int n) {
   c->d_tiles = d;
   c->n_tiles = n;
-  c->grid_sweep = (n + NXCD - 1) / NXCD * NXCD;
+  c->grid_sweep = (n * c->group + NXCD - 1) / NXCD * NXCD;
   c->subsets_valid = false;
 }
 
@@ -1261,9 +1189,7 @@ int srs_ctx_tune(srs_ctx* c, int32_t key, int32_t value) {
     case SRS_TUNE_NT_STATE:
       c->nt_state = value != 0;
       return c->finalized ? drop_graphs(c) : SRS_OK;
-    case SRS_TUNE_LDS:
-      c->lds = value != 0;
-      return c->finalized ? drop_graphs(c) : SRS_OK;
+    case SRS_TUNE_LDS: return SRS_OK;  // tiles are always staged
     case SRS_TUNE_GATED_SWEEP:
       c->gated = value != 0;
       return c->finalized ? drop_graphs(c) : SRS_OK;
@@ -1383,12 +1309,12 @@ int srs_ctx_add_mesh(srs_ctx* c, const srs_mesh_desc* m, int32_t* mesh_id) {
   if (any_br) hm->br.assign(4 * (size_t)np, 0.0);
   for (int k = 0; k < np; ++k) {
     if (k >= n) {  // padding rows point at themselves
-      for (int q = 0; q < 4; ++q) hm->nbr[(size_t)q * np + k] = k < n ? k : 0;
+      for (int q = 0; q < 4; ++q) hm->nbr[4 * (size_t)k + q] = 0;
       continue;
     }
     const int i = hm->perm[k];
     for (int q = 0; q < 5; ++q) hm->coef[(size_t)q * np + k] = m->aij[5 * (size_t)i + q];
-    for (int q = 0; q < 4; ++q) hm->nbr[(size_t)q * np + k] = hm->inv[m->nij[4 * (size_t)i + q]];
+    for (int q = 0; q < 4; ++q) hm->nbr[4 * (size_t)k + q] = hm->inv[m->nij[4 * (size_t)i + q]];
     uint8_t f = 0;
     if (m->domain[i] != 0) f |= F_JSR;
     if (m->tropc[i]) f |= F_TROPC;
@@ -1407,7 +1333,7 @@ int srs_ctx_add_mesh(srs_ctx* c, const srs_mesh_desc* m, int32_t* mesh_id) {
     }
     hm->flags[k] = f;
   }
-  if (c->compact) build_compact(*hm);
+  if (c->compact) build_class_rows(*hm);
   *mesh_id = (int32_t)c->meshes.size();
   c->meshes.push_back(std::move(hm));
   return SRS_OK;
@@ -1490,24 +1416,31 @@ int srs_ctx_finalize(srs_ctx* c, int32_t record_capacity) {
   if (c->reals.empty()) return srs::fail(SRS_E_STATE, "no realizations");
   HIPCHK(hipSetDevice(c->device));
   int rc;
-  if (c->tile == 0) {
-    // 512-element tiles pay on meshes of a million elements and more (the
-    // 3M-element dyad); smaller meshes keep more workgroups in flight with 256
-    int n_max = 0;
-    for (const HostReal& hr : c->reals) n_max = std::max(n_max, c->meshes[hr.mesh]->n);
-    c->tile = n_max >= (1 << 20) ? 512 : 256;
-  }
-  c->compact_all = !c->meshes.empty();
-  for (auto& hmp : c->meshes) c->compact_all &= hmp->compact;
+  // 512-element tiles share the most neighbours inside a tile (halos of 1.4
+  // elements per element in the block order, 0.6 in the Morton order; 1.9 and
+  // 0.8 with 256) and were the fastest
+  // at every size: 927,816 elements 21.5 against 23.3 us per step, 56,250
+  // 9.2 against 9.3, the 48-member ensemble 147 against 171
+  if (c->tile == 0) c->tile = 512;
+  c->class_all = !c->meshes.empty();
+  for (auto& hmp : c->meshes) c->class_all &= hmp->class_rows;
   for (auto& hmp : c->meshes) {
     HostMesh& hm = *hmp;
-    if (!c->compact_all) {
-      if ((rc = dev_upload(c, &hm.d_nbr, hm.nbr))) return rc;
+    // the meshes' channel flags were set by add_realization: what blocks hold
+    std::vector<uint32_t> blk(hm.np / 64, 0);
+    for (size_t b = 0; b < blk.size(); ++b) {
+      bool plain = true;
+      for (size_t k = 64 * b; k < std::min<size_t>(64 * b + 64, hm.n); ++k) plain &= hm.flags[k] == F_TROPC;
+      if (plain) blk[b] |= BLK_PLAIN;
+    }
+    if ((rc = dev_upload(c, &hm.d_nbr, hm.nbr))) return rc;
+    if ((rc = dev_upload(c, &hm.d_blk, blk))) return rc;
+    if ((rc = build_map(c, hm, c->tile, &hm.map))) return rc;
+    c->sweep_lds = std::max(c->sweep_lds, 4 * sizeof(double) * (size_t)hm.map.qcap);
+    if (!c->class_all) {
       if ((rc = dev_upload(c, &hm.d_coef, hm.coef))) return rc;
     } else {
-      if ((rc = dev_upload(c, &hm.d_off, hm.off))) return rc;
-      if ((rc = dev_upload(c, &hm.d_cls, hm.cls))) return rc;
-      if ((rc = dev_upload(c, &hm.d_dq, hm.dq))) return rc;
+      if ((rc = dev_upload(c, &hm.d_row, hm.row))) return rc;
       if ((rc = dev_upload(c, &hm.d_tab, hm.tab))) return rc;
     }
     if ((rc = dev_upload(c, &hm.d_flags, hm.flags))) return rc;
@@ -1559,7 +1492,8 @@ int srs_ctx_finalize(srs_ctx* c, int32_t record_capacity) {
     d.nbr = hm.d_nbr; d.coef = hm.d_coef; d.flags = hm.d_flags; d.V0 = hm.d_V0; d.tt = hm.d_tt; d.br = hm.d_br;
     d.br_mesh = hm.d_br;
     std::copy(hm.br_d, hm.br_d + 4, d.brd);
-    d.off = hm.d_off; d.cls = hm.d_cls; d.dq = hm.d_dq; d.tab = hm.d_tab;
+    d.loc = hm.map.d_loc; d.hal = hm.map.d_hal; d.hoff = hm.map.d_hoff; d.qcap = hm.map.qcap;
+    d.row = hm.d_row; d.tab = hm.d_tab; d.blk = hm.d_blk;
     d.n_class = hm.n_class;
     d.n = hm.n; d.np = hm.np;
     d.X[0] = gx0[real_group[r]]; d.X[1] = gx1[real_group[r]];
@@ -1611,7 +1545,7 @@ int srs_ctx_finalize(srs_ctx* c, int32_t record_capacity) {
     lives.push_back(lv);
   }
   c->n_tiles = (int)tiles.size();
-  c->grid_sweep = (c->n_tiles + NXCD - 1) / NXCD * NXCD;
+  c->grid_sweep = (c->n_tiles * c->group + NXCD - 1) / NXCD * NXCD;
   // the staging buffer of state transfers: the largest realization's fields,
   // at most 32 MB (larger fields go through it in parts)
   for (const HostReal& hr : c->reals) c->stage_len = std::max(c->stage_len, 6 * (size_t)c->meshes[hr.mesh]->n);
@@ -1627,9 +1561,6 @@ int srs_ctx_finalize(srs_ctx* c, int32_t record_capacity) {
   if (c->reals.size() > 1 && (rc = dev_alloc(c, &c->d_sub_rids, c->reals.size()))) return rc;
   c->groups = groups;
   if (c->reals.size() > 1 && (rc = dev_alloc(c, &c->d_tiles_live, tiles.size()))) return rc;
-  // meshes' channel flags were updated by add_realization; refresh them
-  for (auto& hmp : c->meshes)
-    HIPCHK(hipMemcpy(hmp->d_flags, hmp->flags.data(), hmp->flags.size(), hipMemcpyHostToDevice));
   HIPCHK(hipDeviceSynchronize());
   c->finalized = true;
   return SRS_OK;
@@ -1878,7 +1809,7 @@ static int graph_gated(srs_ctx* c, int64_t block, int cur, uint32_t gmode, hipGr
 static int gated_start(srs_ctx* c, uint32_t flags, bool* ok, int* cur) {
   *ok = false;
   const int occ_max = (flags & SRS_STEP_PROTOCOL) ? 0 : 6;
-  if (!c->gated || c->reals.size() != 1 || c->group != 1 || !c->lds || c->occ > occ_max) return SRS_OK;
+  if (!c->gated || c->reals.size() != 1 || c->group != 1 || c->occ > occ_max) return SRS_OK;
   RealLive lv;
   int rc = live_rw(c, 0, &lv, false);
   if (rc) return rc;

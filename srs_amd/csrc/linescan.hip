@@ -20,7 +20,7 @@ __global__ __launch_bounds__(SCAN_BS) void k_scan_blur(const RealDesc* __restric
     const int j = (blockIdx.x * SCAN_CELLS_PER_THREAD + q) * SCAN_BS + threadIdx.x;
     if (j < n) {
       cx[q] = cen[j]; cy[q] = cen[np + j]; cz[q] = cen[2 * np + j];
-      vf[q] = d.V0[j] * X[cq(d, j) + 3];  // V0 * Ca-bound Fluo
+      vf[q] = d.V0[j] * X[cq(d, j) + FLUO_OFF];  // V0 * Ca-bound Fluo
     } else {
       cx[q] = cy[q] = cz[q] = 1e30;  // beyond the 1 um cut-off of every point
       vf[q] = 0.0;
@@ -102,7 +102,7 @@ __global__ void k_scan_final(const RealDesc* __restrict__ D, const RealLive* __r
   }
   for (int i = threadIdx.x; i < n_f; i += blockDim.x) {
     const int e = near_f[i];
-    out[n_ca + i] = e >= 0 ? X[cq(D[r], e) + 3] : f0;
+    out[n_ca + i] = e >= 0 ? X[cq(D[r], e) + FLUO_OFF] : f0;
   }
   for (int i = threadIdx.x; i < n_ca; i += blockDim.x) {
     const int e = near_ca[i];
