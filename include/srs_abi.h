@@ -278,8 +278,9 @@ int srs_ctx_create(int device, srs_ctx** out);
  * never results.  Layout keys must be set before the first mesh is added,
  * the tile before srs_ctx_finalize; the rest at any time. */
 #define SRS_TUNE_TILE 1          /* elements per sweep workgroup: 128, 256 or 512 (default) */
-#define SRS_TUNE_NT_GEOMETRY 2   /* 1 (default): non-temporal loads of operator rows and flags */
-#define SRS_TUNE_NT_STATE 3      /* 1: non-temporal stores of the new state */
+#define SRS_TUNE_NT_GEOMETRY 2   /* 1: non-temporal loads of operator rows and halo lists; by default 0 */
+#define SRS_TUNE_NT_STATE 3      /* 1: non-temporal stores of the new state; by default srs_ctx_finalize
+                                    takes 1 when states and rows exceed 330 MB */
 #define SRS_TUNE_PLANE_PAD 4     /* extra elements (multiple of 64) between SoA planes */
 #define SRS_TUNE_COMPACT 5       /* 1 (default): store operator rows as class + int16 deltas of the
                                     bit patterns where that reproduces them exactly */

@@ -450,6 +450,7 @@ struct DevBuf {
 struct TileMap {
   int tile = 0;       // elements per tile; 0: not built
   int32_t qcap = 0;   // the most quads a tile stages (its elements and its halo)
+  int32_t n_halo = 0; // elements of all halos
   uint16_t* d_loc = nullptr;
   int32_t *d_hal = nullptr, *d_hoff = nullptr;
 };
@@ -511,8 +512,9 @@ struct srs_ctx {
   int device = 0;
   int tile = 0;          // elements per k_sweep workgroup; 0: chosen by srs_ctx_finalize
   size_t sweep_lds = 0;  // LDS bytes of a sweep workgroup (staged quads)
-  int nt_geometry = 1;   // non-temporal loads of operator rows and flags
-  int nt_state = 0;      // non-temporal stores of the new state
+  // cache hints; -1: chosen by srs_ctx_finalize
+  int nt_geometry = -1;  // non-temporal loads of operator rows and halo lists
+  int nt_state = -1;     // non-temporal stores of the new state
   int plane_pad = 0;     // extra elements per SoA plane
   int compact = 1;       // compress operator rows when a mesh allows it
   int occ = 0;           // gated sweep's register budget: 0 compiler's choice, 6 or 8 wavefronts per SIMD

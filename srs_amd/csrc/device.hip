@@ -868,6 +868,7 @@ int build_map(srs_ctx* c, HostMesh& hm, int tile, TileMap* m) {
   if ((rc = dev_upload(c, &m->d_loc, loc)) || (rc = dev_upload(c, &m->d_hal, hal)) ||
       (rc = dev_upload(c, &m->d_hoff, hoff)))
     return rc;
+  m->n_halo = hoff[nt];
   m->tile = tile;
   m->qcap = tile + h_max;
   return SRS_OK;
@@ -1543,6 +1544,22 @@ int srs_ctx_finalize(srs_ctx* c, int32_t record_capacity) {
     lv.ca_nsr = hr.reals[SRS_R_DEFAULT_CA_NSR];
     serca_terms(lv.ca_nsr, hr.reals, lv.serca);
     lives.push_back(lv);
+  }
+  // Cache hints.  A step reads and writes every state buffer in turn with the
+  // one before, so while the buffers and the meshes' rows fit the 256 MB
+  // last-level cache nothing is hinted past it (us per step without hints /
+  // non-temporal stores / non-temporal row loads: 928k-element dyad, 114 MB,
+  // 21.5 / 25.9 / 24.8; 18-member ensemble, 266 MB, 53.6 / 60.8 / 61.2; 21
+  // members in groups, 309 MB, 76.2 / 78.2 / 79.8).  Beyond it plain stores
+  // evict what the next step could still have found (24 members, 351 MB, 78.6 /
+  // 74.9 / 77.4; 3M-element dyad, 362 MB, 69.4 / 61.1 / 61.2; 48 members, 147 /
+  // 138 / 160).  The line lies between 309 and 351 MB.
+  {
+    double ws = 0.0;
+    for (const HostReal& hr : c->reals) ws += 2.0 * 48.0 * c->meshes[hr.mesh]->n;
+    for (auto& hmp : c->meshes) ws += (double)hmp->n * ((c->class_all ? 12 : 40) + 9) + 4.0 * hmp->map.n_halo;
+    if (c->nt_state < 0) c->nt_state = ws > 330e6;
+    if (c->nt_geometry < 0) c->nt_geometry = 0;
   }
   c->n_tiles = (int)tiles.size();
   c->grid_sweep = (c->n_tiles * c->group + NXCD - 1) / NXCD * NXCD;
