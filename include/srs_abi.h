@@ -278,16 +278,15 @@ int srs_ctx_create(int device, srs_ctx** out);
  * never results.  Layout keys must be set before the first mesh is added,
  * the tile before srs_ctx_finalize; the rest at any time. */
 #define SRS_TUNE_TILE 1          /* elements per sweep workgroup: 128, 256 or 512 (default) */
-#define SRS_TUNE_NT_GEOMETRY 2   /* 1: non-temporal loads of operator rows and halo lists; by default 0 */
+#define SRS_TUNE_NT_GEOMETRY 2   /* accepted and ignored: operator rows are read through the caches */
 #define SRS_TUNE_NT_STATE 3      /* 1: non-temporal stores of the new state; by default srs_ctx_finalize
                                     takes 1 when states and rows exceed 330 MB */
 #define SRS_TUNE_PLANE_PAD 4     /* extra elements (multiple of 64) between SoA planes */
 #define SRS_TUNE_COMPACT 5       /* 1 (default): store operator rows as class + int16 deltas of the
                                     bit patterns where that reproduces them exactly */
 #define SRS_TUNE_OCCUPANCY 6     /* register budget of the single-realization step with the gating folded
-                                    in (SRS_TUNE_GATED_SWEEP): 0 compiler's choice; 6: at most 80 VGPRs,
-                                    so that six wavefronts share each SIMD; 8: separate gating launches.
-                                    The sweep itself fits 64 VGPRs and has no budget */
+                                    in (SRS_TUNE_GATED_SWEEP): 0 by the mesh's size; 6 or 8: at most 80
+                                    VGPRs, so that six wavefronts share each SIMD */
 #define SRS_TUNE_GROUP 7         /* 1 (default), 2 or 4: realizations of one mesh whose states are interleaved
                                     per 64 elements and whose tiles are swept side by side, so that the
                                     operator rows come from cache for all but the first (set before
@@ -298,8 +297,7 @@ int srs_ctx_create(int device, srs_ctx** out);
                                     realizations have all finished out of the sweep; 0: sweep them all */
 #define SRS_TUNE_GATED_SWEEP 10  /* 1 (default): a single-realization context runs each
                                     step's gating (and, with SRS_STEP_PROTOCOL, the loop body) inside the
-                                    next step's sweep launch (register budget 0 or 6; 0 with the loop
-                                    body); 0: a gating launch after every sweep */
+                                    next step's sweep launch; 0: a gating launch after every sweep */
 #define SRS_TUNE_SUBSET_MB 12    /* 0 (default): every step sweeps all realizations; > 0: srs_explicit_step
                                     steps runs of realization groups whose state takes at most this many MB
                                     through a whole block of steps (128 with SRS_STEP_GRAPH) each, one after

@@ -177,8 +177,8 @@ __device__ __forceinline__ void adj_step(const RealDesc* __restrict__ D, const R
   double V0 = 1.0;
   SlBuf sb{1.0, 0.0, 0.0};
   if (in) {
-    if constexpr (WMAT) g = load_geo_nbr<false, CLASS>(d, j);
-    else g = load_geo<false, CLASS>(d, am.loc, j, block_flags(d, j));
+    if constexpr (WMAT) g = load_geo_nbr<CLASS>(d, j);
+    else g = load_geo<CLASS>(d, am.loc, j, block_flags(d, j));
     m0 = ld_quad(gp(X), qidx1(j));
     mu = ld_quad(gp(lam), qidx1(j));
     V0 = d.V0[j];
@@ -192,7 +192,7 @@ __device__ __forceinline__ void adj_step(const RealDesc* __restrict__ D, const R
   }
   if constexpr (!WMAT) {
     tw.put(threadIdx.x, w0);
-    const Halo h = load_halo<ADJ_BS, false>(am.hal, am.hoff, tile);
+    const Halo h = load_halo<ADJ_BS>(am.hal, am.hoff, tile);
     auto put_halo = [&](int k, int e) {
       const uint8_t fn = d.flags[e];
       const d4 ln = ld_quad(gp(lam), qidx1(e));
@@ -314,11 +314,12 @@ __device__ __forceinline__ void adj_step(const RealDesc* __restrict__ D, const R
       if (lo < d.n_celem && d.celem[lo] == j) {
         const double a = P[SRS_R_V_RYR] * P[SRS_R_V_CELL];
         for (int e = d.cstart[lo]; e < d.cstart[lo + 1]; ++e) {
-          const int ch = d.centry[e];
+          const ChanEntry en = d.centry[e];
+          const int ch = en.code;
           if (ch >= 0) {
             const int i = ch >> 1;
             if (!ryr[i]) continue;
-            const int ce = d.ryr_ele[i], je = d.ryr_jsr[i];
+            const int ce = en.cyt, je = en.jsr;
             const int p = (ch & 1) ? ce : je;  // the partner element
             const double cp = X[2 * (size_t)qidx1(p)];
             const double up = lam[2 * (size_t)qidx1(p)] / sl_buffer(d, p, cp, d.flags[p]).beta;
@@ -806,7 +807,7 @@ static int loss_grad_run(srs_ctx* c, const std::vector<int32_t>& ids, int32_t sc
     // the steps between two of those through the gated sweep (one launch per
     // step, the replay of each step in the next one's workgroup 0)
     hipLaunchKernelGGL(k_seg_start, dim3(nb), dim3(256), 0, c->stream, c->d_desc, c->d_live, d_rid, (int64_t)0);
-    const bool gated = c->gated && n_real == 1 && c->group == 1 && c->occ <= 6;
+    const bool gated = c->gated && n_real == 1 && c->group == 1;
     int cur = lv[ids[m0]].cur;
     int ks = 0;
     for (int64_t n = 0; n < n_steps && e == hipSuccess;) {

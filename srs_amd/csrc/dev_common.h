@@ -72,6 +72,20 @@ __host__ __device__ inline size_t xoff(int s, size_t e, size_t np, int K = 1, in
 typedef double d2 __attribute__((ext_vector_type(2)));
 typedef double d4 __attribute__((ext_vector_type(4)));
 
+// One channel of an element that carries channel flux, in the reference's order.
+struct ChanEntry {
+  int32_t code;      // >=0: 2*ryr + side (0 cleft, 1 jSR); <0: -(lcc+1)
+  int32_t jsr, cyt;  // a RyR's two elements
+  int32_t pad;
+};
+// Everything about a channel-flux element that is fixed, in one record, for
+// the workgroup that gates and then updates these elements (sweep_gated).
+struct ChanElem {
+  double a[5], v0, tt;
+  int32_t j, nb[4], e0, e1;  // the element, its neighbours, its run of centry
+  uint32_t f;
+};
+
 // Immutable per-realization descriptor (read with scalar loads).
 struct RealDesc {
   const int32_t* nbr;     // [np][4] neighbour indices
@@ -107,7 +121,8 @@ struct RealDesc {
   int32_t n_celem;
   const int32_t* celem;   // sorted element indices that carry channel flux
   const int32_t* cstart;  // [n_celem+1]
-  const int32_t* centry;  // >=0: 2*ryr + side(0 cleft, 1 jSR); <0: -(lcc+1)
+  const ChanEntry* centry;
+  const ChanElem* crec;   // [n_celem] what an element of celem is updated from
   const int32_t* sched;   // replay schedule [n_sched][n_ryr] or null
   int64_t n_sched;
   float* rec;
@@ -188,21 +203,14 @@ __device__ __forceinline__ double wave_sum_dpp(double v) {
   return v;
 }
 
-// Loads of data read once per step (operator rows, flags) may bypass cache
-// allocation so that the state planes stay resident between steps.  Pointers
-// read from the descriptor are generic; casting them to the global address
-// space lets the compiler use global (not flat) memory instructions.
+// Pointers read from the descriptor are generic; casting them to the global
+// address space lets the compiler use global (not flat) memory instructions.
 #define SRS_GLOBAL __attribute__((address_space(1)))
 template <class T>
 __device__ __forceinline__ const SRS_GLOBAL T* gp(const T* p) { return (const SRS_GLOBAL T*)p; }
 template <class T>
 __device__ __forceinline__ SRS_GLOBAL T* gpw(T* p) { return (SRS_GLOBAL T*)p; }
 
-template <bool NT, class T>
-__device__ __forceinline__ T ldg(const SRS_GLOBAL T* p) {
-  if constexpr (NT) return __builtin_nontemporal_load(p);
-  else return *p;
-}
 template <bool NT, class T>
 __device__ __forceinline__ void stg(SRS_GLOBAL T* p, T v) {
   if constexpr (NT) __builtin_nontemporal_store(v, p);
@@ -249,7 +257,7 @@ constexpr int HPRE = 2;
 struct Halo {
   int s, n, e[HPRE];
 };
-template <int BS, bool NTG>
+template <int BS>
 __device__ __forceinline__ Halo load_halo(const int32_t* hal, const int32_t* hoff, const int t) {
   Halo h;
   h.s = sld(hoff + t);
@@ -257,7 +265,7 @@ __device__ __forceinline__ Halo load_halo(const int32_t* hal, const int32_t* hof
 #pragma unroll
   for (int q = 0; q < HPRE; ++q) {
     const int k = (int)threadIdx.x + q * BS;
-    h.e[q] = k < h.n ? ldg<NTG>(gp(hal) + h.s + k) : -1;
+    h.e[q] = k < h.n ? gp(hal)[h.s + k] : -1;
   }
   return h;
 }
@@ -276,12 +284,12 @@ struct Geo {
 __device__ __forceinline__ double ulps_from(const double t, const int delta) {
   return __longlong_as_double(__double_as_longlong(t) + (long long)delta);
 }
-template <bool NTG, bool CLASS>
+template <bool CLASS>
 __device__ __forceinline__ void load_coef(const RealDesc& d, const int j, Geo& g) {
   if constexpr (CLASS) {
     // reproduces the assembled FP64 values exactly (every row was checked
     // when the mesh was added)
-    const i3 r = ldg<NTG>((const SRS_GLOBAL i3*)((const SRS_GLOBAL uint32_t*)d.row + 3 * (size_t)j));
+    const i3 r = *(const SRS_GLOBAL i3*)(gp(d.row) + 3 * (size_t)j);
     const SRS_GLOBAL double* t = gp(d.tab) + 5 * (r.x & 0xffff);
     g.a0 = ulps_from(t[0], r.x >> 16);
     g.a1 = ulps_from(t[1], (int16_t)r.y);
@@ -289,33 +297,32 @@ __device__ __forceinline__ void load_coef(const RealDesc& d, const int j, Geo& g
     g.a3 = ulps_from(t[3], (int16_t)r.z);
     g.a4 = ulps_from(t[4], r.z >> 16);
   } else {
-    const int np = d.np;
+    const size_t np = d.np;
     const SRS_GLOBAL double* cf = gp(d.coef);
-    g.a0 = ldg<NTG>(cf + j); g.a1 = ldg<NTG>(cf + np + j); g.a2 = ldg<NTG>(cf + 2 * np + j);
-    g.a3 = ldg<NTG>(cf + 3 * np + j); g.a4 = ldg<NTG>(cf + 4 * np + j);
+    g.a0 = cf[j]; g.a1 = cf[np + j]; g.a2 = cf[2 * np + j]; g.a3 = cf[3 * np + j]; g.a4 = cf[4 * np + j];
   }
 }
 // The row of an element of the workgroup's tile.  b: the flags of the
 // element's block; in a plain block no element flags are loaded.  A row is two
 // wide loads (places 8 B, class row 12 B).
-template <bool NTG, bool CLASS>
+template <bool CLASS>
 __device__ __forceinline__ Geo load_geo(const RealDesc& d, const uint16_t* loc, const int j, const uint32_t b) {
   Geo g;
-  g.f = (b & BLK_PLAIN) ? (uint8_t)F_TROPC : ldg<NTG>(gp(d.flags) + j);
-  const i2 q = ldg<NTG>((const SRS_GLOBAL i2*)loc + j);
+  g.f = (b & BLK_PLAIN) ? (uint8_t)F_TROPC : gp(d.flags)[j];
+  const i2 q = ((const SRS_GLOBAL i2*)loc)[j];
   g.l1 = q.x & 0xffff; g.l2 = (uint32_t)q.x >> 16;
   g.l3 = q.y & 0xffff; g.l4 = (uint32_t)q.y >> 16;
-  load_coef<NTG, CLASS>(d, j, g);
+  load_coef<CLASS>(d, j, g);
   return g;
 }
 // The row of any element, with neighbour indices in place of tile places.
-template <bool NTG, bool CLASS>
+template <bool CLASS>
 __device__ __forceinline__ Geo load_geo_nbr(const RealDesc& d, const int j) {
   Geo g;
-  g.f = ldg<NTG>(gp(d.flags) + j);
-  const i4 q = ldg<NTG>((const SRS_GLOBAL i4*)d.nbr + j);
+  g.f = gp(d.flags)[j];
+  const i4 q = ((const SRS_GLOBAL i4*)d.nbr)[j];
   g.l1 = q.x; g.l2 = q.y; g.l3 = q.z; g.l4 = q.w;
-  load_coef<NTG, CLASS>(d, j, g);
+  load_coef<CLASS>(d, j, g);
   return g;
 }
 // The flags of the block of element j, j consecutive across the wavefront from
@@ -485,7 +492,8 @@ struct HostReal {
   double* d_br_own = nullptr;  // boundary rates rescaled to this realization's D (srs_params_set)
   srs_extensions ext{0, 0.0, 0.6};
   std::vector<int32_t> ryr_ele, ryr_jsr, ryr_nb, lcc_ele;  // dev numbering
-  std::vector<int32_t> celem, cstart, centry;
+  std::vector<int32_t> celem, cstart;
+  std::vector<ChanEntry> centry;
   int32_t ints[SRS_N_INT];
   double reals[SRS_N_REAL];
   uint64_t key = 0, stream = 0;
@@ -512,12 +520,10 @@ struct srs_ctx {
   int device = 0;
   int tile = 0;          // elements per k_sweep workgroup; 0: chosen by srs_ctx_finalize
   size_t sweep_lds = 0;  // LDS bytes of a sweep workgroup (staged quads)
-  // cache hints; -1: chosen by srs_ctx_finalize
-  int nt_geometry = -1;  // non-temporal loads of operator rows and halo lists
-  int nt_state = -1;     // non-temporal stores of the new state
+  int nt_state = -1;     // non-temporal stores of the new state; -1: chosen by srs_ctx_finalize
   int plane_pad = 0;     // extra elements per SoA plane
   int compact = 1;       // compress operator rows when a mesh allows it
-  int occ = 0;           // gated sweep's register budget: 0 compiler's choice, 6 or 8 wavefronts per SIMD
+  int occ = 0;           // gated sweep's register budget: 0 by size, else six wavefronts per SIMD
   int group = 1;         // realizations per realization group (1, 2 or 4)
   int drop_finished = 1; // sweep without the tiles of groups that have all finished
   int gated = 1;         // fold each step's gating into the next step's sweep (k_sweep_gated) where it applies

@@ -86,35 +86,24 @@ __device__ __forceinline__ size_t qat(const RealDesc& d, const int e) {
 __device__ __forceinline__ bool lives_tr(const uint8_t f) { return (f & (F_JSR | F_TROPC)) == F_TROPC; }
 __device__ __forceinline__ bool lives_cs(const uint8_t f) { return (f & F_JSR) != 0; }
 
-// Element j alone in its group, its neighbours read one by one (g holds their
-// indices).
-__device__ __forceinline__ Loc load_loc(const RealDesc& d, const SRS_GLOBAL double* __restrict__ Xo, const int j,
-                                        const Geo& g) {
-  const size_t np = d.np;
-  Loc c;
-  c.m0 = ld_quad(Xo, qidx1(j));
-  c.c_tr = lives_tr(g.f) ? Xo[4 * np + j] : 0.0;
-  c.c_cs = lives_cs(g.f) ? Xo[5 * np + j] : 0.0;
-  c.s = row_sum(g, c.m0, ld_quad(Xo, qidx1(g.l1)), ld_quad(Xo, qidx1(g.l2)), ld_quad(Xo, qidx1(g.l3)),
-                ld_quad(Xo, qidx1(g.l4)));
-  return c;
-}
+// An element's rates without the channel fluxes, and the divisor of the rapid
+// buffers (B, used where `div`).
+struct Rates {
+  double ca, dy, at, cm, tr, cs, B;
+  bool div;
+};
 
-// The fused step of one element of one realization, from its loaded row and
-// state, in the reference's operation order (cpu/RunSimulation.cpp:591-648).
-template <bool NTS, int FK, bool ONE>
-__device__ __forceinline__ void step_elem(const RealDesc& d, const RealLive& l, const Bufs bf, const int j,
-                                          const Geo& g, const Loc& c) {
-  const int K = ONE ? 1 : d.kst;
+// In the reference's operation order (cpu/RunSimulation.cpp:591-618).  ttj, v0j:
+// the TT area and volume of an element with F_SL.
+template <int FK>
+__device__ __forceinline__ Rates elem_rates(const RealDesc& d, const RealLive& l, const int j, const uint8_t flags,
+                                            const Loc& c, const double ttj, const double v0j) {
   const size_t np = d.np;
-  const SRS_GLOBAL double* __restrict__ Xo = bf.xo;
-  SRS_GLOBAL double* __restrict__ Xn = bf.xn;
   const double* P = d.P;
-  const double dt = P[SRS_R_T_STEP];
-  const uint8_t f = FK >= 0 ? (uint8_t)FK : g.f;
+  const uint8_t f = FK >= 0 ? (uint8_t)FK : flags;
   const double c_ca = c.m0.x, c_at = c.m0.y, c_cm = c.m0.z, c_dy = c.m0.w;
   const double c_tr = c.c_tr, c_cs = c.c_cs;
-  const bool live_tr = lives_tr(f), live_cs = lives_cs(f);
+  const bool live_cs = lives_cs(f);
 
   double br_ca = 0.0, br_dy = 0.0, br_at = 0.0, br_cm = 0.0;
   if (f & F_BR) {
@@ -127,42 +116,98 @@ __device__ __forceinline__ void step_elem(const RealDesc& d, const RealLive& l, 
   // cpu/RunSimulation.cpp:61-71 (Ca uses D_CA in both domains; with the jSR
   // diffusion extension, D_CAJSR in jSR elements)
   const double d_ca = (live_cs && d.jsr_diff) ? P[SRS_R_D_CA_JSR] : P[SRS_R_D_CA];
-  double rca = d_ca * c.s.x + br_ca;
-  double rdy = P[SRS_R_D_DYE] * c.s.w + br_dy;
-  double rat = P[SRS_R_D_ATP] * c.s.y + br_at;
-  double rcm = P[SRS_R_D_CMDN] * c.s.z + br_cm;
-  double rtr = 0, rcs = 0;
-  const double nsr = l.ca_nsr;
+  Rates r;
+  r.ca = d_ca * c.s.x + br_ca;
+  r.dy = P[SRS_R_D_DYE] * c.s.w + br_dy;
+  r.at = P[SRS_R_D_ATP] * c.s.y + br_at;
+  r.cm = P[SRS_R_D_CMDN] * c.s.z + br_cm;
+  r.tr = r.cs = 0.0;
 
   if (!(f & F_JSR)) {
     if (f & F_TROPC) {  // :75-91
-      const double r = P[SRS_R_K_ON_TRPN] * (P[SRS_R_B_TOT_TRPN] - c_tr) * c_ca - P[SRS_R_K_OFF_TRPN] * c_tr;
-      rca += -r;
-      rtr = r;
+      const double q = P[SRS_R_K_ON_TRPN] * (P[SRS_R_B_TOT_TRPN] - c_tr) * c_ca - P[SRS_R_K_OFF_TRPN] * c_tr;
+      r.ca += -q;
+      r.tr = q;
       double K_i = c_ca / P[SRS_R_K_D_I];
       K_i = K_i * K_i;
       const double D_cycle = l.serca[0] + K_i * l.serca[1] + K_i * K_i * l.serca[2];
       const double v_cycle = (K_i * K_i * 3.24873e12 + K_i * l.serca[3] - l.serca[4]) / D_cycle;
-      const double d_ca = (2e-3) * v_cycle * P[SRS_R_A_P];
-      rca -= d_ca;
+      const double d_serca = (2e-3) * v_cycle * P[SRS_R_A_P];
+      r.ca -= d_serca;
     }
-    double r = P[SRS_R_K_ON_DYE] * (P[SRS_R_B_TOT_DYE] - c_dy) * c_ca - P[SRS_R_K_OFF_DYE] * c_dy;
-    rca += -r;
-    rdy += r;
-    r = P[SRS_R_K_ON_ATP] * (P[SRS_R_B_TOT_ATP] - c_at) * c_ca - P[SRS_R_K_OFF_ATP] * c_at;
-    rca += -r;
-    rat += r;
-    r = P[SRS_R_K_ON_CMDN] * (P[SRS_R_B_TOT_CMDN] - c_cm) * c_ca - P[SRS_R_K_OFF_CMDN] * c_cm;
-    rca += -r;
-    rcm += r;
+    double q = P[SRS_R_K_ON_DYE] * (P[SRS_R_B_TOT_DYE] - c_dy) * c_ca - P[SRS_R_K_OFF_DYE] * c_dy;
+    r.ca += -q;
+    r.dy += q;
+    q = P[SRS_R_K_ON_ATP] * (P[SRS_R_B_TOT_ATP] - c_at) * c_ca - P[SRS_R_K_OFF_ATP] * c_at;
+    r.ca += -q;
+    r.at += q;
+    q = P[SRS_R_K_ON_CMDN] * (P[SRS_R_B_TOT_CMDN] - c_cm) * c_ca - P[SRS_R_K_OFF_CMDN] * c_cm;
+    r.ca += -q;
+    r.cm += q;
   } else {  // :113-121
-    const double r = P[SRS_R_K_ON_CSQN] * (P[SRS_R_B_T_JSR] - c_cs) * c_ca - P[SRS_R_K_OFF_CSQN] * c_cs;
-    rca += -r;
-    rcs = r;
-    rca += (nsr - c_ca) * P[SRS_R_V_REFILL];
+    const double q = P[SRS_R_K_ON_CSQN] * (P[SRS_R_B_T_JSR] - c_cs) * c_ca - P[SRS_R_K_OFF_CSQN] * c_cs;
+    r.ca += -q;
+    r.cs = q;
+    r.ca += (l.ca_nsr - c_ca) * P[SRS_R_V_REFILL];
   }
 
-  if (f & F_CHAN) {  // :619-632, contributions in the reference's channel order
+  // SR-site rapid buffer of the cytosol (extension; b_sr == 0 in the reference model)
+  const bool sr = !live_cs && d.b_sr != 0.0;
+  r.B = 1.0;
+  r.div = (f & F_SL) || sr;
+  if (r.div) {
+    if (f & F_SL) {  // :15-22; B == 1 exactly where the TT area is zero
+      const double btothi = ttj * P[SRS_R_B_TOT_SL_HI] / (v0j * (1e-15));
+      const double btotlo = ttj * P[SRS_R_B_TOT_SL_LO] / (v0j * (1e-15));
+      const double kh = P[SRS_R_K_D_SL_HI], kl = P[SRS_R_K_D_SL_LO];
+      r.B = 1 + (btothi * kh / ((kh + c_ca) * (kh + c_ca))) + (btotlo * kl / ((kl + c_ca) * (kl + c_ca)));
+    }
+    if (sr) r.B = r.B + d.b_sr * d.k_sr / ((d.k_sr + c_ca) * (d.k_sr + c_ca));
+  }
+  return r;
+}
+
+// Adds one channel's flux to an element's Ca rate (cpu/RunSimulation.cpp:619-632).
+// dc: Ca of a RyR's jSR element less its cleft element's.
+__device__ __forceinline__ void chan_flux(const RealDesc& d, const RealLive& l, const int code, const bool ryr_open,
+                                          const double dc, const double c_ca, const double v0, double& rca) {
+  const double* P = d.P;
+  if (code >= 0) {
+    if (ryr_open) {
+      const double J = P[SRS_R_V_RYR] * dc * P[SRS_R_V_CELL];
+      if (code & 1) rca -= J / v0; else rca += J / v0;
+    }
+  } else {
+    const int i = -code - 1;
+    if (srs_lcc_open(d.lcc_state[i], d.lccv_state[i])) rca += srs_lcc_flux_raw(l.vm, c_ca, P[SRS_R_CA_0]) / v0;
+  }
+}
+
+// Division by the rapid buffers and forward Euler (:633-644).
+template <bool NTS, int FK, bool ONE>
+__device__ __forceinline__ void elem_store(const RealDesc& d, const Bufs bf, const int j, const uint8_t flags,
+                                           const Loc& c, const Rates& r) {
+  const int K = ONE ? 1 : d.kst;
+  const size_t np = d.np, q = ONE ? (size_t)j : gidx(j, K, d.slot);
+  const uint8_t f = FK >= 0 ? (uint8_t)FK : flags;
+  const double dt = d.P[SRS_R_T_STEP];
+  SRS_GLOBAL double* __restrict__ Xn = bf.xn;
+  const double rca = r.div ? r.ca / r.B : r.ca;
+  st_quad<NTS>(Xn, qat<ONE>(d, j),
+               d4{c.m0.x + rca * dt, c.m0.y + r.at * dt, c.m0.z + r.cm * dt, c.m0.w + r.dy * dt});
+  if (lives_tr(f)) stg<NTS>(Xn + 4 * K * np + q, c.c_tr + r.tr * dt);
+  if (lives_cs(f)) stg<NTS>(Xn + 5 * K * np + q, c.c_cs + r.cs * dt);
+}
+
+// The fused step of one element of one realization, from its loaded row and
+// state, in the reference's operation order (cpu/RunSimulation.cpp:591-648).
+template <bool NTS, int FK, bool ONE>
+__device__ __forceinline__ void step_elem(const RealDesc& d, const RealLive& l, const Bufs bf, const int j,
+                                          const uint8_t flags, const Loc& c) {
+  const uint8_t f = FK >= 0 ? (uint8_t)FK : flags;
+  const bool sl = (f & F_SL) != 0;
+  Rates r = elem_rates<FK>(d, l, j, f, c, sl ? gp(d.tt)[j] : 0.0, sl ? gp(d.V0)[j] : 1.0);
+  if (f & F_CHAN) {  // contributions in the reference's channel order
     int lo = 0, hi = d.n_celem;
     while (lo < hi) {
       const int mid = (lo + hi) >> 1;
@@ -171,43 +216,14 @@ __device__ __forceinline__ void step_elem(const RealDesc& d, const RealLive& l, 
     if (lo < d.n_celem && d.celem[lo] == j) {
       const double v0 = d.V0[j];
       for (int e = d.cstart[lo]; e < d.cstart[lo + 1]; ++e) {
-        const int ch = d.centry[e];
-        if (ch >= 0) {
-          const int i = ch >> 1;
-          if (d.ryr_state[i]) {
-            const double J = P[SRS_R_V_RYR] * (Xo[2 * qat<ONE>(d, d.ryr_jsr[i])] -
-                                               Xo[2 * qat<ONE>(d, d.ryr_ele[i])]) * P[SRS_R_V_CELL];
-            if (ch & 1) rca -= J / v0; else rca += J / v0;
-          }
-        } else {
-          const int i = -ch - 1;
-          if (srs_lcc_open(d.lcc_state[i], d.lccv_state[i])) rca += srs_lcc_flux_raw(l.vm, c_ca, P[SRS_R_CA_0]) / v0;
-        }
+        const ChanEntry en = d.centry[e];
+        const bool open = en.code >= 0 && d.ryr_state[en.code >> 1];
+        const double dc = open ? bf.xo[2 * qat<ONE>(d, en.jsr)] - bf.xo[2 * qat<ONE>(d, en.cyt)] : 0.0;
+        chan_flux(d, l, en.code, open, dc, c.m0.x, v0, r.ca);
       }
     }
   }
-
-  // SR-site rapid buffer of the cytosol (extension; b_sr == 0 in the reference model)
-  const bool sr = !live_cs && d.b_sr != 0.0;
-  if ((f & F_SL) || sr) {
-    double B = 1.0;
-    if (f & F_SL) {  // :15-22; B == 1 exactly where the TT area is zero
-      const double ttj = gp(d.tt)[j], v0j = gp(d.V0)[j];
-      const double btothi = ttj * P[SRS_R_B_TOT_SL_HI] / (v0j * (1e-15));
-      const double btotlo = ttj * P[SRS_R_B_TOT_SL_LO] / (v0j * (1e-15));
-      const double kh = P[SRS_R_K_D_SL_HI], kl = P[SRS_R_K_D_SL_LO];
-      B = 1 + (btothi * kh / ((kh + c_ca) * (kh + c_ca))) + (btotlo * kl / ((kl + c_ca) * (kl + c_ca)));
-    }
-    if (sr) B = B + d.b_sr * d.k_sr / ((d.k_sr + c_ca) * (d.k_sr + c_ca));
-    rca /= B;
-  }
-
-  // :640-644 forward Euler
-  const d4 mn = {c_ca + rca * dt, c_at + rat * dt, c_cm + rcm * dt, c_dy + rdy * dt};
-  const size_t q = ONE ? (size_t)j : gidx(j, K, d.slot);
-  st_quad<NTS>(Xn, qat<ONE>(d, j), mn);
-  if (live_tr) stg<NTS>(Xn + 4 * K * np + q, c_tr + rtr * dt);
-  if (live_cs) stg<NTS>(Xn + 5 * K * np + q, c_cs + rcs * dt);
+  elem_store<NTS, FK, ONE>(d, bf, j, f, c, r);
 }
 
 // The sizes and mesh pointers of a tile's rows and halo, folded for scalars_here.
@@ -234,16 +250,16 @@ extern __shared__ double dyn_lds[];
 // A wavefront whose elements are all plain cytosol with troponin (the bulk of
 // a mesh, known from its block's flags) runs the specialisation with the flags
 // known at compile time.  KG: the realization's group size, s its slot.
-template <int BS, bool NTG, bool NTS, bool CLASS, int KG, bool SKIP_CHAN>
+template <int BS, bool NTS, bool CLASS, int KG, bool SKIP_CHAN>
 __device__ __forceinline__ void sweep_tile(const RealDesc& d, const RealLive& l, const Bufs bf, const int s,
                                            const int t) {
   const QuadTile tq(dyn_lds, d.qcap);
-  const Halo h = load_halo<BS, NTG>(d.hal, d.hoff, t);
+  const Halo h = load_halo<BS>(d.hal, d.hoff, t);
   const int j = t * BS + (int)threadIdx.x;
   // rows and states are padded to whole tiles, so the last tile's lanes past
   // the mesh load (and discard) zeros
   const uint32_t b = block_flags(d, j);
-  const Geo g = load_geo<NTG, CLASS>(d, d.loc, j, b);
+  const Geo g = load_geo<CLASS>(d, d.loc, j, b);
   const SRS_GLOBAL double* Xo = bf.xo;
   const size_t np = d.np, pl = 4 * KG * np + (KG > 1 ? gidx(j, KG, s) : (size_t)j);
   auto quad = [&](int e) { return ld_quad(Xo, KG > 1 ? qidx(e, KG, s) : (size_t)qidx1(e)); };
@@ -261,18 +277,18 @@ __device__ __forceinline__ void sweep_tile(const RealDesc& d, const RealLive& l,
   if (j >= d.n || (SKIP_CHAN && (g.f & F_CHAN))) return;
   c.s = row_sum(g, c.m0, tq.get(g.l1), tq.get(g.l2), tq.get(g.l3), tq.get(g.l4));
   if (b & BLK_PLAIN) {
-    step_elem<NTS, F_TROPC, KG == 1>(d, l, bf, j, g, c);
+    step_elem<NTS, F_TROPC, KG == 1>(d, l, bf, j, g.f, c);
   } else {
     if (!lives_tr(g.f)) c.c_tr = 0.0;
     c.c_cs = lives_cs(g.f) ? Xo[pl + KG * np] : 0.0;
-    step_elem<NTS, -1, KG == 1>(d, l, bf, j, g, c);
+    step_elem<NTS, -1, KG == 1>(d, l, bf, j, g.f, c);
   }
 }
 
 // Workgroup b of a context with groups of KG takes slot b % KG of tile b / KG,
 // so that the slots' workgroups, which read the same rows and halo lists, run
 // side by side on one XCD.
-template <int BS, bool NTG, bool NTS, bool CLASS, int KG>
+template <int BS, bool NTS, bool CLASS, int KG>
 __device__ __forceinline__ void sweep(const RealDesc* __restrict__ D, const RealLive* __restrict__ L,
                                       const int2* __restrict__ tiles, int n_tiles, const int* __restrict__ groups,
                                       int single) {
@@ -290,14 +306,14 @@ __device__ __forceinline__ void sweep(const RealDesc* __restrict__ D, const Real
   const Bufs bf = bufs(d.X[0], d.X[1], l.cur);
   scalars_here(fold(skip, bf.xo, bf.xn) ^ geo_fold<CLASS>(d));
   if (skip) return;
-  sweep_tile<BS, NTG, NTS, CLASS, KG, false>(d, l, bf, s, tl.y);
+  sweep_tile<BS, NTS, CLASS, KG, false>(d, l, bf, s, tl.y);
 }
 
-template <int BS, bool NTG, bool NTS, bool CLASS, int KG>
+template <int BS, bool NTS, bool CLASS, int KG>
 __global__ __launch_bounds__(BS) void k_sweep(const RealDesc* __restrict__ D, const RealLive* __restrict__ L,
                                               const int2* __restrict__ tiles, int n_tiles,
                                               const int* __restrict__ groups, int single) {
-  sweep<BS, NTG, NTS, CLASS, KG>(D, L, tiles, n_tiles, groups, single);
+  sweep<BS, NTS, CLASS, KG>(D, L, tiles, n_tiles, groups, single);
 }
 
 __device__ void write_record(const RealDesc& d, RealLive& l, const double* Ca, double t) {
@@ -339,19 +355,17 @@ __device__ void write_record(const RealDesc& d, RealLive& l, const double* Ca, d
 }
 
 // The gating and loop body of realization r by one workgroup of NT threads.
-// LEAN loads each LCC's inputs when it is updated rather than with the RyRs'
-// before the first barrier: one more memory round trip, fewer live registers.
 // PROTO = false leaves out the loop body (callers that never pass G_PROTOCOL).
-// smem: GATE_LDS bytes.
-constexpr size_t GATE_LDS = 3 * MAX_RYR * sizeof(int);
-template <int NT, bool LEAN = false, bool PROTO = true>
+// smem: GATE_LDS bytes; its last MAX_RYR ints end as the RyR states.
+constexpr size_t GATE_LDS = 4 * MAX_RYR * sizeof(int);
+template <int NT, bool PROTO = true>
 __device__ __forceinline__ void gate_workgroup(const RealDesc* __restrict__ D, RealLive* __restrict__ L, const int r,
                                                const uint32_t mode, int* smem) {
   static_assert(MAX_RYR % NT == 0 && MAX_LCC % NT == 0, "channel slots per thread");
   const RealDesc& d = D[r];
   RealLive& l = L[r];
   if (l.done) return;
-  int *s_old = smem, *s_a = smem + MAX_RYR, *s_b = smem + 2 * MAX_RYR;
+  int *s_old = smem, *s_a = smem + MAX_RYR, *s_b = smem + 2 * MAX_RYR, *s_fin = smem + 3 * MAX_RYR;
   const int tid = threadIdx.x;
   const int cur = l.cur;
   // In the flag_ffwd phase the sweep skipped this realization: the fields are
@@ -374,38 +388,29 @@ __device__ __forceinline__ void gate_workgroup(const RealDesc* __restrict__ D, R
 
   if (gating) {
     // Everything a channel's update reads is loaded before the first barrier
-    // (RyR i by thread i mod 256, LCC i by thread 255 - i mod 256, so RyRs
-    // and LCCs are updated side by side), leaving one memory round trip in
-    // front of the arithmetic.
-    constexpr int RPT = MAX_RYR / NT, LPT = MAX_LCC / NT;
-    double ca_c[RPT], ca_j[RPT], Rr[RPT];
-#pragma unroll
-    for (int k = 0; k < RPT; ++k) {
-      const int i = tid + k * NT;
-      if (i < nr) {
-        const int so = d.ryr_state[i];
-        s_old[i] = so;
-        s_a[i] = so;
-        ca_c[k] = Ca[cq(d, d.ryr_ele[i])];
-        ca_j[k] = Ca[cq(d, d.ryr_jsr[i])];
-        Rr[k] = d.R[i];
-      }
-    }
-    int ls[LPT], lvs[LPT];
-    double ca_l[LPT], Rl[LPT];
-    auto load_lcc = [&](const int k) {
-      const int i = (NT - 1 - tid) + k * NT;
-      if (i < d.n_lcc) {
-        ls[k] = d.lcc_state[i];
-        lvs[k] = d.lccv_state[i];
-        ca_l[k] = Ca[cq(d, d.lcc_ele[i])];
-        Rl[k] = d.R[nr + i];
-      }
+    // (RyR i by thread i mod NT, LCC i by thread NT - 1 - i mod NT, so RyRs and
+    // LCCs are updated side by side), leaving one memory round trip in front
+    // of the arithmetic.  Channels beyond the workgroup's threads are loaded
+    // when their turn comes: holding two of each per thread cost the kernel
+    // this is folded into half of its registers.
+    double ca_c = 0.0, ca_j = 0.0, Rr = 0.0;
+    auto load_ryr = [&](const int i) {
+      ca_c = Ca[cq(d, d.ryr_ele[i])];
+      ca_j = Ca[cq(d, d.ryr_jsr[i])];
+      Rr = d.R[i];
     };
-    if constexpr (!LEAN) {
-#pragma unroll
-      for (int k = 0; k < LPT; ++k) load_lcc(k);
-    }
+    for (int i = tid; i < nr; i += NT) s_old[i] = s_a[i] = d.ryr_state[i];
+    if (tid < nr) load_ryr(tid);
+    int ls = 0, lvs = 0;
+    double ca_l = 0.0, Rl = 0.0;
+    auto load_lcc = [&](const int i) {
+      ls = d.lcc_state[i];
+      lvs = d.lccv_state[i];
+      ca_l = Ca[cq(d, d.lcc_ele[i])];
+      Rl = d.R[nr + i];
+    };
+    const int l0 = NT - 1 - tid;
+    if (l0 < d.n_lcc) load_lcc(l0);
     __syncthreads();
     // RyRs: the reference updates them one after another (later RyRs see
     // earlier flips through the neighbour counts, cpu/RunSimulation.cpp:661-666).
@@ -418,10 +423,9 @@ __device__ __forceinline__ void gate_workgroup(const RealDesc* __restrict__ D, R
     if (coupled) {
       for (int it = 0; it <= nr; ++it) {
         int changed = 0;
-#pragma unroll
-        for (int k = 0; k < RPT; ++k) {
-          const int i = tid + k * NT;
-          if (i >= nr) continue;
+#pragma unroll 1
+        for (int i = tid; i < nr; i += NT) {
+          if (nr > NT) load_ryr(i);
           int no = 0, ncl = 0;
           for (int q = 0; q < 4; ++q) {
             const int nb = d.ryr_nb[4 * i + q];
@@ -430,8 +434,8 @@ __device__ __forceinline__ void gate_workgroup(const RealDesc* __restrict__ D, R
               if (s) no++; else ncl++;
             }
           }
-          const double rate = srs_ryr_rate(s_old[i], no, ncl, ca_c[k], ca_j[k], P);
-          const double Rn = Rr[k] + rate * dt;
+          const double rate = srs_ryr_rate(s_old[i], no, ncl, ca_c, ca_j, P);
+          const double Rn = Rr + rate * dt;
           const int ns = (Rn > 0) ? (s_old[i] == 1 ? 0 : 1) : s_old[i];
           next[i] = ns;
           changed |= (ns != prev[i]);
@@ -443,10 +447,9 @@ __device__ __forceinline__ void gate_workgroup(const RealDesc* __restrict__ D, R
     }
     // Commit with neighbour states from the fixed point (for uncoupled RyRs
     // the neighbour counts do not enter the rate, A* = 0 gives X = 1).
-#pragma unroll
-    for (int k = 0; k < RPT; ++k) {
-      const int i = tid + k * NT;
-      if (i >= nr) continue;
+#pragma unroll 1
+    for (int i = tid; i < nr; i += NT) {
+      if (nr > NT) load_ryr(i);
       int no = 0, ncl = 0;
       if (coupled) {
         for (int q = 0; q < 4; ++q) {
@@ -457,8 +460,8 @@ __device__ __forceinline__ void gate_workgroup(const RealDesc* __restrict__ D, R
           }
         }
       }
-      const double rate = srs_ryr_rate(s_old[i], no, ncl, ca_c[k], ca_j[k], P);
-      double Rn = Rr[k] + rate * dt;
+      const double rate = srs_ryr_rate(s_old[i], no, ncl, ca_c, ca_j, P);
+      double Rn = Rr + rate * dt;
       int ns = s_old[i];
       if (Rn > 0) {
         uint64_t o[4];
@@ -468,19 +471,18 @@ __device__ __forceinline__ void gate_workgroup(const RealDesc* __restrict__ D, R
       }
       d.R[i] = Rn;
       d.ryr_state[i] = ns;
+      s_fin[i] = ns;
     }
     // LCCs, cpu/RunSimulation.cpp:229-400
-#pragma unroll
-    for (int k = 0; k < LPT; ++k) {
-      const int i = (NT - 1 - tid) + k * NT;
-      if (i >= d.n_lcc) continue;
-      if constexpr (LEAN) load_lcc(k);
-      const int s = ls[k], vs = lvs[k];
+#pragma unroll 1
+    for (int i = l0; i < d.n_lcc; i += NT) {
+      if (i != l0) load_lcc(i);
+      const int s = ls, vs = lvs;
       double tr[3];
       int32_t tg[3];
-      const double lr = srs_lcc_rates(s, vs, l.vm, ca_l[k], tr, tg);
+      const double lr = srs_lcc_rates(s, vs, l.vm, ca_l, tr, tg);
       const int ic = nr + i;
-      double Rn = Rl[k] + (tr[0] + tr[1] + tr[2] + lr) * dt;
+      double Rn = Rl + (tr[0] + tr[1] + tr[2] + lr) * dt;
       if (Rn > 0) {
         uint64_t o[4];
         srs_philox4x64_10((uint64_t)step, (uint64_t)ic, d.stream, SRS_PURPOSE_GATING, d.key, SRS_PHILOX_KEY1, o);
@@ -494,12 +496,15 @@ __device__ __forceinline__ void gate_workgroup(const RealDesc* __restrict__ D, R
       d.R[ic] = Rn;
     }
   }
+  else {
+    for (int i = tid; i < nr; i += NT) s_fin[i] = d.ryr_state[i];
+  }
   __syncthreads();
 
   if (mode & G_REPLAY) {
     const int64_t k = step + 1 - l.sched_base;  // schedule row of the next step
     if (k < d.n_sched)
-      for (int i = tid; i < nr; i += NT) d.ryr_state[i] = d.sched[k * nr + i];
+      for (int i = tid; i < nr; i += NT) s_fin[i] = d.ryr_state[i] = d.sched[k * nr + i];
   }
 
   const double iv = P[SRS_R_OUTPUT_STATES_INTERVAL];
@@ -585,7 +590,7 @@ __device__ __forceinline__ void gate_workgroup(const RealDesc* __restrict__ D, R
   if (d.I[SRS_I_FLAG_V_CLAMP]) l.vm = (t <= P[SRS_R_T_CLAMP]) ? P[SRS_R_V_CLAMP] : P[SRS_R_DEFAULT_VM];  // :531-537
   const int ir = d.I[SRS_I_INIT_RYR];
   if (ir != -1 && t < P[SRS_R_INIT_RYR_HOLD] && !d.ryr_state[ir]) {  // :540-542
-    d.ryr_state[ir] = 1;
+    d.ryr_state[ir] = s_fin[ir] = 1;
     ++n_open_all;  // counted closed above
   }
   if (out_due) {  // :552-566
@@ -598,13 +603,13 @@ __device__ __forceinline__ void gate_workgroup(const RealDesc* __restrict__ D, R
 #if SRS_UNIT == 0
 __global__ __launch_bounds__(GATE_THREADS) void k_gate(const RealDesc* __restrict__ D, RealLive* __restrict__ L,
                                                        uint32_t mode) {
-  __shared__ int smem[3 * MAX_RYR];
+  __shared__ int smem[4 * MAX_RYR];
   gate_workgroup<GATE_THREADS>(D, L, blockIdx.x, mode, smem);
 }
 // The gating of the realizations of a list (one subset of the context).
 __global__ __launch_bounds__(GATE_THREADS) void k_gate_list(const RealDesc* __restrict__ D, RealLive* __restrict__ L,
                                                             const int32_t* __restrict__ rids, uint32_t mode) {
-  __shared__ int smem[3 * MAX_RYR];
+  __shared__ int smem[4 * MAX_RYR];
   gate_workgroup<GATE_THREADS>(D, L, rids[blockIdx.x], mode, smem);
 }
 #endif
@@ -627,7 +632,7 @@ __global__ __launch_bounds__(GATE_THREADS) void k_gate_list(const RealDesc* __re
 // reverse order when the index is 1 (alternate steps), so that a step first
 // reads the tiles the step before wrote last, while they may still be in the
 // last-level cache.  The order changes no result.
-template <int BS, bool NTG, bool NTS, bool CLASS, bool LEAN, bool PROTO>
+template <int BS, bool NTS, bool CLASS, bool PROTO, bool PRE>
 __device__ __forceinline__ void sweep_gated(const RealDesc* __restrict__ D, RealLive* __restrict__ L, int n_tiles,
                                             int curx, uint32_t gmode, const double* xo_at, double* xn_at) {
   const int cur = curx & 1;
@@ -642,42 +647,77 @@ __device__ __forceinline__ void sweep_gated(const RealDesc* __restrict__ D, Real
   const Bufs bf = xo_at ? Bufs{gp(xo_at), gpw(xn_at)} : bufs(d.X[0], d.X[1], cur);
   scalars_here(fold(skip, bf.xo, bf.xn) ^ geo_fold<CLASS>(d));
   if (b == 0) {
-    if (gmode) gate_workgroup<BS, LEAN, PROTO>(D, L, 0, gmode, (int*)dyn_lds);
+    // The channel elements: all that does not depend on the gating (every
+    // species but Ca, and Ca's rate without the fluxes) is loaded, computed and
+    // stored before it, by wavefronts that mostly gate no channel, so that its
+    // memory round trips run beside the gating's; a channel-flux element is one
+    // record instead of a search and six tables.  This workgroup's chain of
+    // loads was the step of a small mesh: 9.2 -> 6.5 us on 56,250 elements,
+    // 10.1 -> 7.8 on 172,494.
+    int* s_fin = (int*)dyn_lds + 3 * MAX_RYR;
+    constexpr int FIRST = BS / 4;  // the thread of channel element 0
+    struct Pending { double rca, ca, B, dc, v0; int code, j, e0, e1; };
+    auto fetch = [&](int k) -> Pending {
+      const ChanElem* r = d.crec + k;
+      const SRS_GLOBAL double* Xo = bf.xo;
+      const uint8_t f = (uint8_t)r->f;
+      const size_t np = d.np;
+      Pending p;
+      p.j = r->j;
+      p.e0 = r->e0;
+      p.e1 = r->e1;
+      p.v0 = r->v0;
+      const ChanEntry en = d.centry[p.e0];
+      p.code = en.code;
+      Loc c;
+      c.m0 = ld_quad(Xo, qidx1(p.j));
+      const d4 m1 = ld_quad(Xo, qidx1(r->nb[0])), m2 = ld_quad(Xo, qidx1(r->nb[1]));
+      const d4 m3 = ld_quad(Xo, qidx1(r->nb[2])), m4 = ld_quad(Xo, qidx1(r->nb[3]));
+      c.c_tr = lives_tr(f) ? Xo[4 * np + p.j] : 0.0;
+      c.c_cs = lives_cs(f) ? Xo[5 * np + p.j] : 0.0;
+      p.dc = en.code >= 0 ? Xo[2 * (size_t)qidx1(en.jsr)] - Xo[2 * (size_t)qidx1(en.cyt)] : 0.0;
+      c.s = c.m0 * r->a[0] + m1 * r->a[1] + m2 * r->a[2] + m3 * r->a[3] + m4 * r->a[4];
+      const Rates q = elem_rates<-1>(d, l, p.j, f, c, r->tt, p.v0);
+      elem_store<NTS, -1, true>(d, bf, p.j, f, c, q);  // Ca without its fluxes: replaced by finish
+      p.rca = q.ca;
+      p.ca = c.m0.x;
+      p.B = q.B;  // 1 where nothing divides
+      return p;
+    };
+    auto finish = [&](const Pending& p) {
+      double rca = p.rca;
+      chan_flux(d, l, p.code, p.code >= 0 && s_fin[p.code >> 1], p.dc, p.ca, p.v0, rca);
+      for (int i = p.e0 + 1; i < p.e1; ++i) {
+        const ChanEntry en = d.centry[i];
+        const bool open = en.code >= 0 && s_fin[en.code >> 1];
+        const double dc =
+            open ? bf.xo[2 * (size_t)qidx1(en.jsr)] - bf.xo[2 * (size_t)qidx1(en.cyt)] : 0.0;
+        chan_flux(d, l, en.code, open, dc, p.ca, p.v0, rca);
+      }
+      rca /= p.B;
+      bf.xn[2 * (size_t)qidx1(p.j)] = p.ca + rca * d.P[SRS_R_T_STEP];
+    };
+    const int k0 = ((int)threadIdx.x + BS - FIRST) % BS;
+    Pending p0;
+    if (PRE && !skip && k0 < d.n_celem) p0 = fetch(k0);
+    if (gmode) gate_workgroup<BS, PROTO>(D, L, 0, gmode, (int*)dyn_lds);
+    else
+      for (int i = threadIdx.x; i < d.n_ryr; i += BS) s_fin[i] = d.ryr_state[i];
     __syncthreads();  // the new channel states, written by this workgroup, before the flux reads them
     if (skip) return;
-    for (int k = threadIdx.x; k < d.n_celem; k += BS) {
-      const int j = gp(d.celem)[k];
-      const Geo g = load_geo_nbr<NTG, CLASS>(d, j);
-      const Loc c = load_loc(d, bf.xo, j, g);
-      step_elem<NTS, -1, true>(d, l, bf, j, g, c);
-    }
+    if (PRE && k0 < d.n_celem) finish(p0);
+    for (int k = PRE ? k0 + BS : k0; k < d.n_celem; k += BS) finish(fetch(k));
     return;
   }
   if (skip) return;
-  sweep_tile<BS, NTG, NTS, CLASS, 1, true>(d, l, bf, 0, b - 1);
+  sweep_tile<BS, NTS, CLASS, 1, true>(d, l, bf, 0, b - 1);
 }
-// Register budgets as for the sweep.  The gating workgroup's latency is on
-// the critical path of a small mesh's step, so the compiler's budget keeps
-// all of its loads in one round trip; with a budget the LCC loads wait for
-// the RyR update (LEAN), which is what lets the kernel fit 80 VGPRs.
-template <int BS, bool NTG, bool NTS, bool CLASS>
-__global__ __launch_bounds__(BS) void k_sweep_gated(const RealDesc* __restrict__ D, RealLive* __restrict__ L,
-                                                    int n_tiles, int cur, uint32_t gmode, const double* xo_at,
-                                                    double* xn_at) {
-  sweep_gated<BS, NTG, NTS, CLASS, false, false>(D, L, n_tiles, cur, gmode, xo_at, xn_at);
-}
-template <int BS, bool NTG, bool NTS, bool CLASS, int W>
-__global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W))) void k_sweep_gated_w(
+// W: the register budget, at least W wavefronts per SIMD.
+template <int BS, bool NTS, bool CLASS, bool PROTO, bool PRE, int W>
+__global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W))) void k_sweep_gated(
     const RealDesc* __restrict__ D, RealLive* __restrict__ L, int n_tiles, int cur, uint32_t gmode,
     const double* xo_at, double* xn_at) {
-  sweep_gated<BS, NTG, NTS, CLASS, true, false>(D, L, n_tiles, cur, gmode, xo_at, xn_at);
-}
-// with the loop body (SRS_STEP_PROTOCOL), compiler's register budget only
-template <int BS, bool NTG, bool NTS, bool CLASS>
-__global__ __launch_bounds__(BS) void k_sweep_gated_p(const RealDesc* __restrict__ D, RealLive* __restrict__ L,
-                                                      int n_tiles, int cur, uint32_t gmode, const double* xo_at,
-                                                      double* xn_at) {
-  sweep_gated<BS, NTG, NTS, CLASS, false, true>(D, L, n_tiles, cur, gmode, xo_at, xn_at);
+  sweep_gated<BS, NTS, CLASS, PROTO, PRE>(D, L, n_tiles, cur, gmode, xo_at, xn_at);
 }
 
 // ------------------------------------------------------------ kernel choice
@@ -693,19 +733,15 @@ template <int BS>
 GatedFn pick_gated_bs(const srs_ctx* c, bool proto);
 
 #if SRS_UNIT == 1
-// The sweep kernel for a tile size and cache hints.
 template <int BS, bool CMP, int KG>
-SweepFn pick_nt(int ntg, int nts) {
-  if (ntg) return nts ? k_sweep<BS, true, true, CMP, KG> : k_sweep<BS, true, false, CMP, KG>;
-  return nts ? k_sweep<BS, false, true, CMP, KG> : k_sweep<BS, false, false, CMP, KG>;
-}
+SweepFn pick_nt(int nts) { return nts ? k_sweep<BS, true, CMP, KG> : k_sweep<BS, false, CMP, KG>; }
 
 template <bool CMP, int KG>
 SweepFn pick_tile(const srs_ctx* c) {
   switch (c->tile) {
-    case 128: return pick_nt<128, CMP, KG>(c->nt_geometry, c->nt_state);
-    case 256: return pick_nt<256, CMP, KG>(c->nt_geometry, c->nt_state);
-    default: return pick_nt<512, CMP, KG>(c->nt_geometry, c->nt_state);
+    case 128: return pick_nt<128, CMP, KG>(c->nt_state);
+    case 256: return pick_nt<256, CMP, KG>(c->nt_state);
+    default: return pick_nt<512, CMP, KG>(c->nt_state);
   }
 }
 
@@ -718,33 +754,30 @@ SweepFn pick_sweep(const srs_ctx* c) {
 #endif  // SRS_UNIT == 1
 
 #if SRS_UNIT >= 2
-template <int BS, bool CMP, int W>
-GatedFn pick_gated_w(int ntg, int nts) {
-  if constexpr (W == 0) {
-    if (ntg) return nts ? k_sweep_gated<BS, true, true, CMP> : k_sweep_gated<BS, true, false, CMP>;
-    return nts ? k_sweep_gated<BS, false, true, CMP> : k_sweep_gated<BS, false, false, CMP>;
-  } else {
-    if (ntg) return nts ? k_sweep_gated_w<BS, true, true, CMP, W> : k_sweep_gated_w<BS, true, false, CMP, W>;
-    return nts ? k_sweep_gated_w<BS, false, true, CMP, W> : k_sweep_gated_w<BS, false, false, CMP, W>;
-  }
+template <int BS, bool CMP, bool PROTO, bool PRE, int W>
+GatedFn pick_gated_nt(int nts) {
+  return nts ? k_sweep_gated<BS, true, CMP, PROTO, PRE, W> : k_sweep_gated<BS, false, CMP, PROTO, PRE, W>;
 }
 
-template <int BS, bool CMP>
-GatedFn pick_gated_p(int ntg, int nts) {
-  if (ntg) return nts ? k_sweep_gated_p<BS, true, true, CMP> : k_sweep_gated_p<BS, true, false, CMP>;
-  return nts ? k_sweep_gated_p<BS, false, true, CMP> : k_sweep_gated_p<BS, false, false, CMP>;
-}
-
-template <int BS, bool CMP>
-GatedFn pick_gated_cmp(const srs_ctx* c, bool proto) {
-  if (proto) return pick_gated_p<BS, CMP>(c->nt_geometry, c->nt_state);
-  return c->occ == 6 ? pick_gated_w<BS, CMP, 6>(c->nt_geometry, c->nt_state)
-                     : pick_gated_w<BS, CMP, 0>(c->nt_geometry, c->nt_state);
+// How much the registers of the gating workgroup may cost the tiles.  With no
+// more tiles than CUs (256), each workgroup has a CU to itself: no budget
+// (56,250 elements: 6.5 us per step, 6.9 with four wavefronts per SIMD).  Up to
+// 900,000 elements the gating workgroup is still the longest one: four
+// wavefronts, with its loads ahead of the gating (400,000 elements: 12.5
+// against 17.0 us with six).  Beyond that the tiles' own wavefronts decide: six,
+// the gating's registers spilled and its channel elements loaded after it
+// (928k: 21.3 against 21.9 us; 1.6M: 29.4 / 31.1; 3M: 61.5 / 70.7).
+template <int BS, bool CMP, bool PROTO>
+GatedFn pick_gated_w(const srs_ctx* c) {
+  if (c->occ || (int64_t)c->n_tiles * BS >= 900000) return pick_gated_nt<BS, CMP, PROTO, false, 6>(c->nt_state);
+  return c->n_tiles <= 256 ? pick_gated_nt<BS, CMP, PROTO, true, 2>(c->nt_state)
+                           : pick_gated_nt<BS, CMP, PROTO, true, 4>(c->nt_state);
 }
 
 template <int BS>
 GatedFn pick_gated_bs(const srs_ctx* c, bool proto) {
-  return c->class_all ? pick_gated_cmp<BS, true>(c, proto) : pick_gated_cmp<BS, false>(c, proto);
+  if (c->class_all) return proto ? pick_gated_w<BS, true, true>(c) : pick_gated_w<BS, true, false>(c);
+  return proto ? pick_gated_w<BS, false, true>(c) : pick_gated_w<BS, false, false>(c);
 }
 // one tile size per unit: 128 in unit 2, 256 in unit 3, 512 in unit 4
 template GatedFn pick_gated_bs<SRS_UNIT == 2 ? 128 : SRS_UNIT == 3 ? 256 : 512>(const srs_ctx*, bool);
@@ -1180,9 +1213,7 @@ int srs_ctx_tune(srs_ctx* c, int32_t key, int32_t value) {
       c->compact = value != 0;
       return SRS_OK;
     // kernel keys: captured step graphs hold the old kernels, so they are dropped
-    case SRS_TUNE_NT_GEOMETRY:
-      c->nt_geometry = value != 0;
-      return c->finalized ? drop_graphs(c) : SRS_OK;
+    case SRS_TUNE_NT_GEOMETRY: return SRS_OK;  // rows are read through the caches
     case SRS_TUNE_OCCUPANCY:
       if (value != 0 && value != 6 && value != 8) return srs::fail(SRS_E_ARG, "occupancy must be 0, 6 or 8");
       c->occ = value;
@@ -1356,7 +1387,7 @@ int srs_ctx_add_realization(srs_ctx* c, int32_t mesh_id, const srs_chan_desc* ch
   memcpy(hr.reals, reals, sizeof(hr.reals));
   hr.key = seed_key;
   hr.stream = stream;
-  std::vector<std::pair<int32_t, int32_t>> entries;  // (dev element, code) in reference order
+  std::vector<std::pair<int32_t, ChanEntry>> entries;  // (dev element, channel) in reference order
   for (int i = 0; i < ch->n_ryr; ++i) {
     const int ce = ch->ryr_ele[i], je = ch->ryr_jsr[i];
     if (ce < 0 || ce >= hm.n || je < 0 || je >= hm.n) return srs::fail(SRS_E_ARG, "RyR %d element out of range", i);
@@ -1367,21 +1398,23 @@ int srs_ctx_add_realization(srs_ctx* c, int32_t mesh_id, const srs_chan_desc* ch
       if (nb >= ch->n_ryr || nb < -1) return srs::fail(SRS_E_ARG, "RyR %d neighbour %d out of range", i, nb);
       hr.ryr_nb.push_back(nb);
     }
-    entries.push_back({hm.inv[ce], 2 * i});
-    entries.push_back({hm.inv[je], 2 * i + 1});
+    entries.push_back({hm.inv[ce], {2 * i, hm.inv[je], hm.inv[ce], 0}});
+    entries.push_back({hm.inv[je], {2 * i + 1, hm.inv[je], hm.inv[ce], 0}});
   }
   for (int i = 0; i < ch->n_lcc; ++i) {
     const int e = ch->lcc_ele[i];
     if (e < 0 || e >= hm.n) return srs::fail(SRS_E_ARG, "LCC %d element out of range", i);
     hr.lcc_ele.push_back(hm.inv[e]);
-    entries.push_back({hm.inv[e], -(i + 1)});
+    entries.push_back({hm.inv[e], {-(i + 1), 0, 0, 0}});
   }
   if (ints[SRS_I_INIT_RYR] != -1 && (ints[SRS_I_INIT_RYR] < 0 || ints[SRS_I_INIT_RYR] >= ch->n_ryr))
     return srs::fail(SRS_E_ARG, "ryr_open_init %d must be -1 or in [0, %d)", ints[SRS_I_INIT_RYR], ch->n_ryr);
   if (ints[SRS_I_FLAG_LCC] && (ints[SRS_I_LCC_INDEX] < 0 || ints[SRS_I_LCC_INDEX] >= ch->n_lcc))
     return srs::fail(SRS_E_ARG, "LCC index %d out of range", ints[SRS_I_LCC_INDEX]);
   std::stable_sort(entries.begin(), entries.end(),
-                   [](const std::pair<int32_t, int32_t>& a, const std::pair<int32_t, int32_t>& b) { return a.first < b.first; });
+                   [](const std::pair<int32_t, ChanEntry>& a, const std::pair<int32_t, ChanEntry>& b) {
+                     return a.first < b.first;
+                   });
   for (size_t k = 0; k < entries.size(); ++k) {
     if (k == 0 || entries[k].first != entries[k - 1].first) {
       hr.celem.push_back(entries[k].first);
@@ -1510,7 +1543,22 @@ int srs_ctx_finalize(srs_ctx* c, int32_t record_capacity) {
     if ((rc = dev_upload(c, &p, hr.lcc_ele))) return rc; d.lcc_ele = p;
     if ((rc = dev_upload(c, &p, hr.celem))) return rc; d.celem = p;
     if ((rc = dev_upload(c, &p, hr.cstart))) return rc; d.cstart = p;
-    if ((rc = dev_upload(c, &p, hr.centry))) return rc; d.centry = p;
+    std::vector<ChanElem> crec(hr.celem.size());
+    for (size_t k = 0; k < crec.size(); ++k) {
+      ChanElem& e = crec[k];
+      e.j = hr.celem[k];
+      for (int q = 0; q < 5; ++q) e.a[q] = hm.coef[(size_t)q * hm.np + e.j];
+      for (int q = 0; q < 4; ++q) e.nb[q] = hm.nbr[4 * (size_t)e.j + q];
+      e.v0 = hm.V0[e.j];
+      e.tt = hm.tt[e.j];
+      e.e0 = hr.cstart[k];
+      e.e1 = hr.cstart[k + 1];
+      e.f = hm.flags[e.j];
+    }
+    ChanEntry* pe;
+    ChanElem* pc;
+    if ((rc = dev_upload(c, &pe, hr.centry))) return rc; d.centry = pe;
+    if ((rc = dev_upload(c, &pc, crec))) return rc; d.crec = pc;
     d.n_celem = (int32_t)hr.celem.size();
     std::vector<int32_t> zeros_r(d.n_ryr, 0), ones_l(d.n_lcc, 1), twos_l(d.n_lcc, 2);
     if ((rc = dev_upload(c, &p, zeros_r))) return rc; d.ryr_state = p;
@@ -1553,13 +1601,13 @@ int srs_ctx_finalize(srs_ctx* c, int32_t record_capacity) {
   // members in groups, 309 MB, 76.2 / 78.2 / 79.8).  Beyond it plain stores
   // evict what the next step could still have found (24 members, 351 MB, 78.6 /
   // 74.9 / 77.4; 3M-element dyad, 362 MB, 69.4 / 61.1 / 61.2; 48 members, 147 /
-  // 138 / 160).  The line lies between 309 and 351 MB.
+  // 138 / 160).  The line lies between 309 and 351 MB.  Row loads are never
+  // hinted: nowhere faster than the better of the other two.
   {
     double ws = 0.0;
     for (const HostReal& hr : c->reals) ws += 2.0 * 48.0 * c->meshes[hr.mesh]->n;
     for (auto& hmp : c->meshes) ws += (double)hmp->n * ((c->class_all ? 12 : 40) + 9) + 4.0 * hmp->map.n_halo;
     if (c->nt_state < 0) c->nt_state = ws > 330e6;
-    if (c->nt_geometry < 0) c->nt_geometry = 0;
   }
   c->n_tiles = (int)tiles.size();
   c->grid_sweep = (c->n_tiles * c->group + NXCD - 1) / NXCD * NXCD;
@@ -1825,8 +1873,7 @@ static int graph_gated(srs_ctx* c, int64_t block, int cur, uint32_t gmode, hipGr
 // state waits for the stream.
 static int gated_start(srs_ctx* c, uint32_t flags, bool* ok, int* cur) {
   *ok = false;
-  const int occ_max = (flags & SRS_STEP_PROTOCOL) ? 0 : 6;
-  if (!c->gated || c->reals.size() != 1 || c->group != 1 || c->occ > occ_max) return SRS_OK;
+  if (!c->gated || c->reals.size() != 1 || c->group != 1) return SRS_OK;
   RealLive lv;
   int rc = live_rw(c, 0, &lv, false);
   if (rc) return rc;

@@ -32,8 +32,10 @@ SRS_HD double srs_ryr_rate(int32_t state, int n_open, int n_closed, double ca_ss
     X = exp(0.5 * P[SRS_R_RYR_A_STAR] * (n_open * P[SRS_R_RYR_EPS_OO] - n_closed * P[SRS_R_RYR_EPS_CC]));
     rate = X * P[SRS_R_RYR_K_MINUS];
   } else {
-    double phi = (1.0 - pow(1000.0 / P[SRS_R_RYR_PHI_B], P[SRS_R_RYR_PHI_M])) +
-                 pow(ca_jsr / P[SRS_R_RYR_PHI_B], P[SRS_R_RYR_PHI_M]);
+    double phi = 1.0;  // what both powers give at an exponent of zero
+    if (P[SRS_R_RYR_PHI_M] != 0.0)
+      phi = (1.0 - pow(1000.0 / P[SRS_R_RYR_PHI_B], P[SRS_R_RYR_PHI_M])) +
+            pow(ca_jsr / P[SRS_R_RYR_PHI_B], P[SRS_R_RYR_PHI_M]);
     X = exp(0.5 * P[SRS_R_RYR_A_STAR] * (n_closed * P[SRS_R_RYR_EPS_CC] - n_open * P[SRS_R_RYR_EPS_OO]));
     rate = X * phi * P[SRS_R_RYR_K_PLUS] * pow(ca_ss, P[SRS_R_RYR_ETA]);
   }
