@@ -564,8 +564,9 @@ struct srs_ctx {
   bool tiles_compacted = false;
   int32_t* d_groups = nullptr;  // [n_groups][group] realization ids, -1 pads
   std::vector<int32_t> groups;
-  double* stage = nullptr;       // staging buffer of state transfers (state_xfer)
+  double* stage[2] = {};         // pinned buffers of state transfers (state_xfer), stage_len doubles each
   size_t stage_len = 0;
+  hipEvent_t ev_stage[2] = {};
   double last_total_ms = 0, last_sweep_ms = 0;
   // captured step blocks, keyed by (steps, gate mode)
   std::map<std::pair<int64_t, uint32_t>, hipGraphExec_t> graphs;

@@ -27,8 +27,10 @@
 #define SRS_UNIT 0
 #endif
 
+#include <atomic>
 #include <functional>
 #include <mutex>
+#include <thread>
 
 namespace srs_dev {
 
@@ -1099,23 +1101,99 @@ int tiles_compact(srs_ctx* c) {
 }
 
 
+// Host copies of a transfer's parts by several threads: one thread's copy into
+// fresh pages, not the link, bounded a transfer (15 GB/s).  The threads live
+// for one transfer; with none (too small a transfer, or none to be had) the
+// caller copies alone.
+class CopyTeam {
+ public:
+  explicit CopyTeam(int helpers) {
+    try {
+      for (int k = 0; k < helpers; ++k) th_.emplace_back([this, k] { work(k + 1); });
+    } catch (...) {  // fewer threads than asked for
+    }
+    n_ = (int)th_.size();
+  }
+  ~CopyTeam() {
+    stop_ = true;
+    go_.fetch_add(1, std::memory_order_release);
+    for (std::thread& t : th_) t.join();
+  }
+  CopyTeam(const CopyTeam&) = delete;
+  CopyTeam& operator=(const CopyTeam&) = delete;
+  void copy(void* dst, const void* src, size_t bytes) {
+    dst_ = (char*)dst;
+    src_ = (const char*)src;
+    bytes_ = bytes;
+    parts_ = n_ + 1;
+    left_.store(n_, std::memory_order_relaxed);
+    go_.fetch_add(1, std::memory_order_release);
+    slice(0);
+    while (left_.load(std::memory_order_acquire) > 0) std::this_thread::yield();
+  }
+
+ private:
+  void slice(int k) {
+    const size_t lo = bytes_ / 64 * k / parts_ * 64, hi = k + 1 == parts_ ? bytes_ : bytes_ / 64 * (k + 1) / parts_ * 64;
+    memcpy(dst_ + lo, src_ + lo, hi - lo);
+  }
+  void work(int k) {
+    for (unsigned seen = 0;;) {
+      unsigned g;
+      while ((g = go_.load(std::memory_order_acquire)) == seen) std::this_thread::yield();
+      seen = g;
+      if (stop_) return;
+      slice(k);
+      left_.fetch_sub(1, std::memory_order_release);
+    }
+  }
+  std::vector<std::thread> th_;
+  int n_ = 0, parts_ = 1;
+  std::atomic<unsigned> go_{0};
+  std::atomic<int> left_{0};
+  std::atomic<bool> stop_{false};
+  char* dst_ = nullptr;
+  const char* src_ = nullptr;
+  size_t bytes_ = 0;
+};
+
 // Copies one realization's fields between the caller's array ([6][n], reference
-// numbering) and its state buffers through the context's staging buffer, a
-// staging buffer's worth at a time; the reordering runs on the device.  On the
-// 3M-element dyad a host loop over the same elements, with its own 142 MB
-// copy of the fields, took 75 ms to read and 70 ms to set; this takes 9.4 and 5.4 ms
-// (0.51 and 0.34 ms against 0.21 and 0.13 ms on the 56,250-element spark box).
+// numbering) and its state buffers in parts, through two pinned host buffers
+// that the reordering kernel writes (or reads) over the link while the host
+// copies the part before.  On the 3M-element dyad a host loop over the same
+// elements, with its own 142 MB copy of the fields, took 75 ms to read and 70
+// ms to set; one device staging buffer and plain copies 9.4 and 5.4; this 4.3
+// and 3.2.
 int state_xfer(srs_ctx* c, int32_t r, double* host, bool to_dev) {
   const HostMesh& hm = *c->meshes[c->reals[r].mesh];
-  const size_t total = 6 * (size_t)hm.n;
-  for (size_t t0 = 0; t0 < total; t0 += c->stage_len) {
-    const size_t cnt = std::min(c->stage_len, total - t0);
-    if (to_dev) HIPCHK(hipMemcpy(c->stage, host + t0, cnt * sizeof(double), hipMemcpyHostToDevice));
-    hipLaunchKernelGGL(k_state_xfer, dim3((unsigned)((cnt + 255) / 256)), dim3(256), 0, c->stream, c->d_desc, c->d_live,
-                       r, hm.d_inv, c->stage, t0, cnt, to_dev ? 1 : 0);
+  const size_t total = 6 * (size_t)hm.n, part = c->stage_len;
+  const int n_parts = (int)((total + part - 1) / part);
+  // helper threads from 4 MB up (3M-element dyad, read: none 6.8 ms, one 4.6,
+  // three 4.3, five 4.4)
+  CopyTeam team(total >= (size_t)1 << 19 ? 3 : 0);
+  auto len = [&](int i) { return std::min(part, total - part * (size_t)i); };
+  auto launch = [&](int i) -> int {
+    hipLaunchKernelGGL(k_state_xfer, dim3((unsigned)((len(i) + 255) / 256)), dim3(256), 0, c->stream, c->d_desc,
+                       c->d_live, r, hm.d_inv, c->stage[i & 1], part * (size_t)i, len(i), to_dev ? 1 : 0);
     HIPCHK(hipGetLastError());
-    if (!to_dev) HIPCHK(hipMemcpyAsync(host + t0, c->stage, cnt * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(hipEventRecord(c->ev_stage[i & 1], c->stream));
+    return SRS_OK;
+  };
+  int rc;
+  if (to_dev) {
+    for (int i = 0; i < n_parts; ++i) {
+      if (i >= 2) HIPCHK(hipEventSynchronize(c->ev_stage[i & 1]));  // part i - 2 has left its buffer
+      team.copy(c->stage[i & 1], host + part * (size_t)i, len(i) * sizeof(double));
+      if ((rc = launch(i))) return rc;
+    }
     HIPCHK(hipStreamSynchronize(c->stream));
+    return SRS_OK;
+  }
+  if ((rc = launch(0))) return rc;
+  for (int i = 0; i < n_parts; ++i) {
+    if (i + 1 < n_parts && (rc = launch(i + 1))) return rc;
+    HIPCHK(hipEventSynchronize(c->ev_stage[i & 1]));
+    team.copy(host + part * (size_t)i, c->stage[i & 1], len(i) * sizeof(double));
   }
   return SRS_OK;
 }
@@ -1291,6 +1369,10 @@ int srs_ctx_destroy(srs_ctx* c) {
   (void)hipStreamSynchronize(c->stream);
   for (auto& kv : c->graphs) (void)hipGraphExecDestroy(kv.second);
   for (void* p : c->allocs) (void)hipFree(p);
+  for (int k = 0; k < 2; ++k) {
+    if (c->stage[k]) (void)hipHostFree(c->stage[k]);
+    if (c->ev_stage[k]) (void)hipEventDestroy(c->ev_stage[k]);
+  }
   (void)hipEventDestroy(c->ev0);
   (void)hipEventDestroy(c->ev1);
   (void)hipStreamDestroy(c->stream);
@@ -1611,11 +1693,14 @@ int srs_ctx_finalize(srs_ctx* c, int32_t record_capacity) {
   }
   c->n_tiles = (int)tiles.size();
   c->grid_sweep = (c->n_tiles * c->group + NXCD - 1) / NXCD * NXCD;
-  // the staging buffer of state transfers: the largest realization's fields,
-  // at most 32 MB (larger fields go through it in parts)
+  // state transfers: two pinned buffers of at most 8 MB (larger fields go
+  // through them in parts)
   for (const HostReal& hr : c->reals) c->stage_len = std::max(c->stage_len, 6 * (size_t)c->meshes[hr.mesh]->n);
-  c->stage_len = std::min(c->stage_len, (size_t)1 << 22);
-  if ((rc = dev_alloc(c, &c->stage, c->stage_len))) return rc;
+  c->stage_len = std::min(c->stage_len, (size_t)1 << 20);
+  for (int k = 0; k < 2; ++k) {
+    HIPCHK(hipHostMalloc((void**)&c->stage[k], c->stage_len * sizeof(double), hipHostMallocDefault));
+    HIPCHK(hipEventCreateWithFlags(&c->ev_stage[k], hipEventDisableTiming));
+  }
   if ((rc = dev_upload(c, &c->d_desc, descs))) return rc;
   if ((rc = dev_upload(c, &c->d_live, lives))) return rc;
   if ((rc = dev_upload(c, &c->d_tiles, tiles))) return rc;

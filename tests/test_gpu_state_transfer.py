@@ -1,6 +1,6 @@
-"""Field transfers between the caller's layout and the device's: the staging
-buffer holds 4,194,304 doubles, so fields of more than 699,050 elements cross
-it in parts."""
+"""Field transfers between the caller's layout and the device's: a pinned
+buffer holds 1,048,576 doubles, so fields of more than 174,762 elements cross
+in parts, through two buffers in turn."""
 from __future__ import annotations
 
 import numpy as np
@@ -16,7 +16,7 @@ pytestmark = pytest.mark.gpu
 def test_fields_come_back_as_they_were_set(n_xy, group, members):
     """state_set then state_get returns every bit for each member of a
     realization group, in a shuffled element order, below and above the
-    staging buffer's size; a step then reads what was set (two contexts with
+    buffers' size; a step then reads what was set (two contexts with
     different orders agree)."""
     spec = W.spark_box_spec(h=1.0 / n_xy, n_xy=n_xy)
     g = S.box_grid(spec)
