@@ -305,13 +305,10 @@ int srs_ctx_create(int device, srs_ctx** out);
 #define SRS_TUNE_ALT_ORDER 13    /* 1: the single-realization step (SRS_TUNE_GATED_SWEEP) sweeps its tiles
                                     in reverse order on alternate steps, reading first what the step before
                                     wrote last; 0 (default): one order */
-#define SRS_TUNE_ADJ_WAVES 14    /* adjoint reverse step's register budget: 0 (default) the compiler's, 4: at
-                                    most 128 VGPRs so that four wavefronts share each SIMD */
-#define SRS_TUNE_ADJ_W 15        /* adjoint reverse step's w = (lambda_Ca / beta, lambda_ATP, lambda_CaM,
-                                    lambda_Fluo) / V0: 0 (default) written by each step for the next on
-                                    launches of fewer than 4096 workgroups (tiles x members), else formed
-                                    in the kernel from lambda; 1: always written (two more state-sized
-                                    buffers per member); 2: always formed.  Same results */
+#define SRS_TUNE_ADJ_WAVES 14    /* accepted (0 or 4) and ignored: the adjoint reverse step takes at most
+                                    128 VGPRs, so that four wavefronts share each SIMD */
+#define SRS_TUNE_ADJ_W 15        /* accepted (0, 1 or 2) and ignored: the adjoint reverse step stores lambda
+                                    / V0 and needs no weights of its own */
 #define SRS_TUNE_ADJ_LEVELS 11   /* adjoint checkpoint levels (srs_linescan_loss_grad*): 0 (default) the
                                     fewest whose memory fits the sub-batch, 1..6 forced; each level below the
                                     first is one more forward pass and needs about (L+1) n^(1/(L+1)) states */

@@ -13,14 +13,15 @@ namespace srs_dev {
 // and dL/dtheta += dt (dr/dtheta)^T lambda_{n+1}.  The diffusion operator
 // satisfies V_i A_ij = V_j A_ji (both equal the face coefficient), so
 // (A^T y)_j = V_j (A (y / V))_j: the transpose is another gather over the same
-// rows.  Single-realization layout (quads, then the TnC and CSQ planes); a
-// launch covers the realizations of a table, one workgroup row (blockIdx.y)
-// each, with row y's adjoint, state and weight arrays at y times their size.
+// rows.  The stored adjoint is m = lambda / V0, so that this gather reads it as
+// it is (divided by the SL buffer's beta in the few SL elements); within an
+// element the recursion is linear in lambda and keeps its form, and the
+// gradient terms take one factor V0.  Single-realization layout (quads, then
+// the TnC and CSQ planes); a launch covers the realizations of a table, one
+// workgroup row (blockIdx.y) each, with row y's adjoint and state arrays at y
+// times their size.
 constexpr int ADJ_NT = 13;   // D_CA, D_DYE, kon/koff of CaM, TnC, ATP, Fluo, V_RYR, A_P, K_D_SL_HI
 constexpr int ADJ_BS = 256;
-// Reverse-step launches (tiles x members) below which w is written by each
-// step for the next instead of formed in the kernel (SRS_TUNE_ADJ_W 0).
-constexpr size_t kAdjWrittenWBlocks = 4096;
 __constant__ const int kAdjTheta[ADJ_NT] = {SRS_R_D_CA,     SRS_R_D_DYE,     SRS_R_K_ON_CMDN, SRS_R_K_OFF_CMDN,
                                             SRS_R_K_ON_TRPN, SRS_R_K_OFF_TRPN, SRS_R_K_ON_ATP, SRS_R_K_OFF_ATP,
                                             SRS_R_K_ON_DYE, SRS_R_K_OFF_DYE, SRS_R_V_RYR,     SRS_R_A_P,
@@ -85,175 +86,125 @@ __device__ __forceinline__ double scan_adj_sum(const double* __restrict__ cen, c
   return s;
 }
 
-// w = (lambda_Ca / beta, lambda_ATP, lambda_CaM, lambda_Fluo) / V0 of element j
-// (c, the element's Ca, is read only where the SL buffer makes beta depend on
-// it; callers pass 0 elsewhere and skip the load).
-__device__ __forceinline__ d4 adj_weight(const RealDesc& d, int j, double c, uint8_t f, double la_c, double la_a,
-                                         double la_m, double la_d) {
-  const SlBuf sb = sl_buffer(d, j, c, f);
-  const double iv = 1.0 / d.V0[j];
-  return d4{la_c / sb.beta * iv, la_a * iv, la_m * iv, la_d * iv};
-}
-
-// Written w (small launches): w of the first step of a recomputed segment;
-// the step kernel writes each later one for the step before.
-__global__ __launch_bounds__(ADJ_BS) void k_adj_w(const RealDesc* __restrict__ D, const int32_t* __restrict__ rid,
-                                                  const double* __restrict__ X, const double* __restrict__ lam,
-                                                  double* __restrict__ w) {
-  const RealDesc& d = D[rid[blockIdx.y]];
-  const int j = blockIdx.x * ADJ_BS + threadIdx.x;
-  if (j >= d.n) return;
-  X += blockIdx.y * 6 * (size_t)d.np;
-  lam += blockIdx.y * 6 * (size_t)d.np;
-  w += blockIdx.y * 4 * (size_t)d.np;
-  const d4 m = ld_quad(gp(lam), qidx1(j));
-  const uint8_t f = d.flags[j];
-  st_quad<false>(gpw(w), qidx1(j), adj_weight(d, j, (f & F_SL) ? X[2 * (size_t)qidx1(j)] : 0.0, f, m.x, m.y, m.z, m.w));
-}
-
-// What the step kernel does after lambda_n: add the loss source of a scan
-// sample taken after n steps (SCAN), and, with written w, form w for step
-// n - 1 from lambda_n and that step's state (Xprev, when it is in the
-// recomputed segment).
-struct AdjNext {
-  const double* Xprev;  // state of step n - 1, or null
-  double* wout;         // its w (quads as in a state)
+// The loss source of a scan sample taken after n steps (SCAN), added to
+// lambda_n.
+struct AdjScan {
   const double* cen;    // scan cell centres [3][np]
   const double* gcoef;  // the sample's loss coefficients per point
   ScanGeo g;
   int n_f, gstride;
 };
 
-// The reverse step's tile map on the device.
-struct AdjMap {
-  const uint16_t* loc;
-  const int32_t *hal, *hoff;
-  int32_t qcap;
-};
+// The tiles of each chiplet's workgroups lie next to each other (the grid's
+// remainder modulo eight keeps its place): its L2 then holds most neighbours
+// (8.5 against 9.2 us per step on the 56,124-element mesh, 234 either way on
+// eight 927,816-element members).
+__device__ __forceinline__ int xcd_run(int bid, int grid) {
+  const int whole = grid / NXCD * NXCD;
+  return bid < whole ? xcd_tile(bid, whole) : bid;
+}
 
-// lambda_n and the theta-gradient partials of one step.  The transposed
-// diffusion gathers w = (lambda_Ca / beta, lambda_ATP, lambda_CaM,
-// lambda_Fluo) / V0 of lambda_{n+1} and this step's state.  WMAT: w was
-// written by the step before (or k_adj_w) and is gathered as it is, the
-// shortest dependency chain for a launch too small to fill the GPU.  Else
-// the tile's w and its halo's are formed once each and staged in LDS (each
-// out-of-tile neighbour used to be formed anew by every element it borders:
-// 309 -> 289 us per step of eight 927,816-element members).
-// The operations are the same, so are the bits.
-template <bool CLASS, bool SCAN, bool WMAT>
+// m_n (lambda_n / V0) and the theta-gradient partials of one step.  The
+// transposed diffusion gathers w = (m_Ca / beta, m_ATP, m_CaM, m_Fluo) of
+// m_{n+1} and this step's state, each element its neighbours' itself.
+// Bound by memory traffic and the gathers' lines: m, X and the rows in and m
+// out are 1.16 GB per step of eight 927,816-element members, 211 us at the
+// 5.5 TB/s that a launch of this mix of reads and writes reaches; the step
+// takes 234 us.  It took 309 us with lambda itself stored, whose gather read
+// 1/V0 as well or w written by a launch or a step of its own; storing m took
+// it to 289.  The neighbours staged in LDS with the sweep's halo lists are
+// slower (251 us, and 9.9 against 9.2 us on the 56,124-element mesh): the
+// registers that hold the gradient sums leave four wavefronts per SIMD, too
+// few to cover a barrier, and the second copy of m fits the cache.
+template <bool CLASS, bool SCAN, bool NTS>
 __device__ __forceinline__ void adj_step(const RealDesc* __restrict__ D, const RealLive* __restrict__ L,
                                          const int32_t* __restrict__ rid, const double* __restrict__ X,
-                                         const double* __restrict__ lam, const double* __restrict__ w, int64_t step,
-                                         double* __restrict__ lam_out, double* __restrict__ gpart, AdjNext nx,
-                                         AdjMap am) {
-  __shared__ double red[ADJ_BS / 16][ADJ_NT];  // gradient partials per row of 16 lanes
-  extern __shared__ double adj_lds[];
-  const QuadTile tw(adj_lds, am.qcap);  // w of the tile's elements and of its halo
+                                         const double* __restrict__ lam, int64_t step, double* __restrict__ lam_out,
+                                         double* __restrict__ gpart, const AdjScan& sc) {
+  __shared__ double red[ADJ_BS / 64][ADJ_NT][16];  // gradient partials per wavefront and lane modulo 16
   const int r = rid[blockIdx.y];
   const RealDesc& d = D[r];
   const RealLive& l = L[r];
-  // Tiles in grid order: an XCD-aware order (consecutive tiles on one XCD)
-  // cuts this kernel's L2 misses by 40% but measured 6% slower.
-  const int tile = blockIdx.x;
+  const int tile = xcd_run(blockIdx.x, gridDim.x);
   const int j = tile * ADJ_BS + threadIdx.x;
   const size_t np = d.np;
   X += blockIdx.y * 6 * np;
   lam += blockIdx.y * 6 * np;
   lam_out += blockIdx.y * 6 * np;
-  if (WMAT) w += blockIdx.y * 4 * np;
-  gpart += (size_t)blockIdx.y * gridDim.x * ADJ_NT;
-  // the tile's running partials, loaded now so the final update waits on no load
-  const double gp_old = threadIdx.x < ADJ_NT ? gpart[(size_t)tile * ADJ_NT + threadIdx.x] : 0.0;
+  // the tile's running partials (16 threads per component), loaded now so the
+  // final update waits on no load
+  const bool sums = threadIdx.x < ADJ_NT * 16;
+  double* gsum = gpart + ((size_t)blockIdx.y * gridDim.x + tile) * ADJ_NT + (threadIdx.x >> 4);
+  const double gp_old = sums ? *gsum : 0.0;
   // RyR states during this step: row `step` of the frozen schedule
   const int32_t* ryr = d.n_ryr ? d.sched + step * d.n_ryr : nullptr;
   double gr[ADJ_NT];
 #pragma unroll
   for (int k = 0; k < ADJ_NT; ++k) gr[k] = 0.0;
-  // the element's operator row, state, lambda_{n+1} and w; with w formed
-  // here, the tile's w staged in LDS
+  // the element's operator row, state, m_{n+1} and its neighbours' w
   const bool in = j < d.n;
   Geo g{};
-  d4 m0 = {0.0, 0.0, 0.0, 0.0}, mu = {0.0, 0.0, 0.0, 0.0}, w0 = {0.0, 0.0, 0.0, 0.0};
-  double V0 = 1.0;
+  d4 m0 = {0.0, 0.0, 0.0, 0.0}, mu = {0.0, 0.0, 0.0, 0.0};
+  double V0 = 1.0, u = 0.0;
   SlBuf sb{1.0, 0.0, 0.0};
   if (in) {
-    if constexpr (WMAT) g = load_geo_nbr<CLASS>(d, j);
-    else g = load_geo<CLASS>(d, am.loc, j, block_flags(d, j));
+    g = load_geo_nbr<CLASS>(d, j);
     m0 = ld_quad(gp(X), qidx1(j));
     mu = ld_quad(gp(lam), qidx1(j));
-    V0 = d.V0[j];
-    sb = sl_buffer(d, j, m0.x, g.f);
-    if constexpr (WMAT) {
-      w0 = ld_quad(gp(w), qidx1(j));
-    } else {
-      const double iv = 1.0 / V0;
-      w0 = d4{mu.x / sb.beta * iv, mu.y * iv, mu.z * iv, mu.w * iv};
+    V0 = gp(d.V0)[j];
+    u = mu.x;
+    if (g.f & F_SL) {
+      sb = sl_buffer(d, j, m0.x, g.f);
+      u = mu.x / sb.beta;
     }
   }
-  if constexpr (!WMAT) {
-    tw.put(threadIdx.x, w0);
-    const Halo h = load_halo<ADJ_BS>(am.hal, am.hoff, tile);
-    auto put_halo = [&](int k, int e) {
-      const uint8_t fn = d.flags[e];
-      const d4 ln = ld_quad(gp(lam), qidx1(e));
-      tw.put(ADJ_BS + k, adj_weight(d, e, (fn & F_SL) ? X[2 * (size_t)qidx1(e)] : 0.0, fn, ln.x, ln.y, ln.z, ln.w));
-    };
-#pragma unroll
-    for (int q = 0; q < HPRE; ++q)
-      if (h.e[q] >= 0) put_halo(threadIdx.x + q * ADJ_BS, h.e[q]);
-    for (int k = threadIdx.x + HPRE * ADJ_BS; k < h.n; k += ADJ_BS) put_halo(k, am.hal[h.s + k]);
-    __syncthreads();
-  }
+  auto w_at = [&](uint32_t e) -> d4 {
+    const uint32_t i = idx_of(e);
+    d4 w = ld_quad(gp(lam), qidx1(i));
+    if (e & IDX_SL) w.x /= sl_buffer(d, (int)i, X[2 * (size_t)qidx1(i)], F_SL).beta;
+    return w;
+  };
+  d4 w1{}, w2{}, w3{}, w4{};
+  if (in) w1 = w_at(g.l1), w2 = w_at(g.l2), w3 = w_at(g.l3), w4 = w_at(g.l4);
   // the scan sample's loss source (all lanes of the wavefront take part)
   const double src =
-      SCAN ? scan_adj_sum(nx.cen, nx.g, nx.n_f, nx.gcoef + (size_t)blockIdx.y * nx.gstride, np, j, in) : 0.0;
+      SCAN ? scan_adj_sum(sc.cen, sc.g, sc.n_f, sc.gcoef + (size_t)blockIdx.y * sc.gstride, np, j, in) : 0.0;
   if (in) {
     const double* P = d.P;
-    const double dt = P[SRS_R_T_STEP];
+    const double dt = P[SRS_R_T_STEP], dv0 = dt * V0;
     const uint8_t f = g.f;
-    auto nw = [&](int nb) -> d4 {
-      if constexpr (WMAT) return ld_quad(gp(w), qidx1(nb));
-      else return tw.get(nb);
-    };
-    const d4 w1 = nw(g.l1), w2 = nw(g.l2), w3 = nw(g.l3), w4 = nw(g.l4);
-    const bool live_tr = (f & (F_JSR | F_TROPC)) == F_TROPC;
-    const bool live_cs = (f & F_JSR) != 0;
+    const d4 aw = row_sum(g, d4{u, mu.y, mu.z, mu.w}, w1, w2, w3, w4);
+    const bool live_tr = lives_tr(f), live_cs = lives_cs(f);
     const double bT = live_tr ? X[4 * np + j] : 0.0, bC = live_cs ? X[5 * np + j] : 0.0;
     // the TnC and CSQ adjoints change only where the buffer lives (troponin
-    // cytosol, jSR); both lambda buffers start at zero, so elsewhere they stay
+    // cytosol, jSR); both adjoint buffers start at zero, so elsewhere they stay
     // zero and those planes are neither read nor written
     const double muT = live_tr ? lam[4 * np + j] : 0.0, muC = live_cs ? lam[5 * np + j] : 0.0;
     const double c = m0.x, bA = m0.y, bM = m0.z, bD = m0.w;
-    const double u = mu.x / sb.beta;
 
-    // transposed diffusion: dt D_s V0 (A w_s)_j
-    const double aw_c = g.a0 * w0.x + g.a1 * w1.x + g.a2 * w2.x + g.a3 * w3.x + g.a4 * w4.x;
-    const double aw_a = g.a0 * w0.y + g.a1 * w1.y + g.a2 * w2.y + g.a3 * w3.y + g.a4 * w4.y;
-    const double aw_m = g.a0 * w0.z + g.a1 * w1.z + g.a2 * w2.z + g.a3 * w3.z + g.a4 * w4.z;
-    const double aw_d = g.a0 * w0.w + g.a1 * w1.w + g.a2 * w2.w + g.a3 * w3.w + g.a4 * w4.w;
-    double lc = mu.x + dt * P[SRS_R_D_CA] * V0 * aw_c;
-    double la = mu.y + dt * P[SRS_R_D_ATP] * V0 * aw_a;
-    double lm = mu.z + dt * P[SRS_R_D_CMDN] * V0 * aw_m;
-    double ld = mu.w + dt * P[SRS_R_D_DYE] * V0 * aw_d;
+    // transposed diffusion: dt D_s (A w_s)_j
+    double lc = mu.x + dt * P[SRS_R_D_CA] * aw.x;
+    double la = mu.y + dt * P[SRS_R_D_ATP] * aw.y;
+    double lm = mu.z + dt * P[SRS_R_D_CMDN] * aw.z;
+    double ld = mu.w + dt * P[SRS_R_D_DYE] * aw.w;
     double lT = muT, lC = muC;
 
-    // The D gradients sum u_j (A c)_j and mu_Fluo,j (A b_Fluo)_j over the mesh;
-    // V_i A_ij = V_j A_ji turns those sums into sum_j c_j V0_j (A w_Ca)_j and
+    // The D gradients sum V0_j u_j (A c)_j and V0_j m_Fluo,j (A b_Fluo)_j over the
+    // mesh; V_i A_ij = V_j A_ji turns those sums into sum_j c_j V0_j (A w_Ca)_j and
     // sum_j b_Fluo,j V0_j (A w_Fluo)_j, terms of the element alone.  So the
     // neighbours' states are gathered only for an SL element, whose SL terms
     // need its full Ca rate before the division (rca; unused elsewhere).
     double ac = 0.0;
     if (f & F_SL) {
-      auto ca_at = [&](int e) { return X[2 * (size_t)qidx1(e)]; };
-      const i4 nb = ((const i4*)d.nbr)[j];
-      ac = c * g.a0 + ca_at(nb.x) * g.a1 + ca_at(nb.y) * g.a2 + ca_at(nb.z) * g.a3 + ca_at(nb.w) * g.a4;
+      auto ca_at = [&](uint32_t e) { return X[2 * (size_t)qidx1(idx_of(e))]; };
+      ac = c * g.a0 + ca_at(g.l1) * g.a1 + ca_at(g.l2) * g.a2 + ca_at(g.l3) * g.a3 + ca_at(g.l4) * g.a4;
     }
     // boundary rates are D times a D-free plane: they enter the D gradients
     const double bu_c = (f & F_BR) ? br_unit(d.br_mesh[j], d.brd[0]) : 0.0;
     const double bu_d = (f & F_BR) ? br_unit(d.br_mesh[np + j], d.brd[1]) : 0.0;
     double rca = P[SRS_R_D_CA] * ac + ((f & F_BR) ? d.br[j] : 0.0);
-    gr[0] += dt * (c * V0 * aw_c + u * bu_c);       // D_CA
-    gr[1] += dt * (bD * V0 * aw_d + mu.w * bu_d);   // D_DYE
+    gr[0] += dv0 * (c * aw.x + u * bu_c);       // D_CA
+    gr[1] += dv0 * (bD * aw.w + mu.w * bu_d);   // D_DYE
     if (!(f & F_JSR)) {
       if (f & F_TROPC) {
         const double kon = P[SRS_R_K_ON_TRPN], koff = P[SRS_R_K_OFF_TRPN], B = P[SRS_R_B_TOT_TRPN];
@@ -261,8 +212,8 @@ __device__ __forceinline__ void adj_step(const RealDesc* __restrict__ D, const R
         rca -= r;
         lc += dt * (muT - u) * kon * (B - bT);
         lT += dt * (muT - u) * (-kon * c - koff);
-        gr[4] += dt * (muT - u) * (B - bT) * c;
-        gr[5] += dt * (muT - u) * (-bT);
+        gr[4] += dv0 * (muT - u) * (B - bT) * c;
+        gr[5] += dv0 * (muT - u) * (-bT);
         // SERCA, cpu/RunSimulation.cpp:82-90
         const double kdi = P[SRS_R_K_D_I];
         double K = c / kdi;
@@ -274,29 +225,29 @@ __device__ __forceinline__ void adj_step(const RealDesc* __restrict__ D, const R
         const double dv = ((2 * K * 3.24873e12 + l.serca[3]) * Dn - Nn * (l.serca[1] + 2 * K * l.serca[2])) / (Dn * Dn);
         rca -= (2e-3) * v * P[SRS_R_A_P];
         lc += dt * (-u) * (2e-3) * P[SRS_R_A_P] * dv * dK;
-        gr[11] += dt * u * (-(2e-3) * v);
+        gr[11] += dv0 * u * (-(2e-3) * v);
       }
       const double konD = P[SRS_R_K_ON_DYE], koffD = P[SRS_R_K_OFF_DYE], BD = P[SRS_R_B_TOT_DYE];
       const double rD = konD * (BD - bD) * c - koffD * bD;
       rca -= rD;
       lc += dt * (mu.w - u) * konD * (BD - bD);
       ld += dt * (mu.w - u) * (-konD * c - koffD);
-      gr[8] += dt * (mu.w - u) * (BD - bD) * c;
-      gr[9] += dt * (mu.w - u) * (-bD);
+      gr[8] += dv0 * (mu.w - u) * (BD - bD) * c;
+      gr[9] += dv0 * (mu.w - u) * (-bD);
       const double konA = P[SRS_R_K_ON_ATP], koffA = P[SRS_R_K_OFF_ATP], BA = P[SRS_R_B_TOT_ATP];
       const double rA = konA * (BA - bA) * c - koffA * bA;
       rca -= rA;
       lc += dt * (mu.y - u) * konA * (BA - bA);
       la += dt * (mu.y - u) * (-konA * c - koffA);
-      gr[6] += dt * (mu.y - u) * (BA - bA) * c;
-      gr[7] += dt * (mu.y - u) * (-bA);
+      gr[6] += dv0 * (mu.y - u) * (BA - bA) * c;
+      gr[7] += dv0 * (mu.y - u) * (-bA);
       const double konM = P[SRS_R_K_ON_CMDN], koffM = P[SRS_R_K_OFF_CMDN], BM = P[SRS_R_B_TOT_CMDN];
       const double rM = konM * (BM - bM) * c - koffM * bM;
       rca -= rM;
       lc += dt * (mu.z - u) * konM * (BM - bM);
       lm += dt * (mu.z - u) * (-konM * c - koffM);
-      gr[2] += dt * (mu.z - u) * (BM - bM) * c;
-      gr[3] += dt * (mu.z - u) * (-bM);
+      gr[2] += dv0 * (mu.z - u) * (BM - bM) * c;
+      gr[3] += dv0 * (mu.z - u) * (-bM);
     } else {
       const double kon = P[SRS_R_K_ON_CSQN], koff = P[SRS_R_K_OFF_CSQN], B = P[SRS_R_B_T_JSR];
       const double r = kon * (B - bC) * c - koff * bC;
@@ -325,13 +276,12 @@ __device__ __forceinline__ void adj_step(const RealDesc* __restrict__ D, const R
             const double up = lam[2 * (size_t)qidx1(p)] / sl_buffer(d, p, cp, d.flags[p]).beta;
             const double dc = X[2 * (size_t)qidx1(je)] - X[2 * (size_t)qidx1(ce)];
             const double J = a * dc;
+            lc += dt * (a / V0) * (up - u);
             if (ch & 1) {  // jSR side: r -= J / V0_jsr
               rca -= J / V0;
-              lc += dt * (u * (-a / V0) + up * (a / d.V0[p]));
             } else {       // cleft side: r += J / V0_cyt
               rca += J / V0;
-              lc += dt * (u * (-a / V0) + up * (a / d.V0[p]));
-              gr[10] += dt * (u * P[SRS_R_V_CELL] * dc / V0 - up * P[SRS_R_V_CELL] * dc / d.V0[p]);
+              gr[10] += dt * P[SRS_R_V_CELL] * dc * (u - up);
             }
           } else {
             const int i = -ch - 1;
@@ -346,70 +296,62 @@ __device__ __forceinline__ void adj_step(const RealDesc* __restrict__ D, const R
     if (f & F_SL) {
       const double b2 = sb.beta * sb.beta;
       lc += dt * mu.x * (-rca * sb.dbeta_dc / b2);
-      gr[12] += dt * mu.x * (-rca * sb.dbeta_dkh / b2);
+      gr[12] += dv0 * mu.x * (-rca * sb.dbeta_dkh / b2);
     }
-    if (SCAN) ld += V0 * src;
-    st_quad<false>(gpw(lam_out), qidx1(j), d4{lc, la, lm, ld});
-    if (live_tr) lam_out[4 * np + j] = lT;
-    if (live_cs) lam_out[5 * np + j] = lC;
-    if (WMAT && nx.Xprev) {
-      const double* Xp = nx.Xprev + blockIdx.y * 6 * np;
-      st_quad<false>(gpw(nx.wout) + blockIdx.y * 4 * np, qidx1(j),
-                     adj_weight(d, j, (f & F_SL) ? Xp[2 * (size_t)qidx1(j)] : 0.0, f, lc, la, lm, ld));
-    }
+    if (SCAN) ld += src;
+    st_quad<NTS>(gpw(lam_out), qidx1(j), d4{lc, la, lm, ld});
+    if (live_tr) stg<NTS>(gpw(lam_out) + 4 * np + j, lT);
+    if (live_cs) stg<NTS>(gpw(lam_out) + 5 * np + j, lC);
   }
-  // block reduction of the gradient partials, accumulated per block: DPP
-  // sums within each row of 16 lanes (a component that is zero in every lane
-  // of the wavefront, as the channel and SL terms are in most, is not
-  // summed), then the block's rows in LDS in a fixed order
+  // block reduction of the gradient partials, accumulated per block, in a fixed
+  // order.  A matrix instruction with a matrix of ones adds the four lanes l,
+  // l + 16, l + 32, l + 48 of a wavefront in FP64, on the matrix cores instead
+  // of twelve lane moves and additions per component; the rest goes through
+  // LDS, 16 sums per wavefront and component.  A channel or SL component that
+  // is zero in every lane is not summed.
+  typedef double v4 __attribute__((ext_vector_type(4)));
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
   for (int k = 0; k < ADJ_NT; ++k) {
-    const double v = __builtin_amdgcn_ballot_w64(gr[k] != 0.0) ? row_sum_dpp(gr[k]) : 0.0;
-    if ((threadIdx.x & 15) == 15) red[threadIdx.x >> 4][k] = v;
+    double v = 0.0;
+    if ((k != 10 && k != 12) || __builtin_amdgcn_ballot_w64(gr[k] != 0.0)) {
+      const v4 z = {0.0, 0.0, 0.0, 0.0};
+      v = __builtin_amdgcn_mfma_f64_16x16x4f64(1.0, gr[k], z, 0, 0, 0)[0];
+    }
+    if (lane < 16) red[wave][k][lane] = v;
   }
   __syncthreads();
-  if (threadIdx.x < ADJ_NT) {
-    double s = 0.0;
-    for (int q = 0; q < ADJ_BS / 16; ++q) s += red[q][threadIdx.x];
-    gpart[(size_t)tile * ADJ_NT + threadIdx.x] = gp_old + s;
+  if (sums) {
+    const int k = threadIdx.x >> 4, q = threadIdx.x & 15;
+    double s = red[0][k][q];
+#pragma unroll
+    for (int w = 1; w < ADJ_BS / 64; ++w) s += red[w][k][q];
+    s = row_sum_dpp(s);
+    if (q == 15) *gsum = gp_old + s;
   }
 }
 
-// The compiler's register budget (126 VGPRs: four wavefronts per SIMD), or
-// at most 128 (four) asked for explicitly; the two compile alike.
-template <bool CLASS, bool SCAN, bool WMAT>
-__global__ __launch_bounds__(ADJ_BS) void k_adj_step(const RealDesc* __restrict__ D, const RealLive* __restrict__ L,
-                                                     const int32_t* __restrict__ rid, const double* __restrict__ X,
-                                                     const double* __restrict__ lam, const double* __restrict__ w,
-                                                     int64_t step, double* __restrict__ lam_out,
-                                                     double* __restrict__ gpart, AdjNext nx, AdjMap am) {
-  adj_step<CLASS, SCAN, WMAT>(D, L, rid, X, lam, w, step, lam_out, gpart, nx, am);
-}
-template <bool CLASS, bool SCAN, bool WMAT>
-__global__ __launch_bounds__(ADJ_BS) __attribute__((amdgpu_waves_per_eu(4))) void k_adj_step_w4(
+// At most 128 VGPRs: four wavefronts per SIMD (a budget of five spills 116 B
+// per lane: 366 against 280 us per step of eight 927,816-element members).
+template <bool CLASS, bool SCAN, bool NTS>
+__global__ __launch_bounds__(ADJ_BS) __attribute__((amdgpu_waves_per_eu(4))) void k_adj_step(
     const RealDesc* __restrict__ D, const RealLive* __restrict__ L, const int32_t* __restrict__ rid,
-    const double* __restrict__ X, const double* __restrict__ lam, const double* __restrict__ w, int64_t step,
-    double* __restrict__ lam_out, double* __restrict__ gpart, AdjNext nx, AdjMap am) {
-  adj_step<CLASS, SCAN, WMAT>(D, L, rid, X, lam, w, step, lam_out, gpart, nx, am);
+    const double* __restrict__ X, const double* __restrict__ lam, int64_t step, double* __restrict__ lam_out,
+    double* __restrict__ gpart, AdjScan sc) {
+  adj_step<CLASS, SCAN, NTS>(D, L, rid, X, lam, step, lam_out, gpart, sc);
 }
 
-using AdjStepFn = void (*)(const RealDesc*, const RealLive*, const int32_t*, const double*, const double*,
-                           const double*, int64_t, double*, double*, AdjNext, AdjMap);
-template <bool CLASS, bool SCAN, bool WMAT>
-static AdjStepFn adj_step_fn(bool waves4) {
-  return waves4 ? k_adj_step_w4<CLASS, SCAN, WMAT> : k_adj_step<CLASS, SCAN, WMAT>;
-}
-static AdjStepFn adj_step_kernel(bool compact, bool scan, bool wmat, bool waves4) {
-  if (compact) {
-    if (scan) return wmat ? adj_step_fn<true, true, true>(waves4) : adj_step_fn<true, true, false>(waves4);
-    return wmat ? adj_step_fn<true, false, true>(waves4) : adj_step_fn<true, false, false>(waves4);
-  }
-  if (scan) return wmat ? adj_step_fn<false, true, true>(waves4) : adj_step_fn<false, true, false>(waves4);
-  return wmat ? adj_step_fn<false, false, true>(waves4) : adj_step_fn<false, false, false>(waves4);
+using AdjStepFn = void (*)(const RealDesc*, const RealLive*, const int32_t*, const double*, const double*, int64_t,
+                           double*, double*, AdjScan);
+template <bool CLASS>
+static AdjStepFn adj_step_fn(bool scan, bool nts) {
+  if (scan) return nts ? k_adj_step<CLASS, true, true> : k_adj_step<CLASS, true, false>;
+  return nts ? k_adj_step<CLASS, false, true> : k_adj_step<CLASS, false, false>;
 }
 
 // The loss gradient of one scan sample in the Fluo adjoint:
-// lambda_Fluo,j += V0_j sum_i gcoef_i w(c_j - p_i) over points within 1 um.
+// lambda_Fluo,j += V0_j sum_i gcoef_i w(c_j - p_i) over points within 1 um
+// (m = lambda / V0).
 __global__ __launch_bounds__(ADJ_BS) void k_scan_adj(const RealDesc* __restrict__ D, const int32_t* __restrict__ rid,
                                                      const double* __restrict__ cen, ScanGeo g, int n_f,
                                                      const double* __restrict__ gcoef, int gstride,
@@ -420,7 +362,7 @@ __global__ __launch_bounds__(ADJ_BS) void k_scan_adj(const RealDesc* __restrict_
   const double s = scan_adj_sum(cen, g, n_f, gcoef + (size_t)blockIdx.y * gstride, np, j, j < d.n);
   if (j >= d.n) return;
   lam += blockIdx.y * 6 * np;
-  lam[2 * (size_t)qidx1(j) + FLUO_OFF] += d.V0[j] * s;
+  lam[2 * (size_t)qidx1(j) + FLUO_OFF] += s;
 }
 
 // Copies the current state (X[cur]) of each realization of a table to slot y
@@ -642,7 +584,7 @@ static int loss_grad_run(srs_ctx* c, const std::vector<int32_t>& ids, int32_t sc
                          const double* targets, int32_t ckpt, int32_t max_batch, double* losses, double* grads,
                          double* scans) {
   const HostScan& S = c->scans[scan_id];
-  HostMesh& hm = *c->meshes[S.mesh];
+  const HostMesh& hm = *c->meshes[S.mesh];
   const size_t np = hm.np, n6 = 6 * np;
   const int nf = S.n_f, nca = S.n_ca, nout = nca + 2 * nf;
   const int n_mem = (int)ids.size(), n_real = (int)c->reals.size();
@@ -657,22 +599,13 @@ static int loss_grad_run(srs_ctx* c, const std::vector<int32_t>& ids, int32_t sc
   }
   HIPCHK(hipSetDevice(c->device));
   HIPCHK(hipStreamSynchronize(c->stream));
-  if (want_grad && hm.map.tile != ADJ_BS && hm.map_adj.tile == 0) {  // kept with the mesh
-    const int rc = build_map(c, hm, ADJ_BS, &hm.map_adj);
-    if (rc) return rc;
-  }
-  const TileMap& tm = hm.map.tile == ADJ_BS ? hm.map : hm.map_adj;
-  const AdjMap am{tm.d_loc, tm.d_hal, tm.d_hoff, tm.qcap};
   size_t mem_free = 0, mem_total = 0;
   HIPCHK(hipMemGetInfo(&mem_free, &mem_total));
   const size_t budget = mem_free / 10 * 9;
-  // written w (two buffers) on launches of fewer than kAdjWrittenWBlocks
-  // workgroups, unless SRS_TUNE_ADJ_W forces one form
-  const bool wmat_possible = want_grad && (c->adj_w == 1 || (c->adj_w == 0 && (size_t)nblk < kAdjWrittenWBlocks));
   // device bytes per member of a sub-batch under a plan (a loss alone keeps
   // only the start state)
   auto per_member = [&](const AdjPlan& p) {
-    return 8 * n6 * (size_t)(want_grad ? p.kept() + p.K[p.L - 1] + 2 : 1) + (wmat_possible ? 64 * np : 0) +
+    return 8 * n6 * (size_t)(want_grad ? p.kept() + p.K[p.L - 1] + 2 : 1) +
            8 * (size_t)n_samples * nout + 8 * (size_t)S.n_blocks * nf + 8 * (size_t)nblk * ADJ_NT +
            8 * (size_t)n_samples * nf + 4 * max_sched + 64;
   };
@@ -702,9 +635,10 @@ static int loss_grad_run(srs_ctx* c, const std::vector<int32_t>& ids, int32_t sc
   c->adj_last_levels = plan.L;
   for (int l = 0; l < ADJ_MAX_LEVELS; ++l) c->adj_last_strides[l] = l < plan.L ? plan.K[l] : 0;
   c->adj_last_batch = bs;
-  const bool wmat = wmat_possible && (c->adj_w == 1 || (size_t)nblk * bs < kAdjWrittenWBlocks);
 
-  const size_t adj_lds_bytes = wmat ? 0 : 4 * sizeof(double) * (size_t)tm.qcap;
+  // the reverse step's new lambda past the caches once a step's states no longer
+  // fit them (eight 927,816-element members, 1.07 GB: 238 -> 234 us per step)
+  const bool nts = 8.0 * n6 * bs * 3 > 330e6;
 
   // everything restored at the end
   std::vector<RealLive> live0(n_real);
@@ -721,7 +655,6 @@ static int loss_grad_run(srs_ctx* c, const std::vector<int32_t>& ids, int32_t sc
   double *ck = nullptr, *samp = nullptr, *part = nullptr, *dg = nullptr, *gpart = nullptr;
   double *lam0 = nullptr, *lam1 = nullptr, *seg = nullptr;
   std::vector<double*> ckl(plan.L, nullptr);  // checkpoint levels; ckl[0] = ck, the forward's
-  double *w0 = nullptr, *w1 = nullptr;        // written w of steps n and n - 1
   int32_t *d_sched = nullptr, *d_rid = nullptr;
   int2* d_sub_tiles = nullptr;
   const int nt_mesh = (hm.n + c->tile - 1) / c->tile;
@@ -735,10 +668,6 @@ static int loss_grad_run(srs_ctx* c, const std::vector<int32_t>& ids, int32_t sc
   if (want_grad) {
     HIPCHK(M.alloc(&lam0, (size_t)bs * n6));
     HIPCHK(M.alloc(&lam1, (size_t)bs * n6));
-    if (wmat) {
-      HIPCHK(M.alloc(&w0, 4 * (size_t)bs * np));
-      HIPCHK(M.alloc(&w1, 4 * (size_t)bs * np));
-    }
     HIPCHK(M.alloc(&seg, (size_t)leaf * bs * n6));
     for (int l = 1; l < plan.L; ++l) HIPCHK(M.alloc(&ckl[l], (size_t)plan.slots[l] * bs * n6));
     HIPCHK(M.alloc(&gpart, (size_t)bs * nblk * ADJ_NT));
@@ -858,8 +787,6 @@ static int loss_grad_run(srs_ctx* c, const std::vector<int32_t>& ids, int32_t sc
       if (e == hipSuccess) e = hipMemsetAsync(gpart, 0, (size_t)nb * nblk * ADJ_NT * sizeof(double), c->stream);
       double* lam = lam0;   // lambda_{n+1}
       double* lout = lam1;  // lambda_n
-      double* wcur = w0;        // written w of step n
-      double* wnext = w1;       // written w of step n - 1
       ks = n_samples - 1;
       // the loss source of a sample after the last step; the step kernel
       // adds the others to the lambda it produces
@@ -898,17 +825,13 @@ static int loss_grad_run(srs_ctx* c, const std::vector<int32_t>& ids, int32_t sc
         }
         for (int64_t n = s1 - 1; n >= s0 && e2 == hipSuccess; --n) {
           const double* Xn = seg + (size_t)(n - s0) * nb * n6;
-          if (wmat && n == s1 - 1)
-            hipLaunchKernelGGL(k_adj_w, g_adj, dim3(ADJ_BS), 0, c->stream, c->d_desc, d_rid, Xn, lam, wcur);
           const bool scan = ks >= 0 && sample_steps[ks] == n;
-          AdjNext nx{wmat && n > s0 ? Xn - nb * n6 : nullptr, wnext, S.d_cen, scan ? dg + (size_t)ks * nf : nullptr,
-                     S.geo, nf, n_samples * nf};
+          const AdjScan sc{S.d_cen, scan ? dg + (size_t)ks * nf : nullptr, S.geo, nf, n_samples * nf};
           if (scan) --ks;
-          const AdjStepFn kern = adj_step_kernel(c->class_all, scan, wmat, c->adj_waves == 4);
-          hipLaunchKernelGGL(kern, g_adj, dim3(ADJ_BS), adj_lds_bytes, c->stream, c->d_desc, c->d_live, d_rid, Xn, lam,
-                             wcur, n, lout, gpart, nx, am);
+          const AdjStepFn kern = c->class_all ? adj_step_fn<true>(scan, nts) : adj_step_fn<false>(scan, nts);
+          hipLaunchKernelGGL(kern, g_adj, dim3(ADJ_BS), 0, c->stream, c->d_desc, c->d_live, d_rid, Xn, lam, n, lout,
+                             gpart, sc);
           std::swap(lam, lout);
-          std::swap(wcur, wnext);
           e2 = hipGetLastError();
         }
         if (e2 == hipSuccess) e2 = hipStreamSynchronize(c->stream);

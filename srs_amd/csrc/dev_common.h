@@ -88,11 +88,11 @@ struct ChanElem {
 
 // Immutable per-realization descriptor (read with scalar loads).
 struct RealDesc {
-  const int32_t* nbr;     // [np][4] neighbour indices
+  const uint32_t* nbr;    // [np][4] neighbour indices (IDX_SL)
   // tile map of the sweep (TileMap): where each element's neighbours are among
   // its tile's staged quads
   const uint16_t* loc;    // [np][4]
-  const int32_t* hal;     // halo elements, tile by tile
+  const uint32_t* hal;    // halo elements (IDX_SL), tile by tile
   const int32_t* hoff;    // [tiles + 1] the tiles' runs in hal
   int32_t qcap;           // quads a tile stages at most
   const double* coef;     // [5][np] (plain rows)
@@ -251,24 +251,45 @@ struct QuadTile {
 template <class T>
 __device__ __forceinline__ T sld(const T* p) { return *(const __attribute__((address_space(4))) T*)p; }
 
-// A tile's run of the halo list, and the halo elements of a thread: the first
-// HPRE of them are loaded ahead of everything that does not depend on them.
+// An element index with bit 31 set where the element has F_SL, as the halo
+// lists and the neighbour table hold them.
+constexpr uint32_t IDX_SL = 0x80000000u;
+__device__ __forceinline__ uint32_t idx_of(uint32_t e) { return e & ~IDX_SL; }
+
+// A tile's run of the halo list, and the entries of a thread: the first HPRE
+// of them are loaded ahead of everything that does not depend on them.
 constexpr int HPRE = 2;
 struct Halo {
-  int s, n, e[HPRE];
+  int s, n;
+  uint32_t e[HPRE];
 };
 template <int BS>
-__device__ __forceinline__ Halo load_halo(const int32_t* hal, const int32_t* hoff, const int t) {
+__device__ __forceinline__ Halo load_halo(const uint32_t* hal, const int32_t* hoff, const int t) {
   Halo h;
   h.s = sld(hoff + t);
   h.n = sld(hoff + t + 1) - h.s;
 #pragma unroll
   for (int q = 0; q < HPRE; ++q) {
     const int k = (int)threadIdx.x + q * BS;
-    h.e[q] = k < h.n ? gp(hal)[h.s + k] : -1;
+    h.e[q] = k < h.n ? gp(hal)[h.s + k] : 0u;
   }
   return h;
 }
+// put(i, e) for each of the thread's halo entries e, i its place in the halo.
+template <int BS, class F>
+__device__ __forceinline__ void each_halo(const uint32_t* hal, const Halo& h, F put) {
+#pragma unroll
+  for (int q = 0; q < HPRE; ++q)
+    if ((int)threadIdx.x + q * BS < h.n) put((int)threadIdx.x + q * BS, h.e[q]);
+  for (int k = (int)threadIdx.x + HPRE * BS; k < h.n; k += BS) put(k, gp(hal)[h.s + k]);
+}
+
+// TnC has a nonzero rate only in cytosol elements with troponin, CSQ only in
+// the jSR (cpu/RunSimulation.cpp:45-46 reset both rates to zero).  A zero rate
+// leaves the value unchanged, and both state buffers hold the same value, so
+// those planes are neither read nor written elsewhere.
+__device__ __forceinline__ bool lives_tr(const uint8_t f) { return (f & (F_JSR | F_TROPC)) == F_TROPC; }
+__device__ __forceinline__ bool lives_cs(const uint8_t f) { return (f & F_JSR) != 0; }
 
 // Operator row of one element: coefficients (diagonal first), its neighbours'
 // places among the tile's staged quads, and flags.  Mesh-level data, shared
@@ -315,7 +336,7 @@ __device__ __forceinline__ Geo load_geo(const RealDesc& d, const uint16_t* loc, 
   load_coef<CLASS>(d, j, g);
   return g;
 }
-// The row of any element, with neighbour indices in place of tile places.
+// The row of any element, with neighbour indices (IDX_SL) in place of tile places.
 template <bool CLASS>
 __device__ __forceinline__ Geo load_geo_nbr(const RealDesc& d, const int j) {
   Geo g;
@@ -325,6 +346,13 @@ __device__ __forceinline__ Geo load_geo_nbr(const RealDesc& d, const int j) {
   load_coef<CLASS>(d, j, g);
   return g;
 }
+// The operator row applied to an element's own and its neighbours' quads, in
+// the reference's order (cpu/RunSimulation.cpp:61-71).
+__device__ __forceinline__ d4 row_sum(const Geo& g, const d4& m0, const d4& m1, const d4& m2, const d4& m3,
+                                      const d4& m4) {
+  return m0 * g.a0 + m1 * g.a1 + m2 * g.a2 + m3 * g.a3 + m4 * g.a4;
+}
+
 // The flags of the block of element j, j consecutive across the wavefront from
 // a multiple of 64.
 __device__ __forceinline__ uint32_t block_flags(const RealDesc& d, const int j) {
@@ -459,7 +487,8 @@ struct TileMap {
   int32_t qcap = 0;   // the most quads a tile stages (its elements and its halo)
   int32_t n_halo = 0; // elements of all halos
   uint16_t* d_loc = nullptr;
-  int32_t *d_hal = nullptr, *d_hoff = nullptr;
+  uint32_t* d_hal = nullptr;
+  int32_t* d_hoff = nullptr;
 };
 
 struct HostMesh {
@@ -475,13 +504,14 @@ struct HostMesh {
   // realization added on the mesh, which every later one must share.
   double br_d[4] = {0, 0, 0, 0};
   bool br_d_set = false;
-  TileMap map, map_adj;             // of the sweep's tiles and of the reverse step's
+  TileMap map;                      // of the sweep's tiles
   // compact operator layout
   bool class_rows = false;          // row and tab reproduce every coefficient
   std::vector<uint32_t> row;        // [np][3]
   std::vector<double> tab;
   int32_t n_class = 0;
-  int32_t *d_nbr = nullptr, *d_inv = nullptr;
+  uint32_t* d_nbr = nullptr;
+  int32_t* d_inv = nullptr;
   double *d_coef = nullptr, *d_V0 = nullptr, *d_tt = nullptr, *d_br = nullptr, *d_tab = nullptr;
   uint8_t* d_flags = nullptr;
   uint32_t *d_blk = nullptr, *d_row = nullptr;
@@ -530,8 +560,6 @@ struct srs_ctx {
   int alt_order = 0;      // single-realization gated sweep: tiles in reverse order on alternate steps
   int gpu_layout = 0;     // states records in the GPU program's layout (Ca_cyt at each RyR appended)
   int adj_levels = 0;     // adjoint checkpoint levels, 0: the fewest that fit the sub-batch
-  int adj_waves = 0;      // adjoint reverse-step register budget: 0 compiler's choice, 4 wavefronts per SIMD
-  int adj_w = 0;          // adjoint w: 0 by launch size, 1 written by each step, 2 formed in the kernel
   int adj_last_levels = 0, adj_last_batch = 0;  // the plan of the last loss/gradient call
   int64_t adj_last_strides[6] = {};
   bool class_all = false;  // class rows on every mesh

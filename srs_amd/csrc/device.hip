@@ -42,13 +42,6 @@ struct Loc {
   double c_tr, c_cs;
 };
 
-// The operator row applied to an element's own and its neighbours' quads, in
-// the reference's order (cpu/RunSimulation.cpp:61-71).
-__device__ __forceinline__ d4 row_sum(const Geo& g, const d4& m0, const d4& m1, const d4& m2, const d4& m3,
-                                      const d4& m4) {
-  return m0 * g.a0 + m1 * g.a1 + m2 * g.a2 + m3 * g.a3 + m4 * g.a4;
-}
-
 // A realization's state buffers for one step: read X[cur], write X[cur ^ 1].
 // Both pointers are loaded and one is selected, so that the live index and
 // the pointers arrive in the same round of scalar loads.
@@ -80,13 +73,6 @@ template <bool ONE>
 __device__ __forceinline__ size_t qat(const RealDesc& d, const int e) {
   return ONE ? (size_t)qidx1((uint32_t)e) : qidx((size_t)e, d.kst, d.slot);
 }
-
-// TnC has a nonzero rate only in cytosol elements with troponin, CSQ only in
-// the jSR (cpu/RunSimulation.cpp:45-46 reset both rates to zero).  A zero rate
-// leaves the value unchanged, and both state buffers hold the same value, so
-// those planes are neither read nor written elsewhere.
-__device__ __forceinline__ bool lives_tr(const uint8_t f) { return (f & (F_JSR | F_TROPC)) == F_TROPC; }
-__device__ __forceinline__ bool lives_cs(const uint8_t f) { return (f & F_JSR) != 0; }
 
 // An element's rates without the channel fluxes, and the divisor of the rapid
 // buffers (B, used where `div`).
@@ -271,10 +257,7 @@ __device__ __forceinline__ void sweep_tile(const RealDesc& d, const RealLive& l,
   // is live in all but jSR and troponin-free cytosol elements)
   c.c_tr = Xo[pl];
   tq.put(threadIdx.x, c.m0);
-#pragma unroll
-  for (int q = 0; q < HPRE; ++q)
-    if (h.e[q] >= 0) tq.put(BS + threadIdx.x + q * BS, quad(h.e[q]));
-  for (int k = threadIdx.x + HPRE * BS; k < h.n; k += BS) tq.put(BS + k, quad(gp(d.hal)[h.s + k]));
+  each_halo<BS>(d.hal, h, [&](int i, uint32_t e) { tq.put(BS + i, quad((int)idx_of(e))); });
   __syncthreads();
   if (j >= d.n || (SKIP_CHAN && (g.f & F_CHAN))) return;
   c.s = row_sum(g, c.m0, tq.get(g.l1), tq.get(g.l2), tq.get(g.l3), tq.get(g.l4));
@@ -874,7 +857,8 @@ void build_class_rows(HostMesh& hm) {
 int build_map(srs_ctx* c, HostMesh& hm, int tile, TileMap* m) {
   const int n = hm.n, np = hm.np, nt = (n + tile - 1) / tile;
   std::vector<uint16_t> loc(4 * (size_t)np, 0);
-  std::vector<int32_t> hal, hoff(nt + 1, 0), place(n, -1), out;
+  std::vector<uint32_t> hal;
+  std::vector<int32_t> hoff(nt + 1, 0), place(n, -1), out;
   int h_max = 0;
   for (int t = 0; t < nt; ++t) {
     const int j0 = t * tile, j1 = std::min(n, j0 + tile);
@@ -893,7 +877,7 @@ int build_map(srs_ctx* c, HostMesh& hm, int tile, TileMap* m) {
       loc[k] = (uint16_t)(e >= j0 && e < j0 + tile ? e - j0 : place[e]);
     }
     for (int e : out) place[e] = -1;
-    hal.insert(hal.end(), out.begin(), out.end());
+    for (int e : out) hal.push_back((uint32_t)e | ((hm.flags[e] & F_SL) ? IDX_SL : 0u));
     if (hal.size() > (size_t)INT32_MAX) return srs::fail(SRS_E_ARG, "mesh too large for its halo lists");
     hoff[t + 1] = (int32_t)hal.size();
     h_max = std::max(h_max, (int)out.size());
@@ -1308,12 +1292,10 @@ int srs_ctx_tune(srs_ctx* c, int32_t key, int32_t value) {
       return c->finalized ? tiles_full(c) : SRS_OK;
     case SRS_TUNE_ADJ_WAVES:
       if (value != 0 && value != 4) return srs::fail(SRS_E_ARG, "adjoint register budget must be 0 or 4");
-      c->adj_waves = value;
-      return SRS_OK;
+      return SRS_OK;  // four wavefronts per SIMD either way
     case SRS_TUNE_ADJ_W:
       if (value < 0 || value > 2) return srs::fail(SRS_E_ARG, "adjoint w form must be 0, 1 or 2");
-      c->adj_w = value;
-      return SRS_OK;
+      return SRS_OK;  // the gather reads the stored adjoint: no w
     case SRS_TUNE_ALT_ORDER:
       c->alt_order = value != 0;
       return c->finalized ? drop_graphs(c) : SRS_OK;
@@ -1549,7 +1531,10 @@ int srs_ctx_finalize(srs_ctx* c, int32_t record_capacity) {
       for (size_t k = 64 * b; k < std::min<size_t>(64 * b + 64, hm.n); ++k) plain &= hm.flags[k] == F_TROPC;
       if (plain) blk[b] |= BLK_PLAIN;
     }
-    if ((rc = dev_upload(c, &hm.d_nbr, hm.nbr))) return rc;
+    std::vector<uint32_t> nbr(hm.nbr.begin(), hm.nbr.end());
+    for (uint32_t& e : nbr)
+      if (hm.flags[e] & F_SL) e |= IDX_SL;
+    if ((rc = dev_upload(c, &hm.d_nbr, nbr))) return rc;
     if ((rc = dev_upload(c, &hm.d_blk, blk))) return rc;
     if ((rc = build_map(c, hm, c->tile, &hm.map))) return rc;
     c->sweep_lds = std::max(c->sweep_lds, 4 * sizeof(double) * (size_t)hm.map.qcap);
