@@ -31,6 +31,7 @@
 #include <functional>
 #include <mutex>
 #include <thread>
+#include <unordered_map>
 
 namespace srs_dev {
 
@@ -819,7 +820,19 @@ double quantize(double a, int bits) {
 // class_rows stays false unless every row of the mesh is reproduced exactly.
 void build_class_rows(HostMesh& hm) {
   const int n = hm.n, np = hm.np;
-  std::map<std::array<double, 5>, int> classes;
+  struct Hash {
+    size_t operator()(const std::array<double, 5>& k) const {
+      uint64_t h = 0;
+      for (double v : k) {
+        uint64_t u;
+        memcpy(&u, &v, 8);
+        h = (h ^ u) * 0x9E3779B97F4A7C15ull;
+        h ^= h >> 32;
+      }
+      return h;
+    }
+  };
+  std::unordered_map<std::array<double, 5>, int, Hash> classes;
   std::vector<uint32_t> row(3 * (size_t)np + 1, 0);
   for (int k = 0; k < n; ++k) {
     std::array<double, 5> key;
@@ -852,39 +865,101 @@ void build_class_rows(HostMesh& hm) {
   hm.class_rows = true;
 }
 
-// The tile map of a mesh for `tile` elements per tile, uploaded.  Halos are
-// sorted, so that a wavefront's loads of them fall in runs.
+// body(i) for i in [0, n), on up to eight threads for long work; false if a
+// body threw.
+template <class F>
+bool each_chunk(int n, F body) {
+  std::atomic<int> next{0};
+  std::atomic<bool> ok{true};
+  auto work = [&] {
+    try {
+      for (int i; (i = next.fetch_add(1)) < n && ok;) body(i);
+    } catch (...) {
+      ok = false;
+    }
+  };
+  std::vector<std::thread> th;
+  try {
+    const int helpers = std::min({n - 1, 7, (int)std::thread::hardware_concurrency() - 1});
+    for (int k = 0; k < helpers; ++k) th.emplace_back(work);
+  } catch (...) {  // fewer threads than asked for
+  }
+  work();
+  for (std::thread& t : th) t.join();
+  return ok;
+}
+
+// The tile map of a mesh for `tile` elements per tile, uploaded with the
+// neighbour table and the block flags.  Halos are sorted, so that a
+// wavefront's loads of them fall in runs.  Runs of tiles are independent:
+// finalizing the 3,000,000-element dyad takes 30 ms, 101 with them one after
+// another.
 int build_map(srs_ctx* c, HostMesh& hm, int tile, TileMap* m) {
   const int n = hm.n, np = hm.np, nt = (n + tile - 1) / tile;
+  const int run = (64 * 512 + tile - 1) / tile, n_run = (nt + run - 1) / run;
+  std::vector<uint32_t> nbr(hm.nbr.size()), blk(np / 64, 0);
   std::vector<uint16_t> loc(4 * (size_t)np, 0);
-  std::vector<uint32_t> hal;
-  std::vector<int32_t> hoff(nt + 1, 0), place(n, -1), out;
+  std::vector<std::vector<uint32_t>> halos(n_run);
+  std::vector<int32_t> hoff(nt + 1, 0);
+  const bool ok = each_chunk(n_run, [&](int q) {
+    std::vector<uint32_t>& hal = halos[q];
+    // the tile's foreign elements, and their places by element in a small
+    // open-addressed table (at most 4 tile of them)
+    uint32_t mask = 15;
+    while (mask + 1 < 8u * (uint32_t)tile) mask = 2 * mask + 1;
+    std::vector<int32_t> key(mask + 1, -1), place(mask + 1), out;
+    auto slot = [&](int e) {
+      uint32_t h = ((uint32_t)e * 2654435761u >> 7) & mask;
+      while (key[h] != e && key[h] >= 0) h = (h + 1) & mask;
+      return h;
+    };
+    for (int t = q * run; t < std::min(nt, (q + 1) * run); ++t) {
+      const int j0 = t * tile, j1 = std::min(n, j0 + tile);
+      out.clear();
+      for (size_t k = 4 * (size_t)j0; k < 4 * (size_t)j1; ++k) {
+        const int e = hm.nbr[k];
+        nbr[k] = (uint32_t)e | ((hm.flags[e] & F_SL) ? IDX_SL : 0u);
+        if (e >= j0 && e < j0 + tile) continue;
+        const uint32_t h = slot(e);
+        if (key[h] < 0) {
+          key[h] = e;
+          out.push_back(e);
+        }
+      }
+      std::sort(out.begin(), out.end());
+      for (size_t i = 0; i < out.size(); ++i) place[slot(out[i])] = tile + (int)i;
+      for (size_t k = 4 * (size_t)j0; k < 4 * (size_t)j1; ++k) {
+        const int e = hm.nbr[k];
+        loc[k] = (uint16_t)(e >= j0 && e < j0 + tile ? e - j0 : place[slot(e)]);
+      }
+      for (int e : out) hal.push_back((uint32_t)e | ((hm.flags[e] & F_SL) ? IDX_SL : 0u));
+      hoff[t + 1] = (int32_t)out.size();
+      std::fill(key.begin(), key.end(), -1);
+    }
+  });
+  if (!ok) return srs::fail(SRS_E_STATE, "out of host memory for the tile map");
+  for (size_t k = 4 * (size_t)n; k < nbr.size(); ++k) nbr[k] = (uint32_t)hm.nbr[k];
+  // the meshes' channel flags were set by add_realization: what blocks hold
+  for (size_t b = 0; b < blk.size(); ++b) {
+    bool plain = true;
+    for (size_t k = 64 * b; k < std::min<size_t>(64 * b + 64, n); ++k) plain &= hm.flags[k] == F_TROPC;
+    if (plain) blk[b] |= BLK_PLAIN;
+  }
+  size_t total = 0;
   int h_max = 0;
   for (int t = 0; t < nt; ++t) {
-    const int j0 = t * tile, j1 = std::min(n, j0 + tile);
-    out.clear();
-    for (size_t k = 4 * (size_t)j0; k < 4 * (size_t)j1; ++k) {
-      const int e = hm.nbr[k];
-      if ((e < j0 || e >= j0 + tile) && place[e] < 0) {
-        place[e] = 0;
-        out.push_back(e);
-      }
-    }
-    std::sort(out.begin(), out.end());
-    for (size_t i = 0; i < out.size(); ++i) place[out[i]] = tile + (int)i;
-    for (size_t k = 4 * (size_t)j0; k < 4 * (size_t)j1; ++k) {
-      const int e = hm.nbr[k];
-      loc[k] = (uint16_t)(e >= j0 && e < j0 + tile ? e - j0 : place[e]);
-    }
-    for (int e : out) place[e] = -1;
-    for (int e : out) hal.push_back((uint32_t)e | ((hm.flags[e] & F_SL) ? IDX_SL : 0u));
-    if (hal.size() > (size_t)INT32_MAX) return srs::fail(SRS_E_ARG, "mesh too large for its halo lists");
-    hoff[t + 1] = (int32_t)hal.size();
-    h_max = std::max(h_max, (int)out.size());
+    h_max = std::max(h_max, (int)hoff[t + 1]);
+    total += hoff[t + 1];
+    if (total > (size_t)INT32_MAX) return srs::fail(SRS_E_ARG, "mesh too large for its halo lists");
+    hoff[t + 1] = (int32_t)total;
   }
+  std::vector<uint32_t> hal;
+  hal.reserve(total + 1);
+  for (const auto& h : halos) hal.insert(hal.end(), h.begin(), h.end());
   if (hal.empty()) hal.push_back(0);
   int rc;
-  if ((rc = dev_upload(c, &m->d_loc, loc)) || (rc = dev_upload(c, &m->d_hal, hal)) ||
+  if ((rc = dev_upload(c, &hm.d_nbr, nbr)) || (rc = dev_upload(c, &hm.d_blk, blk)) ||
+      (rc = dev_upload(c, &m->d_loc, loc)) || (rc = dev_upload(c, &m->d_hal, hal)) ||
       (rc = dev_upload(c, &m->d_hoff, hoff)))
     return rc;
   m->n_halo = hoff[nt];
@@ -1524,18 +1599,6 @@ int srs_ctx_finalize(srs_ctx* c, int32_t record_capacity) {
   for (auto& hmp : c->meshes) c->class_all &= hmp->class_rows;
   for (auto& hmp : c->meshes) {
     HostMesh& hm = *hmp;
-    // the meshes' channel flags were set by add_realization: what blocks hold
-    std::vector<uint32_t> blk(hm.np / 64, 0);
-    for (size_t b = 0; b < blk.size(); ++b) {
-      bool plain = true;
-      for (size_t k = 64 * b; k < std::min<size_t>(64 * b + 64, hm.n); ++k) plain &= hm.flags[k] == F_TROPC;
-      if (plain) blk[b] |= BLK_PLAIN;
-    }
-    std::vector<uint32_t> nbr(hm.nbr.begin(), hm.nbr.end());
-    for (uint32_t& e : nbr)
-      if (hm.flags[e] & F_SL) e |= IDX_SL;
-    if ((rc = dev_upload(c, &hm.d_nbr, nbr))) return rc;
-    if ((rc = dev_upload(c, &hm.d_blk, blk))) return rc;
     if ((rc = build_map(c, hm, c->tile, &hm.map))) return rc;
     c->sweep_lds = std::max(c->sweep_lds, 4 * sizeof(double) * (size_t)hm.map.qcap);
     if (!c->class_all) {
