@@ -50,10 +50,22 @@ __device__ __forceinline__ SlBuf sl_buffer(const RealDesc& d, int j, double c, u
 // the blur's own points and weights (the cell's run of points within the
 // cut-off).  Every lane of the wavefront calls it (valid false: no element,
 // sum zero).  The loop runs over the points any lane can reach, the same for
-// the whole wavefront, so gcoef_i is one uniform load per point; each lane's
-// weights walk from anchors at multiples of the anchor spacing, so a lane's
-// weight at a point of its own run is the one its own walk would give (a
-// weight outside the run is never used, so it may be anything).
+// the whole wavefront, so gcoef_i is one uniform load per point (a weight
+// outside a lane's own run is never used, so it may be anything).
+template <bool WALK>
+__device__ __forceinline__ double scan_adj_run(const ScanGeo& g, const ScanCell& c, int n_f,
+                                               const double* __restrict__ gcoef, int lo, int hi, int i_lo, int i_hi) {
+  double s = 0.0;
+  for (int base = scan_seg(lo); base <= hi; base += SCAN_SEG)
+    scan_walk<WALK>(g, c, base, 1.0, [&](int a, int b) { return base + a <= hi && base + b >= lo; },
+                    [&](int m, double t) {
+                      const int i = base + m;
+                      const double gi = gcoef[min(i, n_f - 1)] * scan_power<WALK>(g, m);
+                      if (i >= i_lo && i <= i_hi) s += gi * t;
+                    });
+  return s;
+}
+
 __device__ __forceinline__ double scan_adj_sum(const double* __restrict__ cen, const ScanGeo& g, int n_f,
                                                const double* __restrict__ gcoef, size_t np, int j, bool valid) {
   int i_lo = n_f, i_hi = -1;
@@ -71,19 +83,9 @@ __device__ __forceinline__ double scan_adj_sum(const double* __restrict__ cen, c
   }
   lo = __builtin_amdgcn_readfirstlane(lo);
   hi = __builtin_amdgcn_readfirstlane(hi);
-  double s = 0.0;
-  if (lo > hi) return s;
-  const int i0 = __builtin_amdgcn_readfirstlane(scan_walk_start(g, lo));
-  double w = 0.0, r = 0.0;
-  for (int i = i0; i <= hi; ++i) {
-    const double pa = scan_pa(g, i);
-    if (scan_is_anchor(g, i, i0)) scan_anchor(g, c, pa, &w, &r);
-    const double gi = gcoef[i];
-    if (i >= i_lo && i <= i_hi) s += gi * w;
-    w *= r;
-    r *= g.q;
-  }
-  return s;
+  if (lo > hi) return 0.0;
+  return g.walk ? scan_adj_run<true>(g, c, n_f, gcoef, lo, hi, i_lo, i_hi)
+                : scan_adj_run<false>(g, c, n_f, gcoef, lo, hi, i_lo, i_hi);
 }
 
 // The loss source of a scan sample taken after n steps (SCAN), added to
@@ -725,9 +727,9 @@ static int loss_grad_run(srs_ctx* c, const std::vector<int32_t>& ids, int32_t sc
     HIPCHK(hipMemcpy(c->d_live, lv.data(), n_real * sizeof(RealLive), hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(d_rid, ids.data() + m0, nb * sizeof(int32_t), hipMemcpyHostToDevice));
     auto scan_into = [&](double* out) {
-      hipLaunchKernelGGL(k_scan_blur, dim3(S.n_blocks, nb), dim3(SCAN_BS), 0, c->stream, c->d_desc, c->d_live, 0,
+      hipLaunchKernelGGL(k_scan_blur, dim3(S.n_blocks, nb), dim3(SCAN_BS), scan_lds(nf), c->stream, c->d_desc, c->d_live, 0,
                          d_rid, S.d_cen, S.geo, nf, part);
-      hipLaunchKernelGGL(k_scan_final, dim3(1, nb), dim3(256), 0, c->stream, c->d_desc, c->d_live, 0, d_rid,
+      hipLaunchKernelGGL(k_scan_final, dim3(scan_final_blocks(nf), nb), dim3(SCAN_BS), 0, c->stream, c->d_desc, c->d_live, 0, d_rid,
                          S.n_blocks, nf, nca, part, S.d_pad, S.d_near_f, S.d_near_ca, S.desc.f0, S.desc.c0, out, nout);
     };
     auto ck_at = [&](int l, int64_t k) { return ckl[l] + (size_t)k * nb * n6; };

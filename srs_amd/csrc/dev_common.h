@@ -367,15 +367,18 @@ __device__ __forceinline__ uint32_t block_flags(const RealDesc& d, const int j) 
 // workgroup order; the padding cells' part is a per-point constant.
 //
 // Along the line only the axis term of the PSF's exponent changes, by a
-// quadratic in the point index, so a cell's weights at consecutive points
-// follow w(i+1) = w(i) r(i), r(i+1) = r(i) q with q = exp(-res^2 / s_a^2): two
-// products per point instead of an exponential.  The walk restarts from the
-// closed form at every SCAN_ANCHOR-th point, which keeps the rounding of a
-// weight within a few tens of ulps; a weight is a function of the cell and
-// the point alone, so the blur and the adjoint's loss source use the same
-// numbers.  PSFs so narrow that an anchor could underflow while its segment
-// holds a weight above exp(-260), or a ratio overflow, within a cell's reach
-// take the closed form at every point (walk = 0).
+// quadratic in the point index, so k points from a point of weight w0 and
+// ratio r0 = w(1) / w0 a cell's weight is w0 r0^k q^(k (k - 1) / 2) upwards and
+// w0 r0^-k q^(k (k + 1) / 2) downwards, q = exp(-res^2 / s_a^2): one product
+// per point and cell instead of an exponential, and the powers of q are factors
+// of a point's whole sum.  Points go in segments of SCAN_SEG, with the closed
+// form at the middle one (two exponentials per segment and cell), which keeps
+// the rounding of a weight within a few tens of ulps.  PSFs so narrow that a
+// middle weight could underflow while its segment holds a weight above
+// exp(-260), or a power of the ratio overflow, within a cell's reach take the
+// closed form at every point (walk = 0).
+constexpr int SCAN_SEG = 16, SCAN_HALF = SCAN_SEG / 2;
+
 struct ScanGeo {
   double base[3];   // scan line point with the axis coordinate zero
   int axis;
@@ -385,11 +388,9 @@ struct ScanGeo {
   double ia;        // inv[axis] (device code indexes no array by axis: the
                     // struct then stays in scalar registers)
   double kw;        // alpha / (sx sy sz)
-  double q;         // exp(-res^2 inv[axis])
+  double pw[SCAN_HALF + 1];  // q^(k (k + 1) / 2), q = exp(-res^2 inv[axis])
   int walk;         // 1: the recurrence above; 0: the closed form everywhere
 };
-
-constexpr int SCAN_ANCHOR = 8;
 
 // One cell's terms of the walk: its axis coordinate, the perpendicular
 // squares in the reference's summation order (distance^2 = (da^2 + u) + v,
@@ -429,13 +430,51 @@ __device__ __forceinline__ void scan_exact_range(const ScanGeo& g, const ScanCel
   while (*lo <= *hi && !(scan_dist2(c, scan_pa(g, *lo)) < 1.0)) ++*lo;
   while (*hi >= *lo && !(scan_dist2(c, scan_pa(g, *hi)) < 1.0)) --*hi;
 }
-// The first point of a walk that covers lo: its anchor.
-__device__ __forceinline__ int scan_walk_start(const ScanGeo& g, int lo) {
-  return g.walk ? lo - lo % SCAN_ANCHOR : lo;
+// The reciprocal of a ratio in the normal range, to the last bit or so.
+__device__ __forceinline__ double scan_rcp(double r) {
+  double x = __builtin_amdgcn_rcp(r);
+  x = __builtin_fma(x, __builtin_fma(-r, x, 1.0), x);
+  return __builtin_fma(x, __builtin_fma(-r, x, 1.0), x);
 }
-__device__ __forceinline__ bool scan_is_anchor(const ScanGeo& g, int i, int i0) {
-  return !g.walk || i == i0 || i % SCAN_ANCHOR == 0;
+// f(m, t) at the points base + m of a segment that use(first, last) asks for,
+// half by half: t times scan_power(m) is scale times the cell's weight there.
+template <bool WALK, class U, class F>
+__device__ __forceinline__ void scan_walk(const ScanGeo& g, const ScanCell& c, int base, double scale, U use, F f) {
+  if constexpr (WALK) {
+    double w0, r0;
+    scan_anchor(g, c, scan_pa(g, base + SCAN_HALF), &w0, &r0);
+    w0 *= scale;
+    if (use(SCAN_HALF, SCAN_SEG - 1)) {
+      double t = w0;
+#pragma unroll
+      for (int k = 0; k < SCAN_HALF; ++k) {
+        f(SCAN_HALF + k, t);
+        t *= r0;
+      }
+    }
+    if (use(0, SCAN_HALF - 1)) {
+      const double rd = scan_rcp(r0);
+      double t = w0;
+#pragma unroll
+      for (int k = 1; k <= SCAN_HALF; ++k) {
+        t *= rd;
+        f(SCAN_HALF - k, t);
+      }
+    }
+  } else {
+    for (int m = 0; m < SCAN_SEG; ++m) {
+      double w, r;
+      scan_anchor(g, c, scan_pa(g, base + m), &w, &r);
+      f(m, scale * w);
+    }
+  }
 }
+template <bool WALK>
+__device__ __forceinline__ double scan_power(const ScanGeo& g, int m) {
+  return !WALK ? 1.0 : m >= SCAN_HALF ? g.pw[m > SCAN_HALF ? m - SCAN_HALF - 1 : 0] : g.pw[SCAN_HALF - m];
+}
+// First point of the segment that holds point i.
+__device__ __forceinline__ int scan_seg(int i) { return i & ~(SCAN_SEG - 1); }
 
 // The scan points a cell at (cx, cy, cz) can reach (distance < 1 um): none
 // (lo > hi) when its distance to the line is 1 um or more, else those whose
@@ -462,6 +501,11 @@ __device__ __forceinline__ void scan_point_range(const ScanGeo& g, int n_f, doub
 constexpr int SCAN_BS = 256;
 constexpr int SCAN_MAX_POINTS = 1024;
 constexpr int SCAN_CELLS_PER_THREAD = 4;
+
+// LDS of the blur's workgroup, its wavefronts' sums per point, and the
+// workgroups of the final sum, a wavefront per point.
+inline size_t scan_lds(int n_f) { return sizeof(double) * (SCAN_BS / 64) * (size_t)n_f; }
+inline unsigned scan_final_blocks(int n_f) { return (unsigned)std::max(1, (n_f + SCAN_BS / 64 - 1) / (SCAN_BS / 64)); }
 
 // Realization of workgroup row blockIdx.y in a batched launch: rid[blockIdx.y],
 // or r when there is no table (a launch for one realization).

@@ -896,7 +896,7 @@ bool each_chunk(int n, F body) {
 // another.
 int build_map(srs_ctx* c, HostMesh& hm, int tile, TileMap* m) {
   const int n = hm.n, np = hm.np, nt = (n + tile - 1) / tile;
-  const int run = (64 * 512 + tile - 1) / tile, n_run = (nt + run - 1) / run;
+  const int run = (16 * 512 + tile - 1) / tile, n_run = (nt + run - 1) / run;
   std::vector<uint32_t> nbr(hm.nbr.size()), blk(np / 64, 0);
   std::vector<uint16_t> loc(4 * (size_t)np, 0);
   std::vector<std::vector<uint32_t>> halos(n_run);

@@ -5,111 +5,151 @@
 
 namespace srs_dev {
 
-__global__ __launch_bounds__(SCAN_BS) void k_scan_blur(const RealDesc* __restrict__ D, const RealLive* __restrict__ L,
+// A wavefront's sums at the points of [lo, hi], added up over its cells.
+template <bool WALK>
+__device__ __forceinline__ void blur_points(const ScanGeo& g, int n_f, int lo, int hi,
+                                            const ScanCell (&sc)[SCAN_CELLS_PER_THREAD],
+                                            const double (&vf)[SCAN_CELLS_PER_THREAD],
+                                            const int (&clo)[SCAN_CELLS_PER_THREAD],
+                                            const int (&chi)[SCAN_CELLS_PER_THREAD], double* __restrict__ rw) {
+  typedef double v4 __attribute__((ext_vector_type(4)));
+  const int lane = threadIdx.x & 63;
+  for (int base = scan_seg(lo); base <= hi; base += SCAN_SEG) {
+    double acc[SCAN_SEG];
+#pragma unroll
+    for (int m = 0; m < SCAN_SEG; ++m) acc[m] = 0.0;
+#pragma unroll
+    for (int q = 0; q < SCAN_CELLS_PER_THREAD; ++q) {
+      const int a = clo[q] - base, b = chi[q] - base;  // the cell's points, a <= m <= b
+      auto any = [&](int m0, int m1) { return __builtin_amdgcn_ballot_w64(a <= m1 && b >= m0) != 0; };
+      if (!any(0, SCAN_SEG - 1)) continue;
+      scan_walk<WALK>(g, sc[q], base, vf[q], any, [&](int m, double t) {
+        if (a <= m && m <= b) {
+          acc[m] += t;
+          asm volatile("" : "+v"(acc[m]));  // a branch: skipping lanes beats two selects
+        }
+      });
+    }
+    // Four points at a time: a matrix instruction with a matrix of ones adds the
+    // lanes l, l + 16, l + 32, l + 48 in FP64, the sums of four points are placed
+    // in a row of 16 lanes each, and lane moves add the rows.
+#pragma unroll
+    for (int m0 = 0; m0 < SCAN_SEG; m0 += 4) {
+      double v = 0.0;
+#pragma unroll
+      for (int p = 0; p < 4; ++p) {
+        const v4 z = {0.0, 0.0, 0.0, 0.0};
+        const double s =
+            __builtin_amdgcn_mfma_f64_16x16x4f64(1.0, acc[m0 + p], z, 0, 0, 0)[0] * scan_power<WALK>(g, m0 + p);
+        v = lane >> 4 == p ? s : v;
+      }
+      v = row_sum_dpp(v);
+      const int i = base + m0 + (lane >> 4);
+      if ((lane & 15) == 15 && i < n_f) rw[i] = v;
+    }
+  }
+}
+
+// The blur's partial sums per workgroup and point.  Bound by vector
+// instructions: about 110 per segment and cell for the two exponentials, 5 per
+// point and cell for the walk and the cell's own range, 7 per point and
+// wavefront for the sums.  927,816 cells and 96 points 56 us (80 with a walk
+// of weight and ratio from an exponential every eight points, and a full
+// lane-move sum per point), eight members in one launch 261 us (313).  Four
+// cells per thread: the sums per point cost as much as two more cells (two:
+// 60 and 324 us).
+__global__ __launch_bounds__(SCAN_BS) __attribute__((amdgpu_waves_per_eu(4))) void k_scan_blur(const RealDesc* __restrict__ D, const RealLive* __restrict__ L,
                                                       int r, const int32_t* __restrict__ rid,
                                                       const double* __restrict__ cen, ScanGeo g, int n_f,
                                                       double* __restrict__ part) {
-  __shared__ double red[SCAN_BS / 64][SCAN_MAX_POINTS];
+  constexpr int NC = SCAN_CELLS_PER_THREAD;
+  extern __shared__ double red[];  // [wavefront][point]
   r = batch_real(rid, r);
   part += (size_t)blockIdx.y * gridDim.x * n_f;
   const RealDesc& d = D[r];
   const double* X = d.X[L[r].cur];
   const int n = d.n, np = d.np;
-  double cx[SCAN_CELLS_PER_THREAD], cy[SCAN_CELLS_PER_THREAD], cz[SCAN_CELLS_PER_THREAD], vf[SCAN_CELLS_PER_THREAD];
-  for (int q = 0; q < SCAN_CELLS_PER_THREAD; ++q) {
-    const int j = (blockIdx.x * SCAN_CELLS_PER_THREAD + q) * SCAN_BS + threadIdx.x;
-    if (j < n) {
-      cx[q] = cen[j]; cy[q] = cen[np + j]; cz[q] = cen[2 * np + j];
-      vf[q] = d.V0[j] * X[cq(d, j) + FLUO_OFF];  // V0 * Ca-bound Fluo
-    } else {
-      cx[q] = cy[q] = cz[q] = 1e30;  // beyond the 1 um cut-off of every point
-      vf[q] = 0.0;
-    }
-  }
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  // The points any cell of this wavefront can reach: outside them every
-  // lane's sum is zero, so the wavefront's partial is written as zero
-  // without the loop (the same bits as the full loop).
+  double* rw = red + wave * n_f;
+  for (int i = lane; i < n_f; i += 64) rw[i] = 0.0;
+  // each cell's points within the cut-off, and those any cell of the wavefront
+  // can reach: no other point is visited
+  // (every cell's loads first: a cell beyond the mesh reads the last one's)
   int lo = n_f, hi = -1;
-  ScanCell sc[SCAN_CELLS_PER_THREAD];
-  int clo[SCAN_CELLS_PER_THREAD], chi[SCAN_CELLS_PER_THREAD];  // each cell's points within the cut-off
-  for (int q = 0; q < SCAN_CELLS_PER_THREAD; ++q) {
+  double vf[NC], cx[NC], cy[NC], cz[NC];
+#pragma unroll
+  for (int q = 0; q < NC; ++q) {
+    const int j = min((int)(blockIdx.x * NC + q) * SCAN_BS + (int)threadIdx.x, n - 1);
+    cx[q] = gp(cen)[j], cy[q] = gp(cen)[np + j], cz[q] = gp(cen)[2 * np + j];
+    vf[q] = gp(d.V0)[j] * gp(X)[cq(d, j) + FLUO_OFF];  // V0 * Ca-bound Fluo
+  }
+  ScanCell sc[NC];
+  int clo[NC], chi[NC];
+#pragma unroll
+  for (int q = 0; q < NC; ++q) {
+    const int j = (blockIdx.x * NC + q) * SCAN_BS + threadIdx.x;
     sc[q] = scan_cell(g, cx[q], cy[q], cz[q]);
-    const int j = (blockIdx.x * SCAN_CELLS_PER_THREAD + q) * SCAN_BS + threadIdx.x;
-    clo[q] = n_f;
-    chi[q] = -1;
+    int a = n_f, b = -1;
     if (j < n) {
-      scan_point_range(g, n_f, cx[q], cy[q], cz[q], &clo[q], &chi[q]);
-      scan_exact_range(g, sc[q], &clo[q], &chi[q]);
-      if (clo[q] <= chi[q]) {
-        lo = min(lo, clo[q]);
-        hi = max(hi, chi[q]);
-      }
+      scan_point_range(g, n_f, cx[q], cy[q], cz[q], &a, &b);
+      scan_exact_range(g, sc[q], &a, &b);
     }
+    clo[q] = a <= b ? a : n_f;
+    chi[q] = a <= b ? b : -1;
+    lo = min(lo, clo[q]);
+    hi = max(hi, chi[q]);
   }
   for (int o = 32; o > 0; o >>= 1) {
     lo = min(lo, __shfl_xor(lo, o));
     hi = max(hi, __shfl_xor(hi, o));
   }
-  if (lane == 0) {
-    for (int i = 0; i < min(lo, n_f); ++i) red[wave][i] = 0.0;
-    for (int i = max(hi + 1, 0); i < n_f; ++i) red[wave][i] = 0.0;
-  }
-  // Each cell's weights by the walk from the anchor at or below lo (a weight
-  // outside the cell's run of points within the cut-off is never used, so it
-  // may be anything).
-  const int i0 = scan_walk_start(g, lo);
-  double ww[SCAN_CELLS_PER_THREAD], wr[SCAN_CELLS_PER_THREAD];
-  for (int i = i0; i <= hi; ++i) {
-    const double pa = scan_pa(g, i);
-    const bool anchor = scan_is_anchor(g, i, i0);  // uniform across the wavefront
-    double acc = 0.0;
-    for (int q = 0; q < SCAN_CELLS_PER_THREAD; ++q) {
-      if (anchor) scan_anchor(g, sc[q], pa, &ww[q], &wr[q]);
-      if (i >= clo[q] && i <= chi[q]) acc += vf[q] * ww[q];
-      ww[q] *= wr[q];
-      wr[q] *= g.q;
-    }
-    if (i < lo) continue;
-    acc = wave_sum_dpp(acc);
-    if (lane == 63) red[wave][i] = acc;
-  }
+  lo = __builtin_amdgcn_readfirstlane(lo);
+  hi = __builtin_amdgcn_readfirstlane(hi);
+  if (g.walk) blur_points<true>(g, n_f, lo, hi, sc, vf, clo, chi, rw);
+  else blur_points<false>(g, n_f, lo, hi, sc, vf, clo, chi, rw);
   __syncthreads();
   for (int i = threadIdx.x; i < n_f; i += SCAN_BS) {
     double s = 0.0;
-    for (int w = 0; w < SCAN_BS / 64; ++w) s += red[w][i];
+    for (int w = 0; w < SCAN_BS / 64; ++w) s += red[w * n_f + i];
     part[(size_t)blockIdx.x * n_f + i] = s;
   }
 }
 
-__global__ void k_scan_final(const RealDesc* __restrict__ D, const RealLive* __restrict__ L, int r,
-                             const int32_t* __restrict__ rid, int n_blocks, int n_f, int n_ca,
-                             const double* __restrict__ part, const double* __restrict__ pad,
-                             const int32_t* __restrict__ near_f, const int32_t* __restrict__ near_ca, double f0,
-                             double c0, double* __restrict__ out, int out_stride) {
+// The workgroups' partial sums of each point, with the padding cells' part,
+// and the values at the cells nearest the line.  A wavefront per point: each
+// lane sums every 64th workgroup's partial, then the lanes' sums by DPP (a
+// fixed order: deterministic).  906 partials of 96 points take 7 us; one
+// workgroup for all points took 72.
+__global__ __launch_bounds__(SCAN_BS) void k_scan_final(const RealDesc* __restrict__ D, const RealLive* __restrict__ L,
+                                                       int r, const int32_t* __restrict__ rid, int n_blocks, int n_f,
+                                                       int n_ca, const double* __restrict__ part,
+                                                       const double* __restrict__ pad,
+                                                       const int32_t* __restrict__ near_f,
+                                                       const int32_t* __restrict__ near_ca, double f0, double c0,
+                                                       double* __restrict__ out, int out_stride) {
   r = batch_real(rid, r);
   part += (size_t)blockIdx.y * n_blocks * n_f;
   out += (size_t)blockIdx.y * out_stride;
   const double* X = D[r].X[L[r].cur];
-  // a wavefront per point: each lane sums every 64th workgroup's partial,
-  // then the lanes' sums by DPP (a fixed order: deterministic)
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, n_waves = blockDim.x >> 6;
-  for (int i = wave; i < n_f; i += n_waves) {
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int i = blockIdx.x * (SCAN_BS / 64) + wave;
+  if (i < n_f) {
     double s = 0.0;
+#pragma unroll 4
     for (int b = lane; b < n_blocks; b += 64) s += part[(size_t)b * n_f + i];
     s = wave_sum_dpp(s);
     if (lane == 63) out[n_ca + n_f + i] = s + pad[i];
   }
-  for (int i = threadIdx.x; i < n_f; i += blockDim.x) {
-    const int e = near_f[i];
-    out[n_ca + i] = e >= 0 ? X[cq(D[r], e) + FLUO_OFF] : f0;
+  const int t = blockIdx.x * SCAN_BS + threadIdx.x, nt = gridDim.x * SCAN_BS;
+  for (int k = t; k < n_f; k += nt) {
+    const int e = near_f[k];
+    out[n_ca + k] = e >= 0 ? X[cq(D[r], e) + FLUO_OFF] : f0;
   }
-  for (int i = threadIdx.x; i < n_ca; i += blockDim.x) {
-    const int e = near_ca[i];
-    out[i] = e >= 0 ? X[cq(D[r], e)] : c0;
+  for (int k = t; k < n_ca; k += nt) {
+    const int e = near_ca[k];
+    out[k] = e >= 0 ? X[cq(D[r], e)] : c0;
   }
 }
-
 
 }  // namespace srs_dev
 
@@ -153,15 +193,15 @@ int srs_ctx_add_scan(srs_ctx* c, int32_t mesh_id, const double* centers, const s
   g.ia = g.inv[g.axis];
   g.kw = g.alpha / (g.sx * g.sy * g.sz);
   {
-    // The walk is safe when an anchor SCAN_ANCHOR - 1 points before a point
-    // of weight ~1 has an exponent below 100 (then a weight exp(-x) of the
-    // segment can be lost to the anchor's underflow only for x > 260) and
-    // the ratio stays finite over a cell's reach (|da| < 1 + (SCAN_ANCHOR +
-    // 1) res).
+    // The walk is safe when an anchor SCAN_HALF points away from a point of
+    // weight ~1 has an exponent below 100 (then a weight exp(-x) of the
+    // segment can be lost to the anchor's underflow only for x > 260) and the
+    // powers of the ratio stay finite over a cell's reach (|da| < 1 +
+    // (SCAN_HALF + 1) res).
     const double ia = g.inv[g.axis], h = g.res;
-    const double far = (SCAN_ANCHOR - 1) * h;
-    g.walk = 0.5 * far * far * ia < 100.0 && h * (1.0 + (SCAN_ANCHOR + 1) * h) * ia < 600.0;
-    g.q = std::exp(-h * h * ia);
+    const double far = SCAN_HALF * h;
+    g.walk = 0.5 * far * far * ia < 100.0 && SCAN_HALF * h * (1.0 + (SCAN_HALF + 1) * h) * ia < 600.0;
+    for (int k = 0; k <= SCAN_HALF; ++k) g.pw[k] = (double)std::exp(-(long double)h * h * ia * (k * (k + 1) / 2));
   }
 
   // padding cells, linescan/main.cpp:119-141 and AddPointGrid :268-306
@@ -258,9 +298,9 @@ int srs_scan_sample(srs_ctx* c, int32_t r, int32_t scan_id, double* ca, double* 
   if (c->reals[r].mesh != S.mesh) return srs::fail(SRS_E_ARG, "realization %d is not on the scan's mesh", r);
   HIPCHK(hipSetDevice(c->device));
   if (S.n_f > 0)
-    hipLaunchKernelGGL(k_scan_blur, dim3(S.n_blocks), dim3(SCAN_BS), 0, c->stream, c->d_desc, c->d_live, r, nullptr,
+    hipLaunchKernelGGL(k_scan_blur, dim3(S.n_blocks), dim3(SCAN_BS), scan_lds(S.n_f), c->stream, c->d_desc, c->d_live, r, nullptr,
                        S.d_cen, S.geo, S.n_f, S.d_part);
-  hipLaunchKernelGGL(k_scan_final, dim3(1), dim3(256), 0, c->stream, c->d_desc, c->d_live, r, nullptr, S.n_blocks,
+  hipLaunchKernelGGL(k_scan_final, dim3(scan_final_blocks(S.n_f)), dim3(SCAN_BS), 0, c->stream, c->d_desc, c->d_live, r, nullptr, S.n_blocks,
                      S.n_f, S.n_ca, S.d_part, S.d_pad, S.d_near_f, S.d_near_ca, S.desc.f0, S.desc.c0, S.d_out, 0);
   HIPCHK(hipGetLastError());
   std::vector<double> out((size_t)S.n_ca + 2 * (size_t)S.n_f);
