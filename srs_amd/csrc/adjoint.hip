@@ -411,19 +411,11 @@ __global__ void k_seg_start(const RealDesc* __restrict__ D, RealLive* __restrict
   }
 }
 
-// Writes each step's RyR states (the ones the next step's fluxes use) into a
-// schedule, for srs_record_schedule.
-__global__ void k_sched_out(const RealDesc* __restrict__ D, const RealLive* __restrict__ L,
-                            const int64_t* __restrict__ base, const size_t* __restrict__ off, int32_t* out,
-                            int64_t n_rows) {
-  const int r = blockIdx.x;
-  const RealDesc& d = D[r];
-  const int64_t row = L[r].step - base[r];  // k_gate already advanced the step counter
-  if (row < 1 || row >= n_rows) return;
-  out += off[r];
-  for (int i = threadIdx.x; i < d.n_ryr; i += blockDim.x) out[row * d.n_ryr + i] = d.ryr_state[i];
+// Row 0 of each realization's recorded schedule: its RyR states now.
+__global__ void k_sched_first(const RealDesc* __restrict__ D) {
+  const RealDesc& d = D[blockIdx.x];
+  for (int i = threadIdx.x; i < d.n_ryr; i += blockDim.x) d.sched[i] = d.ryr_state[i];
 }
-
 
 }  // namespace srs_dev
 
@@ -488,36 +480,39 @@ static int record_run(srs_ctx* c, int64_t n_steps, int32_t* out_host) {
   HIPCHK(hipStreamSynchronize(c->stream));
   std::vector<RealLive> lv(n_real);
   HIPCHK(hipMemcpy(lv.data(), c->d_live, n_real * sizeof(RealLive), hipMemcpyDeviceToHost));
-  std::vector<int64_t> base(n_real);
   std::vector<size_t> off(n_real + 1, 0);
   for (int r = 0; r < n_real; ++r) {
     if (lv[r].done) return srs::fail(SRS_E_ARG, "record schedule: realization %d has finished its protocol", r);
-    base[r] = lv[r].step;
     off[r + 1] = off[r] + (size_t)n_steps * c->reals[r].ryr_ele.size();
   }
+  bool gated;
+  int cur;
+  int rc = gated_start(c, &gated, &cur);
+  if (rc) return rc;
   DevMem M;
   int32_t* d_out = nullptr;
-  int64_t* d_base = nullptr;
-  size_t* d_off = nullptr;
   HIPCHK(M.alloc(&d_out, off[n_real]));
-  HIPCHK(M.alloc(&d_base, (size_t)n_real));
-  HIPCHK(M.alloc(&d_off, (size_t)n_real));
-  HIPCHK(hipMemcpy(d_base, base.data(), n_real * sizeof(int64_t), hipMemcpyHostToDevice));
-  HIPCHK(hipMemcpy(d_off, off.data(), n_real * sizeof(size_t), hipMemcpyHostToDevice));
-  for (int r = 0; r < n_real; ++r)
-    if (off[r + 1] > off[r])
-      HIPCHK(hipMemcpy(d_out + off[r], c->reals[r].desc.ryr_state, c->reals[r].ryr_ele.size() * sizeof(int32_t),
-                       hipMemcpyDeviceToDevice));
-  hipError_t e = hipSuccess;
-  for (int64_t k = 0; k < n_steps && e == hipSuccess; ++k) {
-    launch_step(c, G_AFTER_SWEEP);
-    hipLaunchKernelGGL(k_sched_out, dim3(n_real), dim3(256), 0, c->stream, c->d_desc, c->d_live, d_base, d_off,
-                       d_out, n_steps);
-    e = hipGetLastError();
-    if (e == hipSuccess && (k & 1023) == 1023) e = hipStreamSynchronize(c->stream);
+  // the gating writes each step's row to the descriptors' schedules
+  std::vector<RealDesc> own(n_real), rec(n_real);
+  for (int r = 0; r < n_real; ++r) {
+    own[r] = rec[r] = c->reals[r].desc;
+    rec[r].sched = d_out + off[r];
+    rec[r].n_sched = n_steps;
+    rec[r].rec_step0 = lv[r].step;
   }
-  if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+  HIPCHK(hipMemcpy(c->d_desc, rec.data(), n_real * sizeof(RealDesc), hipMemcpyHostToDevice));
+  hipLaunchKernelGGL(k_sched_first, dim3(n_real), dim3(256), 0, c->stream, c->d_desc);
+  hipError_t e = hipGetLastError();
+  for (int64_t k = 0; k < n_steps && e == hipSuccess; k += 1024) {
+    const int64_t m = std::min<int64_t>(1024, n_steps - k);
+    launch_steps(c, m, G_AFTER_SWEEP | G_RECORD, gated, cur);  // an even count leaves cur as it was
+    e = hipGetLastError();
+    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+  }
+  (void)hipStreamSynchronize(c->stream);
   if (e == hipSuccess) e = hipMemcpy(out_host, d_out, off[n_real] * sizeof(int32_t), hipMemcpyDeviceToHost);
+  const hipError_t e2 = hipMemcpy(c->d_desc, own.data(), n_real * sizeof(RealDesc), hipMemcpyHostToDevice);
+  if (e == hipSuccess) e = e2;
   if (e != hipSuccess) return srs::fail(SRS_E_HIP, "record schedule: %s", hipGetErrorString(e));
   return SRS_OK;
 }

@@ -8,6 +8,7 @@
 
 #include <algorithm>
 #include <array>
+#include <atomic>
 #include <cstddef>
 #include <cmath>
 #include <cstdio>
@@ -15,6 +16,7 @@
 #include <map>
 #include <memory>
 #include <numeric>
+#include <thread>
 #include <vector>
 
 #include "kinetics.h"
@@ -123,8 +125,9 @@ struct RealDesc {
   const int32_t* cstart;  // [n_celem+1]
   const ChanEntry* centry;
   const ChanElem* crec;   // [n_celem] what an element of celem is updated from
-  const int32_t* sched;   // replay schedule [n_sched][n_ryr] or null
+  int32_t* sched;         // replay or recorded schedule [n_sched][n_ryr] or null
   int64_t n_sched;
+  int64_t rec_step0;      // the step that row 0 of a recorded schedule is before
   float* rec;
   int32_t rec_cap, rec_len, ryr_out, gpu_layout;
   uint64_t key, stream;
@@ -169,6 +172,7 @@ enum : uint32_t {
   G_PROTOCOL = 2,     // run the loop body for the next time
   G_NO_GATING = 4,    // skip gating regardless of the parameter flag
   G_REPLAY = 8,       // load RyR states for the next step from the schedule
+  G_RECORD = 16,      // write RyR states for the next step to the schedule
 };
 
 __device__ __forceinline__ int xcd_tile(int bid, int grid) {
@@ -524,6 +528,30 @@ struct DevBuf {
   size_t bytes = 0;
 };
 
+// body(i) for i in [0, n), on up to eight threads for long work; false if a
+// body threw.
+template <class F>
+bool each_chunk(int n, F body) {
+  std::atomic<int> next{0};
+  std::atomic<bool> ok{true};
+  auto work = [&] {
+    try {
+      for (int i; (i = next.fetch_add(1)) < n && ok;) body(i);
+    } catch (...) {
+      ok = false;
+    }
+  };
+  std::vector<std::thread> th;
+  try {
+    const int helpers = std::min({n - 1, 7, (int)std::thread::hardware_concurrency() - 1});
+    for (int k = 0; k < helpers; ++k) th.emplace_back(work);
+  } catch (...) {  // fewer threads than asked for
+  }
+  work();
+  for (std::thread& t : th) t.join();
+  return ok;
+}
+
 // Where the neighbours of a tile's elements are once the tile is staged: place
 // k < tile is the tile's own element k, place tile + i the i-th of its halo.
 struct TileMap {
@@ -695,6 +723,8 @@ int tiles_full(srs_ctx* c);
 int tiles_compact(srs_ctx* c);
 int plan_subsets(srs_ctx* c);
 void launch_subset_block(srs_ctx* c, int64_t m, uint32_t gmode);
+int gated_start(srs_ctx* c, bool* ok, int* cur);
+void launch_steps(srs_ctx* c, int64_t n_steps, uint32_t gmode, bool gated, int cur);
 int live_rw(srs_ctx* c, int32_t r, RealLive* lv, bool write);
 int state_xfer(srs_ctx* c, int32_t r, double* host, bool to_dev);
 

@@ -252,25 +252,30 @@ int srs_ctx_add_scan(srs_ctx* c, int32_t mesh_id, const double* centers, const s
   };
   std::vector<int32_t> near_f(S.n_f), near_ca(S.n_ca);
   std::vector<double> pad(S.n_f);
-  for (int i = 0; i < S.n_f; ++i) {
-    double p[3] = {g.base[0], g.base[1], g.base[2]};
-    p[g.axis] = sd->x_min + i * sd->res_x_f;
-    near_f[i] = nearest(p);
-    double sum = 0.0;
-    for (size_t k = 0; k < pc.size(); ++k) {
-      const double rx = pc[k][0] - p[0], ry = pc[k][1] - p[1], rz = pc[k][2] - p[2];
-      if (rx * rx + ry * ry + rz * rz < 1.0)
-        sum += pv[k] * sd->f0 *
-               (g.alpha * std::exp(-0.5 * ((rx * rx / (g.sx * g.sx)) + (ry * ry / (g.sy * g.sy)) + (rz * rz / (g.sz * g.sz)))) /
-                (g.sx * g.sy * g.sz));
+  // 16 points at a time, on several threads
+  const bool ok = each_chunk((S.n_f + S.n_ca + 15) / 16, [&](int q) {
+    for (int i = 16 * q; i < std::min(16 * q + 16, S.n_f + S.n_ca); ++i) {
+      double p[3] = {g.base[0], g.base[1], g.base[2]};
+      if (i >= S.n_f) {
+        p[g.axis] = sd->x_min + (i - S.n_f) * sd->res_x_ca;
+        near_ca[i - S.n_f] = nearest(p);
+        continue;
+      }
+      p[g.axis] = sd->x_min + i * sd->res_x_f;
+      near_f[i] = nearest(p);
+      double sum = 0.0;
+      for (size_t k = 0; k < pc.size(); ++k) {
+        const double rx = pc[k][0] - p[0], ry = pc[k][1] - p[1], rz = pc[k][2] - p[2];
+        if (rx * rx + ry * ry + rz * rz < 1.0)
+          sum += pv[k] * sd->f0 *
+                 (g.alpha *
+                  std::exp(-0.5 * ((rx * rx / (g.sx * g.sx)) + (ry * ry / (g.sy * g.sy)) + (rz * rz / (g.sz * g.sz)))) /
+                  (g.sx * g.sy * g.sz));
+      }
+      pad[i] = sum;
     }
-    pad[i] = sum;
-  }
-  for (int i = 0; i < S.n_ca; ++i) {
-    double p[3] = {g.base[0], g.base[1], g.base[2]};
-    p[g.axis] = sd->x_min + i * sd->res_x_ca;
-    near_ca[i] = nearest(p);
-  }
+  });
+  if (!ok) return srs::fail(SRS_E_STATE, "out of host memory for the scan line");
   std::vector<double> cen(3 * (size_t)np, 1e30);
   for (int k = 0; k < n; ++k)
     for (int q = 0; q < 3; ++q) cen[(size_t)q * np + k] = centers[3 * (size_t)hm.perm[k] + q];
