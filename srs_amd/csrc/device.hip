@@ -811,16 +811,26 @@ __global__ __launch_bounds__(256) void k_state_xfer(const RealDesc* __restrict__
 
 // ----------------------------------------------------------------- host side
 
-// Rounds the significand to `bits` bits (class key of a coefficient).
-double quantize(double a, int bits) {
+// Rounds the significand to 40 bits, ties to even (class key of a coefficient).
+double quantize(double a) {
+  uint64_t u;
+  memcpy(&u, &a, 8);
+  const uint64_t e = u >> 52 & 0x7ff;
+  if (e != 0 && e < 0x7fe) {  // normal, and so after a carry: 13 bits go
+    u = (u + 0xfff + (u >> 13 & 1)) & ~(uint64_t)0x1fff;
+    memcpy(&a, &u, 8);
+    return a;
+  }
   if (a == 0.0 || !std::isfinite(a)) return a;
-  int e;
-  const double m = std::frexp(a, &e);
-  return std::ldexp(std::nearbyint(std::ldexp(m, bits)), e - bits);
+  int x;
+  const double m = std::frexp(a, &x);
+  return std::ldexp(std::nearbyint(std::ldexp(m, 40)), x - 40);
 }
 
 // Each coefficient row as a class row plus int16 deltas of the bit patterns.
-// class_rows stays false unless every row of the mesh is reproduced exactly.
+// class_rows stays false unless every row of the mesh is reproduced exactly,
+// and where classes are hardly fewer than rows (an irregular mesh), so that
+// the table would be as much to read as the rows.
 void build_class_rows(HostMesh& hm) {
   const int n = hm.n, np = hm.np;
   struct Hash {
@@ -843,7 +853,7 @@ void build_class_rows(HostMesh& hm) {
     for (int q = 0; q < 5; ++q) {
       const double a = hm.coef[(size_t)q * np + k];
       if (!std::isfinite(a) || (a == 0.0 && std::signbit(a))) return;  // the classes are keyed by value
-      key[q] = quantize(a, 40);
+      key[q] = quantize(a);
       int64_t ka, kt;
       memcpy(&ka, &a, 8);
       memcpy(&kt, &key[q], 8);
@@ -852,7 +862,7 @@ void build_class_rows(HostMesh& hm) {
     }
     auto it = classes.find(key);
     if (it == classes.end()) {
-      if (classes.size() >= 65535) return;
+      if (classes.size() >= 65535 || (classes.size() >= 8192 && 2 * classes.size() > (size_t)k)) return;
       it = classes.emplace(key, (int)classes.size()).first;
     }
     auto u = [](int64_t v) { return (uint32_t)(uint16_t)v; };
