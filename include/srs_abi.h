@@ -287,14 +287,13 @@ int srs_ctx_create(int device, srs_ctx** out);
 #define SRS_TUNE_OCCUPANCY 6     /* register budget of the single-realization step with the gating folded
                                     in (SRS_TUNE_GATED_SWEEP): 0 by the mesh's size; 6 or 8: at most 80
                                     VGPRs, so that six wavefronts share each SIMD */
-#define SRS_TUNE_GROUP 7         /* 1 (default), 2 or 4: realizations of one mesh whose states are interleaved
-                                    per 64 elements and whose tiles are swept side by side, so that the
-                                    operator rows come from cache for all but the first (set before
-                                    srs_ctx_finalize) */
+#define SRS_TUNE_GROUP 7         /* accepted (1, 2 or 4; set before srs_ctx_finalize): results and speed do not
+                                    depend on it.  The adjoint needs 1.  Every realization has buffers of
+                                    its own; the order of the tiles is chosen by size */
 #define SRS_TUNE_LDS 8           /* accepted and ignored: each sweep tile's diffusing species, and those
                                     of the elements its own neighbour, are always staged in LDS */
-#define SRS_TUNE_DROP_FINISHED 9 /* 1 (default): srs_explicit_step leaves the tiles of groups whose
-                                    realizations have all finished out of the sweep; 0: sweep them all */
+#define SRS_TUNE_DROP_FINISHED 9 /* 1 (default): srs_explicit_step leaves the tiles of finished
+                                    realizations out of the sweep; 0: sweeps them all */
 #define SRS_TUNE_GATED_SWEEP 10  /* 1 (default): a single-realization context runs each
                                     step's gating (and, with SRS_STEP_PROTOCOL, the loop body) inside the
                                     next step's sweep launch; 0: a gating launch after every sweep */

@@ -692,7 +692,7 @@ static int loss_grad_run(srs_ctx* c, const std::vector<int32_t>& ids, int32_t sc
     if (n_real > 1) {
       sub_tiles.clear();
       for (int y = 0; y < nb; ++y)
-        for (int t = 0; t < nt_mesh; ++t) sub_tiles.push_back(make_int2(c->reals[ids[m0 + y]].group, t));
+        for (int t = 0; t < nt_mesh; ++t) sub_tiles.push_back(make_int2(ids[m0 + y], t));
       HIPCHK(hipMemcpy(d_sub_tiles, sub_tiles.data(), sub_tiles.size() * sizeof(int2), hipMemcpyHostToDevice));
       c->d_tiles = d_sub_tiles;
       c->n_tiles = (int)sub_tiles.size();

@@ -50,25 +50,14 @@ enum : uint32_t {
 // against 6.3, and the write requests to L2 were 72 per wavefront instead of
 // 40 (48-member ensemble: 175.7 -> 171.8 us per step; with non-temporal
 // stores, which that form had made slower, 154 us).
-// A realization group holds K realizations of one mesh block by block: the
-// block of slot 0, then slot 1, ...  Element e of slot `slot` is pair
-// qidx(e, K, slot) of the array, its second pair 64 pairs on; in the TnC and
-// CSQ planes (K*np entries each) that follow the 4*K*np doubles it is entry
-// ((e/64)*K + slot)*64 + e%64.
 constexpr int QHALF = 64;              // pairs from an element's first pair to its second
 constexpr int FLUO_OFF = 2 * QHALF + 1;  // doubles from an element's Ca to its Fluo
-__host__ __device__ inline size_t gidx(size_t e, int K, int slot) {
-  return ((e >> 6) * (size_t)K + (size_t)slot) * 64 + (e & 63);
-}
-__host__ __device__ inline size_t qidx(size_t e, int K, int slot) {
-  return ((e >> 6) * (size_t)K + (size_t)slot) * (2 * QHALF) + (e & 63);
-}
-// Groups of one: pairs of 2^31 elements still count in 32 bits.
+// Element e's first pair (pairs of 2^31 elements still count in 32 bits).
 __host__ __device__ inline uint32_t qidx1(uint32_t e) { return e + (e & ~63u); }
-__host__ __device__ inline size_t xoff(int s, size_t e, size_t np, int K = 1, int slot = 0) {
-  if (s == srs::TRPN) return 4 * (size_t)K * np + gidx(e, K, slot);
-  if (s == srs::CSQN) return 5 * (size_t)K * np + gidx(e, K, slot);
-  const size_t q = 2 * qidx(e, K, slot);
+__host__ __device__ inline size_t xoff(int s, size_t e, size_t np) {
+  if (s == srs::TRPN) return 4 * np + e;
+  if (s == srs::CSQN) return 5 * np + e;
+  const size_t q = 2 * (size_t)qidx1((uint32_t)e);
   return s == srs::CA ? q : s == srs::ATP ? q + 1 : s == srs::CMDN ? q + FLUO_OFF - 1 : q + FLUO_OFF;
 }
 typedef double d2 __attribute__((ext_vector_type(2)));
@@ -110,7 +99,6 @@ struct RealDesc {
   double brd[4];          // the D_Ca, D_Fluo, D_ATP, D_CaM the mesh's boundary rates were built with
   double* X[2];           // [6][np] ping-pong state
   int32_t n, np;
-  int32_t kst, slot;      // realization group: K realizations interleaved, this one in slot `slot`
   int32_t n_ryr, n_lcc;
   const int32_t* ryr_ele;
   const int32_t* ryr_jsr;
@@ -152,7 +140,7 @@ __host__ __device__ inline double br_scaled(double v, double D, double D_b) {
 __host__ __device__ inline double br_unit(double v, double D_b) { return D_b == 0.0 ? 0.0 : v / D_b; }
 
 // Offset of element e's Ca in a realization's state buffer; Fluo is at +FLUO_OFF.
-__device__ __forceinline__ size_t cq(const RealDesc& d, int e) { return 2 * qidx((size_t)e, d.kst, d.slot); }
+__device__ __forceinline__ size_t cq(int e) { return 2 * (size_t)qidx1((uint32_t)e); }
 
 // Mutable per-realization loop state.
 struct RealLive {
@@ -297,7 +285,7 @@ __device__ __forceinline__ bool lives_cs(const uint8_t f) { return (f & F_JSR) !
 
 // Operator row of one element: coefficients (diagonal first), its neighbours'
 // places among the tile's staged quads, and flags.  Mesh-level data, shared
-// by every realization of a realization group.
+// by every realization of the mesh.
 struct Geo {
   double a0, a1, a2, a3, a4;
   int l1, l2, l3, l4;
@@ -599,7 +587,7 @@ struct HostReal {
   int32_t ints[SRS_N_INT];
   double reals[SRS_N_REAL];
   uint64_t key = 0, stream = 0;
-  int32_t group = 0;  // realization group (index into the sweep's group table)
+  int32_t band = 0;   // index into srs_ctx::bands
   RealDesc desc{};
 };
 
@@ -626,8 +614,8 @@ struct srs_ctx {
   int plane_pad = 0;     // extra elements per SoA plane
   int compact = 1;       // compress operator rows when a mesh allows it
   int occ = 0;           // gated sweep's register budget: 0 by size, else six wavefronts per SIMD
-  int group = 1;         // realizations per realization group (1, 2 or 4)
-  int drop_finished = 1; // sweep without the tiles of groups that have all finished
+  int group = 1;         // SRS_TUNE_GROUP
+  int drop_finished = 1; // sweep without the tiles of finished realizations
   int gated = 1;         // fold each step's gating into the next step's sweep (k_sweep_gated) where it applies
   int alt_order = 0;      // single-realization gated sweep: tiles in reverse order on alternate steps
   int gpu_layout = 0;     // states records in the GPU program's layout (Ca_cyt at each RyR appended)
@@ -644,14 +632,14 @@ struct srs_ctx {
   std::vector<void*> allocs;
   RealDesc* d_desc = nullptr;
   RealLive* d_live = nullptr;
-  int2* d_tiles = nullptr;   // {group, tile} of the sweep
+  int2* d_tiles = nullptr;   // {realization, tile} of the sweep
   int n_tiles = 0, grid_sweep = 0;
-  // Every group's tiles; when the groups whose members have all finished hold
-  // enough of them, the sweep runs over a list without them (d_tiles_live).
+  // Every realization's tiles; when the finished ones hold enough of them, the
+  // sweep runs over a list without them (d_tiles_live).
   std::vector<int2> tiles_all;
   int2* d_tiles_all = nullptr;
   std::vector<int2> tiles_cur;    // host copy of the tile list the sweep runs over (d_tiles)
-  // Realization subsets (SRS_TUNE_SUBSET_MB): consecutive groups of the tile
+  // Realization subsets (SRS_TUNE_SUBSET_MB): consecutive bands of the tile
   // list whose state takes at most subset_mb MB, each stepped through a
   // whole block of steps before the next, so that its state stays in the
   // last-level cache between steps.
@@ -662,8 +650,7 @@ struct srs_ctx {
   int32_t* d_sub_rids = nullptr;  // realization ids of the subsets, concatenated
   int2* d_tiles_live = nullptr;
   bool tiles_compacted = false;
-  int32_t* d_groups = nullptr;  // [n_groups][group] realization ids, -1 pads
-  std::vector<int32_t> groups;
+  std::vector<std::vector<int32_t>> bands;  // realizations of one mesh whose tiles are side by side in the list
   double* stage[2] = {};         // pinned buffers of state transfers (state_xfer), stage_len doubles each
   size_t stage_len = 0;
   hipEvent_t ev_stage[2] = {};

@@ -67,12 +67,6 @@ __device__ __forceinline__ uint64_t fold(const T... v) {
 }
 __device__ __forceinline__ void scalars_here(const uint64_t folded) { __asm__ volatile("" ::"s"(folded)); }
 
-// Pair index of an element; ONE: the realization is alone in its group.
-template <bool ONE>
-__device__ __forceinline__ size_t qat(const RealDesc& d, const int e) {
-  return ONE ? (size_t)qidx1((uint32_t)e) : qidx((size_t)e, d.kst, d.slot);
-}
-
 // An element's rates without the channel fluxes, and the divisor of the rapid
 // buffers (B, used where `div`).
 struct Rates {
@@ -171,24 +165,23 @@ __device__ __forceinline__ void chan_flux(const RealDesc& d, const RealLive& l, 
 }
 
 // Division by the rapid buffers and forward Euler (:633-644).
-template <bool NTS, int FK, bool ONE>
+template <bool NTS, int FK>
 __device__ __forceinline__ void elem_store(const RealDesc& d, const Bufs bf, const int j, const uint8_t flags,
                                            const Loc& c, const Rates& r) {
-  const int K = ONE ? 1 : d.kst;
-  const size_t np = d.np, q = ONE ? (size_t)j : gidx(j, K, d.slot);
+  const size_t np = d.np;
   const uint8_t f = FK >= 0 ? (uint8_t)FK : flags;
   const double dt = d.P[SRS_R_T_STEP];
   SRS_GLOBAL double* __restrict__ Xn = bf.xn;
   const double rca = r.div ? r.ca / r.B : r.ca;
-  st_quad<NTS>(Xn, qat<ONE>(d, j),
+  st_quad<NTS>(Xn, qidx1(j),
                d4{c.m0.x + rca * dt, c.m0.y + r.at * dt, c.m0.z + r.cm * dt, c.m0.w + r.dy * dt});
-  if (lives_tr(f)) stg<NTS>(Xn + 4 * K * np + q, c.c_tr + r.tr * dt);
-  if (lives_cs(f)) stg<NTS>(Xn + 5 * K * np + q, c.c_cs + r.cs * dt);
+  if (lives_tr(f)) stg<NTS>(Xn + 4 * np + j, c.c_tr + r.tr * dt);
+  if (lives_cs(f)) stg<NTS>(Xn + 5 * np + j, c.c_cs + r.cs * dt);
 }
 
 // The fused step of one element of one realization, from its loaded row and
 // state, in the reference's operation order (cpu/RunSimulation.cpp:591-648).
-template <bool NTS, int FK, bool ONE>
+template <bool NTS, int FK>
 __device__ __forceinline__ void step_elem(const RealDesc& d, const RealLive& l, const Bufs bf, const int j,
                                           const uint8_t flags, const Loc& c) {
   const uint8_t f = FK >= 0 ? (uint8_t)FK : flags;
@@ -205,12 +198,12 @@ __device__ __forceinline__ void step_elem(const RealDesc& d, const RealLive& l, 
       for (int e = d.cstart[lo]; e < d.cstart[lo + 1]; ++e) {
         const ChanEntry en = d.centry[e];
         const bool open = en.code >= 0 && d.ryr_state[en.code >> 1];
-        const double dc = open ? bf.xo[2 * qat<ONE>(d, en.jsr)] - bf.xo[2 * qat<ONE>(d, en.cyt)] : 0.0;
+        const double dc = open ? bf.xo[cq(en.jsr)] - bf.xo[cq(en.cyt)] : 0.0;
         chan_flux(d, l, en.code, open, dc, c.m0.x, v0, r.ca);
       }
     }
   }
-  elem_store<NTS, FK, ONE>(d, bf, j, f, c, r);
+  elem_store<NTS, FK>(d, bf, j, f, c, r);
 }
 
 // The sizes and mesh pointers of a tile's rows and halo, folded for scalars_here.
@@ -236,10 +229,9 @@ extern __shared__ double dyn_lds[];
 // 3M-element dyad).
 // A wavefront whose elements are all plain cytosol with troponin (the bulk of
 // a mesh, known from its block's flags) runs the specialisation with the flags
-// known at compile time.  KG: the realization's group size, s its slot.
-template <int BS, bool NTS, bool CLASS, int KG, bool SKIP_CHAN>
-__device__ __forceinline__ void sweep_tile(const RealDesc& d, const RealLive& l, const Bufs bf, const int s,
-                                           const int t) {
+// known at compile time.
+template <int BS, bool NTS, bool CLASS, bool SKIP_CHAN>
+__device__ __forceinline__ void sweep_tile(const RealDesc& d, const RealLive& l, const Bufs bf, const int t) {
   const QuadTile tq(dyn_lds, d.qcap);
   const Halo h = load_halo<BS>(d.hal, d.hoff, t);
   const int j = t * BS + (int)threadIdx.x;
@@ -248,8 +240,8 @@ __device__ __forceinline__ void sweep_tile(const RealDesc& d, const RealLive& l,
   const uint32_t b = block_flags(d, j);
   const Geo g = load_geo<CLASS>(d, d.loc, j, b);
   const SRS_GLOBAL double* Xo = bf.xo;
-  const size_t np = d.np, pl = 4 * KG * np + (KG > 1 ? gidx(j, KG, s) : (size_t)j);
-  auto quad = [&](int e) { return ld_quad(Xo, KG > 1 ? qidx(e, KG, s) : (size_t)qidx1(e)); };
+  const size_t np = d.np, pl = 4 * np + (size_t)j;
+  auto quad = [&](int e) { return ld_quad(Xo, qidx1(e)); };
   Loc c;
   c.m0 = quad(j);
   // the element's TnC is loaded with its quad, before its flags are known (it
@@ -261,43 +253,29 @@ __device__ __forceinline__ void sweep_tile(const RealDesc& d, const RealLive& l,
   if (j >= d.n || (SKIP_CHAN && (g.f & F_CHAN))) return;
   c.s = row_sum(g, c.m0, tq.get(g.l1), tq.get(g.l2), tq.get(g.l3), tq.get(g.l4));
   if (b & BLK_PLAIN) {
-    step_elem<NTS, F_TROPC, KG == 1>(d, l, bf, j, g.f, c);
+    step_elem<NTS, F_TROPC>(d, l, bf, j, g.f, c);
   } else {
     if (!lives_tr(g.f)) c.c_tr = 0.0;
-    c.c_cs = lives_cs(g.f) ? Xo[pl + KG * np] : 0.0;
-    step_elem<NTS, -1, KG == 1>(d, l, bf, j, g.f, c);
+    c.c_cs = lives_cs(g.f) ? Xo[pl + np] : 0.0;
+    step_elem<NTS, -1>(d, l, bf, j, g.f, c);
   }
 }
 
-// Workgroup b of a context with groups of KG takes slot b % KG of tile b / KG,
-// so that the slots' workgroups, which read the same rows and halo lists, run
-// side by side on one XCD.
-template <int BS, bool NTS, bool CLASS, int KG>
-__device__ __forceinline__ void sweep(const RealDesc* __restrict__ D, const RealLive* __restrict__ L,
-                                      const int2* __restrict__ tiles, int n_tiles, const int* __restrict__ groups,
-                                      int single) {
+template <int BS, bool NTS, bool CLASS>
+__global__ __launch_bounds__(BS) void k_sweep(const RealDesc* __restrict__ D, const RealLive* __restrict__ L,
+                                              const int2* __restrict__ tiles, int n_tiles, int single) {
   const int b = xcd_tile(blockIdx.x, gridDim.x);
-  if (b >= n_tiles * KG) return;
-  const int2 tl = single ? make_int2(0, b / KG) : tiles[b / KG];  // {group, tile}
-  const int s = b % KG;
-  const int r = single ? (s == 0 ? 0 : -1) : groups[KG * tl.x + s];
-  if (KG > 1 && r < 0) return;
-  const RealDesc& d = D[r];
-  const RealLive& l = L[r];
+  if (b >= n_tiles) return;
+  const int2 tl = single ? make_int2(0, b) : tiles[b];  // {realization, tile}
+  const RealDesc& d = D[tl.x];
+  const RealLive& l = L[tl.x];
   // a finished realization (done) or one in the gating-only ffwd phase keeps
   // its fields
   const int skip = l.done | l.ffwd;
   const Bufs bf = bufs(d.X[0], d.X[1], l.cur);
   scalars_here(fold(skip, bf.xo, bf.xn) ^ geo_fold<CLASS>(d));
   if (skip) return;
-  sweep_tile<BS, NTS, CLASS, KG, false>(d, l, bf, s, tl.y);
-}
-
-template <int BS, bool NTS, bool CLASS, int KG>
-__global__ __launch_bounds__(BS) void k_sweep(const RealDesc* __restrict__ D, const RealLive* __restrict__ L,
-                                              const int2* __restrict__ tiles, int n_tiles,
-                                              const int* __restrict__ groups, int single) {
-  sweep<BS, NTS, CLASS, KG>(D, L, tiles, n_tiles, groups, single);
+  sweep_tile<BS, NTS, CLASS, false>(d, l, bf, tl.y);
 }
 
 __device__ void write_record(const RealDesc& d, RealLive& l, const double* Ca, double t) {
@@ -308,7 +286,7 @@ __device__ void write_record(const RealDesc& d, RealLive& l, const double* Ca, d
   rec[k++] = (float)t;
   double i_ryr = 0;
   for (int i = 0; i < d.n_ryr; ++i)
-    i_ryr += d.ryr_state[i] * d.P[SRS_R_V_RYR] * (Ca[cq(d, d.ryr_jsr[i])] - Ca[cq(d, d.ryr_ele[i])]) * (d.P[SRS_R_V_CELL]) * 96485 *
+    i_ryr += d.ryr_state[i] * d.P[SRS_R_V_RYR] * (Ca[cq(d.ryr_jsr[i])] - Ca[cq(d.ryr_ele[i])]) * (d.P[SRS_R_V_CELL]) * 96485 *
              2 * (1e-6);
   rec[k++] = (float)i_ryr;
   int n_open = 0;
@@ -321,18 +299,18 @@ __device__ void write_record(const RealDesc& d, RealLive& l, const double* Ca, d
   double i_lcc = 0;
   for (int i = 0; i < d.n_lcc; ++i)
     if (srs_lcc_open(d.lcc_state[i], d.lccv_state[i]))
-      i_lcc += srs_lcc_flux_raw(l.vm, Ca[cq(d, d.lcc_ele[i])], d.P[SRS_R_CA_0]) * 96485 * 2 * (1e-6);
+      i_lcc += srs_lcc_flux_raw(l.vm, Ca[cq(d.lcc_ele[i])], d.P[SRS_R_CA_0]) * 96485 * 2 * (1e-6);
   rec[k++] = (float)i_lcc;
   double m = 0;
-  for (int i = 0; i < d.n_ryr; ++i) m += Ca[cq(d, d.ryr_jsr[i])];
+  for (int i = 0; i < d.n_ryr; ++i) m += Ca[cq(d.ryr_jsr[i])];
   m /= d.n_ryr;
   rec[k++] = (float)m;
   m = 0;
-  for (int i = 0; i < d.n_ryr; ++i) m += Ca[cq(d, d.ryr_ele[i])];
+  for (int i = 0; i < d.n_ryr; ++i) m += Ca[cq(d.ryr_ele[i])];
   m /= d.n_ryr;
   rec[k++] = (float)m;
   if (d.gpu_layout)
-    for (int i = 0; i < d.n_ryr; ++i) rec[k++] = (float)Ca[cq(d, d.ryr_ele[i])];
+    for (int i = 0; i < d.n_ryr; ++i) rec[k++] = (float)Ca[cq(d.ryr_ele[i])];
   if (d.ryr_out)
     for (int i = 0; i < d.n_ryr; ++i) rec[k++] = (float)d.ryr_state[i];
   l.rec_count++;
@@ -357,7 +335,7 @@ __device__ __forceinline__ void gate_workgroup(const RealDesc* __restrict__ D, R
   const bool ff = l.ffwd != 0;
   const bool swept = (mode & G_AFTER_SWEEP) && !ff;
   const double* Xn = swept ? d.X[cur ^ 1] : d.X[cur];
-  const double* Ca = Xn;  // Ca of element e at Ca[cq(d, e)] (interleaved diffusing species)
+  const double* Ca = Xn;  // Ca of element e at Ca[cq(e)] (interleaved diffusing species)
   const double* P = d.P;
   const double dt = P[SRS_R_T_STEP];
   const int64_t step = l.step;
@@ -379,8 +357,8 @@ __device__ __forceinline__ void gate_workgroup(const RealDesc* __restrict__ D, R
     // this is folded into half of its registers.
     double ca_c = 0.0, ca_j = 0.0, Rr = 0.0;
     auto load_ryr = [&](const int i) {
-      ca_c = Ca[cq(d, d.ryr_ele[i])];
-      ca_j = Ca[cq(d, d.ryr_jsr[i])];
+      ca_c = Ca[cq(d.ryr_ele[i])];
+      ca_j = Ca[cq(d.ryr_jsr[i])];
       Rr = d.R[i];
     };
     for (int i = tid; i < nr; i += NT) s_old[i] = s_a[i] = d.ryr_state[i];
@@ -390,7 +368,7 @@ __device__ __forceinline__ void gate_workgroup(const RealDesc* __restrict__ D, R
     auto load_lcc = [&](const int i) {
       ls = d.lcc_state[i];
       lvs = d.lccv_state[i];
-      ca_l = Ca[cq(d, d.lcc_ele[i])];
+      ca_l = Ca[cq(d.lcc_ele[i])];
       Rl = d.R[nr + i];
     };
     const int l0 = NT - 1 - tid;
@@ -515,7 +493,7 @@ __device__ __forceinline__ void gate_workgroup(const RealDesc* __restrict__ D, R
       const bool open = i < nr && d.ryr_state[i] != 0;
       cr += __builtin_popcountll(__builtin_amdgcn_ballot_w64(open));
       if (i < nr) {
-        const double c = Ca[cq(d, d.ryr_ele[i])];
+        const double c = Ca[cq(d.ryr_ele[i])];
         if (c > m) m = c;
       }
     }
@@ -667,7 +645,7 @@ __device__ __forceinline__ void sweep_gated(const RealDesc* __restrict__ D, Real
       p.dc = en.code >= 0 ? Xo[2 * (size_t)qidx1(en.jsr)] - Xo[2 * (size_t)qidx1(en.cyt)] : 0.0;
       c.s = c.m0 * r->a[0] + m1 * r->a[1] + m2 * r->a[2] + m3 * r->a[3] + m4 * r->a[4];
       const Rates q = elem_rates<-1>(d, l, p.j, f, c, r->tt, p.v0);
-      elem_store<NTS, -1, true>(d, bf, p.j, f, c, q);  // Ca without its fluxes: replaced by finish
+      elem_store<NTS, -1>(d, bf, p.j, f, c, q);  // Ca without its fluxes: replaced by finish
       p.rca = q.ca;
       p.ca = c.m0.x;
       p.B = q.B;  // 1 where nothing divides
@@ -699,7 +677,7 @@ __device__ __forceinline__ void sweep_gated(const RealDesc* __restrict__ D, Real
     return;
   }
   if (skip) return;
-  sweep_tile<BS, NTS, CLASS, 1, true>(d, l, bf, 0, b - 1);
+  sweep_tile<BS, NTS, CLASS, true>(d, l, bf, b - 1);
 }
 // W: the register budget, at least W wavefronts per SIMD.
 template <int BS, bool NTS, bool CLASS, bool PROTO, bool PRE, int W>
@@ -715,31 +693,26 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W))) void k_
 // gated sweeps of 128-, 256- and 512-element tiles), which the build
 // compiles in parallel.
 
-using SweepFn = void (*)(const RealDesc*, const RealLive*, const int2*, int, const int*, int);
+using SweepFn = void (*)(const RealDesc*, const RealLive*, const int2*, int, int);
 using GatedFn = void (*)(const RealDesc*, RealLive*, int, int, uint32_t, const double*, double*);
 SweepFn pick_sweep(const srs_ctx* c);
 template <int BS>
 GatedFn pick_gated_bs(const srs_ctx* c, bool proto);
 
 #if SRS_UNIT == 1
-template <int BS, bool CMP, int KG>
-SweepFn pick_nt(int nts) { return nts ? k_sweep<BS, true, CMP, KG> : k_sweep<BS, false, CMP, KG>; }
+template <int BS, bool CMP>
+SweepFn pick_nt(int nts) { return nts ? k_sweep<BS, true, CMP> : k_sweep<BS, false, CMP>; }
 
-template <bool CMP, int KG>
+template <bool CMP>
 SweepFn pick_tile(const srs_ctx* c) {
   switch (c->tile) {
-    case 128: return pick_nt<128, CMP, KG>(c->nt_state);
-    case 256: return pick_nt<256, CMP, KG>(c->nt_state);
-    default: return pick_nt<512, CMP, KG>(c->nt_state);
+    case 128: return pick_nt<128, CMP>(c->nt_state);
+    case 256: return pick_nt<256, CMP>(c->nt_state);
+    default: return pick_nt<512, CMP>(c->nt_state);
   }
 }
 
-template <int KG>
-SweepFn pick_kg(const srs_ctx* c) { return c->class_all ? pick_tile<true, KG>(c) : pick_tile<false, KG>(c); }
-
-SweepFn pick_sweep(const srs_ctx* c) {
-  return c->group == 4 ? pick_kg<4>(c) : c->group == 2 ? pick_kg<2>(c) : pick_kg<1>(c);
-}
+SweepFn pick_sweep(const srs_ctx* c) { return c->class_all ? pick_tile<true>(c) : pick_tile<false>(c); }
 #endif  // SRS_UNIT == 1
 
 #if SRS_UNIT >= 2
@@ -776,12 +749,12 @@ template GatedFn pick_gated_bs<SRS_UNIT == 2 ? 128 : SRS_UNIT == 3 ? 256 : 512>(
 // Gathers Ca at the channel elements of one realization.
 __global__ void k_channel_ca(const RealDesc* __restrict__ D, const RealLive* __restrict__ L, int r, double* out) {
   const RealDesc& d = D[r];
-  const double* Ca = d.X[L[r].cur];  // Ca of element e at Ca[cq(d, e)]
+  const double* Ca = d.X[L[r].cur];  // Ca of element e at Ca[cq(e)]
   for (int i = threadIdx.x; i < d.n_ryr; i += blockDim.x) {
-    out[i] = Ca[cq(d, d.ryr_ele[i])];
-    out[d.n_ryr + i] = Ca[cq(d, d.ryr_jsr[i])];
+    out[i] = Ca[cq(d.ryr_ele[i])];
+    out[d.n_ryr + i] = Ca[cq(d.ryr_jsr[i])];
   }
-  for (int i = threadIdx.x; i < d.n_lcc; i += blockDim.x) out[2 * d.n_ryr + i] = Ca[cq(d, d.lcc_ele[i])];
+  for (int i = threadIdx.x; i < d.n_lcc; i += blockDim.x) out[2 * d.n_ryr + i] = Ca[cq(d.lcc_ele[i])];
 }
 
 
@@ -799,7 +772,7 @@ __global__ __launch_bounds__(256) void k_state_xfer(const RealDesc* __restrict__
   const RealDesc& d = D[r];
   const size_t t = t0 + i, n = d.n;
   const int s = (int)(t / n);
-  const size_t x = xoff(s, inv[t - s * n], d.np, d.kst, d.slot);
+  const size_t x = xoff(s, inv[t - s * n], d.np);
   if (to_dev) {
     const double v = stage[i];
     d.X[0][x] = v;
@@ -980,7 +953,7 @@ void launch_sweep(srs_ctx* c) {
   // one realization: tile b is tile b of realization 0, no table lookups
   const int single = c->reals.size() == 1 ? 1 : 0;
   hipLaunchKernelGGL(pick_sweep(c), dim3(c->grid_sweep), dim3(c->tile), c->sweep_lds, c->stream, c->d_desc, c->d_live,
-                     c->d_tiles, c->n_tiles, (const int*)c->d_groups, single);
+                     c->d_tiles, c->n_tiles, single);
 }
 
 // m steps of every subset, one subset after another: the sweep over the
@@ -991,50 +964,45 @@ void launch_subset_block(srs_ctx* c, int64_t m, uint32_t gmode) {
   for (const srs_ctx::Subset& sb : c->subsets)
     for (int64_t k = 0; k < m; ++k) {
       if (sb.nt > 0)
-        hipLaunchKernelGGL(pick_sweep(c), dim3((sb.nt * c->group + NXCD - 1) / NXCD * NXCD), dim3(c->tile), c->sweep_lds, c->stream,
-                           c->d_desc, c->d_live, c->d_tiles + sb.t0, sb.nt, (const int*)c->d_groups, 0);
+        hipLaunchKernelGGL(pick_sweep(c), dim3((sb.nt + NXCD - 1) / NXCD * NXCD), dim3(c->tile), c->sweep_lds, c->stream,
+                           c->d_desc, c->d_live, c->d_tiles + sb.t0, sb.nt, 0);
       hipLaunchKernelGGL(k_gate_list, dim3((unsigned)sb.nr), dim3(GATE_THREADS), 0, c->stream, c->d_desc, c->d_live,
                          (const int32_t*)c->d_sub_rids + sb.r0, gmode);
     }
 }
 
-// Splits the current tile list into subsets: runs of whole groups (in list
+// Splits the current tile list into subsets: runs of whole bands (in list
 // order) whose realizations' state buffers (two of 48 B per element each)
-// take at most subset_mb MB; realizations whose groups have no tile left
+// take at most subset_mb MB; realizations whose bands have no tile left
 // (all finished) are gated with the last subset, as k_gate would.
 int plan_subsets(srs_ctx* c) {
   c->subsets.clear();
   c->subsets_valid = true;
   if (c->subset_mb <= 0 || c->reals.size() < 2) return SRS_OK;
   const size_t budget = (size_t)c->subset_mb << 20;
-  const int KG = c->group;
+  auto band_of = [&](int t) { return c->reals[c->tiles_cur[t].x].band; };
   std::vector<int32_t> rids;
   std::vector<char> listed(c->reals.size(), 0);
   srs_ctx::Subset cur{0, 0, 0, 0};
   size_t bytes = 0;
   const int n = (int)c->tiles_cur.size();
   for (int t = 0; t < n;) {
-    const int g = c->tiles_cur[t].x;
+    const int g = band_of(t);
     int t1 = t;
-    while (t1 < n && c->tiles_cur[t1].x == g) ++t1;
+    while (t1 < n && band_of(t1) == g) ++t1;
     size_t gb = 0;
-    for (int s = 0; s < KG; ++s) {
-      const int r = c->groups[(size_t)KG * g + s];
-      if (r >= 0) gb += 2 * 48 * (size_t)c->meshes[c->reals[r].mesh]->np;
-    }
+    for (int r : c->bands[g]) gb += 2 * 48 * (size_t)c->meshes[c->reals[r].mesh]->np;
     if (cur.nt > 0 && bytes + gb > budget) {
       c->subsets.push_back(cur);
       cur = srs_ctx::Subset{t, 0, (int)rids.size(), 0};
       bytes = 0;
     }
-    for (int s = 0; s < KG; ++s) {
-      const int r = c->groups[(size_t)KG * g + s];
-      if (r >= 0 && !listed[r]) {
+    for (int r : c->bands[g])
+      if (!listed[r]) {
         listed[r] = 1;
         rids.push_back(r);
         cur.nr++;
       }
-    }
     cur.nt += t1 - t;
     bytes += gb;
     t = t1;
@@ -1071,20 +1039,20 @@ void launch_gated(srs_ctx* c, int cur, uint32_t gmode, bool proto, const double*
                      cur | (c->alt_order ? 2 : 0), gmode, xo_at, xn_at);
 }
 
-// m steps through k_sweep_gated: the first without gating (nothing is
-// pending when a block starts), each later one gating the step before it,
-// then k_gate for the last step, so that a block leaves no gating pending.
-// cur is the live state index when the block starts; gmode is the step's
-// gating mode (G_AFTER_SWEEP, with G_PROTOCOL for the loop body).
 // The gating of a single realization's last gated step (k_gate alone).
 void launch_gate_single(srs_ctx* c, uint32_t gmode) {
   hipLaunchKernelGGL(k_gate, dim3(1), dim3(GATE_THREADS), 0, c->stream, c->d_desc, c->d_live, gmode);
 }
 
+// m steps through k_sweep_gated: the first without gating (nothing is
+// pending when a block starts), each later one gating the step before it,
+// then k_gate for the last step, so that a block leaves no gating pending.
+// cur is the live state index when the block starts; gmode is the step's
+// gating mode (G_AFTER_SWEEP, with G_PROTOCOL for the loop body).
 void launch_gated_block(srs_ctx* c, int64_t m, int cur, uint32_t gmode) {
   const bool proto = (gmode & G_PROTOCOL) != 0;
   for (int64_t k = 0; k < m; ++k) launch_gated(c, cur ^ (int)(k & 1), k ? gmode : 0u, proto);
-  hipLaunchKernelGGL(k_gate, dim3(1), dim3(GATE_THREADS), 0, c->stream, c->d_desc, c->d_live, gmode);
+  launch_gate_single(c, gmode);
 }
 
 // Captured step blocks hold the sweep's tile list and grid; they are dropped
@@ -1099,7 +1067,7 @@ int drop_graphs(srs_ctx* c) {
 void set_tiles(srs_ctx* c, int2* d, int n) {
   c->d_tiles = d;
   c->n_tiles = n;
-  c->grid_sweep = (n * c->group + NXCD - 1) / NXCD * NXCD;
+  c->grid_sweep = (n + NXCD - 1) / NXCD * NXCD;
   c->subsets_valid = false;
 }
 
@@ -1127,17 +1095,9 @@ int tiles_compact(srs_ctx* c) {
   HIPCHK(hipStreamSynchronize(c->stream));
   std::vector<RealLive> lv(n_real);
   HIPCHK(hipMemcpy(lv.data(), c->d_live, n_real * sizeof(RealLive), hipMemcpyDeviceToHost));
-  const int KG = c->group;
-  const int n_groups = (int)c->groups.size() / KG;
-  std::vector<char> live(n_groups, 0);
-  for (int g = 0; g < n_groups; ++g)
-    for (int s = 0; s < KG; ++s) {
-      const int r = c->groups[(size_t)KG * g + s];
-      if (r >= 0 && !lv[r].done) live[g] = 1;
-    }
   std::vector<int2> t;
   for (const int2& x : c->tiles_all)
-    if (live[x.x]) t.push_back(x);
+    if (!lv[x.x].done) t.push_back(x);
   if ((int64_t)t.size() == c->n_tiles || (int64_t)t.size() * 8 > (int64_t)c->n_tiles * 7) return SRS_OK;
   int rc = drop_graphs(c);
   if (rc) return rc;
@@ -1259,13 +1219,12 @@ int live_rw(srs_ctx* c, int32_t r, RealLive* lv, bool write) {
 }
 
 // Whether steps run through k_sweep_gated, and the live state index they
-// start from: single-realization contexts with the LDS sweep of groups of
-// one and a register budget of 0 or 6 (0 with the loop body), while the
-// realization is neither finished nor in the ffwd phase.  Reading the live
-// state waits for the stream.
+// start from: single-realization contexts while the realization is neither
+// finished nor in the ffwd phase.  Reading the live state waits for the
+// stream.
 int gated_start(srs_ctx* c, bool* ok, int* cur) {
   *ok = false;
-  if (!c->gated || c->reals.size() != 1 || c->group != 1) return SRS_OK;
+  if (!c->gated || c->reals.size() != 1) return SRS_OK;
   RealLive lv;
   int rc = live_rw(c, 0, &lv, false);
   if (rc) return rc;
@@ -1630,38 +1589,36 @@ int srs_ctx_finalize(srs_ctx* c, int32_t record_capacity) {
   std::vector<RealDesc> descs;
   std::vector<RealLive> lives;
   std::vector<int2> tiles;
-  // Realization groups: up to c->group realizations of one mesh, in the
-  // order they were added, share interleaved state buffers and each sweep
-  // tile of the group loads the operator rows once for all of them.
-  const int KG = c->group;
-  std::vector<int32_t> groups;     // [n_groups][KG], -1 pads
-  std::vector<int32_t> real_group(c->reals.size()), real_slot(c->reals.size());
-  std::vector<int32_t> group_mesh;
+  // bytes a step works on: the state buffers, and rows and halo lists
+  double ws = 0.0;
+  for (const HostReal& hr : c->reals) ws += 2.0 * 48.0 * c->meshes[hr.mesh]->n;
+  for (auto& hmp : c->meshes) ws += (double)hmp->n * ((c->class_all ? 12 : 40) + 9) + 4.0 * hmp->map.n_halo;
+  // Tile order.  Up to four realizations of a mesh form a band whose tiles lie
+  // side by side, so that rows and halo lists come from the L2 for all but the
+  // first, while everything a step touches fits the 256 MB last-level cache (us
+  // per step in bands of one / four: 14-member ensemble, 207 MB, 40.9 / 37.8;
+  // 16 members, 237 MB, 45.2 / 43.4; two 928k-element dyads, 200 MB, 40.4 /
+  // 38.5).  Beyond it four state streams at a time cost more than the rows (18
+  // members, 266 MB, 52.7 / 56.6; 48, 137 / 142; twelve 214k-element dyads, 241
+  // MB, 53.7 / 48.5 in one run and 57.4 in another).
+  const int width = ws > 220e6 ? 1 : 4;
   for (size_t m = 0; m < c->meshes.size(); ++m) {
-    int cur_g = -1, fill = KG;
-    for (size_t r = 0; r < c->reals.size(); ++r) {
+    for (size_t r = 0, fill = width; r < c->reals.size(); ++r) {
       if (c->reals[r].mesh != (int)m) continue;
-      if (fill == KG) {
-        cur_g = (int)group_mesh.size();
-        group_mesh.push_back((int)m);
-        groups.insert(groups.end(), KG, -1);
+      if (fill == (size_t)width) {
+        c->bands.emplace_back();
         fill = 0;
       }
-      groups[(size_t)KG * cur_g + fill] = (int32_t)r;
-      real_group[r] = cur_g;
-      real_slot[r] = fill++;
+      c->bands.back().push_back((int32_t)r);
+      c->reals[r].band = (int32_t)c->bands.size() - 1;
+      ++fill;
     }
   }
-  const int n_groups = (int)group_mesh.size();
-  std::vector<double*> gx0(n_groups), gx1(n_groups);
-  for (int gi = 0; gi < n_groups; ++gi) {
-    const HostMesh& hm = *c->meshes[group_mesh[gi]];
-    const size_t cnt = 6 * (size_t)KG * hm.np;
-    if ((rc = dev_alloc(c, &gx0[gi], cnt)) || (rc = dev_alloc(c, &gx1[gi], cnt))) return rc;
-    HIPCHK(hipMemset(gx0[gi], 0, cnt * sizeof(double)));
-    HIPCHK(hipMemset(gx1[gi], 0, cnt * sizeof(double)));
+  for (const auto& band : c->bands) {
+    const HostMesh& hm = *c->meshes[c->reals[band[0]].mesh];
     const int nt = (hm.n + c->tile - 1) / c->tile;
-    for (int t = 0; t < nt; ++t) tiles.push_back(make_int2(gi, t));
+    for (int t = 0; t < nt; ++t)
+      for (int r : band) tiles.push_back(make_int2(r, t));
   }
   for (size_t r = 0; r < c->reals.size(); ++r) {
     HostReal& hr = c->reals[r];
@@ -1674,10 +1631,10 @@ int srs_ctx_finalize(srs_ctx* c, int32_t record_capacity) {
     d.row = hm.d_row; d.tab = hm.d_tab; d.blk = hm.d_blk;
     d.n_class = hm.n_class;
     d.n = hm.n; d.np = hm.np;
-    d.X[0] = gx0[real_group[r]]; d.X[1] = gx1[real_group[r]];
-    hr.group = real_group[r];
-    d.kst = KG;
-    d.slot = real_slot[r];
+    for (int k = 0; k < 2; ++k) {
+      if ((rc = dev_alloc(c, &d.X[k], 6 * (size_t)hm.np))) return rc;
+      HIPCHK(hipMemset(d.X[k], 0, 6 * (size_t)hm.np * sizeof(double)));
+    }
     d.n_ryr = (int32_t)hr.ryr_ele.size();
     d.n_lcc = (int32_t)hr.lcc_ele.size();
     int32_t *p;
@@ -1741,20 +1698,15 @@ int srs_ctx_finalize(srs_ctx* c, int32_t record_capacity) {
   // one before, so while the buffers and the meshes' rows fit the 256 MB
   // last-level cache nothing is hinted past it (us per step without hints /
   // non-temporal stores / non-temporal row loads: 928k-element dyad, 114 MB,
-  // 21.5 / 25.9 / 24.8; 18-member ensemble, 266 MB, 53.6 / 60.8 / 61.2; 21
-  // members in groups, 309 MB, 76.2 / 78.2 / 79.8).  Beyond it plain stores
+  // 21.5 / 25.9 / 24.8; 18-member ensemble, 266 MB, 53.6 / 60.8 / 61.2; 20
+  // members, 295 MB, 62.0 / 62.5 / -).  Beyond it plain stores
   // evict what the next step could still have found (24 members, 351 MB, 78.6 /
   // 74.9 / 77.4; 3M-element dyad, 362 MB, 69.4 / 61.1 / 61.2; 48 members, 147 /
-  // 138 / 160).  The line lies between 309 and 351 MB.  Row loads are never
+  // 138 / 160).  The line lies between 295 and 351 MB.  Row loads are never
   // hinted: nowhere faster than the better of the other two.
-  {
-    double ws = 0.0;
-    for (const HostReal& hr : c->reals) ws += 2.0 * 48.0 * c->meshes[hr.mesh]->n;
-    for (auto& hmp : c->meshes) ws += (double)hmp->n * ((c->class_all ? 12 : 40) + 9) + 4.0 * hmp->map.n_halo;
-    if (c->nt_state < 0) c->nt_state = ws > 330e6;
-  }
+  if (c->nt_state < 0) c->nt_state = ws > 330e6;
   c->n_tiles = (int)tiles.size();
-  c->grid_sweep = (c->n_tiles * c->group + NXCD - 1) / NXCD * NXCD;
+  c->grid_sweep = (c->n_tiles + NXCD - 1) / NXCD * NXCD;
   // state transfers: two pinned buffers of at most 8 MB (larger fields go
   // through them in parts)
   for (const HostReal& hr : c->reals) c->stage_len = std::max(c->stage_len, 6 * (size_t)c->meshes[hr.mesh]->n);
@@ -1766,12 +1718,10 @@ int srs_ctx_finalize(srs_ctx* c, int32_t record_capacity) {
   if ((rc = dev_upload(c, &c->d_desc, descs))) return rc;
   if ((rc = dev_upload(c, &c->d_live, lives))) return rc;
   if ((rc = dev_upload(c, &c->d_tiles, tiles))) return rc;
-  if ((rc = dev_upload(c, &c->d_groups, groups))) return rc;
   c->tiles_all = tiles;
   c->tiles_cur = tiles;
   c->d_tiles_all = c->d_tiles;
   if (c->reals.size() > 1 && (rc = dev_alloc(c, &c->d_sub_rids, c->reals.size()))) return rc;
-  c->groups = groups;
   if (c->reals.size() > 1 && (rc = dev_alloc(c, &c->d_tiles_live, tiles.size()))) return rc;
   HIPCHK(hipDeviceSynchronize());
   c->finalized = true;
@@ -2118,7 +2068,8 @@ static int replay_from(srs_ctx* c, int32_t r, int64_t n_steps, const int32_t* sc
   HIPCHK(hipMemcpy(c->d_live + r, &lv, sizeof(lv), hipMemcpyHostToDevice));
   const uint32_t gmode = G_AFTER_SWEEP | G_NO_GATING | G_REPLAY;
   // through the gated sweep, a launch per step with the replay of the step
-  // before in its workgroup 0: 400 steps of 98,010 elements MEASURED
+  // before in its workgroup 0: 400 steps of 124,146 elements 3.3 ms, 4.8 with
+  // two launches
   bool gated;
   int cur;
   const int rc = gated_start(c, &gated, &cur);

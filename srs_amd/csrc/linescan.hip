@@ -81,7 +81,7 @@ __global__ __launch_bounds__(SCAN_BS) __attribute__((amdgpu_waves_per_eu(4))) vo
   for (int q = 0; q < NC; ++q) {
     const int j = min((int)(blockIdx.x * NC + q) * SCAN_BS + (int)threadIdx.x, n - 1);
     cx[q] = gp(cen)[j], cy[q] = gp(cen)[np + j], cz[q] = gp(cen)[2 * np + j];
-    vf[q] = gp(d.V0)[j] * gp(X)[cq(d, j) + FLUO_OFF];  // V0 * Ca-bound Fluo
+    vf[q] = gp(d.V0)[j] * gp(X)[cq(j) + FLUO_OFF];  // V0 * Ca-bound Fluo
   }
   ScanCell sc[NC];
   int clo[NC], chi[NC];
@@ -143,11 +143,11 @@ __global__ __launch_bounds__(SCAN_BS) void k_scan_final(const RealDesc* __restri
   const int t = blockIdx.x * SCAN_BS + threadIdx.x, nt = gridDim.x * SCAN_BS;
   for (int k = t; k < n_f; k += nt) {
     const int e = near_f[k];
-    out[n_ca + k] = e >= 0 ? X[cq(D[r], e) + FLUO_OFF] : f0;
+    out[n_ca + k] = e >= 0 ? X[cq(e) + FLUO_OFF] : f0;
   }
   for (int k = t; k < n_ca; k += nt) {
     const int e = near_ca[k];
-    out[k] = e >= 0 ? X[cq(D[r], e)] : c0;
+    out[k] = e >= 0 ? X[cq(e)] : c0;
   }
 }
 
