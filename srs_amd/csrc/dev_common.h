@@ -75,6 +75,7 @@ struct ChanElem {
   double a[5], v0, tt;
   int32_t j, nb[4], e0, e1;  // the element, its neighbours, its run of centry
   uint32_t f;
+  int32_t code, jsr, cyt, pad;  // centry[e0]
 };
 
 // Immutable per-realization descriptor (read with scalar loads).

@@ -150,17 +150,15 @@ __device__ __forceinline__ Rates elem_rates(const RealDesc& d, const RealLive& l
 
 // Adds one channel's flux to an element's Ca rate (cpu/RunSimulation.cpp:619-632).
 // dc: Ca of a RyR's jSR element less its cleft element's.
-__device__ __forceinline__ void chan_flux(const RealDesc& d, const RealLive& l, const int code, const bool ryr_open,
+__device__ __forceinline__ void chan_flux(const RealDesc& d, const RealLive& l, const int code, const bool open,
                                           const double dc, const double c_ca, const double v0, double& rca) {
   const double* P = d.P;
+  if (!open) return;
   if (code >= 0) {
-    if (ryr_open) {
-      const double J = P[SRS_R_V_RYR] * dc * P[SRS_R_V_CELL];
-      if (code & 1) rca -= J / v0; else rca += J / v0;
-    }
+    const double J = P[SRS_R_V_RYR] * dc * P[SRS_R_V_CELL];
+    if (code & 1) rca -= J / v0; else rca += J / v0;
   } else {
-    const int i = -code - 1;
-    if (srs_lcc_open(d.lcc_state[i], d.lccv_state[i])) rca += srs_lcc_flux_raw(l.vm, c_ca, P[SRS_R_CA_0]) / v0;
+    rca += srs_lcc_flux_raw(l.vm, c_ca, P[SRS_R_CA_0]) / v0;
   }
 }
 
@@ -197,8 +195,9 @@ __device__ __forceinline__ void step_elem(const RealDesc& d, const RealLive& l, 
       const double v0 = d.V0[j];
       for (int e = d.cstart[lo]; e < d.cstart[lo + 1]; ++e) {
         const ChanEntry en = d.centry[e];
-        const bool open = en.code >= 0 && d.ryr_state[en.code >> 1];
-        const double dc = open ? bf.xo[cq(en.jsr)] - bf.xo[cq(en.cyt)] : 0.0;
+        const int i = en.code >= 0 ? en.code >> 1 : -en.code - 1;
+        const bool open = en.code >= 0 ? d.ryr_state[i] != 0 : srs_lcc_open(d.lcc_state[i], d.lccv_state[i]);
+        const double dc = open && en.code >= 0 ? bf.xo[cq(en.jsr)] - bf.xo[cq(en.cyt)] : 0.0;
         chan_flux(d, l, en.code, open, dc, c.m0.x, v0, r.ca);
       }
     }
@@ -316,18 +315,31 @@ __device__ void write_record(const RealDesc& d, RealLive& l, const double* Ca, d
   l.rec_count++;
 }
 
+constexpr int GATE_RYR = 3 * MAX_RYR, GATE_LCC = 4 * MAX_RYR;
+constexpr size_t GATE_LDS = (GATE_LCC + MAX_LCC) * sizeof(int);
+// Where a step does not gate: the LCCs as they are.
+template <int NT>
+__device__ __forceinline__ void held_lccs(const RealDesc& d, int* smem) {
+  for (int i = NT - 1 - threadIdx.x; i < d.n_lcc; i += NT)
+    smem[GATE_LCC + i] = srs_lcc_open(d.lcc_state[i], d.lccv_state[i]);
+}
+
 // The gating and loop body of realization r by one workgroup of NT threads.
 // PROTO = false leaves out the loop body (callers that never pass G_PROTOCOL).
-// smem: GATE_LDS bytes; its last MAX_RYR ints end as the RyR states.
-constexpr size_t GATE_LDS = 4 * MAX_RYR * sizeof(int);
-template <int NT, bool PROTO = true>
+// smem: GATE_LDS bytes; from GATE_RYR its ints end as the RyR states, from
+// GATE_LCC as whether the LCCs are open.  mid() runs once, by every thread,
+// after the first barrier: work of other wavefronts than the first and the
+// last, which mostly gate no channel, done while those two are at theirs.
+struct NoMid { __device__ void operator()() const {} };
+template <int NT, bool PROTO = true, class Mid = NoMid>
 __device__ __forceinline__ void gate_workgroup(const RealDesc* __restrict__ D, RealLive* __restrict__ L, const int r,
-                                               const uint32_t mode, int* smem) {
+                                               const uint32_t mode, int* smem, Mid mid = NoMid()) {
   static_assert(MAX_RYR % NT == 0 && MAX_LCC % NT == 0, "channel slots per thread");
   const RealDesc& d = D[r];
   RealLive& l = L[r];
   if (l.done) return;
-  int *s_old = smem, *s_a = smem + MAX_RYR, *s_b = smem + 2 * MAX_RYR, *s_fin = smem + 3 * MAX_RYR;
+  int *s_old = smem, *s_a = smem + MAX_RYR, *s_b = smem + 2 * MAX_RYR, *s_fin = smem + GATE_RYR;
+  int* s_lcc = smem + GATE_LCC;
   const int tid = threadIdx.x;
   const int cur = l.cur;
   // In the flag_ffwd phase the sweep skipped this realization: the fields are
@@ -374,43 +386,49 @@ __device__ __forceinline__ void gate_workgroup(const RealDesc* __restrict__ D, R
     const int l0 = NT - 1 - tid;
     if (l0 < d.n_lcc) load_lcc(l0);
     __syncthreads();
+    mid();
+    // LCCs, cpu/RunSimulation.cpp:229-400; first, so that their wavefronts work
+    // while the RyRs' do
+#pragma unroll 1
+    for (int i = l0; i < d.n_lcc; i += NT) {
+      if (i != l0) load_lcc(i);
+      const int s = ls, vs = lvs;
+      double tr[3];
+      int32_t tg[3];
+      const double lr = srs_lcc_rates(s, vs, l.vm, ca_l, tr, tg);
+      const int ic = nr + i;
+      double Rn = Rl + (tr[0] + tr[1] + tr[2] + lr) * dt;
+      int sn = s, vn = vs;
+      if (Rn > 0) {
+        uint64_t o[4];
+        srs_philox4x64_10((uint64_t)step, (uint64_t)ic, d.stream, SRS_PURPOSE_GATING, d.key, SRS_PHILOX_KEY1, o);
+        Rn = log(srs_open01(o[0]));
+        const double u = srs_open01(o[1]) * (tr[0] + tr[1] + tr[2] + lr);
+        if (u < tr[0]) sn = tg[0];
+        else if (u < tr[0] + tr[1]) sn = tg[1];
+        else if (u < tr[0] + tr[1] + tr[2]) sn = tg[2];
+        else vn = (vs == 1) ? 2 : 1;
+        d.lcc_state[i] = sn;
+        d.lccv_state[i] = vn;
+      }
+      s_lcc[i] = srs_lcc_open(sn, vn);
+      d.R[ic] = Rn;
+    }
     // RyRs: the reference updates them one after another (later RyRs see
     // earlier flips through the neighbour counts, cpu/RunSimulation.cpp:661-666).
     // Each sweep below recomputes every RyR with lower-index neighbours taken
     // from the previous sweep's result and higher-index ones from the old
     // states; the first sweep that changes nothing is the sequential result.
+    // (For uncoupled RyRs the neighbour counts do not enter the rate, A* = 0
+    // gives X = 1.)  A rate is some 250 dependent instructions, 0.9 us: with at
+    // most one RyR per thread the last sweep's values are committed as they are
+    // instead of being computed once more.
     const bool coupled = P[SRS_R_RYR_A_STAR] != 0.0;
     int* prev = s_a;
     int* next = s_b;
-    if (coupled) {
-      for (int it = 0; it <= nr; ++it) {
-        int changed = 0;
-#pragma unroll 1
-        for (int i = tid; i < nr; i += NT) {
-          if (nr > NT) load_ryr(i);
-          int no = 0, ncl = 0;
-          for (int q = 0; q < 4; ++q) {
-            const int nb = d.ryr_nb[4 * i + q];
-            if (nb >= 0) {
-              const int s = (nb < i) ? prev[nb] : s_old[nb];
-              if (s) no++; else ncl++;
-            }
-          }
-          const double rate = srs_ryr_rate(s_old[i], no, ncl, ca_c, ca_j, P);
-          const double Rn = Rr + rate * dt;
-          const int ns = (Rn > 0) ? (s_old[i] == 1 ? 0 : 1) : s_old[i];
-          next[i] = ns;
-          changed |= (ns != prev[i]);
-        }
-        changed = __syncthreads_or(changed);
-        int* tmp = prev; prev = next; next = tmp;
-        if (!changed) break;
-      }
-    }
-    // Commit with neighbour states from the fixed point (for uncoupled RyRs
-    // the neighbour counts do not enter the rate, A* = 0 gives X = 1).
-#pragma unroll 1
-    for (int i = tid; i < nr; i += NT) {
+    double Rn = 0.0;
+    int ns = 0;
+    auto update = [&](const int i) {
       if (nr > NT) load_ryr(i);
       int no = 0, ncl = 0;
       if (coupled) {
@@ -422,52 +440,49 @@ __device__ __forceinline__ void gate_workgroup(const RealDesc* __restrict__ D, R
           }
         }
       }
-      const double rate = srs_ryr_rate(s_old[i], no, ncl, ca_c, ca_j, P);
-      double Rn = Rr + rate * dt;
-      int ns = s_old[i];
+      Rn = Rr + srs_ryr_rate(s_old[i], no, ncl, ca_c, ca_j, P) * dt;
+      ns = (Rn > 0) ? (s_old[i] == 1 ? 0 : 1) : s_old[i];
+    };
+    if (coupled) {
+      for (int it = 0; it <= nr; ++it) {
+        int changed = 0;
+#pragma unroll 1
+        for (int i = tid; i < nr; i += NT) {
+          update(i);
+          next[i] = ns;
+          changed |= (ns != prev[i]);
+        }
+        changed = __syncthreads_or(changed);
+        int* tmp = prev; prev = next; next = tmp;
+        if (!changed) break;
+      }
+    }
+    // commit
+#pragma unroll 1
+    for (int i = tid; i < nr; i += NT) {
+      if (!coupled || nr > NT) update(i);
       if (Rn > 0) {
         uint64_t o[4];
         srs_philox4x64_10((uint64_t)step, (uint64_t)i, d.stream, SRS_PURPOSE_GATING, d.key, SRS_PHILOX_KEY1, o);
         Rn = log(srs_open01(o[0]));
-        ns = (s_old[i] == 1) ? 0 : 1;
       }
       d.R[i] = Rn;
       d.ryr_state[i] = ns;
       s_fin[i] = ns;
     }
-    // LCCs, cpu/RunSimulation.cpp:229-400
-#pragma unroll 1
-    for (int i = l0; i < d.n_lcc; i += NT) {
-      if (i != l0) load_lcc(i);
-      const int s = ls, vs = lvs;
-      double tr[3];
-      int32_t tg[3];
-      const double lr = srs_lcc_rates(s, vs, l.vm, ca_l, tr, tg);
-      const int ic = nr + i;
-      double Rn = Rl + (tr[0] + tr[1] + tr[2] + lr) * dt;
-      if (Rn > 0) {
-        uint64_t o[4];
-        srs_philox4x64_10((uint64_t)step, (uint64_t)ic, d.stream, SRS_PURPOSE_GATING, d.key, SRS_PHILOX_KEY1, o);
-        Rn = log(srs_open01(o[0]));
-        const double u = srs_open01(o[1]) * (tr[0] + tr[1] + tr[2] + lr);
-        if (u < tr[0]) d.lcc_state[i] = tg[0];
-        else if (u < tr[0] + tr[1]) d.lcc_state[i] = tg[1];
-        else if (u < tr[0] + tr[1] + tr[2]) d.lcc_state[i] = tg[2];
-        else d.lccv_state[i] = (vs == 1) ? 2 : 1;
-      }
-      d.R[ic] = Rn;
-    }
   }
   else {
-    for (int i = tid; i < nr; i += NT) s_fin[i] = d.ryr_state[i];
+    // a replay (never with gating) takes the row of the next step, if there is one
+    const int64_t k = step + 1 - l.sched_base;
+    if ((mode & G_REPLAY) && k < d.n_sched)
+      for (int i = tid; i < nr; i += NT) s_fin[i] = d.ryr_state[i] = d.sched[k * nr + i];
+    else
+      for (int i = tid; i < nr; i += NT) s_fin[i] = d.ryr_state[i];
+    held_lccs<NT>(d, smem);
+    mid();
   }
   __syncthreads();
 
-  if (mode & G_REPLAY) {
-    const int64_t k = step + 1 - l.sched_base;  // schedule row of the next step
-    if (k < d.n_sched)
-      for (int i = tid; i < nr; i += NT) s_fin[i] = d.ryr_state[i] = d.sched[k * nr + i];
-  }
   if (mode & G_RECORD) {  // a launch of its own after each step took 4.7 us
     const int64_t k = step + 1 - d.rec_step0;
     if (k < d.n_sched)
@@ -553,6 +568,7 @@ __device__ __forceinline__ void gate_workgroup(const RealDesc* __restrict__ D, R
   if (d.I[SRS_I_FLAG_LCC] && l.lcc_open && t >= l.t_lcc_close) {  // :525-528
     l.lcc_open = 0;
     d.lcc_state[d.I[SRS_I_LCC_INDEX]] = 1;
+    s_lcc[d.I[SRS_I_LCC_INDEX]] = 0;
   }
   if (d.I[SRS_I_FLAG_V_CLAMP]) l.vm = (t <= P[SRS_R_T_CLAMP]) ? P[SRS_R_V_CLAMP] : P[SRS_R_DEFAULT_VM];  // :531-537
   const int ir = d.I[SRS_I_INIT_RYR];
@@ -570,13 +586,13 @@ __device__ __forceinline__ void gate_workgroup(const RealDesc* __restrict__ D, R
 #if SRS_UNIT == 0
 __global__ __launch_bounds__(GATE_THREADS) void k_gate(const RealDesc* __restrict__ D, RealLive* __restrict__ L,
                                                        uint32_t mode) {
-  __shared__ int smem[4 * MAX_RYR];
+  __shared__ int smem[GATE_LDS / sizeof(int)];
   gate_workgroup<GATE_THREADS>(D, L, blockIdx.x, mode, smem);
 }
 // The gating of the realizations of a list (one subset of the context).
 __global__ __launch_bounds__(GATE_THREADS) void k_gate_list(const RealDesc* __restrict__ D, RealLive* __restrict__ L,
                                                             const int32_t* __restrict__ rids, uint32_t mode) {
-  __shared__ int smem[4 * MAX_RYR];
+  __shared__ int smem[GATE_LDS / sizeof(int)];
   gate_workgroup<GATE_THREADS>(D, L, rids[blockIdx.x], mode, smem);
 }
 #endif
@@ -616,64 +632,83 @@ __device__ __forceinline__ void sweep_gated(const RealDesc* __restrict__ D, Real
   if (b == 0) {
     // The channel elements: all that does not depend on the gating (every
     // species but Ca, and Ca's rate without the fluxes) is loaded, computed and
-    // stored before it, by wavefronts that mostly gate no channel, so that its
-    // memory round trips run beside the gating's; a channel-flux element is one
-    // record instead of a search and six tables.  This workgroup's chain of
-    // loads was the step of a small mesh: 9.2 -> 6.5 us on 56,250 elements,
-    // 10.1 -> 7.8 on 172,494.
-    int* s_fin = (int*)dyn_lds + 3 * MAX_RYR;
+    // stored beside the gating, by wavefronts that mostly gate no channel; a
+    // channel-flux element is one record instead of a search and six tables.
+    // This workgroup's chain is the step of a small mesh (the tiles alone take
+    // 4.7 us on 56,250 elements, an empty launch 1.6): 9.2 us with everything
+    // after the gating, 6.5 with the first half ahead of the gating's first
+    // barrier, which then waits for it, 5.3 with it behind that barrier; 10.1,
+    // 7.8 and 7.4 on 172,494 elements.  Only its loads ahead of the barrier is no
+    // faster and spills in the four-wavefront variant (5.5 and 11.9).
+    int* smem = (int*)dyn_lds;
     constexpr int FIRST = BS / 4;  // the thread of channel element 0
+    struct Raw { d4 m0, m1, m2, m3, m4; double tr, cs, xj, xc, a[5], v0, tt; int code, j, e0, e1; uint8_t f; };
     struct Pending { double rca, ca, B, dc, v0; int code, j, e0, e1; };
-    auto fetch = [&](int k) -> Pending {
+    auto load = [&](int k) -> Raw {
       const ChanElem* r = d.crec + k;
       const SRS_GLOBAL double* Xo = bf.xo;
-      const uint8_t f = (uint8_t)r->f;
       const size_t np = d.np;
-      Pending p;
-      p.j = r->j;
-      p.e0 = r->e0;
-      p.e1 = r->e1;
-      p.v0 = r->v0;
-      const ChanEntry en = d.centry[p.e0];
-      p.code = en.code;
+      Raw w;
+      w.f = (uint8_t)r->f;
+      w.j = r->j;
+      w.e0 = r->e0;
+      w.e1 = r->e1;
+      w.v0 = r->v0;
+      w.tt = r->tt;
+      w.code = r->code;
+      for (int q = 0; q < 5; ++q) w.a[q] = r->a[q];
+      w.m0 = ld_quad(Xo, qidx1(w.j));
+      w.m1 = ld_quad(Xo, qidx1(r->nb[0])), w.m2 = ld_quad(Xo, qidx1(r->nb[1]));
+      w.m3 = ld_quad(Xo, qidx1(r->nb[2])), w.m4 = ld_quad(Xo, qidx1(r->nb[3]));
+      w.tr = lives_tr(w.f) ? Xo[4 * np + w.j] : 0.0;
+      w.cs = lives_cs(w.f) ? Xo[5 * np + w.j] : 0.0;
+      w.xj = w.xc = 0.0;
+      if (w.code >= 0) w.xj = Xo[cq(r->jsr)], w.xc = Xo[cq(r->cyt)];
+      return w;
+    };
+    auto half = [&](const Raw& w) -> Pending {
+      Pending p{0.0, w.m0.x, 0.0, w.xj - w.xc, w.v0, w.code, w.j, w.e0, w.e1};
       Loc c;
-      c.m0 = ld_quad(Xo, qidx1(p.j));
-      const d4 m1 = ld_quad(Xo, qidx1(r->nb[0])), m2 = ld_quad(Xo, qidx1(r->nb[1]));
-      const d4 m3 = ld_quad(Xo, qidx1(r->nb[2])), m4 = ld_quad(Xo, qidx1(r->nb[3]));
-      c.c_tr = lives_tr(f) ? Xo[4 * np + p.j] : 0.0;
-      c.c_cs = lives_cs(f) ? Xo[5 * np + p.j] : 0.0;
-      p.dc = en.code >= 0 ? Xo[2 * (size_t)qidx1(en.jsr)] - Xo[2 * (size_t)qidx1(en.cyt)] : 0.0;
-      c.s = c.m0 * r->a[0] + m1 * r->a[1] + m2 * r->a[2] + m3 * r->a[3] + m4 * r->a[4];
-      const Rates q = elem_rates<-1>(d, l, p.j, f, c, r->tt, p.v0);
-      elem_store<NTS, -1>(d, bf, p.j, f, c, q);  // Ca without its fluxes: replaced by finish
+      c.m0 = w.m0;
+      c.c_tr = w.tr;
+      c.c_cs = w.cs;
+      c.s = w.m0 * w.a[0] + w.m1 * w.a[1] + w.m2 * w.a[2] + w.m3 * w.a[3] + w.m4 * w.a[4];
+      const Rates q = elem_rates<-1>(d, l, w.j, w.f, c, w.tt, w.v0);
+      elem_store<NTS, -1>(d, bf, w.j, w.f, c, q);  // Ca without its fluxes: replaced by finish
       p.rca = q.ca;
-      p.ca = c.m0.x;
       p.B = q.B;  // 1 where nothing divides
       return p;
     };
+    auto is_open = [&](int code) { return code >= 0 ? smem[GATE_RYR + (code >> 1)] : smem[GATE_LCC - code - 1]; };
     auto finish = [&](const Pending& p) {
       double rca = p.rca;
-      chan_flux(d, l, p.code, p.code >= 0 && s_fin[p.code >> 1], p.dc, p.ca, p.v0, rca);
+      chan_flux(d, l, p.code, is_open(p.code), p.dc, p.ca, p.v0, rca);
       for (int i = p.e0 + 1; i < p.e1; ++i) {
         const ChanEntry en = d.centry[i];
-        const bool open = en.code >= 0 && s_fin[en.code >> 1];
-        const double dc =
-            open ? bf.xo[2 * (size_t)qidx1(en.jsr)] - bf.xo[2 * (size_t)qidx1(en.cyt)] : 0.0;
+        const bool open = is_open(en.code);
+        const double dc = open && en.code >= 0 ? bf.xo[cq(en.jsr)] - bf.xo[cq(en.cyt)] : 0.0;
         chan_flux(d, l, en.code, open, dc, p.ca, p.v0, rca);
       }
       rca /= p.B;
-      bf.xn[2 * (size_t)qidx1(p.j)] = p.ca + rca * d.P[SRS_R_T_STEP];
+      bf.xn[cq(p.j)] = p.ca + rca * d.P[SRS_R_T_STEP];
     };
     const int k0 = ((int)threadIdx.x + BS - FIRST) % BS;
+    const bool pre = PRE && !skip && k0 < d.n_celem;
     Pending p0;
-    if (PRE && !skip && k0 < d.n_celem) p0 = fetch(k0);
-    if (gmode) gate_workgroup<BS, PROTO>(D, L, 0, gmode, (int*)dyn_lds);
-    else
-      for (int i = threadIdx.x; i < d.n_ryr; i += BS) s_fin[i] = d.ryr_state[i];
+    auto mid = [&] {
+      if (pre) p0 = half(load(k0));
+    };
+    if (gmode) {
+      gate_workgroup<BS, PROTO>(D, L, 0, gmode, smem, mid);
+    } else {
+      for (int i = threadIdx.x; i < d.n_ryr; i += BS) smem[GATE_RYR + i] = d.ryr_state[i];
+      held_lccs<BS>(d, smem);
+      mid();
+    }
     __syncthreads();  // the new channel states, written by this workgroup, before the flux reads them
     if (skip) return;
-    if (PRE && k0 < d.n_celem) finish(p0);
-    for (int k = PRE ? k0 + BS : k0; k < d.n_celem; k += BS) finish(fetch(k));
+    if (pre) finish(p0);
+    for (int k = PRE ? k0 + BS : k0; k < d.n_celem; k += BS) finish(half(load(k)));
     return;
   }
   if (skip) return;
@@ -723,7 +758,7 @@ GatedFn pick_gated_nt(int nts) {
 
 // How much the registers of the gating workgroup may cost the tiles.  With no
 // more tiles than CUs (256), each workgroup has a CU to itself: no budget
-// (56,250 elements: 6.5 us per step, 6.9 with four wavefronts per SIMD).  Up to
+// (56,250 elements: 5.3 us per step).  Up to
 // 900,000 elements the gating workgroup is still the longest one: four
 // wavefronts, with its loads ahead of the gating (400,000 elements: 12.5
 // against 17.0 us with six).  Beyond that the tiles' own wavefronts decide: six,
@@ -1655,6 +1690,10 @@ int srs_ctx_finalize(srs_ctx* c, int32_t record_capacity) {
       e.e0 = hr.cstart[k];
       e.e1 = hr.cstart[k + 1];
       e.f = hm.flags[e.j];
+      const ChanEntry& en = hr.centry[e.e0];
+      e.code = en.code;
+      e.jsr = en.jsr;
+      e.cyt = en.cyt;
     }
     ChanEntry* pe;
     ChanElem* pc;
