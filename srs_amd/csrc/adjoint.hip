@@ -27,22 +27,23 @@ __constant__ const int kAdjTheta[ADJ_NT] = {SRS_R_D_CA,     SRS_R_D_DYE,     SRS
                                             SRS_R_K_ON_DYE, SRS_R_K_OFF_DYE, SRS_R_V_RYR,     SRS_R_A_P,
                                             SRS_R_K_D_SL_HI};
 
-// 1 / beta of the rapid SL buffer at element j and its derivatives in c and
-// in K_D_SL_HI (cpu/RunSimulation.cpp:15-22).
-struct SlBuf { double beta, dbeta_dc, dbeta_dkh; };
-__device__ __forceinline__ SlBuf sl_buffer(const RealDesc& d, int j, double c, uint8_t f) {
-  SlBuf s{1.0, 0.0, 0.0};
-  if (!(f & F_SL)) return s;
-  const double* P = d.P;
-  const double ttj = d.tt[j], v0j = d.V0[j];
-  const double bhi = ttj * P[SRS_R_B_TOT_SL_HI] / (v0j * (1e-15));
-  const double blo = ttj * P[SRS_R_B_TOT_SL_LO] / (v0j * (1e-15));
+// 1 / beta of the rapid SL buffer (cpu/RunSimulation.cpp:15-22) at an element
+// with F_SL, beta = 1 + q (B_hi K_hi / (K_hi + c)^2 + B_lo K_lo / (K_lo + c)^2),
+// q = TT area / (V0 1e-15): over the common denominator, one division instead
+// of six (a neighbour's w is on the step's critical path).
+__device__ __forceinline__ double sl_inv_beta(const double* P, double tt, double v0, double c) {
   const double kh = P[SRS_R_K_D_SL_HI], kl = P[SRS_R_K_D_SL_LO];
-  const double eh = kh + c, el = kl + c;
-  s.beta = 1 + (bhi * kh / (eh * eh)) + (blo * kl / (el * el));
-  s.dbeta_dc = -2 * bhi * kh / (eh * eh * eh) - 2 * blo * kl / (el * el * el);
-  s.dbeta_dkh = bhi * (c - kh) / (eh * eh * eh);
-  return s;
+  const double eh = kh + c, el = kl + c, eh2 = eh * eh, el2 = el * el;
+  const double D = eh2 * el2 * (v0 * 1e-15);
+  return D / (D + tt * (P[SRS_R_B_TOT_SL_HI] * kh * el2 + P[SRS_R_B_TOT_SL_LO] * kl * eh2));
+}
+// Derivatives of beta in c and in K_D_SL_HI.
+struct SlDer { double dc, dkh; };
+__device__ __forceinline__ SlDer sl_derivs(const double* P, double tt, double v0, double c) {
+  const double q = tt / (v0 * 1e-15), kh = P[SRS_R_K_D_SL_HI], kl = P[SRS_R_K_D_SL_LO];
+  const double eh = kh + c, el = kl + c, r = 1.0 / (eh * el), ih = r * el, il = r * eh;
+  const double hi = q * P[SRS_R_B_TOT_SL_HI] * ih * ih * ih, lo = q * P[SRS_R_B_TOT_SL_LO] * il * il * il;
+  return SlDer{-2.0 * (hi * kh + lo * kl), hi * (c - kh)};
 }
 
 // The loss source of one scan sample at element j: sum_i gcoef_i w(c_j - p_i)
@@ -99,8 +100,8 @@ struct AdjScan {
 
 // The tiles of each chiplet's workgroups lie next to each other (the grid's
 // remainder modulo eight keeps its place): its L2 then holds most neighbours
-// (8.5 against 9.2 us per step on the 56,124-element mesh, 234 either way on
-// eight 927,816-element members).
+// (8.5 against 9.2 us per step on the 56,124-element mesh when it was measured,
+// the same on eight 927,816-element members).
 __device__ __forceinline__ int xcd_run(int bid, int grid) {
   const int whole = grid / NXCD * NXCD;
   return bid < whole ? xcd_tile(bid, whole) : bid;
@@ -112,9 +113,8 @@ __device__ __forceinline__ int xcd_run(int bid, int grid) {
 // Bound by memory traffic and the gathers' lines: m, X and the rows in and m
 // out are 1.16 GB per step of eight 927,816-element members, 211 us at the
 // 5.5 TB/s that a launch of this mix of reads and writes reaches; the step
-// takes 234 us.  It took 309 us with lambda itself stored, whose gather read
-// 1/V0 as well or w written by a launch or a step of its own; storing m took
-// it to 289.  The neighbours staged in LDS with the sweep's halo lists are
+// takes 229 us, and 309 with lambda itself stored, whose gather read 1/V0 as
+// well or w written by a pass of its own.  The neighbours staged in LDS with the sweep's halo lists are
 // slower (251 us, and 9.9 against 9.2 us on the 56,124-element mesh): the
 // registers that hold the gradient sums leave four wavefronts per SIMD, too
 // few to cover a barrier, and the second copy of m fits the cache.
@@ -147,8 +147,7 @@ __device__ __forceinline__ void adj_step(const RealDesc* __restrict__ D, const R
   const bool in = j < d.n;
   Geo g{};
   d4 m0 = {0.0, 0.0, 0.0, 0.0}, mu = {0.0, 0.0, 0.0, 0.0};
-  double V0 = 1.0, u = 0.0;
-  SlBuf sb{1.0, 0.0, 0.0};
+  double V0 = 1.0, u = 0.0, ttj = 0.0, inv_beta = 1.0;
   if (in) {
     g = load_geo_nbr<CLASS>(d, j);
     m0 = ld_quad(gp(X), qidx1(j));
@@ -156,18 +155,47 @@ __device__ __forceinline__ void adj_step(const RealDesc* __restrict__ D, const R
     V0 = gp(d.V0)[j];
     u = mu.x;
     if (g.f & F_SL) {
-      sb = sl_buffer(d, j, m0.x, g.f);
-      u = mu.x / sb.beta;
+      ttj = gp(d.tt)[j];
+      inv_beta = sl_inv_beta(d.P, ttj, V0, m0.x);
+      u = mu.x * inv_beta;
     }
   }
   auto w_at = [&](uint32_t e) -> d4 {
     const uint32_t i = idx_of(e);
     d4 w = ld_quad(gp(lam), qidx1(i));
-    if (e & IDX_SL) w.x /= sl_buffer(d, (int)i, X[2 * (size_t)qidx1(i)], F_SL).beta;
+    if (e & IDX_SL) w.x *= sl_inv_beta(d.P, gp(d.tt)[i], gp(d.V0)[i], X[cq(i)]);
     return w;
   };
   d4 w1{}, w2{}, w3{}, w4{};
   if (in) w1 = w_at(g.l1), w2 = w_at(g.l2), w3 = w_at(g.l3), w4 = w_at(g.l4);
+  // The realization's record of a channel element: those of the wavefront's 64
+  // elements follow each other in crec, so one round of loads counts the
+  // records before them and the flags below a lane give its place (a mesh
+  // shared with other clusters: a search).  A binary search and the tables it
+  // led to were ten loads in a chain: 8.5 -> 7.6 us per step of the 56,124-element
+  // mesh, with one division per SL neighbour instead of six.
+  int own = -1;
+  ChanElem ce{};
+  const uint64_t chan = __builtin_amdgcn_ballot_w64(in && (g.f & F_CHAN));
+  if (chan) {
+    const int lane = threadIdx.x & 63, j0 = j - lane;
+    int before = 0;
+    for (int k = 0; k < d.n_celem; k += 64)
+      before += __builtin_popcountll(__builtin_amdgcn_ballot_w64(k + lane < d.n_celem && d.celem[min(k + lane, d.n_celem - 1)] < j0));
+    if (chan >> lane & 1) {
+      own = before + __builtin_popcountll(chan & ((1ull << lane) - 1));
+      if (own < d.n_celem) ce = d.crec[own];
+      if (own >= d.n_celem || ce.j != j) {
+        int lo = before, hi = min(own, d.n_celem);
+        while (lo < hi) {
+          const int mid = (lo + hi) >> 1;
+          if (d.celem[mid] < j) lo = mid + 1; else hi = mid;
+        }
+        own = lo < d.n_celem && d.celem[lo] == j ? lo : -1;
+        if (own >= 0) ce = d.crec[own];
+      }
+    }
+  }
   // the scan sample's loss source (all lanes of the wavefront take part)
   const double src =
       SCAN ? scan_adj_sum(sc.cen, sc.g, sc.n_f, sc.gcoef + (size_t)blockIdx.y * sc.gstride, np, j, in) : 0.0;
@@ -258,25 +286,19 @@ __device__ __forceinline__ void adj_step(const RealDesc* __restrict__ D, const R
       lc += dt * ((muC - u) * kon * (B - bC) - u * P[SRS_R_V_REFILL]);
       lC += dt * (muC - u) * (-kon * c - koff);
     }
-    if (f & F_CHAN) {
-      int lo = 0, hi = d.n_celem;
-      while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (d.celem[mid] < j) lo = mid + 1; else hi = mid;
-      }
-      if (lo < d.n_celem && d.celem[lo] == j) {
-        const double a = P[SRS_R_V_RYR] * P[SRS_R_V_CELL];
-        for (int e = d.cstart[lo]; e < d.cstart[lo + 1]; ++e) {
-          const ChanEntry en = d.centry[e];
-          const int ch = en.code;
-          if (ch >= 0) {
-            const int i = ch >> 1;
-            if (!ryr[i]) continue;
-            const int ce = en.cyt, je = en.jsr;
-            const int p = (ch & 1) ? ce : je;  // the partner element
-            const double cp = X[2 * (size_t)qidx1(p)];
-            const double up = lam[2 * (size_t)qidx1(p)] / sl_buffer(d, p, cp, d.flags[p]).beta;
-            const double dc = X[2 * (size_t)qidx1(je)] - X[2 * (size_t)qidx1(ce)];
+    if (own >= 0) {
+      const double a = P[SRS_R_V_RYR] * P[SRS_R_V_CELL];
+      ChanEntry en = ce.first;
+      for (int e = ce.e0;;) {
+        const int ch = en.code;
+        if (ch >= 0) {
+          const int p = (ch & 1) ? en.cyt : en.jsr;  // the partner element
+          if (ryr[ch >> 1]) {
+            const double xj = X[cq(en.jsr)], xc = X[cq(en.cyt)];
+            double up = lam[cq(p)];
+            if (en.sl & ((ch & 1) ? 2 : 1))
+              up *= sl_inv_beta(P, gp(d.tt)[p], gp(d.V0)[p], (ch & 1) ? xc : xj);
+            const double dc = xj - xc;
             const double J = a * dc;
             lc += dt * (a / V0) * (up - u);
             if (ch & 1) {  // jSR side: r -= J / V0_jsr
@@ -285,20 +307,23 @@ __device__ __forceinline__ void adj_step(const RealDesc* __restrict__ D, const R
               rca += J / V0;
               gr[10] += dt * P[SRS_R_V_CELL] * dc * (u - up);
             }
-          } else {
-            const int i = -ch - 1;
-            if (srs_lcc_open(d.lcc_state[i], d.lccv_state[i])) {
-              rca += srs_lcc_flux_raw(l.vm, c, P[SRS_R_CA_0]) / V0;
-              lc += dt * u * srs_lcc_flux_raw(l.vm, 1.0, 0.0) / V0;
-            }
+          }
+        } else {
+          const int i = -ch - 1;
+          if (srs_lcc_open(d.lcc_state[i], d.lccv_state[i])) {
+            rca += srs_lcc_flux_raw(l.vm, c, P[SRS_R_CA_0]) / V0;
+            lc += dt * u * srs_lcc_flux_raw(l.vm, 1.0, 0.0) / V0;
           }
         }
+        if (++e >= ce.e1) break;
+        en = d.centry[e];
       }
     }
     if (f & F_SL) {
-      const double b2 = sb.beta * sb.beta;
-      lc += dt * mu.x * (-rca * sb.dbeta_dc / b2);
-      gr[12] += dv0 * mu.x * (-rca * sb.dbeta_dkh / b2);
+      const SlDer sd = sl_derivs(P, ttj, V0, c);
+      const double k = mu.x * (-rca * inv_beta * inv_beta);
+      lc += dt * k * sd.dc;
+      gr[12] += dv0 * k * sd.dkh;
     }
     if (SCAN) ld += src;
     st_quad<NTS>(gpw(lam_out), qidx1(j), d4{lc, la, lm, ld});

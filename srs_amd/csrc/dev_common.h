@@ -67,7 +67,7 @@ typedef double d4 __attribute__((ext_vector_type(4)));
 struct ChanEntry {
   int32_t code;      // >=0: 2*ryr + side (0 cleft, 1 jSR); <0: -(lcc+1)
   int32_t jsr, cyt;  // a RyR's two elements
-  int32_t pad;
+  int32_t sl;        // bit 0: jsr has F_SL, bit 1: cyt has
 };
 // Everything about a channel-flux element that is fixed, in one record, for
 // the workgroup that gates and then updates these elements (sweep_gated).
@@ -75,7 +75,7 @@ struct ChanElem {
   double a[5], v0, tt;
   int32_t j, nb[4], e0, e1;  // the element, its neighbours, its run of centry
   uint32_t f;
-  int32_t code, jsr, cyt, pad;  // centry[e0]
+  ChanEntry first;  // centry[e0]
 };
 
 // Immutable per-realization descriptor (read with scalar loads).

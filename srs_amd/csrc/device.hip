@@ -655,7 +655,7 @@ __device__ __forceinline__ void sweep_gated(const RealDesc* __restrict__ D, Real
       w.e1 = r->e1;
       w.v0 = r->v0;
       w.tt = r->tt;
-      w.code = r->code;
+      w.code = r->first.code;
       for (int q = 0; q < 5; ++q) w.a[q] = r->a[q];
       w.m0 = ld_quad(Xo, qidx1(w.j));
       w.m1 = ld_quad(Xo, qidx1(r->nb[0])), w.m2 = ld_quad(Xo, qidx1(r->nb[1]));
@@ -663,7 +663,7 @@ __device__ __forceinline__ void sweep_gated(const RealDesc* __restrict__ D, Real
       w.tr = lives_tr(w.f) ? Xo[4 * np + w.j] : 0.0;
       w.cs = lives_cs(w.f) ? Xo[5 * np + w.j] : 0.0;
       w.xj = w.xc = 0.0;
-      if (w.code >= 0) w.xj = Xo[cq(r->jsr)], w.xc = Xo[cq(r->cyt)];
+      if (w.code >= 0) w.xj = Xo[cq(r->first.jsr)], w.xc = Xo[cq(r->first.cyt)];
       return w;
     };
     auto half = [&](const Raw& w) -> Pending {
@@ -1679,6 +1679,8 @@ int srs_ctx_finalize(srs_ctx* c, int32_t record_capacity) {
     if ((rc = dev_upload(c, &p, hr.lcc_ele))) return rc; d.lcc_ele = p;
     if ((rc = dev_upload(c, &p, hr.celem))) return rc; d.celem = p;
     if ((rc = dev_upload(c, &p, hr.cstart))) return rc; d.cstart = p;
+    for (ChanEntry& en : hr.centry)
+      if (en.code >= 0) en.sl = (hm.flags[en.jsr] & F_SL ? 1 : 0) | (hm.flags[en.cyt] & F_SL ? 2 : 0);
     std::vector<ChanElem> crec(hr.celem.size());
     for (size_t k = 0; k < crec.size(); ++k) {
       ChanElem& e = crec[k];
@@ -1690,10 +1692,7 @@ int srs_ctx_finalize(srs_ctx* c, int32_t record_capacity) {
       e.e0 = hr.cstart[k];
       e.e1 = hr.cstart[k + 1];
       e.f = hm.flags[e.j];
-      const ChanEntry& en = hr.centry[e.e0];
-      e.code = en.code;
-      e.jsr = en.jsr;
-      e.cyt = en.cyt;
+      e.first = hr.centry[e.e0];
     }
     ChanEntry* pe;
     ChanElem* pc;
