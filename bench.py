@@ -197,8 +197,7 @@ def bench_cpu_ensemble(procs=16, budget_s=8.0):
 
 def bench_batched(n_real, steps, warmup, order, tune=None, n_tune=512):
     """The batched leg and its plain-sequential reference.  Unless `tune` is
-    given, the batched sweep is autotuned (tile, realization group, cache
-    hints, LDS staging) on the first `n_tune` members of the same ensemble,
+    given, the batched sweep is autotuned (tile, cache hints) on the first `n_tune` members of the same ensemble,
     and the plain path on each of the three meshes on its own."""
     import srs_amd as S
     from srs_amd import workloads as W
@@ -284,9 +283,8 @@ def bench_adjoint_batch(n_real=256, n_steps=256, n_points=64, n_samples=8, max_b
     from theta moved by +-10%.  Times the batched loss alone and the loss with
     every member's gradient (the library's checkpoint plan, at most max_batch
     members stepped at once).  sweep_tune: sweep tunables set after the set-up
-    (nt_geometry, nt_state, occupancy, lds), for the forward and recomputed
-    steps; adj_w: the reverse step's w form (0 by launch size, 1 written by
-    each step, 2 formed in the kernel)."""
+    (nt_state, occupancy), for the forward and recomputed steps; adj_waves and
+    adj_w are accepted by the library and change nothing."""
     from srs_amd import workloads as W
 
     t0 = time.perf_counter()
@@ -543,10 +541,8 @@ def main():
         f" gating {gate_ms * 1e3:.2f} us")
     value = args.steps * dt / wall
     # The library folds each step's gating into the next step's sweep launch
-    # (k_sweep_gated) for a single realization with the LDS sweep and a
-    # register budget of 0 or 6; time_sweep then times that kernel.
-    eff = {"lds": 1, "occupancy": 0, "gated_sweep": 1, **tune}
-    kernel = "k_sweep_gated" if eff["gated_sweep"] and eff["lds"] and eff["occupancy"] in (0, 6) else "k_sweep"
+    # (k_sweep_gated) for a single realization; time_sweep then times that kernel.
+    kernel = "k_sweep_gated" if tune.get("gated_sweep", 1) else "k_sweep"
     nbytes = algorithmic_bytes(N)
     achieved = nbytes / (sweep_ms * 1e-3) / 1e9
     traffic = profiled_traffic(os.path.join(ROOT, "profiles", f"k_sweep_{args.workload}_traffic.md"))

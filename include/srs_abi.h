@@ -298,7 +298,7 @@ int srs_ctx_create(int device, srs_ctx** out);
                                     step's gating (and, with SRS_STEP_PROTOCOL, the loop body) inside the
                                     next step's sweep launch; 0: a gating launch after every sweep */
 #define SRS_TUNE_SUBSET_MB 12    /* 0 (default): every step sweeps all realizations; > 0: srs_explicit_step
-                                    steps runs of realization groups whose state takes at most this many MB
+                                    steps runs of realizations whose state takes at most this many MB
                                     through a whole block of steps (128 with SRS_STEP_GRAPH) each, one after
                                     another, so that a run's state stays in the last-level cache */
 #define SRS_TUNE_ALT_ORDER 13    /* 1: the single-realization step (SRS_TUNE_GATED_SWEEP) sweeps its tiles

@@ -358,9 +358,10 @@ class Context:
 
     def tune(self, **kw):
         """Sweep tunables (srs_ctx_tune): tile=, plane_pad=, compact=, group=
-        before the meshes / srs_ctx_finalize; nt_geometry=, nt_state=,
-        occupancy=, lds=, drop_finished=, gated_sweep= at any time.  None changes
-        results."""
+        before the meshes / srs_ctx_finalize; nt_state=, occupancy=,
+        drop_finished=, gated_sweep= and the rest at any time.  None changes
+        results; group=, nt_geometry=, lds=, adj_waves= and adj_w= are accepted
+        and change nothing."""
         keys = dict(tile=TUNE_TILE, nt_geometry=TUNE_NT_GEOMETRY, nt_state=TUNE_NT_STATE, plane_pad=TUNE_PLANE_PAD,
                     compact=TUNE_COMPACT, occupancy=TUNE_OCCUPANCY, group=TUNE_GROUP, lds=TUNE_LDS,
                     drop_finished=TUNE_DROP_FINISHED, gated_sweep=TUNE_GATED_SWEEP, adj_levels=TUNE_ADJ_LEVELS,

@@ -1,10 +1,9 @@
 """Autotuner for the sweep kernel's launch shape and cache hints.
 
-Candidates: elements per workgroup (tile), realizations per realization
-group (group, for batches), non-temporal loads of the read-once operator rows
-(nt_geometry), non-temporal stores of the new state (nt_state), SoA plane
-padding (plane_pad), the compact row format, the register budget and LDS
-staging.  Every candidate computes the
+Candidates: elements per workgroup (tile), non-temporal stores of the new
+state (nt_state), SoA plane padding (plane_pad), the compact row format and the
+gated step's register budget (occupancy); group, nt_geometry and lds are
+accepted by the library and change nothing.  Every candidate computes the
 same bits; only speed differs.  Each trial runs on a scratch context built
 by the caller's factory, so the context that is finally used has taken no
 steps.  Timing is the step as it runs, a captured graph of steps timed by
@@ -35,7 +34,7 @@ def autotune(make: Callable[[dict], Context], tiles=(128, 256, 512), pads=(0,), 
         try:
             for g, s, o, ld in itertools.product(nt_geometry, nt_state, occupancy, lds):
                 if ld and grp != 1:
-                    continue  # the LDS-staged sweep: groups of 1 only
+                    continue
                 ctx.tune(nt_geometry=g, nt_state=s, occupancy=o, lds=ld)
                 ctx.explicit_step(warm)
                 t0 = time.perf_counter()

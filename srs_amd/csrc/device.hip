@@ -10,9 +10,9 @@
 //             optionally, the RunSimulation loop body for the next time
 //             (while-condition, LCC trigger, voltage clamp, RyR hold,
 //             states-record output).
-// A single realization stepping without the loop body runs each step as one
-// launch instead, k_sweep_gated: its workgroup 0 runs k_gate's body for the
-// previous step before updating the channel elements.
+// A single realization runs each step as one launch instead, k_sweep_gated:
+// its workgroup 0 runs k_gate's body for the previous step beside the channel
+// elements' update.
 // The reference runs the same step as nine kernels with a state-sized rate
 // buffer (gpu/RunSimulation.cu:781-852); here the rates never leave registers.
 //
@@ -893,7 +893,7 @@ void build_class_rows(HostMesh& hm) {
 // another.
 int build_map(srs_ctx* c, HostMesh& hm, int tile, TileMap* m) {
   const int n = hm.n, np = hm.np, nt = (n + tile - 1) / tile;
-  const int run = (16 * 512 + tile - 1) / tile, n_run = (nt + run - 1) / run;
+  const int run = (4 * 512 + tile - 1) / tile, n_run = (nt + run - 1) / run;
   std::vector<uint32_t> nbr(hm.nbr.size()), blk(np / 64, 0);
   std::vector<uint16_t> loc(4 * (size_t)np, 0);
   std::vector<std::vector<uint32_t>> halos(n_run);
@@ -1748,6 +1748,7 @@ int srs_ctx_finalize(srs_ctx* c, int32_t record_capacity) {
   // state transfers: two pinned buffers of at most 8 MB (larger fields go
   // through them in parts)
   for (const HostReal& hr : c->reals) c->stage_len = std::max(c->stage_len, 6 * (size_t)c->meshes[hr.mesh]->n);
+  if (c->stage_len > (size_t)1 << 17) c->stage_len = (c->stage_len + 1) / 2;  // two parts, one copied while one moves
   c->stage_len = std::min(c->stage_len, (size_t)1 << 20);
   for (int k = 0; k < 2; ++k) {
     HIPCHK(hipHostMalloc((void**)&c->stage[k], c->stage_len * sizeof(double), hipHostMallocDefault));
