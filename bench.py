@@ -207,7 +207,7 @@ def bench_batched(n_real, steps, warmup, order, tune=None, n_tune=512):
     if tune is None:
         sample = list(range(min(n_real, n_tune)))
         tune, trials = autotune(lambda cfg: W.ensemble_context(n_real, order=order, tune=cfg, only=sample)[0],
-                                tiles=(128, 256), compact=(1,), occupancy=(0, 6), groups=(1, 2, 4))
+                                tiles=(256, 512), compact=(1,), occupancy=(0,), nt_geometry=(0,), lds=(1,))
         log(f"batched autotune: {tune}")
     ctx, dts, n_ele, nbytes = W.ensemble_context(n_real, order=order, tune=tune, log=log)
     log(f"batched: {n_real} realizations, {n_ele} elements, group {tune.get('group', 1)}")
@@ -598,8 +598,7 @@ def main():
             "group": b["tune"].get("group", 1), "tuning": b["tune"],
             "sweep_ms": b["sweep_ms"], "sweep_gbs": bach, "sweep_frac": bach / HBM_PEAK_GBS,
             "sweep_traffic": {"bytes": profiled_traffic(os.path.join(ROOT, "profiles", "k_sweep_batched_traffic.md")),
-                              "profiled_tuning": {"tile": 256, "compact": 1, "group": 1, "nt_geometry": 0,
-                                                  "nt_state": 1, "occupancy": 6, "lds": 1}},
+                              "profiled_tuning": {"tile": 512, "compact": 1, "group": 1, "nt_state": 1}},
             "plain_sequential_value": b["plain_rate"], "speedup_vs_plain_sequential": brate / b["plain_rate"],
             "plain_per_mesh": {"h40": b["plain_per_mesh"][0], "h30": b["plain_per_mesh"][1],
                                "h25": b["plain_per_mesh"][2]},

@@ -100,7 +100,7 @@ struct AdjScan {
 
 // The tiles of each chiplet's workgroups lie next to each other (the grid's
 // remainder modulo eight keeps its place): its L2 then holds most neighbours
-// (8.5 against 9.2 us per step on the 56,124-element mesh when it was measured,
+// (8.5 against 9.2 us per step on the 56,250-element mesh when it was measured,
 // the same on eight 927,816-element members).
 __device__ __forceinline__ int xcd_run(int bid, int grid) {
   const int whole = grid / NXCD * NXCD;
@@ -115,7 +115,7 @@ __device__ __forceinline__ int xcd_run(int bid, int grid) {
 // 5.5 TB/s that a launch of this mix of reads and writes reaches; the step
 // takes 229 us, and 309 with lambda itself stored, whose gather read 1/V0 as
 // well or w written by a pass of its own.  The neighbours staged in LDS with the sweep's halo lists are
-// slower (251 us, and 9.9 against 9.2 us on the 56,124-element mesh): the
+// slower (251 us, and 9.9 against 9.2 us on the 56,250-element mesh): the
 // registers that hold the gradient sums leave four wavefronts per SIMD, too
 // few to cover a barrier, and the second copy of m fits the cache.
 template <bool CLASS, bool SCAN, bool NTS>
@@ -168,33 +168,15 @@ __device__ __forceinline__ void adj_step(const RealDesc* __restrict__ D, const R
   };
   d4 w1{}, w2{}, w3{}, w4{};
   if (in) w1 = w_at(g.l1), w2 = w_at(g.l2), w3 = w_at(g.l3), w4 = w_at(g.l4);
-  // The realization's record of a channel element: those of the wavefront's 64
-  // elements follow each other in crec, so one round of loads counts the
-  // records before them and the flags below a lane give its place (a mesh
-  // shared with other clusters: a search).  A binary search and the tables it
-  // led to were ten loads in a chain: 8.5 -> 7.6 us per step of the 56,124-element
-  // mesh, with one division per SL neighbour instead of six.
+  // The realization's record of a channel element.  A binary search and the
+  // tables it led to were ten loads in a chain: 8.5 -> 7.6 us per step of the
+  // 56,250-element mesh, with one division per SL neighbour instead of six.
   int own = -1;
   ChanElem ce{};
   const uint64_t chan = __builtin_amdgcn_ballot_w64(in && (g.f & F_CHAN));
   if (chan) {
-    const int lane = threadIdx.x & 63, j0 = j - lane;
-    int before = 0;
-    for (int k = 0; k < d.n_celem; k += 64)
-      before += __builtin_popcountll(__builtin_amdgcn_ballot_w64(k + lane < d.n_celem && d.celem[min(k + lane, d.n_celem - 1)] < j0));
-    if (chan >> lane & 1) {
-      own = before + __builtin_popcountll(chan & ((1ull << lane) - 1));
-      if (own < d.n_celem) ce = d.crec[own];
-      if (own >= d.n_celem || ce.j != j) {
-        int lo = before, hi = min(own, d.n_celem);
-        while (lo < hi) {
-          const int mid = (lo + hi) >> 1;
-          if (d.celem[mid] < j) lo = mid + 1; else hi = mid;
-        }
-        own = lo < d.n_celem && d.celem[lo] == j ? lo : -1;
-        if (own >= 0) ce = d.crec[own];
-      }
-    }
+    own = chan_place(d, j, chan);
+    if (own >= 0) ce = d.crec[own];
   }
   // the scan sample's loss source (all lanes of the wavefront take part)
   const double src =
@@ -405,22 +387,6 @@ __global__ void k_batch_state(const RealDesc* __restrict__ D, const RealLive* __
     if (to_buf) B[i] = X[i];
     else X[i] = B[i];
   }
-}
-
-// Points the ping-pong buffers of each realization y of a table at slots of a
-// recomputed segment (slot i of y at seg + (i * nb + y) * 6 np): the current
-// state at slot step - s0, the next one at the slot after, so the sweep writes
-// the segment in place.
-__global__ void k_seg_ptrs(RealDesc* __restrict__ D, const RealLive* __restrict__ L, const int32_t* __restrict__ rid,
-                           double* seg, int64_t s0, int nb) {
-  const int y = blockIdx.x * blockDim.x + threadIdx.x;
-  if (y >= nb) return;
-  const int r = rid[y];
-  const int cur = L[r].cur;
-  const size_t n6 = 6 * (size_t)D[r].np;
-  const size_t i = (size_t)(L[r].step - s0);
-  D[r].X[cur] = seg + (i * nb + y) * n6;
-  D[r].X[cur ^ 1] = seg + ((i + 1) * nb + y) * n6;
 }
 
 // Starts a replayed segment at `step` for each realization of a table: the
@@ -728,7 +694,6 @@ static int loss_grad_run(srs_ctx* c, const std::vector<int32_t>& ids, int32_t sc
       lv[q] = live0[q];
       lv[q].done = 1;
     }
-    std::vector<RealDesc> dsc_sub(nb);  // the members' descriptors with their schedules, own state buffers
     for (int y = 0; y < nb; ++y) {
       const int r = ids[m0 + y];
       lv[r].done = 0;
@@ -736,8 +701,7 @@ static int loss_grad_run(srs_ctx* c, const std::vector<int32_t>& ids, int32_t sc
       lv[r].step = 0;
       lv[r].sched_base = 0;
       HostReal& hr = c->reals[r];
-      RealDesc& dsc = dsc_sub[y];
-      dsc = hr.desc;
+      RealDesc dsc = hr.desc;
       dsc.sched = d_sched + (size_t)y * max_sched;
       dsc.n_sched = n_steps;
       HIPCHK(hipMemcpy(d_sched + (size_t)y * max_sched, schedules + soff[m0 + y],
@@ -754,27 +718,27 @@ static int loss_grad_run(srs_ctx* c, const std::vector<int32_t>& ids, int32_t sc
     };
     auto ck_at = [&](int l, int64_t k) { return ckl[l] + (size_t)k * nb * n6; };
 
-    // forward, with checkpoints and scan samples; a single realization runs
-    // the steps between two of those through the gated sweep (one launch per
-    // step, the replay of each step in the next one's workgroup 0)
-    hipLaunchKernelGGL(k_seg_start, dim3(nb), dim3(256), 0, c->stream, c->d_desc, c->d_live, d_rid, (int64_t)0);
-    const bool gated = c->gated && n_real == 1 && c->group == 1;
+    // forward, with checkpoints and scan samples; the steps between two of those
+    // are one launch each: a single realization's through the gated sweep (whose
+    // workgroup 0 replays the step before), several through sweeps that read the
+    // schedules
+    const bool gated = c->gated && n_real == 1;
     int cur = lv[ids[m0]].cur;
+    auto replay_block = [&](int64_t m, int64_t n) {
+      if (gated) launch_gated_block(c, m, cur, gmode);
+      else launch_replay_block(c, m, n, d_rid, nb);
+      cur ^= (int)(m & 1);
+    };
+    hipLaunchKernelGGL(k_seg_start, dim3(nb), dim3(256), 0, c->stream, c->d_desc, c->d_live, d_rid, (int64_t)0);
     int ks = 0;
     for (int64_t n = 0; n < n_steps && e == hipSuccess;) {
       if (n % K0 == 0 && n / K0 < n_ck_kept)
         hipLaunchKernelGGL(k_batch_state, g_cp, dim3(256), 0, c->stream, c->d_desc, c->d_live, d_rid,
                            ck_at(0, n / K0), 1);
-      int64_t m = 1;
-      if (gated) {
-        int64_t next = std::min<int64_t>(n_steps, (n / K0 + 1) * K0);
-        if (ks < n_samples && sample_steps[ks] > n) next = std::min<int64_t>(next, sample_steps[ks]);
-        m = std::max<int64_t>(1, next - n);
-        launch_gated_block(c, m, cur, gmode);
-        cur ^= (int)(m & 1);
-      } else {
-        launch_step(c, gmode);
-      }
+      int64_t next = std::min<int64_t>(n_steps, (n / K0 + 1) * K0);
+      if (ks < n_samples && sample_steps[ks] > n) next = std::min<int64_t>(next, sample_steps[ks]);
+      const int64_t m = std::min<int64_t>(4096, std::max<int64_t>(1, next - n));
+      replay_block(m, n);
       n += m;
       if (ks < n_samples && sample_steps[ks] == n) scan_into(samp + (size_t)(ks++) * nb * nout);
       e = hipGetLastError();
@@ -824,25 +788,17 @@ static int loss_grad_run(srs_ctx* c, const std::vector<int32_t>& ids, int32_t sc
         hipLaunchKernelGGL(k_seg_start, dim3(nb), dim3(256), 0, c->stream, c->d_desc, c->d_live, d_rid, s0);
         hipError_t e2 = hipMemcpyAsync(seg, ckq, (size_t)nb * n6 * sizeof(double), hipMemcpyDeviceToDevice,
                                        c->stream);
-        if (gated) {
-          // a single realization: one gated-sweep launch per step, from slot
-          // n - s0 into slot n - s0 + 1, whose workgroup 0 replays the step
-          // before; k_gate replays the last one (the same live state as
-          // below, and the same fields)
-          for (int64_t n = s0; n < s1 - 1 && e2 == hipSuccess; ++n) {
-            launch_gated(c, 0, n > s0 ? gmode : 0u, false, seg + (size_t)(n - s0) * n6,
-                         seg + (size_t)(n - s0 + 1) * n6);
-            e2 = hipGetLastError();
-          }
-          if (s1 - 1 > s0 && e2 == hipSuccess) {
-            launch_gate_single(c, gmode);
-            e2 = hipGetLastError();
-          }
+        for (int64_t n = s0; n < s1 - 1 && e2 == hipSuccess; ++n) {
+          // from slot n - s0 into slot n - s0 + 1
+          const double* from = seg + (size_t)(n - s0) * nb * n6;
+          double* to = seg + (size_t)(n - s0 + 1) * nb * n6;
+          if (gated) launch_gated(c, 0, n > s0 ? gmode : 0u, false, from, to);
+          else launch_replay(c, n, 0, from, to, n6, nt_mesh);
+          e2 = hipGetLastError();
         }
-        for (int64_t n = s0; !gated && n < s1 - 1 && e2 == hipSuccess; ++n) {
-          hipLaunchKernelGGL(k_seg_ptrs, dim3((nb + 63) / 64), dim3(64), 0, c->stream, c->d_desc, c->d_live, d_rid,
-                             seg, s0, nb);
-          launch_step(c, gmode);
+        if (gated && s1 - 1 > s0 && e2 == hipSuccess) {
+          launch_gate_single(c, gmode);  // moves the live index on
+          cur ^= (int)((s1 - 1 - s0) & 1);
           e2 = hipGetLastError();
         }
         for (int64_t n = s1 - 1; n >= s0 && e2 == hipSuccess; --n) {
@@ -870,24 +826,23 @@ static int loss_grad_run(srs_ctx* c, const std::vector<int32_t>& ids, int32_t sc
             e2 = leaf_back(s0, s1, ck_at(l, q));
             continue;
           }
-          // recompute [s0, s1) in the members' own state buffers (the last
-          // level's recomputation pointed them into the segment), keeping
-          // the next level's checkpoints
-          e2 = hipStreamSynchronize(c->stream);
-          for (int y = 0; y < nb && e2 == hipSuccess; ++y)
-            e2 = hipMemcpy(c->d_desc + ids[m0 + y], &dsc_sub[y], sizeof(RealDesc), hipMemcpyHostToDevice);
-          if (e2 != hipSuccess) break;
+          // recompute [s0, s1) in the members' own state buffers, keeping the
+          // next level's checkpoints
           hipLaunchKernelGGL(k_seg_start, dim3(nb), dim3(256), 0, c->stream, c->d_desc, c->d_live, d_rid, s0);
           hipLaunchKernelGGL(k_batch_state, g_cp, dim3(256), 0, c->stream, c->d_desc, c->d_live, d_rid,
                              (double*)ck_at(l, q), 0);
           const int64_t K1 = plan.K[l + 1];
-          for (int64_t n = s0; n < s1 && e2 == hipSuccess; ++n) {
-            if ((n - s0) % K1 == 0)
-              hipLaunchKernelGGL(k_batch_state, g_cp, dim3(256), 0, c->stream, c->d_desc, c->d_live, d_rid,
-                                 ck_at(l + 1, (n - s0) / K1), 1);
-            launch_step(c, gmode);
+          int64_t queued = 0;
+          for (int64_t n = s0; n < s1 && e2 == hipSuccess; n += K1) {
+            hipLaunchKernelGGL(k_batch_state, g_cp, dim3(256), 0, c->stream, c->d_desc, c->d_live, d_rid,
+                               ck_at(l + 1, (n - s0) / K1), 1);
+            replay_block(std::min<int64_t>(K1, s1 - n), n);
             e2 = hipGetLastError();
-            if (e2 == hipSuccess && (n - s0) % 4096 == 4095) e2 = hipStreamSynchronize(c->stream);
+            queued += K1;
+            if (e2 == hipSuccess && queued >= 4096) {
+              e2 = hipStreamSynchronize(c->stream);
+              queued = 0;
+            }
           }
           if (e2 == hipSuccess) e2 = back(l + 1, s0, s1);
         }

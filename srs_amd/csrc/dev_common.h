@@ -346,6 +346,29 @@ __device__ __forceinline__ d4 row_sum(const Geo& g, const d4& m0, const d4& m1, 
   return m0 * g.a0 + m1 * g.a1 + m2 * g.a2 + m3 * g.a3 + m4 * g.a4;
 }
 
+// Index in celem of each F_CHAN lane's element (chan: those lanes, j the
+// lane's element, consecutive across a wavefront of 64 active lanes), -1 where
+// the element is another realization's.  The records of a wavefront's
+// elements follow each other, so one round of loads counts those before them
+// and the flags below a lane give its place; on a mesh shared with other
+// clusters, a search.
+__device__ __forceinline__ int chan_place(const RealDesc& d, const int j, const uint64_t chan) {
+  const int lane = threadIdx.x & 63, j0 = j - lane;
+  int before = 0;
+  for (int k = 0; k < d.n_celem; k += 64)
+    before += __builtin_popcountll(
+        __builtin_amdgcn_ballot_w64(k + lane < d.n_celem && d.celem[min(k + lane, d.n_celem - 1)] < j0));
+  if (!(chan >> lane & 1)) return -1;
+  const int own = before + __builtin_popcountll(chan & ((1ull << lane) - 1));
+  if (own < d.n_celem && d.celem[own] == j) return own;
+  int lo = before, hi = min(own, d.n_celem);
+  while (lo < hi) {
+    const int mid = (lo + hi) >> 1;
+    if (d.celem[mid] < j) lo = mid + 1; else hi = mid;
+  }
+  return lo < d.n_celem && d.celem[lo] == j ? lo : -1;
+}
+
 // The flags of the block of element j, j consecutive across the wavefront from
 // a multiple of 64.
 __device__ __forceinline__ uint32_t block_flags(const RealDesc& d, const int j) {
@@ -703,6 +726,9 @@ int launch_step(srs_ctx* c, uint32_t gmode);
 void launch_gated_block(srs_ctx* c, int64_t m, int cur, uint32_t gmode);
 // One step through the single-realization gated sweep; xo_at/xn_at (both or
 // neither) replace X[cur] -> X[cur ^ 1] as the step's state buffers.
+void launch_replay(srs_ctx* c, int64_t row, int par, const double* xo = nullptr, double* xn = nullptr,
+                   size_t stride = 0, int n_tiles = 1);
+void launch_replay_block(srs_ctx* c, int64_t m, int64_t row, const int32_t* rid, int n_rid);
 void launch_gated(srs_ctx* c, int cur, uint32_t gmode, bool proto, const double* xo_at = nullptr,
                   double* xn_at = nullptr);
 void launch_gate_single(srs_ctx* c, uint32_t gmode);

@@ -179,9 +179,10 @@ __device__ __forceinline__ void elem_store(const RealDesc& d, const Bufs bf, con
 
 // The fused step of one element of one realization, from its loaded row and
 // state, in the reference's operation order (cpu/RunSimulation.cpp:591-648).
+// ryr: the RyR states that the fluxes read.
 template <bool NTS, int FK>
 __device__ __forceinline__ void step_elem(const RealDesc& d, const RealLive& l, const Bufs bf, const int j,
-                                          const uint8_t flags, const Loc& c) {
+                                          const uint8_t flags, const Loc& c, const int32_t* ryr) {
   const uint8_t f = FK >= 0 ? (uint8_t)FK : flags;
   const bool sl = (f & F_SL) != 0;
   Rates r = elem_rates<FK>(d, l, j, f, c, sl ? gp(d.tt)[j] : 0.0, sl ? gp(d.V0)[j] : 1.0);
@@ -196,7 +197,7 @@ __device__ __forceinline__ void step_elem(const RealDesc& d, const RealLive& l, 
       for (int e = d.cstart[lo]; e < d.cstart[lo + 1]; ++e) {
         const ChanEntry en = d.centry[e];
         const int i = en.code >= 0 ? en.code >> 1 : -en.code - 1;
-        const bool open = en.code >= 0 ? d.ryr_state[i] != 0 : srs_lcc_open(d.lcc_state[i], d.lccv_state[i]);
+        const bool open = en.code >= 0 ? ryr[i] != 0 : srs_lcc_open(d.lcc_state[i], d.lccv_state[i]);
         const double dc = open && en.code >= 0 ? bf.xo[cq(en.jsr)] - bf.xo[cq(en.cyt)] : 0.0;
         chan_flux(d, l, en.code, open, dc, c.m0.x, v0, r.ca);
       }
@@ -219,8 +220,8 @@ extern __shared__ double dyn_lds[];
 // LDS (every lane's own by consecutive loads, the halo's by the tile's sorted
 // list, each element once) and each element reads its neighbours from there.
 // Bound by the memory system, not by arithmetic (with the reactions left out
-// the step takes as long): a 48-member ensemble (7.05M elements) moves 107 B
-// per element-step at 5.0 TB/s, a copy of the same shape runs at 5.5.  When each
+// the step takes as long): a 48-member ensemble (6.68M elements) moves 110 B
+// per element-step at 5.5 TB/s, a copy of the same shape runs at 5.5.  When each
 // element gathered its out-of-tile neighbours itself, a neighbour of several
 // elements was fetched for each of them, and every wavefront held four quads
 // in flight in registers: 84 VGPRs against 64, 175 us against 160 us per step of
@@ -230,7 +231,8 @@ extern __shared__ double dyn_lds[];
 // a mesh, known from its block's flags) runs the specialisation with the flags
 // known at compile time.
 template <int BS, bool NTS, bool CLASS, bool SKIP_CHAN>
-__device__ __forceinline__ void sweep_tile(const RealDesc& d, const RealLive& l, const Bufs bf, const int t) {
+__device__ __forceinline__ void sweep_tile(const RealDesc& d, const RealLive& l, const Bufs bf, const int t,
+                                           const int32_t* ryr) {
   const QuadTile tq(dyn_lds, d.qcap);
   const Halo h = load_halo<BS>(d.hal, d.hoff, t);
   const int j = t * BS + (int)threadIdx.x;
@@ -252,17 +254,36 @@ __device__ __forceinline__ void sweep_tile(const RealDesc& d, const RealLive& l,
   if (j >= d.n || (SKIP_CHAN && (g.f & F_CHAN))) return;
   c.s = row_sum(g, c.m0, tq.get(g.l1), tq.get(g.l2), tq.get(g.l3), tq.get(g.l4));
   if (b & BLK_PLAIN) {
-    step_elem<NTS, F_TROPC>(d, l, bf, j, g.f, c);
+    step_elem<NTS, F_TROPC>(d, l, bf, j, g.f, c, ryr);
   } else {
     if (!lives_tr(g.f)) c.c_tr = 0.0;
     c.c_cs = lives_cs(g.f) ? Xo[pl + np] : 0.0;
-    step_elem<NTS, -1>(d, l, bf, j, g.f, c);
+    step_elem<NTS, -1>(d, l, bf, j, g.f, c, ryr);
   }
 }
 
-template <int BS, bool NTS, bool CLASS>
+// A replayed step: the RyR states of schedule row `row`, from X[cur ^ par] (or,
+// with xo, realization y of the tile list's from xo + y stride to xn + y
+// stride, each with n_tiles tiles in turn).
+struct ReplayAt {
+  int64_t row;
+  const double* xo;
+  double* xn;
+  size_t stride;
+  int par, n_tiles;
+};
+
+// REPLAY: the step takes its RyR states from the schedule itself, so that no
+// gating launch lies between replayed steps and nothing but the fields changes
+// until k_replay_end: fitting call of three 90,540-element members, 724 steps,
+// 35.0 -> 29.0 ms (a step was sweep and gating forward, and those two and an
+// update of the state pointers when recomputed), of eight of 927,816, 39.5 ->
+// 39.1.  A single realization's replay is faster through the gated sweep (call
+// of 56,250 elements, 39.3 against 42.9 ms: its channel elements are the longest
+// chain there).
+template <int BS, bool NTS, bool CLASS, bool REPLAY>
 __global__ __launch_bounds__(BS) void k_sweep(const RealDesc* __restrict__ D, const RealLive* __restrict__ L,
-                                              const int2* __restrict__ tiles, int n_tiles, int single) {
+                                              const int2* __restrict__ tiles, int n_tiles, int single, ReplayAt at) {
   const int b = xcd_tile(blockIdx.x, gridDim.x);
   if (b >= n_tiles) return;
   const int2 tl = single ? make_int2(0, b) : tiles[b];  // {realization, tile}
@@ -271,10 +292,15 @@ __global__ __launch_bounds__(BS) void k_sweep(const RealDesc* __restrict__ D, co
   // a finished realization (done) or one in the gating-only ffwd phase keeps
   // its fields
   const int skip = l.done | l.ffwd;
-  const Bufs bf = bufs(d.X[0], d.X[1], l.cur);
+  Bufs bf = bufs(d.X[0], d.X[1], REPLAY ? l.cur ^ at.par : l.cur);
+  if (REPLAY && at.xo) {
+    const size_t y = (size_t)(b / at.n_tiles) * at.stride;
+    bf = Bufs{gp(at.xo + y), gpw(at.xn + y)};
+  }
+  const int32_t* ryr = REPLAY ? d.sched + at.row * d.n_ryr : d.ryr_state;
   scalars_here(fold(skip, bf.xo, bf.xn) ^ geo_fold<CLASS>(d));
   if (skip) return;
-  sweep_tile<BS, NTS, CLASS, false>(d, l, bf, tl.y);
+  sweep_tile<BS, NTS, CLASS, false>(d, l, bf, tl.y, ryr);
 }
 
 __device__ void write_record(const RealDesc& d, RealLive& l, const double* Ca, double t) {
@@ -712,7 +738,7 @@ __device__ __forceinline__ void sweep_gated(const RealDesc* __restrict__ D, Real
     return;
   }
   if (skip) return;
-  sweep_tile<BS, NTS, CLASS, true>(d, l, bf, b - 1);
+  sweep_tile<BS, NTS, CLASS, true>(d, l, bf, b - 1, nullptr);
 }
 // W: the register budget, at least W wavefronts per SIMD.
 template <int BS, bool NTS, bool CLASS, bool PROTO, bool PRE, int W>
@@ -728,26 +754,29 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W))) void k_
 // gated sweeps of 128-, 256- and 512-element tiles), which the build
 // compiles in parallel.
 
-using SweepFn = void (*)(const RealDesc*, const RealLive*, const int2*, int, int);
+using SweepFn = void (*)(const RealDesc*, const RealLive*, const int2*, int, int, ReplayAt);
 using GatedFn = void (*)(const RealDesc*, RealLive*, int, int, uint32_t, const double*, double*);
-SweepFn pick_sweep(const srs_ctx* c);
+SweepFn pick_sweep(const srs_ctx* c, bool replay = false);
 template <int BS>
 GatedFn pick_gated_bs(const srs_ctx* c, bool proto);
 
 #if SRS_UNIT == 1
-template <int BS, bool CMP>
-SweepFn pick_nt(int nts) { return nts ? k_sweep<BS, true, CMP> : k_sweep<BS, false, CMP>; }
+template <int BS, bool CMP, bool REPLAY>
+SweepFn pick_nt(int nts) { return nts ? k_sweep<BS, true, CMP, REPLAY> : k_sweep<BS, false, CMP, REPLAY>; }
 
-template <bool CMP>
+template <bool CMP, bool REPLAY>
 SweepFn pick_tile(const srs_ctx* c) {
   switch (c->tile) {
-    case 128: return pick_nt<128, CMP>(c->nt_state);
-    case 256: return pick_nt<256, CMP>(c->nt_state);
-    default: return pick_nt<512, CMP>(c->nt_state);
+    case 128: return pick_nt<128, CMP, REPLAY>(c->nt_state);
+    case 256: return pick_nt<256, CMP, REPLAY>(c->nt_state);
+    default: return pick_nt<512, CMP, REPLAY>(c->nt_state);
   }
 }
 
-SweepFn pick_sweep(const srs_ctx* c) { return c->class_all ? pick_tile<true>(c) : pick_tile<false>(c); }
+SweepFn pick_sweep(const srs_ctx* c, bool replay) {
+  if (replay) return c->class_all ? pick_tile<true, true>(c) : pick_tile<false, true>(c);
+  return c->class_all ? pick_tile<true, false>(c) : pick_tile<false, false>(c);
+}
 #endif  // SRS_UNIT == 1
 
 #if SRS_UNIT >= 2
@@ -781,6 +810,26 @@ template GatedFn pick_gated_bs<SRS_UNIT == 2 ? 128 : SRS_UNIT == 3 ? 256 : 512>(
 #endif  // SRS_UNIT >= 2
 
 #if SRS_UNIT == 0
+// Ends a block of m replayed steps of the listed realizations (all without a
+// list) from schedule row `row`: time, step and live index, and the RyR states
+// of the row after it, as m gating launches leave them.
+__global__ __launch_bounds__(64) void k_replay_end(const RealDesc* __restrict__ D, RealLive* __restrict__ L,
+                                                   const int32_t* __restrict__ rid, int64_t m, int64_t row) {
+  const int r = rid ? rid[blockIdx.x] : blockIdx.x;
+  const RealDesc& d = D[r];
+  RealLive& l = L[r];
+  const int64_t k = row + m < d.n_sched ? row + m : d.n_sched - 1;
+  for (int i = threadIdx.x; i < d.n_ryr; i += 64) d.ryr_state[i] = d.sched[k * d.n_ryr + i];
+  if (threadIdx.x != 0) return;
+  const double dt = d.P[SRS_R_T_STEP];
+  double t = l.t;
+  for (int64_t q = 0; q < m; ++q) t += dt;
+  l.t = t;
+  l.dt_last = dt;
+  l.step += m;
+  l.cur ^= (int)(m & 1);
+}
+
 // Gathers Ca at the channel elements of one realization.
 __global__ void k_channel_ca(const RealDesc* __restrict__ D, const RealLive* __restrict__ L, int r, double* out) {
   const RealDesc& d = D[r];
@@ -889,7 +938,7 @@ void build_class_rows(HostMesh& hm) {
 // The tile map of a mesh for `tile` elements per tile, uploaded with the
 // neighbour table and the block flags.  Halos are sorted, so that a
 // wavefront's loads of them fall in runs.  Runs of tiles are independent:
-// finalizing the 3,000,000-element dyad takes 30 ms, 101 with them one after
+// finalizing the 2,952,000-element dyad takes 30 ms, 101 with them one after
 // another.
 int build_map(srs_ctx* c, HostMesh& hm, int tile, TileMap* m) {
   const int n = hm.n, np = hm.np, nt = (n + tile - 1) / tile;
@@ -988,7 +1037,20 @@ void launch_sweep(srs_ctx* c) {
   // one realization: tile b is tile b of realization 0, no table lookups
   const int single = c->reals.size() == 1 ? 1 : 0;
   hipLaunchKernelGGL(pick_sweep(c), dim3(c->grid_sweep), dim3(c->tile), c->sweep_lds, c->stream, c->d_desc, c->d_live,
-                     c->d_tiles, c->n_tiles, single);
+                     c->d_tiles, c->n_tiles, single, ReplayAt{});
+}
+
+// One replayed step of the tile list (ReplayAt), and m of them with the live
+// state brought up to date.
+void launch_replay(srs_ctx* c, int64_t row, int par, const double* xo, double* xn, size_t stride, int n_tiles) {
+  if (c->grid_sweep == 0) return;
+  hipLaunchKernelGGL(pick_sweep(c, true), dim3(c->grid_sweep), dim3(c->tile), c->sweep_lds, c->stream, c->d_desc,
+                     c->d_live, c->d_tiles, c->n_tiles, c->reals.size() == 1 ? 1 : 0,
+                     (ReplayAt{row, xo, xn, stride, par, n_tiles}));
+}
+void launch_replay_block(srs_ctx* c, int64_t m, int64_t row, const int32_t* rid, int n_rid) {
+  for (int64_t k = 0; k < m; ++k) launch_replay(c, row + k, (int)(k & 1));
+  hipLaunchKernelGGL(k_replay_end, dim3(n_rid), dim3(64), 0, c->stream, c->d_desc, c->d_live, rid, m, row);
 }
 
 // m steps of every subset, one subset after another: the sweep over the
@@ -1000,7 +1062,7 @@ void launch_subset_block(srs_ctx* c, int64_t m, uint32_t gmode) {
     for (int64_t k = 0; k < m; ++k) {
       if (sb.nt > 0)
         hipLaunchKernelGGL(pick_sweep(c), dim3((sb.nt + NXCD - 1) / NXCD * NXCD), dim3(c->tile), c->sweep_lds, c->stream,
-                           c->d_desc, c->d_live, c->d_tiles + sb.t0, sb.nt, 0);
+                           c->d_desc, c->d_live, c->d_tiles + sb.t0, sb.nt, 0, ReplayAt{});
       hipLaunchKernelGGL(k_gate_list, dim3((unsigned)sb.nr), dim3(GATE_THREADS), 0, c->stream, c->d_desc, c->d_live,
                          (const int32_t*)c->d_sub_rids + sb.r0, gmode);
     }

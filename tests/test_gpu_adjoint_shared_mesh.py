@@ -23,5 +23,9 @@ def test_shared_mesh_gradients_equal_those_of_a_mesh_of_their_own(members):
     for k, m in enumerate(mem):
         one, s1, _, _ = _batch_ctx(pr, [m])
         l1, g1 = one.loss_grad_batch([0], s1, [m[2]], samples, tg[k:k + 1], ckpt=32)
+        for levels in (2, 3):  # recomputed in blocks from checkpoints of checkpoints
+            one.tune(adj_levels=levels)
+            l2, g2 = one.loss_grad_batch([0], s1, [m[2]], samples, tg[k:k + 1])
+            assert l2[0] == l1[0] and np.array_equal(g2, g1)
         one.close()
         assert l1[0] == loss[k] and np.array_equal(g1[0], grad[k]) and np.any(g1[0] != 0)
