@@ -1490,16 +1490,23 @@ int srs_ctx_extensions(srs_ctx* c, int32_t r, const srs_extensions* e) {
   return SRS_OK;
 }
 
+static void release_stage(srs_ctx* c) {
+  for (int k = 0; k < 2; ++k) {
+    if (c->stage[k]) (void)hipHostFree(c->stage[k]);
+    if (c->ev_stage[k]) (void)hipEventDestroy(c->ev_stage[k]);
+    c->stage[k] = nullptr;
+    c->ev_stage[k] = nullptr;
+  }
+  c->stage_len = 0;
+}
+
 int srs_ctx_destroy(srs_ctx* c) {
   if (!c) return SRS_OK;
   (void)hipSetDevice(c->device);
   (void)hipStreamSynchronize(c->stream);
   for (auto& kv : c->graphs) (void)hipGraphExecDestroy(kv.second);
   for (void* p : c->allocs) (void)hipFree(p);
-  for (int k = 0; k < 2; ++k) {
-    if (c->stage[k]) (void)hipHostFree(c->stage[k]);
-    if (c->ev_stage[k]) (void)hipEventDestroy(c->ev_stage[k]);
-  }
+  release_stage(c);
   (void)hipEventDestroy(c->ev0);
   (void)hipEventDestroy(c->ev1);
   (void)hipStreamDestroy(c->stream);
@@ -1659,6 +1666,10 @@ int srs_ctx_finalize(srs_ctx* c, int32_t record_capacity) {
   if (c->reals.empty()) return srs::fail(SRS_E_STATE, "no realizations");
   HIPCHK(hipSetDevice(c->device));
   int rc;
+  // nothing of a call that failed part way stays: it may be repeated
+  c->bands.clear();
+  c->sweep_lds = 0;
+  release_stage(c);
   // 512-element tiles share the most neighbours inside a tile (halos of 1.4
   // elements per element in the block order, 0.6 in the Morton order; 1.9 and
   // 0.8 with 256) and were the fastest
@@ -1804,7 +1815,7 @@ int srs_ctx_finalize(srs_ctx* c, int32_t record_capacity) {
   // 74.9 / 77.4; 3M-element dyad, 362 MB, 69.4 / 61.1 / 61.2; 48 members, 147 /
   // 138 / 160).  The line lies between 295 and 351 MB.  Row loads are never
   // hinted: nowhere faster than the better of the other two.
-  if (c->nt_state < 0) c->nt_state = ws > 330e6;
+  const int nt_state = c->nt_state < 0 ? ws > 330e6 : c->nt_state;
   c->n_tiles = (int)tiles.size();
   c->grid_sweep = (c->n_tiles + NXCD - 1) / NXCD * NXCD;
   // state transfers: two pinned buffers of at most 8 MB (larger fields go
@@ -1825,6 +1836,7 @@ int srs_ctx_finalize(srs_ctx* c, int32_t record_capacity) {
   if (c->reals.size() > 1 && (rc = dev_alloc(c, &c->d_sub_rids, c->reals.size()))) return rc;
   if (c->reals.size() > 1 && (rc = dev_alloc(c, &c->d_tiles_live, tiles.size()))) return rc;
   HIPCHK(hipDeviceSynchronize());
+  c->nt_state = nt_state;
   c->finalized = true;
   return SRS_OK;
 }
