@@ -118,11 +118,12 @@ __device__ __forceinline__ int xcd_run(int bid, int grid) {
 // slower (251 us, and 9.9 against 9.2 us on the 56,250-element mesh): the
 // registers that hold the gradient sums leave four wavefronts per SIMD, too
 // few to cover a barrier, and the second copy of m fits the cache.
-template <bool CLASS, bool SCAN, bool NTS>
+template <bool CLASS, bool SCAN, bool NTS, int QB>
 __device__ __forceinline__ void adj_step(const RealDesc* __restrict__ D, const RealLive* __restrict__ L,
                                          const int32_t* __restrict__ rid, const double* __restrict__ X,
                                          const double* __restrict__ lam, int64_t step, double* __restrict__ lam_out,
                                          double* __restrict__ gpart, const AdjScan& sc) {
+  constexpr Quads<QB> lay;
   __shared__ double red[ADJ_BS / 64][ADJ_NT][16];  // gradient partials per wavefront and lane modulo 16
   const int r = rid[blockIdx.y];
   const RealDesc& d = D[r];
@@ -150,8 +151,8 @@ __device__ __forceinline__ void adj_step(const RealDesc* __restrict__ D, const R
   double V0 = 1.0, u = 0.0, ttj = 0.0, inv_beta = 1.0;
   if (in) {
     g = load_geo_nbr<CLASS>(d, j);
-    m0 = ld_quad(gp(X), qidx1(j));
-    mu = ld_quad(gp(lam), qidx1(j));
+    m0 = ld_quad(gp(X), lay, j);
+    mu = ld_quad(gp(lam), lay, j);
     V0 = gp(d.V0)[j];
     u = mu.x;
     if (g.f & F_SL) {
@@ -162,8 +163,8 @@ __device__ __forceinline__ void adj_step(const RealDesc* __restrict__ D, const R
   }
   auto w_at = [&](uint32_t e) -> d4 {
     const uint32_t i = idx_of(e);
-    d4 w = ld_quad(gp(lam), qidx1(i));
-    if (e & IDX_SL) w.x *= sl_inv_beta(d.P, gp(d.tt)[i], gp(d.V0)[i], X[cq(i)]);
+    d4 w = ld_quad(gp(lam), lay, i);
+    if (e & IDX_SL) w.x *= sl_inv_beta(d.P, gp(d.tt)[i], gp(d.V0)[i], X[lay.ca(i)]);
     return w;
   };
   d4 w1{}, w2{}, w3{}, w4{};
@@ -208,7 +209,7 @@ __device__ __forceinline__ void adj_step(const RealDesc* __restrict__ D, const R
     // need its full Ca rate before the division (rca; unused elsewhere).
     double ac = 0.0;
     if (f & F_SL) {
-      auto ca_at = [&](uint32_t e) { return X[2 * (size_t)qidx1(idx_of(e))]; };
+      auto ca_at = [&](uint32_t e) { return X[lay.ca(idx_of(e))]; };
       ac = c * g.a0 + ca_at(g.l1) * g.a1 + ca_at(g.l2) * g.a2 + ca_at(g.l3) * g.a3 + ca_at(g.l4) * g.a4;
     }
     // boundary rates are D times a D-free plane: they enter the D gradients
@@ -276,8 +277,8 @@ __device__ __forceinline__ void adj_step(const RealDesc* __restrict__ D, const R
         if (ch >= 0) {
           const int p = (ch & 1) ? en.cyt : en.jsr;  // the partner element
           if (ryr[ch >> 1]) {
-            const double xj = X[cq(en.jsr)], xc = X[cq(en.cyt)];
-            double up = lam[cq(p)];
+            const double xj = X[lay.ca(en.jsr)], xc = X[lay.ca(en.cyt)];
+            double up = lam[lay.ca(p)];
             if (en.sl & ((ch & 1) ? 2 : 1))
               up *= sl_inv_beta(P, gp(d.tt)[p], gp(d.V0)[p], (ch & 1) ? xc : xj);
             const double dc = xj - xc;
@@ -308,7 +309,7 @@ __device__ __forceinline__ void adj_step(const RealDesc* __restrict__ D, const R
       gr[12] += dv0 * k * sd.dkh;
     }
     if (SCAN) ld += src;
-    st_quad<NTS>(gpw(lam_out), qidx1(j), d4{lc, la, lm, ld});
+    st_quad<NTS>(gpw(lam_out), lay, j, d4{lc, la, lm, ld});
     if (live_tr) stg<NTS>(gpw(lam_out) + 4 * np + j, lT);
     if (live_cs) stg<NTS>(gpw(lam_out) + 5 * np + j, lC);
   }
@@ -342,20 +343,24 @@ __device__ __forceinline__ void adj_step(const RealDesc* __restrict__ D, const R
 
 // At most 128 VGPRs: four wavefronts per SIMD (a budget of five spills 116 B
 // per lane: 366 against 280 us per step of eight 927,816-element members).
-template <bool CLASS, bool SCAN, bool NTS>
+template <bool CLASS, bool SCAN, bool NTS, int QB>
 __global__ __launch_bounds__(ADJ_BS) __attribute__((amdgpu_waves_per_eu(4))) void k_adj_step(
     const RealDesc* __restrict__ D, const RealLive* __restrict__ L, const int32_t* __restrict__ rid,
     const double* __restrict__ X, const double* __restrict__ lam, int64_t step, double* __restrict__ lam_out,
     double* __restrict__ gpart, AdjScan sc) {
-  adj_step<CLASS, SCAN, NTS>(D, L, rid, X, lam, step, lam_out, gpart, sc);
+  adj_step<CLASS, SCAN, NTS, QB>(D, L, rid, X, lam, step, lam_out, gpart, sc);
 }
 
 using AdjStepFn = void (*)(const RealDesc*, const RealLive*, const int32_t*, const double*, const double*, int64_t,
                            double*, double*, AdjScan);
-template <bool CLASS>
+template <bool CLASS, int QB>
 static AdjStepFn adj_step_fn(bool scan, bool nts) {
-  if (scan) return nts ? k_adj_step<CLASS, true, true> : k_adj_step<CLASS, true, false>;
-  return nts ? k_adj_step<CLASS, false, true> : k_adj_step<CLASS, false, false>;
+  if (scan) return nts ? k_adj_step<CLASS, true, true, QB> : k_adj_step<CLASS, true, false, QB>;
+  return nts ? k_adj_step<CLASS, false, true, QB> : k_adj_step<CLASS, false, false, QB>;
+}
+static AdjStepFn adj_step_fn(const srs_ctx* c, bool scan, bool nts) {
+  if (c->quad_block == 1) return c->class_all ? adj_step_fn<true, 1>(scan, nts) : adj_step_fn<false, 1>(scan, nts);
+  return c->class_all ? adj_step_fn<true, 64>(scan, nts) : adj_step_fn<false, 64>(scan, nts);
 }
 
 // The loss gradient of one scan sample in the Fluo adjoint:
@@ -371,7 +376,7 @@ __global__ __launch_bounds__(ADJ_BS) void k_scan_adj(const RealDesc* __restrict_
   const double s = scan_adj_sum(cen, g, n_f, gcoef + (size_t)blockIdx.y * gstride, np, j, j < d.n);
   if (j >= d.n) return;
   lam += blockIdx.y * 6 * np;
-  lam[2 * (size_t)qidx1(j) + FLUO_OFF] += s;
+  lam[QuadsOf{(uint32_t)d.qb}.fluo(j)] += s;
 }
 
 // Copies the current state (X[cur]) of each realization of a table to slot y
@@ -806,7 +811,7 @@ static int loss_grad_run(srs_ctx* c, const std::vector<int32_t>& ids, int32_t sc
           const bool scan = ks >= 0 && sample_steps[ks] == n;
           const AdjScan sc{S.d_cen, scan ? dg + (size_t)ks * nf : nullptr, S.geo, nf, n_samples * nf};
           if (scan) --ks;
-          const AdjStepFn kern = c->class_all ? adj_step_fn<true>(scan, nts) : adj_step_fn<false>(scan, nts);
+          const AdjStepFn kern = adj_step_fn(c, scan, nts);
           hipLaunchKernelGGL(kern, g_adj, dim3(ADJ_BS), 0, c->stream, c->d_desc, c->d_live, d_rid, Xn, lam, n, lout,
                              gpart, sc);
           std::swap(lam, lout);

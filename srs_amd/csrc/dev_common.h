@@ -41,24 +41,39 @@ enum : uint32_t {
 };
 
 // State layout of one realization (6*np doubles): the four diffusing species
-// of 64 elements form a block of two halves, 64 pairs (Ca, ATP) and then 64
-// pairs (CaM, Fluo), so that each of a wavefront's 16-byte loads and stores of
-// consecutive elements covers 1 KB without gaps and a neighbour costs two
-// such loads; then the TnC and CSQ planes, which are never gathered.  With
-// the four species side by side (32 B per element) every access covered half
-// of each cache line it touched: a plain copy in that form ran at 5.7 TB/s
-// against 6.3, and the write requests to L2 were 72 per wavefront instead of
-// 40 (48-member ensemble: 175.7 -> 171.8 us per step; with non-temporal
-// stores, which that form had made slower, 154 us).
-constexpr int QHALF = 64;              // pairs from an element's first pair to its second
-constexpr int FLUO_OFF = 2 * QHALF + 1;  // doubles from an element's Ca to its Fluo
-// Element e's first pair (pairs of 2^31 elements still count in 32 bits).
-__host__ __device__ inline uint32_t qidx1(uint32_t e) { return e + (e & ~63u); }
-__host__ __device__ inline size_t xoff(int s, size_t e, size_t np) {
+// of QB elements form a block of two halves, QB pairs (Ca, ATP) and then QB
+// pairs (CaM, Fluo); then the TnC and CSQ planes, which are never gathered.
+//  QB = 64: each of a wavefront's 16-byte loads and stores of consecutive
+//    elements covers 1 KB without gaps.  With the four species side by side
+//    every access covered half of each cache line it touched: a plain copy in
+//    that form ran at 5.7 TB/s against 6.3, and the write requests to L2 were
+//    72 per wavefront instead of 40 (48-member ensemble: 175.7 -> 171.8 us per
+//    step; with non-temporal stores, which that form had made slower, 154 us).
+//  QB = 1: an element's four species side by side (32 B), for element orders
+//    whose neighbours lie scattered.  A neighbour with no other of the tile's
+//    near it costs one cache line here and two there (quad_block_for).
+template <int QB>
+struct Quads {
+  __host__ __device__ static constexpr uint32_t half() { return QB; }  // pairs from an element's first to its second
+  // element e's first pair (pairs of 2^31 elements still count in 32 bits)
+  __host__ __device__ static uint32_t at(uint32_t e) { return e + (e & ~(uint32_t)(QB - 1)); }
+  // offsets of its Ca and its Fluo in doubles
+  __host__ __device__ static size_t ca(uint32_t e) { return 2 * (size_t)at(e); }
+  __host__ __device__ static size_t fluo(uint32_t e) { return ca(e) + 2 * QB + 1; }
+};
+// The same for a layout that is known at run time only (RealDesc::qb).
+struct QuadsOf {
+  uint32_t qb;
+  __host__ __device__ uint32_t half() const { return qb; }
+  __host__ __device__ uint32_t at(uint32_t e) const { return e + (e & ~(qb - 1)); }
+  __host__ __device__ size_t ca(uint32_t e) const { return 2 * (size_t)at(e); }
+  __host__ __device__ size_t fluo(uint32_t e) const { return ca(e) + 2 * qb + 1; }
+};
+__host__ __device__ inline size_t xoff(QuadsOf lay, int s, size_t e, size_t np) {
   if (s == srs::TRPN) return 4 * np + e;
   if (s == srs::CSQN) return 5 * np + e;
-  const size_t q = 2 * (size_t)qidx1((uint32_t)e);
-  return s == srs::CA ? q : s == srs::ATP ? q + 1 : s == srs::CMDN ? q + FLUO_OFF - 1 : q + FLUO_OFF;
+  const size_t q = lay.ca((uint32_t)e), f = lay.fluo((uint32_t)e);
+  return s == srs::CA ? q : s == srs::ATP ? q + 1 : s == srs::CMDN ? f - 1 : f;
 }
 typedef double d2 __attribute__((ext_vector_type(2)));
 typedef double d4 __attribute__((ext_vector_type(4)));
@@ -87,6 +102,7 @@ struct RealDesc {
   const uint32_t* hal;    // halo elements (IDX_SL), tile by tile
   const int32_t* hoff;    // [tiles + 1] the tiles' runs in hal
   int32_t qcap;           // quads a tile stages at most
+  int32_t qb;             // the state layout's block (Quads)
   const double* coef;     // [5][np] (plain rows)
   const uint32_t* row;    // class rows: [np][3] words, the row's class and five deltas (int16 each)
   const double* tab;      // class rows: [n_class][5] class values
@@ -139,9 +155,6 @@ __host__ __device__ inline double br_scaled(double v, double D, double D_b) {
 }
 // The D-free part Face_C b / V0 of a boundary rate (its derivative in D).
 __host__ __device__ inline double br_unit(double v, double D_b) { return D_b == 0.0 ? 0.0 : v / D_b; }
-
-// Offset of element e's Ca in a realization's state buffer; Fluo is at +FLUO_OFF.
-__device__ __forceinline__ size_t cq(int e) { return 2 * (size_t)qidx1((uint32_t)e); }
 
 // Mutable per-realization loop state.
 struct RealLive {
@@ -210,18 +223,19 @@ __device__ __forceinline__ void stg(SRS_GLOBAL T* p, T v) {
   else *p = v;
 }
 
-// The diffusing species (Ca, ATP, CaM, Fluo) at pair index q of a state or
+// The diffusing species (Ca, ATP, CaM, Fluo) of element e in a state or
 // adjoint buffer.
-__device__ __forceinline__ d4 ld_quad(const SRS_GLOBAL double* X, size_t q) {
-  const SRS_GLOBAL d2* p = (const SRS_GLOBAL d2*)X + q;
-  const d2 a = p[0], b = p[QHALF];
+template <class Lay>
+__device__ __forceinline__ d4 ld_quad(const SRS_GLOBAL double* X, const Lay lay, uint32_t e) {
+  const SRS_GLOBAL d2* p = (const SRS_GLOBAL d2*)X + lay.at(e);
+  const d2 a = p[0], b = p[lay.half()];
   return d4{a.x, a.y, b.x, b.y};
 }
-template <bool NT>
-__device__ __forceinline__ void st_quad(SRS_GLOBAL double* X, size_t q, const d4 m) {
-  SRS_GLOBAL d2* p = (SRS_GLOBAL d2*)X + q;
+template <bool NT, class Lay>
+__device__ __forceinline__ void st_quad(SRS_GLOBAL double* X, const Lay lay, uint32_t e, const d4 m) {
+  SRS_GLOBAL d2* p = (SRS_GLOBAL d2*)X + lay.at(e);
   stg<NT>(p, d2{m.x, m.y});
-  stg<NT>(p + QHALF, d2{m.z, m.w});
+  stg<NT>(p + lay.half(), d2{m.z, m.w});
 }
 typedef int i2 __attribute__((ext_vector_type(2)));
 typedef int i4 __attribute__((ext_vector_type(4)));
@@ -632,8 +646,10 @@ using namespace srs_dev;
 
 struct srs_ctx {
   int device = 0;
-  int tile = 0;          // elements per k_sweep workgroup; 0: chosen by srs_ctx_finalize
+  int tile_set = 0;      // SRS_TUNE_TILE, 0: chosen by srs_ctx_finalize
+  int tile = 0;          // elements per k_sweep workgroup
   size_t sweep_lds = 0;  // LDS bytes of a sweep workgroup (staged quads)
+  int quad_block = 64;   // the state layout's block (Quads), chosen by srs_ctx_finalize
   int nt_state = -1;     // non-temporal stores of the new state; -1: chosen by srs_ctx_finalize
   int plane_pad = 0;     // extra elements per SoA plane
   int compact = 1;       // compress operator rows when a mesh allows it

@@ -163,7 +163,7 @@ __device__ __forceinline__ void chan_flux(const RealDesc& d, const RealLive& l, 
 }
 
 // Division by the rapid buffers and forward Euler (:633-644).
-template <bool NTS, int FK>
+template <bool NTS, int QB, int FK>
 __device__ __forceinline__ void elem_store(const RealDesc& d, const Bufs bf, const int j, const uint8_t flags,
                                            const Loc& c, const Rates& r) {
   const size_t np = d.np;
@@ -171,7 +171,7 @@ __device__ __forceinline__ void elem_store(const RealDesc& d, const Bufs bf, con
   const double dt = d.P[SRS_R_T_STEP];
   SRS_GLOBAL double* __restrict__ Xn = bf.xn;
   const double rca = r.div ? r.ca / r.B : r.ca;
-  st_quad<NTS>(Xn, qidx1(j),
+  st_quad<NTS>(Xn, Quads<QB>(), j,
                d4{c.m0.x + rca * dt, c.m0.y + r.at * dt, c.m0.z + r.cm * dt, c.m0.w + r.dy * dt});
   if (lives_tr(f)) stg<NTS>(Xn + 4 * np + j, c.c_tr + r.tr * dt);
   if (lives_cs(f)) stg<NTS>(Xn + 5 * np + j, c.c_cs + r.cs * dt);
@@ -180,7 +180,7 @@ __device__ __forceinline__ void elem_store(const RealDesc& d, const Bufs bf, con
 // The fused step of one element of one realization, from its loaded row and
 // state, in the reference's operation order (cpu/RunSimulation.cpp:591-648).
 // ryr: the RyR states that the fluxes read.
-template <bool NTS, int FK>
+template <bool NTS, int QB, int FK>
 __device__ __forceinline__ void step_elem(const RealDesc& d, const RealLive& l, const Bufs bf, const int j,
                                           const uint8_t flags, const Loc& c, const int32_t* ryr) {
   const uint8_t f = FK >= 0 ? (uint8_t)FK : flags;
@@ -198,12 +198,12 @@ __device__ __forceinline__ void step_elem(const RealDesc& d, const RealLive& l, 
         const ChanEntry en = d.centry[e];
         const int i = en.code >= 0 ? en.code >> 1 : -en.code - 1;
         const bool open = en.code >= 0 ? ryr[i] != 0 : srs_lcc_open(d.lcc_state[i], d.lccv_state[i]);
-        const double dc = open && en.code >= 0 ? bf.xo[cq(en.jsr)] - bf.xo[cq(en.cyt)] : 0.0;
+        const double dc = open && en.code >= 0 ? bf.xo[Quads<QB>::ca(en.jsr)] - bf.xo[Quads<QB>::ca(en.cyt)] : 0.0;
         chan_flux(d, l, en.code, open, dc, c.m0.x, v0, r.ca);
       }
     }
   }
-  elem_store<NTS, FK>(d, bf, j, f, c, r);
+  elem_store<NTS, QB, FK>(d, bf, j, f, c, r);
 }
 
 // The sizes and mesh pointers of a tile's rows and halo, folded for scalars_here.
@@ -230,7 +230,7 @@ extern __shared__ double dyn_lds[];
 // A wavefront whose elements are all plain cytosol with troponin (the bulk of
 // a mesh, known from its block's flags) runs the specialisation with the flags
 // known at compile time.
-template <int BS, bool NTS, bool CLASS, bool SKIP_CHAN>
+template <int BS, bool NTS, bool CLASS, int QB, bool SKIP_CHAN>
 __device__ __forceinline__ void sweep_tile(const RealDesc& d, const RealLive& l, const Bufs bf, const int t,
                                            const int32_t* ryr) {
   const QuadTile tq(dyn_lds, d.qcap);
@@ -242,7 +242,7 @@ __device__ __forceinline__ void sweep_tile(const RealDesc& d, const RealLive& l,
   const Geo g = load_geo<CLASS>(d, d.loc, j, b);
   const SRS_GLOBAL double* Xo = bf.xo;
   const size_t np = d.np, pl = 4 * np + (size_t)j;
-  auto quad = [&](int e) { return ld_quad(Xo, qidx1(e)); };
+  auto quad = [&](int e) { return ld_quad(Xo, Quads<QB>(), e); };
   Loc c;
   c.m0 = quad(j);
   // the element's TnC is loaded with its quad, before its flags are known (it
@@ -254,11 +254,11 @@ __device__ __forceinline__ void sweep_tile(const RealDesc& d, const RealLive& l,
   if (j >= d.n || (SKIP_CHAN && (g.f & F_CHAN))) return;
   c.s = row_sum(g, c.m0, tq.get(g.l1), tq.get(g.l2), tq.get(g.l3), tq.get(g.l4));
   if (b & BLK_PLAIN) {
-    step_elem<NTS, F_TROPC>(d, l, bf, j, g.f, c, ryr);
+    step_elem<NTS, QB, F_TROPC>(d, l, bf, j, g.f, c, ryr);
   } else {
     if (!lives_tr(g.f)) c.c_tr = 0.0;
     c.c_cs = lives_cs(g.f) ? Xo[pl + np] : 0.0;
-    step_elem<NTS, -1>(d, l, bf, j, g.f, c, ryr);
+    step_elem<NTS, QB, -1>(d, l, bf, j, g.f, c, ryr);
   }
 }
 
@@ -281,7 +281,7 @@ struct ReplayAt {
 // 39.1.  A single realization's replay is faster through the gated sweep (call
 // of 56,250 elements, 39.3 against 42.9 ms: its channel elements are the longest
 // chain there).
-template <int BS, bool NTS, bool CLASS, bool REPLAY>
+template <int BS, bool NTS, bool CLASS, int QB, bool REPLAY>
 __global__ __launch_bounds__(BS) void k_sweep(const RealDesc* __restrict__ D, const RealLive* __restrict__ L,
                                               const int2* __restrict__ tiles, int n_tiles, int single, ReplayAt at) {
   const int b = xcd_tile(blockIdx.x, gridDim.x);
@@ -300,10 +300,11 @@ __global__ __launch_bounds__(BS) void k_sweep(const RealDesc* __restrict__ D, co
   const int32_t* ryr = REPLAY ? d.sched + at.row * d.n_ryr : d.ryr_state;
   scalars_here(fold(skip, bf.xo, bf.xn) ^ geo_fold<CLASS>(d));
   if (skip) return;
-  sweep_tile<BS, NTS, CLASS, false>(d, l, bf, tl.y, ryr);
+  sweep_tile<BS, NTS, CLASS, QB, false>(d, l, bf, tl.y, ryr);
 }
 
-__device__ void write_record(const RealDesc& d, RealLive& l, const double* Ca, double t) {
+template <class Lay>
+__device__ void write_record(const RealDesc& d, RealLive& l, const double* Ca, const Lay lay, double t) {
   // Called by one thread: sums run sequentially, in the reference's order.
   if (l.rec_count >= d.rec_cap) { l.rec_overflow = 1; return; }
   float* rec = d.rec + (size_t)l.rec_count * d.rec_len;
@@ -311,7 +312,7 @@ __device__ void write_record(const RealDesc& d, RealLive& l, const double* Ca, d
   rec[k++] = (float)t;
   double i_ryr = 0;
   for (int i = 0; i < d.n_ryr; ++i)
-    i_ryr += d.ryr_state[i] * d.P[SRS_R_V_RYR] * (Ca[cq(d.ryr_jsr[i])] - Ca[cq(d.ryr_ele[i])]) * (d.P[SRS_R_V_CELL]) * 96485 *
+    i_ryr += d.ryr_state[i] * d.P[SRS_R_V_RYR] * (Ca[lay.ca(d.ryr_jsr[i])] - Ca[lay.ca(d.ryr_ele[i])]) * (d.P[SRS_R_V_CELL]) * 96485 *
              2 * (1e-6);
   rec[k++] = (float)i_ryr;
   int n_open = 0;
@@ -324,18 +325,18 @@ __device__ void write_record(const RealDesc& d, RealLive& l, const double* Ca, d
   double i_lcc = 0;
   for (int i = 0; i < d.n_lcc; ++i)
     if (srs_lcc_open(d.lcc_state[i], d.lccv_state[i]))
-      i_lcc += srs_lcc_flux_raw(l.vm, Ca[cq(d.lcc_ele[i])], d.P[SRS_R_CA_0]) * 96485 * 2 * (1e-6);
+      i_lcc += srs_lcc_flux_raw(l.vm, Ca[lay.ca(d.lcc_ele[i])], d.P[SRS_R_CA_0]) * 96485 * 2 * (1e-6);
   rec[k++] = (float)i_lcc;
   double m = 0;
-  for (int i = 0; i < d.n_ryr; ++i) m += Ca[cq(d.ryr_jsr[i])];
+  for (int i = 0; i < d.n_ryr; ++i) m += Ca[lay.ca(d.ryr_jsr[i])];
   m /= d.n_ryr;
   rec[k++] = (float)m;
   m = 0;
-  for (int i = 0; i < d.n_ryr; ++i) m += Ca[cq(d.ryr_ele[i])];
+  for (int i = 0; i < d.n_ryr; ++i) m += Ca[lay.ca(d.ryr_ele[i])];
   m /= d.n_ryr;
   rec[k++] = (float)m;
   if (d.gpu_layout)
-    for (int i = 0; i < d.n_ryr; ++i) rec[k++] = (float)Ca[cq(d.ryr_ele[i])];
+    for (int i = 0; i < d.n_ryr; ++i) rec[k++] = (float)Ca[lay.ca(d.ryr_ele[i])];
   if (d.ryr_out)
     for (int i = 0; i < d.n_ryr; ++i) rec[k++] = (float)d.ryr_state[i];
   l.rec_count++;
@@ -357,9 +358,9 @@ __device__ __forceinline__ void held_lccs(const RealDesc& d, int* smem) {
 // after the first barrier: work of other wavefronts than the first and the
 // last, which mostly gate no channel, done while those two are at theirs.
 struct NoMid { __device__ void operator()() const {} };
-template <int NT, bool PROTO = true, class Mid = NoMid>
+template <int NT, bool PROTO = true, class Lay, class Mid = NoMid>
 __device__ __forceinline__ void gate_workgroup(const RealDesc* __restrict__ D, RealLive* __restrict__ L, const int r,
-                                               const uint32_t mode, int* smem, Mid mid = NoMid()) {
+                                               const uint32_t mode, int* smem, const Lay lay, Mid mid = NoMid()) {
   static_assert(MAX_RYR % NT == 0 && MAX_LCC % NT == 0, "channel slots per thread");
   const RealDesc& d = D[r];
   RealLive& l = L[r];
@@ -373,7 +374,7 @@ __device__ __forceinline__ void gate_workgroup(const RealDesc* __restrict__ D, R
   const bool ff = l.ffwd != 0;
   const bool swept = (mode & G_AFTER_SWEEP) && !ff;
   const double* Xn = swept ? d.X[cur ^ 1] : d.X[cur];
-  const double* Ca = Xn;  // Ca of element e at Ca[cq(e)] (interleaved diffusing species)
+  const double* Ca = Xn;  // Ca of element e at Ca[lay.ca(e)]
   const double* P = d.P;
   const double dt = P[SRS_R_T_STEP];
   const int64_t step = l.step;
@@ -395,8 +396,8 @@ __device__ __forceinline__ void gate_workgroup(const RealDesc* __restrict__ D, R
     // this is folded into half of its registers.
     double ca_c = 0.0, ca_j = 0.0, Rr = 0.0;
     auto load_ryr = [&](const int i) {
-      ca_c = Ca[cq(d.ryr_ele[i])];
-      ca_j = Ca[cq(d.ryr_jsr[i])];
+      ca_c = Ca[lay.ca(d.ryr_ele[i])];
+      ca_j = Ca[lay.ca(d.ryr_jsr[i])];
       Rr = d.R[i];
     };
     for (int i = tid; i < nr; i += NT) s_old[i] = s_a[i] = d.ryr_state[i];
@@ -406,7 +407,7 @@ __device__ __forceinline__ void gate_workgroup(const RealDesc* __restrict__ D, R
     auto load_lcc = [&](const int i) {
       ls = d.lcc_state[i];
       lvs = d.lccv_state[i];
-      ca_l = Ca[cq(d.lcc_ele[i])];
+      ca_l = Ca[lay.ca(d.lcc_ele[i])];
       Rl = d.R[nr + i];
     };
     const int l0 = NT - 1 - tid;
@@ -534,7 +535,7 @@ __device__ __forceinline__ void gate_workgroup(const RealDesc* __restrict__ D, R
       const bool open = i < nr && d.ryr_state[i] != 0;
       cr += __builtin_popcountll(__builtin_amdgcn_ballot_w64(open));
       if (i < nr) {
-        const double c = Ca[cq(d.ryr_ele[i])];
+        const double c = Ca[lay.ca(d.ryr_ele[i])];
         if (c > m) m = c;
       }
     }
@@ -572,7 +573,7 @@ __device__ __forceinline__ void gate_workgroup(const RealDesc* __restrict__ D, R
   if (ff) {  // the rest of the ffwd loop body, cpu/RunSimulation.cpp:480-518
     const int n_open = n_open_all, n_open_lcc = n_lcc_all;
     const bool stop = n_open > 0 || n_open_lcc > 0 || t > P[SRS_R_T_FINAL];
-    if (!stop && out_due) write_record(d, l, Ca, t);
+    if (!stop && out_due) write_record(d, l, Ca, lay, t);
     if (d.I[SRS_I_FLAG_V_CLAMP]) l.vm = (t <= P[SRS_R_T_CLAMP]) ? P[SRS_R_V_CLAMP] : P[SRS_R_DEFAULT_VM];
     if (!stop) return;
     // The main loop starts at this t with N_RyR_Open from the last ffwd
@@ -588,7 +589,7 @@ __device__ __forceinline__ void gate_workgroup(const RealDesc* __restrict__ D, R
                               l.n_open_last < d.I[SRS_I_N_RYR_FIDELITY]));
   if (!cont) {
     l.done = 1;
-    write_record(d, l, Ca, t);  // final states output, :584
+    write_record(d, l, Ca, lay, t);  // final states output, :584
     return;
   }
   if (d.I[SRS_I_FLAG_LCC] && l.lcc_open && t >= l.t_lcc_close) {  // :525-528
@@ -605,7 +606,7 @@ __device__ __forceinline__ void gate_workgroup(const RealDesc* __restrict__ D, R
   if (out_due) {  // :552-566
     l.n_open_last = n_open_all;
     l.ca_max_last = cmax_all;
-    write_record(d, l, Ca, t);
+    write_record(d, l, Ca, lay, t);
   }
 }
 
@@ -613,13 +614,14 @@ __device__ __forceinline__ void gate_workgroup(const RealDesc* __restrict__ D, R
 __global__ __launch_bounds__(GATE_THREADS) void k_gate(const RealDesc* __restrict__ D, RealLive* __restrict__ L,
                                                        uint32_t mode) {
   __shared__ int smem[GATE_LDS / sizeof(int)];
-  gate_workgroup<GATE_THREADS>(D, L, blockIdx.x, mode, smem);
+  gate_workgroup<GATE_THREADS>(D, L, blockIdx.x, mode, smem, QuadsOf{(uint32_t)D[blockIdx.x].qb});
 }
 // The gating of the realizations of a list (one subset of the context).
 __global__ __launch_bounds__(GATE_THREADS) void k_gate_list(const RealDesc* __restrict__ D, RealLive* __restrict__ L,
                                                             const int32_t* __restrict__ rids, uint32_t mode) {
   __shared__ int smem[GATE_LDS / sizeof(int)];
-  gate_workgroup<GATE_THREADS>(D, L, rids[blockIdx.x], mode, smem);
+  const int r = rids[blockIdx.x];
+  gate_workgroup<GATE_THREADS>(D, L, r, mode, smem, QuadsOf{(uint32_t)D[r].qb});
 }
 #endif
 
@@ -641,10 +643,11 @@ __global__ __launch_bounds__(GATE_THREADS) void k_gate_list(const RealDesc* __re
 // reverse order when the index is 1 (alternate steps), so that a step first
 // reads the tiles the step before wrote last, while they may still be in the
 // last-level cache.  The order changes no result.
-template <int BS, bool NTS, bool CLASS, bool PROTO, bool PRE>
+template <int BS, bool NTS, bool CLASS, int QB, bool PROTO, bool PRE>
 __device__ __forceinline__ void sweep_gated(const RealDesc* __restrict__ D, RealLive* __restrict__ L, int n_tiles,
                                             int curx, uint32_t gmode, const double* xo_at, double* xn_at) {
   const int cur = curx & 1;
+  constexpr Quads<QB> lay;
   int b = xcd_tile(blockIdx.x, gridDim.x);
   if (b > n_tiles) return;  // b = 0: the gating workgroup; b = 1..n_tiles: tile b - 1
   if (b > 0 && curx == 3) b = n_tiles + 1 - b;
@@ -683,13 +686,13 @@ __device__ __forceinline__ void sweep_gated(const RealDesc* __restrict__ D, Real
       w.tt = r->tt;
       w.code = r->first.code;
       for (int q = 0; q < 5; ++q) w.a[q] = r->a[q];
-      w.m0 = ld_quad(Xo, qidx1(w.j));
-      w.m1 = ld_quad(Xo, qidx1(r->nb[0])), w.m2 = ld_quad(Xo, qidx1(r->nb[1]));
-      w.m3 = ld_quad(Xo, qidx1(r->nb[2])), w.m4 = ld_quad(Xo, qidx1(r->nb[3]));
+      w.m0 = ld_quad(Xo, lay, w.j);
+      w.m1 = ld_quad(Xo, lay, r->nb[0]), w.m2 = ld_quad(Xo, lay, r->nb[1]);
+      w.m3 = ld_quad(Xo, lay, r->nb[2]), w.m4 = ld_quad(Xo, lay, r->nb[3]);
       w.tr = lives_tr(w.f) ? Xo[4 * np + w.j] : 0.0;
       w.cs = lives_cs(w.f) ? Xo[5 * np + w.j] : 0.0;
       w.xj = w.xc = 0.0;
-      if (w.code >= 0) w.xj = Xo[cq(r->first.jsr)], w.xc = Xo[cq(r->first.cyt)];
+      if (w.code >= 0) w.xj = Xo[lay.ca(r->first.jsr)], w.xc = Xo[lay.ca(r->first.cyt)];
       return w;
     };
     auto half = [&](const Raw& w) -> Pending {
@@ -700,7 +703,7 @@ __device__ __forceinline__ void sweep_gated(const RealDesc* __restrict__ D, Real
       c.c_cs = w.cs;
       c.s = w.m0 * w.a[0] + w.m1 * w.a[1] + w.m2 * w.a[2] + w.m3 * w.a[3] + w.m4 * w.a[4];
       const Rates q = elem_rates<-1>(d, l, w.j, w.f, c, w.tt, w.v0);
-      elem_store<NTS, -1>(d, bf, w.j, w.f, c, q);  // Ca without its fluxes: replaced by finish
+      elem_store<NTS, QB, -1>(d, bf, w.j, w.f, c, q);  // Ca without its fluxes: replaced by finish
       p.rca = q.ca;
       p.B = q.B;  // 1 where nothing divides
       return p;
@@ -712,11 +715,11 @@ __device__ __forceinline__ void sweep_gated(const RealDesc* __restrict__ D, Real
       for (int i = p.e0 + 1; i < p.e1; ++i) {
         const ChanEntry en = d.centry[i];
         const bool open = is_open(en.code);
-        const double dc = open && en.code >= 0 ? bf.xo[cq(en.jsr)] - bf.xo[cq(en.cyt)] : 0.0;
+        const double dc = open && en.code >= 0 ? bf.xo[lay.ca(en.jsr)] - bf.xo[lay.ca(en.cyt)] : 0.0;
         chan_flux(d, l, en.code, open, dc, p.ca, p.v0, rca);
       }
       rca /= p.B;
-      bf.xn[cq(p.j)] = p.ca + rca * d.P[SRS_R_T_STEP];
+      bf.xn[lay.ca(p.j)] = p.ca + rca * d.P[SRS_R_T_STEP];
     };
     const int k0 = ((int)threadIdx.x + BS - FIRST) % BS;
     const bool pre = PRE && !skip && k0 < d.n_celem;
@@ -725,7 +728,7 @@ __device__ __forceinline__ void sweep_gated(const RealDesc* __restrict__ D, Real
       if (pre) p0 = half(load(k0));
     };
     if (gmode) {
-      gate_workgroup<BS, PROTO>(D, L, 0, gmode, smem, mid);
+      gate_workgroup<BS, PROTO>(D, L, 0, gmode, smem, lay, mid);
     } else {
       for (int i = threadIdx.x; i < d.n_ryr; i += BS) smem[GATE_RYR + i] = d.ryr_state[i];
       held_lccs<BS>(d, smem);
@@ -738,14 +741,14 @@ __device__ __forceinline__ void sweep_gated(const RealDesc* __restrict__ D, Real
     return;
   }
   if (skip) return;
-  sweep_tile<BS, NTS, CLASS, true>(d, l, bf, b - 1, nullptr);
+  sweep_tile<BS, NTS, CLASS, QB, true>(d, l, bf, b - 1, nullptr);
 }
 // W: the register budget, at least W wavefronts per SIMD.
-template <int BS, bool NTS, bool CLASS, bool PROTO, bool PRE, int W>
+template <int BS, bool NTS, bool CLASS, int QB, bool PROTO, bool PRE, int W>
 __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(W))) void k_sweep_gated(
     const RealDesc* __restrict__ D, RealLive* __restrict__ L, int n_tiles, int cur, uint32_t gmode,
     const double* xo_at, double* xn_at) {
-  sweep_gated<BS, NTS, CLASS, PROTO, PRE>(D, L, n_tiles, cur, gmode, xo_at, xn_at);
+  sweep_gated<BS, NTS, CLASS, QB, PROTO, PRE>(D, L, n_tiles, cur, gmode, xo_at, xn_at);
 }
 
 // ------------------------------------------------------------ kernel choice
@@ -762,14 +765,17 @@ GatedFn pick_gated_bs(const srs_ctx* c, bool proto);
 
 #if SRS_UNIT == 1
 template <int BS, bool CMP, bool REPLAY>
-SweepFn pick_nt(int nts) { return nts ? k_sweep<BS, true, CMP, REPLAY> : k_sweep<BS, false, CMP, REPLAY>; }
+SweepFn pick_nt(const srs_ctx* c) {
+  if (c->quad_block == 1) return c->nt_state ? k_sweep<BS, true, CMP, 1, REPLAY> : k_sweep<BS, false, CMP, 1, REPLAY>;
+  return c->nt_state ? k_sweep<BS, true, CMP, 64, REPLAY> : k_sweep<BS, false, CMP, 64, REPLAY>;
+}
 
 template <bool CMP, bool REPLAY>
 SweepFn pick_tile(const srs_ctx* c) {
   switch (c->tile) {
-    case 128: return pick_nt<128, CMP, REPLAY>(c->nt_state);
-    case 256: return pick_nt<256, CMP, REPLAY>(c->nt_state);
-    default: return pick_nt<512, CMP, REPLAY>(c->nt_state);
+    case 128: return pick_nt<128, CMP, REPLAY>(c);
+    case 256: return pick_nt<256, CMP, REPLAY>(c);
+    default: return pick_nt<512, CMP, REPLAY>(c);
   }
 }
 
@@ -781,8 +787,10 @@ SweepFn pick_sweep(const srs_ctx* c, bool replay) {
 
 #if SRS_UNIT >= 2
 template <int BS, bool CMP, bool PROTO, bool PRE, int W>
-GatedFn pick_gated_nt(int nts) {
-  return nts ? k_sweep_gated<BS, true, CMP, PROTO, PRE, W> : k_sweep_gated<BS, false, CMP, PROTO, PRE, W>;
+GatedFn pick_gated_nt(const srs_ctx* c) {
+  if (c->quad_block == 1)
+    return c->nt_state ? k_sweep_gated<BS, true, CMP, 1, PROTO, PRE, W> : k_sweep_gated<BS, false, CMP, 1, PROTO, PRE, W>;
+  return c->nt_state ? k_sweep_gated<BS, true, CMP, 64, PROTO, PRE, W> : k_sweep_gated<BS, false, CMP, 64, PROTO, PRE, W>;
 }
 
 // How much the registers of the gating workgroup may cost the tiles.  With no
@@ -795,9 +803,9 @@ GatedFn pick_gated_nt(int nts) {
 // (928k: 21.3 against 21.9 us; 1.6M: 29.4 / 31.1; 3M: 61.5 / 70.7).
 template <int BS, bool CMP, bool PROTO>
 GatedFn pick_gated_w(const srs_ctx* c) {
-  if (c->occ || (int64_t)c->n_tiles * BS >= 900000) return pick_gated_nt<BS, CMP, PROTO, false, 6>(c->nt_state);
-  return c->n_tiles <= 256 ? pick_gated_nt<BS, CMP, PROTO, true, 2>(c->nt_state)
-                           : pick_gated_nt<BS, CMP, PROTO, true, 4>(c->nt_state);
+  if (c->occ || (int64_t)c->n_tiles * BS >= 900000) return pick_gated_nt<BS, CMP, PROTO, false, 6>(c);
+  return c->n_tiles <= 256 ? pick_gated_nt<BS, CMP, PROTO, true, 2>(c)
+                           : pick_gated_nt<BS, CMP, PROTO, true, 4>(c);
 }
 
 template <int BS>
@@ -833,12 +841,13 @@ __global__ __launch_bounds__(64) void k_replay_end(const RealDesc* __restrict__ 
 // Gathers Ca at the channel elements of one realization.
 __global__ void k_channel_ca(const RealDesc* __restrict__ D, const RealLive* __restrict__ L, int r, double* out) {
   const RealDesc& d = D[r];
-  const double* Ca = d.X[L[r].cur];  // Ca of element e at Ca[cq(e)]
+  const double* Ca = d.X[L[r].cur];  // Ca of element e at Ca[lay.ca(e)]
+  const QuadsOf lay{(uint32_t)d.qb};
   for (int i = threadIdx.x; i < d.n_ryr; i += blockDim.x) {
-    out[i] = Ca[cq(d.ryr_ele[i])];
-    out[d.n_ryr + i] = Ca[cq(d.ryr_jsr[i])];
+    out[i] = Ca[lay.ca(d.ryr_ele[i])];
+    out[d.n_ryr + i] = Ca[lay.ca(d.ryr_jsr[i])];
   }
-  for (int i = threadIdx.x; i < d.n_lcc; i += blockDim.x) out[2 * d.n_ryr + i] = Ca[cq(d.lcc_ele[i])];
+  for (int i = threadIdx.x; i < d.n_lcc; i += blockDim.x) out[2 * d.n_ryr + i] = Ca[lay.ca(d.lcc_ele[i])];
 }
 
 
@@ -846,8 +855,8 @@ __global__ void k_channel_ca(const RealDesc* __restrict__ D, const RealLive* __r
 // buffers and a staging buffer in the caller's layout, [6][n] in the reference
 // numbering (inv: reference -> device position).  to_dev writes both
 // ping-pong buffers; otherwise the live one is read.  Bound by the host link:
-// the kernel's scattered side is 32 B quads (each read for four of the six
-// species, the repeats from L2), the staging side is contiguous.
+// the kernel's scattered side is the elements' pairs (each read for two of the
+// six species, the repeats from L2), the staging side is contiguous.
 __global__ __launch_bounds__(256) void k_state_xfer(const RealDesc* __restrict__ D, const RealLive* __restrict__ L,
                                                     int r, const int32_t* __restrict__ inv, double* __restrict__ stage,
                                                     size_t t0, size_t cnt, int to_dev) {
@@ -856,7 +865,7 @@ __global__ __launch_bounds__(256) void k_state_xfer(const RealDesc* __restrict__
   const RealDesc& d = D[r];
   const size_t t = t0 + i, n = d.n;
   const int s = (int)(t / n);
-  const size_t x = xoff(s, inv[t - s * n], d.np);
+  const size_t x = xoff(QuadsOf{(uint32_t)d.qb}, s, inv[t - s * n], d.np);
   if (to_dev) {
     const double v = stage[i];
     d.X[0][x] = v;
@@ -933,6 +942,48 @@ void build_class_rows(HostMesh& hm) {
     for (int q = 0; q < 5; ++q) hm.tab[5 * (size_t)kv.second + q] = kv.first[q];
   hm.row.swap(row);
   hm.class_rows = true;
+}
+
+// The cache lines per element that the halos of 512-element tiles cost more
+// with blocks of 64 (two lines for up to eight neighbours that follow each
+// other, one in each half) than with an element's species side by side (one
+// line for up to four), from at most eight tiles spread over the mesh.
+double scattered_lines(const HostMesh& hm) {
+  constexpr int T = 512;
+  const int nt = (hm.n + T - 1) / T, take = std::min(nt, 8);
+  std::vector<int32_t> e;
+  int64_t lines = 0, elements = 0;
+  for (int q = 0; q < take; ++q) {
+    const int t = (int)((int64_t)q * nt / take), j0 = t * T, j1 = std::min(hm.n, j0 + T);
+    e.clear();
+    for (size_t k = 4 * (size_t)j0; k < 4 * (size_t)j1; ++k)
+      if (hm.nbr[k] < j0 || hm.nbr[k] >= j1) e.push_back(hm.nbr[k] >> 2);
+    std::sort(e.begin(), e.end());
+    for (size_t k = 0; k < e.size(); ++k) {
+      if (k == 0 || e[k] >> 1 != e[k - 1] >> 1) lines += 2;
+      if (k == 0 || e[k] != e[k - 1]) lines -= 1;
+    }
+    elements += j1 - j0;
+  }
+  return (double)lines / elements;
+}
+
+// The state layout's block: 64, or 1 where the halos of an average element
+// cost 0.6 cache lines less with it.  us per step, blocks of 64 / 1 (lines):
+// 927,816 elements in Morton order 20.0 / 20.3 (0.17), with 5% of the elements
+// anywhere 25.4 / 22.9 (0.41), with 10% 31.9 / 26.4 (0.65), shuffled within
+// 2,048 27.1 / 28.5 (0.46), within 131,072 58.5 / 53.4 (3.6), all of them 116 /
+// 75 (3.9); 2,952,000 with 5% 77.6 / 78.8, 10% 96.9 / 87.9, all 436 / 290;
+// 172,494 shuffled within 2,048 8.8 / 8.7, all 17.6 / 15.3.
+int quad_block_for(const srs_ctx* c) {
+  std::vector<double> lines;
+  for (const auto& hmp : c->meshes) lines.push_back(scattered_lines(*hmp));
+  double sum = 0.0, n = 0.0;
+  for (const HostReal& hr : c->reals) {
+    sum += lines[hr.mesh] * c->meshes[hr.mesh]->n;
+    n += c->meshes[hr.mesh]->n;
+  }
+  return sum > 0.6 * n ? 1 : 64;
 }
 
 // The tile map of a mesh for `tile` elements per tile, uploaded with the
@@ -1408,7 +1459,7 @@ int srs_ctx_tune(srs_ctx* c, int32_t key, int32_t value) {
     case SRS_TUNE_TILE:
       if (value != 128 && value != 256 && value != 512) return srs::fail(SRS_E_ARG, "tile must be 128, 256 or 512");
       if (c->finalized) return srs::fail(SRS_E_STATE, "tile must be set before srs_ctx_finalize");
-      c->tile = value;
+      c->tile_set = value;
       return SRS_OK;
     case SRS_TUNE_PLANE_PAD:
       if (value < 0 || value % 64 || value > 1 << 20) return srs::fail(SRS_E_ARG, "plane pad must be a multiple of 64");
@@ -1675,7 +1726,12 @@ int srs_ctx_finalize(srs_ctx* c, int32_t record_capacity) {
   // 0.8 with 256) and were the fastest
   // at every size: 927,816 elements 21.5 against 23.3 us per step, 56,250
   // 9.2 against 9.3, the 48-member ensemble 147 against 171
-  if (c->tile == 0) c->tile = 512;
+  // Scattered orders have no neighbours to share: there 128 is the fastest (a
+  // 512-element tile's halo then takes half of a CU's LDS; us per step with 128
+  // / 512 elements shuffled: 2,952,000 250 / 290, sixteen members of 172,494 131
+  // / 144, 172,494 13.7 / 15.3).
+  c->quad_block = quad_block_for(c);
+  c->tile = c->tile_set ? c->tile_set : c->quad_block == 1 ? 128 : 512;
   c->class_all = !c->meshes.empty();
   for (auto& hmp : c->meshes) c->class_all &= hmp->class_rows;
   for (auto& hmp : c->meshes) {
@@ -1708,8 +1764,10 @@ int srs_ctx_finalize(srs_ctx* c, int32_t record_capacity) {
   // 16 members, 237 MB, 45.2 / 43.4; two 928k-element dyads, 200 MB, 40.4 /
   // 38.5).  Beyond it four state streams at a time cost more than the rows (18
   // members, 266 MB, 52.7 / 56.6; 48, 137 / 142; twelve 214k-element dyads, 241
-  // MB, 53.7 / 48.5 in one run and 57.4 in another).
-  const int width = ws > 220e6 ? 1 : 4;
+  // MB, 53.7 / 48.5 in one run and 57.4 in another).  Nor with scattered orders,
+  // whose halos fill the L2 (four members of 56,250 elements 19.0 / 21.6, of
+  // 172,494, recording, 45 / 58).
+  const int width = ws > 220e6 || c->quad_block == 1 ? 1 : 4;
   for (size_t m = 0; m < c->meshes.size(); ++m) {
     for (size_t r = 0, fill = width; r < c->reals.size(); ++r) {
       if (c->reals[r].mesh != (int)m) continue;
@@ -1736,6 +1794,7 @@ int srs_ctx_finalize(srs_ctx* c, int32_t record_capacity) {
     d.br_mesh = hm.d_br;
     std::copy(hm.br_d, hm.br_d + 4, d.brd);
     d.loc = hm.map.d_loc; d.hal = hm.map.d_hal; d.hoff = hm.map.d_hoff; d.qcap = hm.map.qcap;
+    d.qb = c->quad_block;
     d.row = hm.d_row; d.tab = hm.d_tab; d.blk = hm.d_blk;
     d.n_class = hm.n_class;
     d.n = hm.n; d.np = hm.np;

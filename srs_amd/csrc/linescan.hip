@@ -68,6 +68,7 @@ __global__ __launch_bounds__(SCAN_BS) __attribute__((amdgpu_waves_per_eu(4))) vo
   part += (size_t)blockIdx.y * gridDim.x * n_f;
   const RealDesc& d = D[r];
   const double* X = d.X[L[r].cur];
+  const QuadsOf lay{(uint32_t)d.qb};
   const int n = d.n, np = d.np;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   double* rw = red + wave * n_f;
@@ -81,7 +82,7 @@ __global__ __launch_bounds__(SCAN_BS) __attribute__((amdgpu_waves_per_eu(4))) vo
   for (int q = 0; q < NC; ++q) {
     const int j = min((int)(blockIdx.x * NC + q) * SCAN_BS + (int)threadIdx.x, n - 1);
     cx[q] = gp(cen)[j], cy[q] = gp(cen)[np + j], cz[q] = gp(cen)[2 * np + j];
-    vf[q] = gp(d.V0)[j] * gp(X)[cq(j) + FLUO_OFF];  // V0 * Ca-bound Fluo
+    vf[q] = gp(d.V0)[j] * gp(X)[lay.fluo(j)];  // V0 * Ca-bound Fluo
   }
   ScanCell sc[NC];
   int clo[NC], chi[NC];
@@ -131,6 +132,7 @@ __global__ __launch_bounds__(SCAN_BS) void k_scan_final(const RealDesc* __restri
   part += (size_t)blockIdx.y * n_blocks * n_f;
   out += (size_t)blockIdx.y * out_stride;
   const double* X = D[r].X[L[r].cur];
+  const QuadsOf lay{(uint32_t)D[r].qb};
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int i = blockIdx.x * (SCAN_BS / 64) + wave;
   if (i < n_f) {
@@ -143,11 +145,11 @@ __global__ __launch_bounds__(SCAN_BS) void k_scan_final(const RealDesc* __restri
   const int t = blockIdx.x * SCAN_BS + threadIdx.x, nt = gridDim.x * SCAN_BS;
   for (int k = t; k < n_f; k += nt) {
     const int e = near_f[k];
-    out[n_ca + k] = e >= 0 ? X[cq(e) + FLUO_OFF] : f0;
+    out[n_ca + k] = e >= 0 ? X[lay.fluo(e)] : f0;
   }
   for (int k = t; k < n_ca; k += nt) {
     const int e = near_ca[k];
-    out[k] = e >= 0 ? X[cq(e)] : c0;
+    out[k] = e >= 0 ? X[lay.ca(e)] : c0;
   }
 }
 
