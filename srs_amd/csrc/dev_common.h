@@ -261,7 +261,7 @@ __device__ __forceinline__ T sld(const T* p) { return *(const __attribute__((add
 // An element index with bit 31 set where the element has F_SL, as the halo
 // lists and the neighbour table hold them.
 constexpr uint32_t IDX_SL = 0x80000000u;
-__device__ __forceinline__ uint32_t idx_of(uint32_t e) { return e & ~IDX_SL; }
+__host__ __device__ __forceinline__ uint32_t idx_of(uint32_t e) { return e & ~IDX_SL; }
 
 // A tile's run of the halo list, and the entries of a thread: the first HPRE
 // of them are loaded ahead of everything that does not depend on them.
@@ -593,7 +593,7 @@ struct HostMesh {
   int32_t n = 0, np = 0;
   std::vector<int32_t> perm;  // dev -> ref
   std::vector<int32_t> inv;   // ref -> dev
-  std::vector<int32_t> nbr;   // [np][4] dev numbering
+  std::vector<uint32_t> nbr;  // [np][4] dev numbering (IDX_SL)
   std::vector<double> coef;   // [5][np]
   std::vector<uint8_t> flags;
   std::vector<double> V0, tt, br;  // br [4][np] or empty
@@ -691,7 +691,7 @@ struct srs_ctx {
   int2* d_tiles_live = nullptr;
   bool tiles_compacted = false;
   std::vector<std::vector<int32_t>> bands;  // realizations of one mesh whose tiles are side by side in the list
-  double* stage[2] = {};         // pinned buffers of state transfers (state_xfer), stage_len doubles each
+  double* stage[2] = {};         // pinned buffers of state transfers (state_xfer), stage_len doubles each, one allocation
   size_t stage_len = 0;
   hipEvent_t ev_stage[2] = {};
   double last_total_ms = 0, last_sweep_ms = 0;
@@ -733,7 +733,6 @@ struct DevMem {
 };
 
 // Context helpers (device.hip).
-int build_map(srs_ctx* c, HostMesh& hm, int tile, TileMap* m);
 int check_real(srs_ctx* c, int32_t r);
 void launch_sweep(srs_ctx* c);
 int launch_step(srs_ctx* c, uint32_t gmode);

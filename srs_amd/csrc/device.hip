@@ -944,125 +944,191 @@ void build_class_rows(HostMesh& hm) {
   hm.class_rows = true;
 }
 
-// The cache lines per element that the halos of 512-element tiles cost more
-// with blocks of 64 (two lines for up to eight neighbours that follow each
-// other, one in each half) than with an element's species side by side (one
-// line for up to four), from at most eight tiles spread over the mesh.
-double scattered_lines(const HostMesh& hm) {
-  constexpr int T = 512;
-  const int nt = (hm.n + T - 1) / T, take = std::min(nt, 8);
-  std::vector<int32_t> e;
-  int64_t lines = 0, elements = 0;
-  for (int q = 0; q < take; ++q) {
-    const int t = (int)((int64_t)q * nt / take), j0 = t * T, j1 = std::min(hm.n, j0 + T);
-    e.clear();
-    for (size_t k = 4 * (size_t)j0; k < 4 * (size_t)j1; ++k)
-      if (hm.nbr[k] < j0 || hm.nbr[k] >= j1) e.push_back(hm.nbr[k] >> 2);
-    std::sort(e.begin(), e.end());
-    for (size_t k = 0; k < e.size(); ++k) {
-      if (k == 0 || e[k] >> 1 != e[k - 1] >> 1) lines += 2;
-      if (k == 0 || e[k] != e[k - 1]) lines -= 1;
-    }
-    elements += j1 - j0;
-  }
-  return (double)lines / elements;
-}
+// Where the neighbours of a mesh's elements are, for `tile` elements per tile,
+// on the host.
+struct HostMap {
+  int tile = 0, qcap = 0;      // as in TileMap
+  std::vector<uint32_t> hal;
+  std::vector<uint16_t> loc;
+  std::vector<int32_t> hoff;
+  // Cache lines that the halos cost more with blocks of 64 (two for up to eight
+  // neighbours that follow each other, one in each half) than with an element's
+  // species side by side (one for up to four), of all tiles.
+  int64_t lines = 0;
+};
 
-// The state layout's block: 64, or 1 where the halos of an average element
-// cost 0.6 cache lines less with it.  us per step, blocks of 64 / 1 (lines):
-// 927,816 elements in Morton order 20.0 / 20.3 (0.17), with 5% of the elements
-// anywhere 25.4 / 22.9 (0.41), with 10% 31.9 / 26.4 (0.65), shuffled within
-// 2,048 27.1 / 28.5 (0.46), within 131,072 58.5 / 53.4 (3.6), all of them 116 /
-// 75 (3.9); 2,952,000 with 5% 77.6 / 78.8, 10% 96.9 / 87.9, all 436 / 290;
-// 172,494 shuffled within 2,048 8.8 / 8.7, all 17.6 / 15.3.
-int quad_block_for(const srs_ctx* c) {
-  std::vector<double> lines;
-  for (const auto& hmp : c->meshes) lines.push_back(scattered_lines(*hmp));
-  double sum = 0.0, n = 0.0;
-  for (const HostReal& hr : c->reals) {
-    sum += lines[hr.mesh] * c->meshes[hr.mesh]->n;
-    n += c->meshes[hr.mesh]->n;
-  }
-  return sum > 0.6 * n ? 1 : 64;
-}
-
-// The tile map of a mesh for `tile` elements per tile, uploaded with the
-// neighbour table and the block flags.  Halos are sorted, so that a
-// wavefront's loads of them fall in runs.  Runs of tiles are independent:
-// finalizing the 2,952,000-element dyad takes 30 ms, 101 with them one after
-// another.
-int build_map(srs_ctx* c, HostMesh& hm, int tile, TileMap* m) {
+// Halos are sorted, so that a wavefront's loads of them fall in runs.  The
+// elements that a tile needs are bits of a bitmap, its own all set, and an
+// element's place is the rank of its bit: no branch per neighbour.  From 128k
+// elements up, runs of tiles on several threads (below, a thread costs more to
+// start than its tiles take).
+int make_map(const HostMesh& hm, int tile, HostMap* m) {
   const int n = hm.n, np = hm.np, nt = (n + tile - 1) / tile;
-  const int run = (4 * 512 + tile - 1) / tile, n_run = (nt + run - 1) / run;
-  std::vector<uint32_t> nbr(hm.nbr.size()), blk(np / 64, 0);
-  std::vector<uint16_t> loc(4 * (size_t)np, 0);
+  const int n_run = n < 1 << 17 ? 1 : std::min(nt, 32);
+  m->tile = tile;
+  m->lines = 0;
+  m->loc.assign(4 * (size_t)np, 0);
+  m->hoff.assign(nt + 1, 0);
   std::vector<std::vector<uint32_t>> halos(n_run);
-  std::vector<int32_t> hoff(nt + 1, 0);
+  std::vector<int64_t> lines(n_run, 0);
+  static_assert(MAX_TILE % 64 == 0, "tiles are whole words of the bitmap");
   const bool ok = each_chunk(n_run, [&](int q) {
     std::vector<uint32_t>& hal = halos[q];
-    // the tile's foreign elements, and their places by element in a small
-    // open-addressed table (at most 4 tile of them)
-    uint32_t mask = 15;
-    while (mask + 1 < 8u * (uint32_t)tile) mask = 2 * mask + 1;
-    std::vector<int32_t> key(mask + 1, -1), place(mask + 1), out;
-    auto slot = [&](int e) {
-      uint32_t h = ((uint32_t)e * 2654435761u >> 7) & mask;
-      while (key[h] != e && key[h] >= 0) h = (h + 1) & mask;
-      return h;
-    };
-    for (int t = q * run; t < std::min(nt, (q + 1) * run); ++t) {
+    std::vector<uint64_t> bits((size_t)np / 64, 0);
+    std::vector<int32_t> rank(bits.size()), words;
+    int64_t more = 0;
+    const int t0 = (int)((int64_t)nt * q / n_run), t1 = (int)((int64_t)nt * (q + 1) / n_run);
+    for (int t = t0; t < t1; ++t) {
       const int j0 = t * tile, j1 = std::min(n, j0 + tile);
-      out.clear();
-      for (size_t k = 4 * (size_t)j0; k < 4 * (size_t)j1; ++k) {
-        const int e = hm.nbr[k];
-        nbr[k] = (uint32_t)e | ((hm.flags[e] & F_SL) ? IDX_SL : 0u);
-        if (e >= j0 && e < j0 + tile) continue;
-        const uint32_t h = slot(e);
-        if (key[h] < 0) {
-          key[h] = e;
-          out.push_back(e);
+      const int w0 = j0 / 64, w1 = std::min(w0 + tile / 64, np / 64);
+      for (int w = w0; w < w1; ++w) {
+        bits[w] = ~0ull;
+        rank[w] = 64 * (w - w0);
+      }
+      words.clear();
+      const uint32_t *nb0 = hm.nbr.data() + 4 * (size_t)j0, *nb1 = hm.nbr.data() + 4 * (size_t)j1;
+      for (const uint32_t* p = nb0; p < nb1; ++p) {
+        const uint32_t e = idx_of(*p);
+        uint64_t& w = bits[e >> 6];
+        if (!w) words.push_back((int32_t)(e >> 6));
+        w |= 1ull << (e & 63);
+      }
+      std::sort(words.begin(), words.end());
+      const size_t h0 = hal.size();
+      for (int w : words) {
+        rank[w] = tile + (int)(hal.size() - h0);
+        uint64_t four = bits[w] | bits[w] >> 1;
+        four = (four | four >> 2) & 0x1111111111111111ull;  // any of four neighbours in a row
+        more += 2 * __builtin_popcountll((four | four >> 4) & 0x0101010101010101ull) - __builtin_popcountll(four);
+        for (uint64_t b = bits[w]; b; b &= b - 1) {
+          const int e = 64 * w + __builtin_ctzll(b);
+          hal.push_back((uint32_t)e | ((hm.flags[e] & F_SL) ? IDX_SL : 0u));
         }
       }
-      std::sort(out.begin(), out.end());
-      for (size_t i = 0; i < out.size(); ++i) place[slot(out[i])] = tile + (int)i;
-      for (size_t k = 4 * (size_t)j0; k < 4 * (size_t)j1; ++k) {
-        const int e = hm.nbr[k];
-        loc[k] = (uint16_t)(e >= j0 && e < j0 + tile ? e - j0 : place[slot(e)]);
+      m->hoff[t + 1] = (int32_t)(hal.size() - h0);
+      uint16_t* loc = m->loc.data() + 4 * (size_t)j0;
+      for (const uint32_t* p = nb0; p < nb1; ++p) {
+        const uint32_t e = idx_of(*p);
+        *loc++ = (uint16_t)(rank[e >> 6] + __builtin_popcountll(bits[e >> 6] & ((1ull << (e & 63)) - 1)));
       }
-      for (int e : out) hal.push_back((uint32_t)e | ((hm.flags[e] & F_SL) ? IDX_SL : 0u));
-      hoff[t + 1] = (int32_t)out.size();
-      std::fill(key.begin(), key.end(), -1);
+      for (int w : words) bits[w] = 0;
+      for (int w = w0; w < w1; ++w) bits[w] = 0;
     }
+    lines[q] = more;
   });
   if (!ok) return srs::fail(SRS_E_STATE, "out of host memory for the tile map");
-  for (size_t k = 4 * (size_t)n; k < nbr.size(); ++k) nbr[k] = (uint32_t)hm.nbr[k];
-  // the meshes' channel flags were set by add_realization: what blocks hold
-  for (size_t b = 0; b < blk.size(); ++b) {
-    bool plain = true;
-    for (size_t k = 64 * b; k < std::min<size_t>(64 * b + 64, n); ++k) plain &= hm.flags[k] == F_TROPC;
-    if (plain) blk[b] |= BLK_PLAIN;
-  }
-  size_t total = 0;
+  int64_t total = 0;
   int h_max = 0;
   for (int t = 0; t < nt; ++t) {
-    h_max = std::max(h_max, (int)hoff[t + 1]);
-    total += hoff[t + 1];
-    if (total > (size_t)INT32_MAX) return srs::fail(SRS_E_ARG, "mesh too large for its halo lists");
-    hoff[t + 1] = (int32_t)total;
+    h_max = std::max(h_max, (int)m->hoff[t + 1]);
+    total += m->hoff[t + 1];
+    if (total > INT32_MAX) return srs::fail(SRS_E_ARG, "mesh too large for its halo lists");
+    m->hoff[t + 1] = (int32_t)total;
   }
-  std::vector<uint32_t> hal;
-  hal.reserve(total + 1);
-  for (const auto& h : halos) hal.insert(hal.end(), h.begin(), h.end());
-  if (hal.empty()) hal.push_back(0);
-  int rc;
-  if ((rc = dev_upload(c, &hm.d_nbr, nbr)) || (rc = dev_upload(c, &hm.d_blk, blk)) ||
-      (rc = dev_upload(c, &m->d_loc, loc)) || (rc = dev_upload(c, &m->d_hal, hal)) ||
-      (rc = dev_upload(c, &m->d_hoff, hoff)))
-    return rc;
-  m->n_halo = hoff[nt];
-  m->tile = tile;
+  m->hal.clear();
+  if (n_run == 1) m->hal.swap(halos[0]);
+  else {
+    m->hal.reserve(total + 1);
+    for (const auto& h : halos) m->hal.insert(m->hal.end(), h.begin(), h.end());
+  }
+  if (m->hal.empty()) m->hal.push_back(0);
+  for (int64_t l : lines) m->lines += l;
   m->qcap = tile + h_max;
   return SRS_OK;
+}
+
+// The maps of every mesh for the context's tile, which is chosen here with the
+// state layout unless SRS_TUNE_TILE gave one.
+//
+// Layout: blocks of 64, or an element's species side by side where the halos of
+// an average element cost 0.6 cache lines less with it.  us per step, blocks of
+// 64 / 1 (lines): 927,816 elements in Morton order 20.0 / 20.3 (0.17), with 5% of
+// the elements anywhere 25.4 / 22.9 (0.41), with 10% 31.9 / 26.4 (0.65), shuffled
+// within 2,048 27.1 / 28.5 (0.46), within 131,072 58.5 / 53.4 (3.6), all of them
+// 116 / 75 (3.9); 2,952,000 with 5% 77.6 / 78.8, 10% 96.9 / 87.9, all 436 / 290;
+// 172,494 shuffled within 2,048 8.8 / 8.7, all 17.6 / 15.3.
+//
+// Tile: 512 elements share the most neighbours inside a tile (halos of 1.4
+// elements per element in the block order, 0.6 in the Morton order, 2.0 in RCM;
+// 1.9, 0.8 and 2.1 with 256) and are the fastest:
+// 2,952,000 elements 61.6 us per step in the block order, 64.2 with 256, 59.2
+// and 60.8 in the Morton order; a hundred 56,250-element members 111 and 128.
+// Scattered orders have no neighbours to share: there 128 is the fastest (us per
+// step with 128 / 512 elements shuffled: 2,952,000 250 / 290, sixteen members of
+// 172,494 131 / 144, 172,494 13.7 / 15.3).
+int plan_tiles(srs_ctx* c, std::vector<HostMap>* maps) {
+  maps->resize(c->meshes.size());
+  auto make = [&](int tile) {
+    c->tile = tile;
+    for (size_t k = 0; k < maps->size(); ++k)
+      if (int rc = make_map(*c->meshes[k], tile, &(*maps)[k])) return rc;
+    return (int)SRS_OK;
+  };
+  int rc = make(c->tile_set ? c->tile_set : 512);
+  if (rc) return rc;
+  double lines = 0.0, n = 0.0;
+  for (const HostReal& hr : c->reals) {
+    lines += (double)(*maps)[hr.mesh].lines;
+    n += c->meshes[hr.mesh]->n;
+  }
+  c->quad_block = lines > 0.6 * n ? 1 : 64;
+  if (c->tile_set) return SRS_OK;
+  return c->quad_block == 1 ? make(128) : (int)SRS_OK;
+}
+
+// Small tables in one device allocation and one copy (an allocation and a copy
+// of each took 10 us); larger ones get their own.  The pointers are set by
+// upload().
+class Pack {
+ public:
+  explicit Pack(srs_ctx* c) : c_(c) {}
+  template <class T>
+  int add(T** p, const std::vector<T>& v) {
+    const size_t bytes = v.size() * sizeof(T), at = (host_.size() + 255) / 256 * 256;
+    if (bytes == 0 || bytes > (size_t)1 << 18) return dev_upload(c_, p, v);
+    host_.resize(at + bytes);
+    memcpy(host_.data() + at, v.data(), bytes);
+    set_.push_back([p, at](char* base) { *p = (T*)(base + at); });
+    return SRS_OK;
+  }
+  int upload() {
+    char* base;
+    if (int rc = dev_upload(c_, &base, host_)) return rc;
+    for (const auto& s : set_) s(base);
+    return SRS_OK;
+  }
+
+ private:
+  srs_ctx* c_;
+  std::vector<char> host_;
+  std::vector<std::function<void(char*)>> set_;
+};
+
+// The tables of a mesh on the device.
+int upload_mesh(srs_ctx* c, HostMesh& hm, const HostMap& m) {
+  // the meshes' channel flags were set by add_realization: what blocks hold
+  std::vector<uint32_t> blk(hm.np / 64, 0);
+  for (size_t b = 0; b < blk.size(); ++b) {
+    bool plain = true;
+    for (size_t k = 64 * b; k < std::min<size_t>(64 * b + 64, hm.n); ++k) plain &= hm.flags[k] == F_TROPC;
+    if (plain) blk[b] |= BLK_PLAIN;
+  }
+  TileMap& t = hm.map;
+  t.tile = m.tile;
+  t.qcap = m.qcap;
+  t.n_halo = m.hoff.back();
+  Pack pk(c);
+  int rc;
+  if ((rc = pk.add(&hm.d_nbr, hm.nbr)) || (rc = pk.add(&hm.d_blk, blk)) || (rc = pk.add(&t.d_loc, m.loc)) ||
+      (rc = pk.add(&t.d_hal, m.hal)) || (rc = pk.add(&t.d_hoff, m.hoff)))
+    return rc;
+  if (c->class_all ? (rc = pk.add(&hm.d_row, hm.row)) || (rc = pk.add(&hm.d_tab, hm.tab))
+                   : (rc = pk.add(&hm.d_coef, hm.coef)))
+    return rc;
+  if ((rc = pk.add(&hm.d_flags, hm.flags)) || (rc = pk.add(&hm.d_inv, hm.inv)) || (rc = pk.add(&hm.d_V0, hm.V0)) ||
+      (rc = pk.add(&hm.d_tt, hm.tt)) || (rc = pk.add(&hm.d_br, hm.br)))
+    return rc;
+  return pk.upload();
 }
 
 // cpu/RunSimulation.cpp:85-88, the parts that depend on CaNSR only.
@@ -1542,8 +1608,8 @@ int srs_ctx_extensions(srs_ctx* c, int32_t r, const srs_extensions* e) {
 }
 
 static void release_stage(srs_ctx* c) {
+  if (c->stage[0]) (void)hipHostFree(c->stage[0]);
   for (int k = 0; k < 2; ++k) {
-    if (c->stage[k]) (void)hipHostFree(c->stage[k]);
     if (c->ev_stage[k]) (void)hipEventDestroy(c->ev_stage[k]);
     c->stage[k] = nullptr;
     c->ev_stage[k] = nullptr;
@@ -1613,7 +1679,10 @@ int srs_ctx_add_mesh(srs_ctx* c, const srs_mesh_desc* m, int32_t* mesh_id) {
     }
     const int i = hm->perm[k];
     for (int q = 0; q < 5; ++q) hm->coef[(size_t)q * np + k] = m->aij[5 * (size_t)i + q];
-    for (int q = 0; q < 4; ++q) hm->nbr[4 * (size_t)k + q] = hm->inv[m->nij[4 * (size_t)i + q]];
+    for (int q = 0; q < 4; ++q) {
+      const int32_t nb = m->nij[4 * (size_t)i + q];
+      hm->nbr[4 * (size_t)k + q] = (uint32_t)hm->inv[nb] | (m->tt_area[nb] != 0.0 ? IDX_SL : 0u);
+    }
     uint8_t f = 0;
     if (m->domain[i] != 0) f |= F_JSR;
     if (m->tropc[i]) f |= F_TROPC;
@@ -1721,35 +1790,15 @@ int srs_ctx_finalize(srs_ctx* c, int32_t record_capacity) {
   c->bands.clear();
   c->sweep_lds = 0;
   release_stage(c);
-  // 512-element tiles share the most neighbours inside a tile (halos of 1.4
-  // elements per element in the block order, 0.6 in the Morton order; 1.9 and
-  // 0.8 with 256) and were the fastest
-  // at every size: 927,816 elements 21.5 against 23.3 us per step, 56,250
-  // 9.2 against 9.3, the 48-member ensemble 147 against 171
-  // Scattered orders have no neighbours to share: there 128 is the fastest (a
-  // 512-element tile's halo then takes half of a CU's LDS; us per step with 128
-  // / 512 elements shuffled: 2,952,000 250 / 290, sixteen members of 172,494 131
-  // / 144, 172,494 13.7 / 15.3).
-  c->quad_block = quad_block_for(c);
-  c->tile = c->tile_set ? c->tile_set : c->quad_block == 1 ? 128 : 512;
+  std::vector<HostMap> maps;
+  if ((rc = plan_tiles(c, &maps))) return rc;
   c->class_all = !c->meshes.empty();
   for (auto& hmp : c->meshes) c->class_all &= hmp->class_rows;
-  for (auto& hmp : c->meshes) {
-    HostMesh& hm = *hmp;
-    if ((rc = build_map(c, hm, c->tile, &hm.map))) return rc;
-    c->sweep_lds = std::max(c->sweep_lds, 4 * sizeof(double) * (size_t)hm.map.qcap);
-    if (!c->class_all) {
-      if ((rc = dev_upload(c, &hm.d_coef, hm.coef))) return rc;
-    } else {
-      if ((rc = dev_upload(c, &hm.d_row, hm.row))) return rc;
-      if ((rc = dev_upload(c, &hm.d_tab, hm.tab))) return rc;
-    }
-    if ((rc = dev_upload(c, &hm.d_flags, hm.flags))) return rc;
-    if ((rc = dev_upload(c, &hm.d_inv, hm.inv))) return rc;
-    if ((rc = dev_upload(c, &hm.d_V0, hm.V0))) return rc;
-    if ((rc = dev_upload(c, &hm.d_tt, hm.tt))) return rc;
-    if (!hm.br.empty() && (rc = dev_upload(c, &hm.d_br, hm.br))) return rc;
+  for (size_t k = 0; k < c->meshes.size(); ++k) {
+    if ((rc = upload_mesh(c, *c->meshes[k], maps[k]))) return rc;
+    c->sweep_lds = std::max(c->sweep_lds, 4 * sizeof(double) * (size_t)maps[k].qcap);
   }
+  maps.clear();
   std::vector<RealDesc> descs;
   std::vector<RealLive> lives;
   std::vector<int2> tiles;
@@ -1804,13 +1853,6 @@ int srs_ctx_finalize(srs_ctx* c, int32_t record_capacity) {
     }
     d.n_ryr = (int32_t)hr.ryr_ele.size();
     d.n_lcc = (int32_t)hr.lcc_ele.size();
-    int32_t *p;
-    if ((rc = dev_upload(c, &p, hr.ryr_ele))) return rc; d.ryr_ele = p;
-    if ((rc = dev_upload(c, &p, hr.ryr_jsr))) return rc; d.ryr_jsr = p;
-    if ((rc = dev_upload(c, &p, hr.ryr_nb))) return rc; d.ryr_nb = p;
-    if ((rc = dev_upload(c, &p, hr.lcc_ele))) return rc; d.lcc_ele = p;
-    if ((rc = dev_upload(c, &p, hr.celem))) return rc; d.celem = p;
-    if ((rc = dev_upload(c, &p, hr.cstart))) return rc; d.cstart = p;
     for (ChanEntry& en : hr.centry)
       if (en.code >= 0) en.sl = (hm.flags[en.jsr] & F_SL ? 1 : 0) | (hm.flags[en.cyt] & F_SL ? 2 : 0);
     std::vector<ChanElem> crec(hr.celem.size());
@@ -1818,7 +1860,7 @@ int srs_ctx_finalize(srs_ctx* c, int32_t record_capacity) {
       ChanElem& e = crec[k];
       e.j = hr.celem[k];
       for (int q = 0; q < 5; ++q) e.a[q] = hm.coef[(size_t)q * hm.np + e.j];
-      for (int q = 0; q < 4; ++q) e.nb[q] = hm.nbr[4 * (size_t)e.j + q];
+      for (int q = 0; q < 4; ++q) e.nb[q] = (int32_t)idx_of(hm.nbr[4 * (size_t)e.j + q]);
       e.v0 = hm.V0[e.j];
       e.tt = hm.tt[e.j];
       e.e0 = hr.cstart[k];
@@ -1826,18 +1868,20 @@ int srs_ctx_finalize(srs_ctx* c, int32_t record_capacity) {
       e.f = hm.flags[e.j];
       e.first = hr.centry[e.e0];
     }
-    ChanEntry* pe;
-    ChanElem* pc;
-    if ((rc = dev_upload(c, &pe, hr.centry))) return rc; d.centry = pe;
-    if ((rc = dev_upload(c, &pc, crec))) return rc; d.crec = pc;
     d.n_celem = (int32_t)hr.celem.size();
-    std::vector<int32_t> zeros_r(d.n_ryr, 0), ones_l(d.n_lcc, 1), twos_l(d.n_lcc, 2);
-    if ((rc = dev_upload(c, &p, zeros_r))) return rc; d.ryr_state = p;
-    if ((rc = dev_upload(c, &p, ones_l))) return rc; d.lcc_state = p;
-    if ((rc = dev_upload(c, &p, twos_l))) return rc; d.lccv_state = p;
-    std::vector<double> zr(d.n_ryr + d.n_lcc, -1.0);
-    double* pr;
-    if ((rc = dev_upload(c, &pr, zr))) return rc; d.R = pr;
+    struct { int32_t *ryr_ele, *ryr_jsr, *ryr_nb, *lcc_ele, *celem, *cstart; ChanEntry* centry; ChanElem* crec; } t{};
+    const std::vector<int32_t> closed(d.n_ryr, 0), ones(d.n_lcc, 1), twos(d.n_lcc, 2);
+    const std::vector<double> resid(d.n_ryr + d.n_lcc, -1.0);
+    Pack pk(c);
+    if ((rc = pk.add(&t.ryr_ele, hr.ryr_ele)) || (rc = pk.add(&t.ryr_jsr, hr.ryr_jsr)) ||
+        (rc = pk.add(&t.ryr_nb, hr.ryr_nb)) || (rc = pk.add(&t.lcc_ele, hr.lcc_ele)) ||
+        (rc = pk.add(&t.celem, hr.celem)) || (rc = pk.add(&t.cstart, hr.cstart)) ||
+        (rc = pk.add(&t.centry, hr.centry)) || (rc = pk.add(&t.crec, crec)) || (rc = pk.add(&d.ryr_state, closed)) ||
+        (rc = pk.add(&d.lcc_state, ones)) || (rc = pk.add(&d.lccv_state, twos)) || (rc = pk.add(&d.R, resid)) ||
+        (rc = pk.upload()))
+      return rc;
+    d.ryr_ele = t.ryr_ele; d.ryr_jsr = t.ryr_jsr; d.ryr_nb = t.ryr_nb; d.lcc_ele = t.lcc_ele;
+    d.celem = t.celem; d.cstart = t.cstart; d.centry = t.centry; d.crec = t.crec;
     d.ryr_out = hr.ints[SRS_I_FLAG_RYR_OUT] ? 1 : 0;
     d.gpu_layout = c->gpu_layout;
     d.rec_len = 7 + (d.gpu_layout ? d.n_ryr : 0) + (d.ryr_out ? d.n_ryr : 0);
@@ -1877,15 +1921,16 @@ int srs_ctx_finalize(srs_ctx* c, int32_t record_capacity) {
   const int nt_state = c->nt_state < 0 ? ws > 330e6 : c->nt_state;
   c->n_tiles = (int)tiles.size();
   c->grid_sweep = (c->n_tiles + NXCD - 1) / NXCD * NXCD;
-  // state transfers: two pinned buffers of at most 8 MB (larger fields go
-  // through them in parts)
-  for (const HostReal& hr : c->reals) c->stage_len = std::max(c->stage_len, 6 * (size_t)c->meshes[hr.mesh]->n);
-  if (c->stage_len > (size_t)1 << 17) c->stage_len = (c->stage_len + 1) / 2;  // two parts, one copied while one moves
-  c->stage_len = std::min(c->stage_len, (size_t)1 << 20);
-  for (int k = 0; k < 2; ++k) {
-    HIPCHK(hipHostMalloc((void**)&c->stage[k], c->stage_len * sizeof(double), hipHostMallocDefault));
-    HIPCHK(hipEventCreateWithFlags(&c->ev_stage[k], hipEventDisableTiming));
-  }
+  // State transfers: the largest fields in eight parts, of 0.5 to 8 MB each, one
+  // copied while one moves.  Two halves of 1.3 MB moved 56,250 elements as fast
+  // as this, but a new pinned page costs 0.75 us when it is first touched: 1.0 ms
+  // for the first fields set against 0.4.
+  size_t fields = 0;
+  for (const HostReal& hr : c->reals) fields = std::max(fields, 6 * (size_t)c->meshes[hr.mesh]->n);
+  c->stage_len = std::min(fields, std::min(std::max(fields / 8, (size_t)1 << 16), (size_t)1 << 20));
+  HIPCHK(hipHostMalloc((void**)&c->stage[0], 2 * c->stage_len * sizeof(double), hipHostMallocDefault));
+  c->stage[1] = c->stage[0] + c->stage_len;
+  for (int k = 0; k < 2; ++k) HIPCHK(hipEventCreateWithFlags(&c->ev_stage[k], hipEventDisableTiming));
   if ((rc = dev_upload(c, &c->d_desc, descs))) return rc;
   if ((rc = dev_upload(c, &c->d_live, lives))) return rc;
   if ((rc = dev_upload(c, &c->d_tiles, tiles))) return rc;

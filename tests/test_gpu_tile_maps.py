@@ -1,0 +1,63 @@
+"""Where a tile's neighbours are staged: the maps that srs_ctx_finalize builds,
+on one thread and on several, for every tile size and padding, and the fields'
+way in and out in parts.  An element's step reads its neighbours in the order of
+its own row, so fields are the same bits whatever the order, tile and padding."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import srs_amd as S
+from srs_amd import workloads as W
+
+pytestmark = pytest.mark.gpu
+
+
+def _mesh(n_xy):
+    g = S.box_grid(W.spark_box_spec(h=1.0 / n_xy, n_xy=n_xy))
+    aij, nij = S.assemble_operator(g)
+    p = W.spark_params(dt=W.stable_dt(aij, 0.22))
+    X = S.equilibrium_state(g, p.reals)[0]
+    return g, aij, nij, p, X * np.random.default_rng(8).uniform(0.9, 1.0, X.shape)
+
+
+def _stepped(m, members=1, tune=None, **order):
+    g, aij, nij, p, X = m
+    with S.Context(0) as ctx:
+        ctx.tune(**(tune or {}))
+        mid = ctx.add_mesh_grid(g, aij, nij, **order)
+        for k in range(members):
+            ctx.add_realization(mid, g.ryr_ele, g.ryr_jsr, g.ryr_nb, g.lcc_ele, p, seed=3, stream=k)
+        ctx.finalize()
+        for k in range(members):
+            ctx.state_set(k, X)
+        ctx.explicit_step(12)
+        return ctx.state_get(members - 1)
+
+
+# 124,146 and 138,720 elements: either side of 131,072, from where several
+# threads build the map
+@pytest.mark.parametrize("n_xy", [10, 33, 34])
+def test_maps_of_every_tile_and_padding(n_xy):
+    m = _mesh(n_xy)
+    want = _stepped(m, order=S.ORDER_AS_GIVEN)
+    assert not np.array_equal(want, m[4])
+    for tile in (128, 256, 512):
+        for pad in (0, 64):
+            assert np.array_equal(_stepped(m, tune=dict(tile=tile, plane_pad=pad)), want), (tile, pad)
+
+
+# one part (63,504 doubles), two (72,900), eight of more than 0.5 MB; the small
+# mesh's fields move through buffers that the large one's set
+@pytest.mark.parametrize("n_xys", [(14,), (15,), (10, 37)])
+def test_fields_in_parts(n_xys):
+    meshes = [_mesh(n) for n in n_xys]
+    with S.Context(0) as ctx:
+        for g, aij, nij, p, _ in meshes:
+            ctx.add_realization(ctx.add_mesh_grid(g, aij, nij), g.ryr_ele, g.ryr_jsr, g.ryr_nb, g.lcc_ele, p, seed=1, stream=0)
+        ctx.finalize()
+        for _ in range(2):
+            for r, m in enumerate(meshes):
+                ctx.state_set(r, m[4])
+            for r, m in enumerate(meshes):
+                assert np.array_equal(ctx.state_get(r), m[4])
