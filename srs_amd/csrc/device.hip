@@ -1050,9 +1050,14 @@ int make_map(const HostMesh& hm, int tile, HostMap* m) {
 //
 // Tile: 512 elements share the most neighbours inside a tile (halos of 1.4
 // elements per element in the block order, 0.6 in the Morton order, 2.0 in RCM;
-// 1.9, 0.8 and 2.1 with 256) and are the fastest:
-// 2,952,000 elements 61.6 us per step in the block order, 64.2 with 256, 59.2
+// 1.9, 0.8 and 2.1 with 256) and are the fastest while three workgroups share a
+// CU: 2,952,000 elements 61.6 us per step in the block order, 64.2 with 256, 59.2
 // and 60.8 in the Morton order; a hundred 56,250-element members 111 and 128.
+// The staged quads of the worst tile decide that.  In a breadth-first order of
+// the 2,952,000 they pass a third of the LDS, and 256 elements take 70.3 us
+// against 77.0 (rows that all differ: 77.7 against 86.1), of 3,930,960 93.8
+// against 102.6; with runs of 64 elements of the block order shuffled, 927,816
+// take 38.6 against 47.9.
 // Scattered orders have no neighbours to share: there 128 is the fastest (us per
 // step with 128 / 512 elements shuffled: 2,952,000 250 / 290, sixteen members of
 // 172,494 131 / 144, 172,494 13.7 / 15.3).
@@ -1067,13 +1072,19 @@ int plan_tiles(srs_ctx* c, std::vector<HostMap>* maps) {
   int rc = make(c->tile_set ? c->tile_set : 512);
   if (rc) return rc;
   double lines = 0.0, n = 0.0;
+  int qcap = 0;
   for (const HostReal& hr : c->reals) {
     lines += (double)(*maps)[hr.mesh].lines;
     n += c->meshes[hr.mesh]->n;
   }
+  for (const HostMap& m : *maps) qcap = std::max(qcap, m.qcap);
   c->quad_block = lines > 0.6 * n ? 1 : 64;
   if (c->tile_set) return SRS_OK;
-  return c->quad_block == 1 ? make(128) : (int)SRS_OK;
+  if (c->quad_block == 1) return make(128);
+  // a CU's 160 KB in granules of 1280 B, 42 for each of three workgroups; the
+  // gated sweep has 256 or 384 B of its own
+  const size_t lds = 4 * sizeof(double) * (size_t)qcap + (c->reals.size() == 1 && c->gated ? 384 : 0);
+  return lds > 42 * 1280 ? make(256) : (int)SRS_OK;
 }
 
 // Small tables in one device allocation and one copy (an allocation and a copy

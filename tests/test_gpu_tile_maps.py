@@ -61,3 +61,17 @@ def test_fields_in_parts(n_xys):
                 ctx.state_set(r, m[4])
             for r, m in enumerate(meshes):
                 assert np.array_equal(ctx.state_get(r), m[4])
+
+
+# Runs of 64 elements of the block order, shuffled: a 512-element tile stages 2,500
+# quads, of which two workgroups, not three, fit a CU's LDS, so 256 are taken
+@pytest.mark.parametrize("members", [1, 3])
+def test_tile_of_an_order_with_large_halos(members):
+    m = _mesh(22)
+    n = m[0].n_ele
+    block = W.kuhn_block_order(m[0])
+    runs = [block[i:i + 64] for i in range(0, n, 64)]
+    perm = np.concatenate([runs[i] for i in np.random.default_rng(0).permutation(len(runs))])
+    want = _stepped(m, members, order=S.ORDER_AS_GIVEN)
+    for tune in ({}, dict(tile=512), dict(tile=256), dict(gated_sweep=0)):
+        assert np.array_equal(_stepped(m, members, tune, perm=perm), want), tune
