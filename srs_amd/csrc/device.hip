@@ -795,15 +795,18 @@ GatedFn pick_gated_nt(const srs_ctx* c) {
 
 // How much the registers of the gating workgroup may cost the tiles.  With no
 // more tiles than CUs (256), each workgroup has a CU to itself: no budget
-// (56,250 elements: 5.3 us per step).  Up to
-// 900,000 elements the gating workgroup is still the longest one: four
-// wavefronts, with its loads ahead of the gating (400,000 elements: 12.5
-// against 17.0 us with six).  Beyond that the tiles' own wavefronts decide: six,
-// the gating's registers spilled and its channel elements loaded after it
-// (928k: 21.3 against 21.9 us; 1.6M: 29.4 / 31.1; 3M: 61.5 / 70.7).
+// (56,250 elements: 5.3 us per step).  Then four wavefronts, with the first half
+// of its channel elements behind the gating's first barrier, while the gating
+// workgroup is the longest one; beyond, the tiles' own wavefronts decide: six,
+// the gating's registers spilled and its channel elements updated after it.  us
+// per step with four / six, RCM, block and Morton order: 354,816 elements
+// 12.5 / 13.2, -, 10.3 / 13.3; 638,262 18.8 / 17.4, 17.2 / 16.2, 15.9 / 16.8;
+// 703,452 19.9 / 18.5, 18.4 / 17.2, 17.2 / 17.1; 750,708 20.7 / 19.3, 19.1 /
+// 17.8, 17.5 / 17.5; with rows that all differ 704,184 22.1 / 20.7, 21.0 / 19.6,
+// 19.6 / 18.5.  The line is where six are slower in no order.
 template <int BS, bool CMP, bool PROTO>
 GatedFn pick_gated_w(const srs_ctx* c) {
-  if (c->occ || (int64_t)c->n_tiles * BS >= 900000) return pick_gated_nt<BS, CMP, PROTO, false, 6>(c);
+  if (c->occ || (int64_t)c->n_tiles * BS >= 700000) return pick_gated_nt<BS, CMP, PROTO, false, 6>(c);
   return c->n_tiles <= 256 ? pick_gated_nt<BS, CMP, PROTO, true, 2>(c)
                            : pick_gated_nt<BS, CMP, PROTO, true, 4>(c);
 }

@@ -75,3 +75,16 @@ def test_tile_of_an_order_with_large_halos(members):
     want = _stepped(m, members, order=S.ORDER_AS_GIVEN)
     for tune in ({}, dict(tile=512), dict(tile=256), dict(gated_sweep=0)):
         assert np.array_equal(_stepped(m, members, tune, perm=perm), want), tune
+
+
+# 658,080 and 703,452 elements: the gated step's register budget changes at 700,000
+@pytest.mark.parametrize("n_xy", [60, 61])
+def test_register_budgets_either_side_of_their_line(n_xy):
+    g = S.box_grid(W.dyad_box_spec(h=2.0 / n_xy))
+    assert (g.n_ele < 700_000) == (n_xy == 60) and abs(g.n_ele - 700_000) < 50_000
+    aij, nij = S.assemble_operator(g)
+    p = W.spark_params(dt=W.stable_dt(aij, 0.22))
+    m = g, aij, nij, p, S.equilibrium_state(g, p.reals)[0]
+    got = _stepped(m)
+    assert np.array_equal(got, _stepped(m, tune=dict(occupancy=6)))
+    assert np.array_equal(got, _stepped(m, tune=dict(gated_sweep=0)))
