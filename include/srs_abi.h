@@ -279,8 +279,9 @@ int srs_ctx_create(int device, srs_ctx** out);
  * the tile before srs_ctx_finalize; the rest at any time. */
 #define SRS_TUNE_TILE 1          /* elements per sweep workgroup: 128, 256 or 512; by default srs_ctx_finalize
                                     takes 512, 256 where a 512-element tile has so many neighbours that
-                                    fewer than three workgroups fit a CU's LDS, and 128 where the element
-                                    order scatters the neighbours */
+                                    fewer than three workgroups fit a CU's LDS or several realizations have
+                                    no more tiles than CUs, and 128 where they still have not or the
+                                    element order scatters the neighbours */
 #define SRS_TUNE_NT_GEOMETRY 2   /* accepted and ignored: operator rows are read through the caches */
 #define SRS_TUNE_NT_STATE 3      /* 1: non-temporal stores of the new state; by default srs_ctx_finalize
                                     takes 1 when states and rows exceed 330 MB */

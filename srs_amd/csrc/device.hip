@@ -1061,6 +1061,11 @@ int make_map(const HostMesh& hm, int tile, HostMap* m) {
 // against 77.0 (rows that all differ: 77.7 against 86.1), of 3,930,960 93.8
 // against 102.6; with runs of 64 elements of the block order shuffled, 927,816
 // take 38.6 against 47.9.
+// Several realizations with no more tiles than CUs (256) take the smallest such
+// tile: each has a CU to itself, and what it waits for is its own chain of loads
+// and barriers.  us per step with 128 / 256 / 512: two members of 3,600 elements
+// 10.3 / 10.9 / 11.5, eight 10.6 / 11.0 / 11.7, eight of 8,112 (512, 256 and 128
+// tiles) 10.9 / 10.9 / 11.3, of 15,360 (960, 480, 240) 11.2 / 11.4 / 11.3.
 // Scattered orders have no neighbours to share: there 128 is the fastest (us per
 // step with 128 / 512 elements shuffled: 2,952,000 250 / 290, sixteen members of
 // 172,494 131 / 144, 172,494 13.7 / 15.3).
@@ -1072,7 +1077,12 @@ int plan_tiles(srs_ctx* c, std::vector<HostMap>* maps) {
       if (int rc = make_map(*c->meshes[k], tile, &(*maps)[k])) return rc;
     return (int)SRS_OK;
   };
-  int rc = make(c->tile_set ? c->tile_set : 512);
+  auto one_each = [&](int tile) {
+    int64_t nt = 0;
+    for (const HostReal& hr : c->reals) nt += (c->meshes[hr.mesh]->n + tile - 1) / tile;
+    return c->reals.size() > 1 && nt <= 256;
+  };
+  int rc = make(c->tile_set ? c->tile_set : one_each(128) ? 128 : one_each(256) ? 256 : 512);
   if (rc) return rc;
   double lines = 0.0, n = 0.0;
   int qcap = 0;
@@ -1082,12 +1092,12 @@ int plan_tiles(srs_ctx* c, std::vector<HostMap>* maps) {
   }
   for (const HostMap& m : *maps) qcap = std::max(qcap, m.qcap);
   c->quad_block = lines > 0.6 * n ? 1 : 64;
-  if (c->tile_set) return SRS_OK;
+  if (c->tile_set || c->tile == 128) return SRS_OK;
   if (c->quad_block == 1) return make(128);
   // a CU's 160 KB in granules of 1280 B, 42 for each of three workgroups; the
   // gated sweep has 256 or 384 B of its own
   const size_t lds = 4 * sizeof(double) * (size_t)qcap + (c->reals.size() == 1 && c->gated ? 384 : 0);
-  return lds > 42 * 1280 ? make(256) : (int)SRS_OK;
+  return c->tile == 512 && lds > 42 * 1280 ? make(256) : (int)SRS_OK;
 }
 
 // Small tables in one device allocation and one copy (an allocation and a copy

@@ -21,7 +21,7 @@ def _mesh(n_xy):
     return g, aij, nij, p, X * np.random.default_rng(8).uniform(0.9, 1.0, X.shape)
 
 
-def _stepped(m, members=1, tune=None, **order):
+def _stepped(m, members=1, tune=None, flags=0, **order):
     g, aij, nij, p, X = m
     with S.Context(0) as ctx:
         ctx.tune(**(tune or {}))
@@ -31,7 +31,7 @@ def _stepped(m, members=1, tune=None, **order):
         ctx.finalize()
         for k in range(members):
             ctx.state_set(k, X)
-        ctx.explicit_step(12)
+        ctx.explicit_step(16, flags)
         return ctx.state_get(members - 1)
 
 
@@ -88,3 +88,13 @@ def test_register_budgets_either_side_of_their_line(n_xy):
     got = _stepped(m)
     assert np.array_equal(got, _stepped(m, tune=dict(occupancy=6)))
     assert np.array_equal(got, _stepped(m, tune=dict(gated_sweep=0)))
+
+
+# 253 and 276 tiles of 128 elements; 256 and 288 of 256
+@pytest.mark.parametrize("n_xy,members", [(9, 11), (9, 12), (13, 8), (13, 9)])
+def test_tiles_of_small_ensembles(n_xy, members):
+    m = _mesh(n_xy)
+    want = _stepped(m, order=S.ORDER_AS_GIVEN)
+    for tune in ({}, dict(tile=512)):
+        for flags in (0, S.STEP_GRAPH):
+            assert np.array_equal(_stepped(m, members, tune, flags), want), (tune, flags)
