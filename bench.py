@@ -207,7 +207,7 @@ def bench_batched(n_real, steps, warmup, order, tune=None, n_tune=512):
     if tune is None:
         sample = list(range(min(n_real, n_tune)))
         tune, trials = autotune(lambda cfg: W.ensemble_context(n_real, order=order, tune=cfg, only=sample)[0],
-                                tiles=(256, 512), compact=(1,), occupancy=(0,), nt_geometry=(0,), lds=(1,))
+                                tiles=(256, 512), compact=(1,), occupancy=(0,))
         log(f"batched autotune: {tune}")
     ctx, dts, n_ele, nbytes = W.ensemble_context(n_real, order=order, tune=tune, log=log)
     log(f"batched: {n_real} realizations, {n_ele} elements, group {tune.get('group', 1)}")
@@ -362,17 +362,16 @@ def bench_adjoint_full(n_real=8, t_sim=20.0, n_points=64, n_samples=50, per_call
 
 def bench_size_scan(steps=400):
     """Cost per element-step against working-set size: the plain path on the
-    dyad box at h = 40/30/25/20 nm (tuned sweep, block order), the ensemble
+    dyad box at h = 40/30/25/20 nm (the library's choices, block order), the ensemble
     with 8..256 members stepped together, and the 2048-member ensemble with
     realization subsets of 0/64/128/192 MB stepped block by block."""
     import srs_amd as S
     from srs_amd import workloads as W
 
     out = []
-    tune = dict(tile=512, compact=1, nt_geometry=1, nt_state=0, occupancy=6, lds=1)
     for h in (0.04, 0.03, 0.025, 0.02):
         pr = W.prepare_dyad(h=h)
-        ctx = setup_plain(pr, "block", tune)
+        ctx = setup_plain(pr, "block", {})
         ctx.explicit_step(50, S.STEP_GRAPH)
         ctx.prepare(steps, S.STEP_GRAPH)
         ctx.sync()
@@ -385,9 +384,8 @@ def bench_size_scan(steps=400):
         out.append(dict(workload=f"dyad h={h}", n_elements=n, state_mb=96 * n / 1e6, us_per_step=1e6 * wall / steps,
                         ps_per_element_step=1e12 * wall / steps / n))
         log(json.dumps(out[-1]))
-    btune = dict(tile=256, compact=1, group=1, nt_geometry=0, nt_state=1, occupancy=6, lds=1)
     for k, mb in ((8, 0), (16, 0), (64, 0), (256, 0), (2048, 0), (2048, 64), (2048, 128), (2048, 192)):
-        ctx, _, n_ele, _ = W.ensemble_context(k, tune=btune)
+        ctx, _, n_ele, _ = W.ensemble_context(k)
         ctx.tune(subset_mb=mb)
         m = 128
         ctx.explicit_step(16, S.STEP_GRAPH)

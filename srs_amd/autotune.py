@@ -2,9 +2,10 @@
 
 Candidates: elements per workgroup (tile), non-temporal stores of the new
 state (nt_state), SoA plane padding (plane_pad), the compact row format and the
-gated step's register budget (occupancy); group, nt_geometry and lds are
-accepted by the library and change nothing.  Every candidate computes the
-same bits; only speed differs.  Each trial runs on a scratch context built
+gated step's register budget (occupancy).  The library accepts group,
+nt_geometry and lds and does the same whatever they are, so of these the first
+value given goes into the configuration and no others are timed.  Every
+candidate computes the same bits; only speed differs.  Each trial runs on a scratch context built
 by the caller's factory, so the context that is finally used has taken no
 steps.  Timing is the step as it runs, a captured graph of steps timed by
 HIP events around the call.
@@ -21,21 +22,20 @@ LAYOUT_KEYS = ("tile", "plane_pad", "compact", "group")
 KERNEL_KEYS = ("nt_geometry", "nt_state", "occupancy", "lds")
 
 
-def autotune(make: Callable[[dict], Context], tiles=(128, 256, 512), pads=(0,), compact=(1, 0), nt_geometry=(0, 1),
-             nt_state=(0, 1), occupancy=(0, 6), lds=(0, 1), groups=(1,), reps: int = 20, warm: int = 3,
+def autotune(make: Callable[[dict], Context], tiles=(128, 256, 512), pads=(0,), compact=(1, 0), nt_geometry=(0,),
+             nt_state=(0, 1), occupancy=(0, 6), lds=(1,), groups=(1,), reps: int = 20, warm: int = 3,
              log=None) -> tuple[dict, list]:
     """Returns (best configuration, all trials as (config, step_ms))."""
     trials = []
-    for tile, pad, cmp, grp in itertools.product(tiles, pads, compact, groups):
+    for tile, pad, cmp in itertools.product(tiles, pads, compact):
         layout = {"tile": tile, "plane_pad": pad, "compact": cmp}
-        if len(groups) > 1 or grp != 1:
-            layout["group"] = grp
+        if len(groups) > 1 or groups[0] != 1:
+            layout["group"] = groups[0]
         ctx = make(layout)
         try:
-            for g, s, o, ld in itertools.product(nt_geometry, nt_state, occupancy, lds):
-                if ld and grp != 1:
-                    continue
-                ctx.tune(nt_geometry=g, nt_state=s, occupancy=o, lds=ld)
+            for s, o in itertools.product(nt_state, occupancy):
+                kernel = {"nt_geometry": nt_geometry[0], "nt_state": s, "occupancy": o, "lds": lds[0]}
+                ctx.tune(**kernel)
                 ctx.explicit_step(warm)
                 t0 = time.perf_counter()
                 # ranked by the step as it runs: a captured graph of n steps
@@ -47,7 +47,7 @@ def autotune(make: Callable[[dict], Context], tiles=(128, 256, 512), pads=(0,), 
                 ctx.explicit_step(n, STEP_GRAPH)
                 total, _ = ctx.last_timing()
                 ms = total / n
-                cfg = {**layout, "nt_geometry": g, "nt_state": s, "occupancy": o, "lds": ld}
+                cfg = {**layout, **kernel}
                 trials.append((cfg, ms))
                 if log:
                     log(f"autotune {cfg}: step {ms * 1e3:.2f} us ({time.perf_counter() - t0:.2f} s)")
