@@ -1945,13 +1945,17 @@ int srs_ctx_finalize(srs_ctx* c, int32_t record_capacity) {
   const int nt_state = c->nt_state < 0 ? ws > 330e6 : c->nt_state;
   c->n_tiles = (int)tiles.size();
   c->grid_sweep = (c->n_tiles + NXCD - 1) / NXCD * NXCD;
-  // State transfers: the largest fields in eight parts, of 0.5 to 8 MB each, one
-  // copied while one moves.  Two halves of 1.3 MB moved 56,250 elements as fast
-  // as this, but a new pinned page costs 0.75 us when it is first touched: 1.0 ms
-  // for the first fields set against 0.4.
+  // State transfers: up to 4 MB of fields in parts of 0.5 MB, larger ones in
+  // halves of at most 8 MB, one part copied while one moves.  A pinned page costs
+  // 0.75 us when it is first touched: with two halves of 1.3 MB the first fields
+  // set of 56,250 elements took 1.0 ms against 0.4, later ones no less (read 0.17
+  // against 0.13).  Eight parts of 1.3 MB, each with its launch, wait and
+  // helpers, read 219,000 elements 0.07 ms slower than halves.
   size_t fields = 0;
   for (const HostReal& hr : c->reals) fields = std::max(fields, 6 * (size_t)c->meshes[hr.mesh]->n);
-  c->stage_len = std::min(fields, std::min(std::max(fields / 8, (size_t)1 << 16), (size_t)1 << 20));
+  c->stage_len = fields <= (size_t)1 << 19 ? std::min(fields, (size_t)1 << 16)
+                                           : std::min((fields + 1) / 2, (size_t)1 << 20);
+  c->stage_len = (c->stage_len + 511) / 512 * 512;  // the second buffer on a page
   HIPCHK(hipHostMalloc((void**)&c->stage[0], 2 * c->stage_len * sizeof(double), hipHostMallocDefault));
   c->stage[1] = c->stage[0] + c->stage_len;
   for (int k = 0; k < 2; ++k) HIPCHK(hipEventCreateWithFlags(&c->ev_stage[k], hipEventDisableTiming));

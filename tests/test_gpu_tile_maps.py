@@ -47,9 +47,9 @@ def test_maps_of_every_tile_and_padding(n_xy):
             assert np.array_equal(_stepped(m, tune=dict(tile=tile, plane_pad=pad)), want), (tile, pad)
 
 
-# one part (63,504 doubles), two (72,900), eight of more than 0.5 MB; the small
-# mesh's fields move through buffers that the large one's set
-@pytest.mark.parametrize("n_xys", [(14,), (15,), (10, 37)])
+# one part (63,504 doubles), two (72,900), eight (514,692 doubles), two halves (550,800
+# doubles); a small mesh's fields move through buffers that the large one's set
+@pytest.mark.parametrize("n_xys", [(14,), (15,), (29,), (30,), (10, 37)])
 def test_fields_in_parts(n_xys):
     meshes = [_mesh(n) for n in n_xys]
     with S.Context(0) as ctx:
