@@ -866,9 +866,9 @@ static int loss_grad_run(srs_ctx* c, const std::vector<int32_t>& ids, int32_t sc
           grads[(size_t)(m0 + y) * ADJ_NT + k] = sum;
         }
     }
-    // the members' states as they were: descriptors (the recomputation
-    // pointed their buffers into the segment) and live state (it names the
-    // current buffer) first, then the start state into that buffer
+    // the members' states as they were: descriptors (their schedules were this
+    // call's) and live state (it names the current buffer) first, then the start
+    // state into that buffer
     for (int y = 0; y < nb; ++y) {
       const HostReal& hr = c->reals[ids[m0 + y]];
       HIPCHK(hipMemcpy(c->d_desc + ids[m0 + y], &hr.desc, sizeof(hr.desc), hipMemcpyHostToDevice));

@@ -697,7 +697,6 @@ struct srs_ctx {
   double last_total_ms = 0, last_sweep_ms = 0;
   // captured step blocks, keyed by (steps, gate mode)
   std::map<std::pair<int64_t, uint32_t>, hipGraphExec_t> graphs;
-  int32_t* d_sched = nullptr;
   std::vector<HostScan> scans;
 };
 
@@ -739,11 +738,13 @@ int launch_step(srs_ctx* c, uint32_t gmode);
 // m steps of a single-realization context through the gated sweep, starting
 // from live state index cur, ending with the gating of the last step
 void launch_gated_block(srs_ctx* c, int64_t m, int cur, uint32_t gmode);
-// One step through the single-realization gated sweep; xo_at/xn_at (both or
-// neither) replace X[cur] -> X[cur ^ 1] as the step's state buffers.
+// One replayed step of the tile list from schedule row `row` (ReplayAt), and m of
+// them with the live state of the listed realizations moved on
 void launch_replay(srs_ctx* c, int64_t row, int par, const double* xo = nullptr, double* xn = nullptr,
                    size_t stride = 0, int n_tiles = 1);
 void launch_replay_block(srs_ctx* c, int64_t m, int64_t row, const int32_t* rid, int n_rid);
+// One step through the single-realization gated sweep; xo_at/xn_at (both or
+// neither) replace X[cur] -> X[cur ^ 1] as the step's state buffers.
 void launch_gated(srs_ctx* c, int cur, uint32_t gmode, bool proto, const double* xo_at = nullptr,
                   double* xn_at = nullptr);
 void launch_gate_single(srs_ctx* c, uint32_t gmode);

@@ -821,12 +821,12 @@ template GatedFn pick_gated_bs<SRS_UNIT == 2 ? 128 : SRS_UNIT == 3 ? 256 : 512>(
 #endif  // SRS_UNIT >= 2
 
 #if SRS_UNIT == 0
-// Ends a block of m replayed steps of the listed realizations (all without a
-// list) from schedule row `row`: time, step and live index, and the RyR states
-// of the row after it, as m gating launches leave them.
+// Ends a block of m replayed steps of the listed realizations from schedule row
+// `row`: time, step and live index, and the RyR states of the row after it, as m
+// gating launches leave them.
 __global__ __launch_bounds__(64) void k_replay_end(const RealDesc* __restrict__ D, RealLive* __restrict__ L,
                                                    const int32_t* __restrict__ rid, int64_t m, int64_t row) {
-  const int r = rid ? rid[blockIdx.x] : blockIdx.x;
+  const int r = rid[blockIdx.x];
   const RealDesc& d = D[r];
   RealLive& l = L[r];
   const int64_t k = row + m < d.n_sched ? row + m : d.n_sched - 1;
