@@ -916,28 +916,50 @@ void build_class_rows(HostMesh& hm) {
   };
   std::unordered_map<std::array<double, 5>, int, Hash> classes;
   std::vector<uint32_t> row(3 * (size_t)np + 1, 0);
+  // A regular mesh's few classes are found again without rounding and comparing: a
+  // value less than half a rounding interval from a class's (12 bits; equal to a
+  // zero) rounds to it.
+  struct Seen { int64_t t[5], tol[5]; int id; };
+  std::vector<Seen> seen(512, Seen{{}, {}, -1});
   for (int k = 0; k < n; ++k) {
-    std::array<double, 5> key;
-    int64_t d[5];
+    int64_t u[5], d[5];
+    for (int q = 0; q < 5; ++q) memcpy(&u[q], &hm.coef[(size_t)q * np + k], 8);
+    uint64_t h = 0;
+    for (int q = 0; q < 5; ++q) h += (((uint64_t)u[q] + 4096) >> 13) * (2 * q + 1);
+    Seen& sn = seen[h * 0x9E3779B97F4A7C15ull >> 55];
+    int id = sn.id;
+    bool same = id >= 0;
     for (int q = 0; q < 5; ++q) {
-      const double a = hm.coef[(size_t)q * np + k];
-      if (!std::isfinite(a) || (a == 0.0 && std::signbit(a))) return;  // the classes are keyed by value
-      key[q] = quantize(a);
-      int64_t ka, kt;
-      memcpy(&ka, &a, 8);
-      memcpy(&kt, &key[q], 8);
-      d[q] = ka - kt;  // as the kernel adds it back, for any pair of patterns
-      if (d[q] < -32768 || d[q] > 32767) return;
+      d[q] = (int64_t)((uint64_t)u[q] - (uint64_t)sn.t[q]);  // as the kernel adds it back, for any pair of patterns
+      same &= (uint64_t)d[q] + (uint64_t)sn.tol[q] <= 2 * (uint64_t)sn.tol[q];
     }
-    auto it = classes.find(key);
-    if (it == classes.end()) {
-      if (classes.size() >= 65535 || (classes.size() >= 8192 && 2 * classes.size() > (size_t)k)) return;
-      it = classes.emplace(key, (int)classes.size()).first;
+    if (!same) {
+      std::array<double, 5> key;
+      Seen cls;
+      bool normal = true;
+      for (int q = 0; q < 5; ++q) {
+        const double a = hm.coef[(size_t)q * np + k];
+        if (!std::isfinite(a) || (a == 0.0 && std::signbit(a))) return;  // the classes are keyed by value
+        key[q] = quantize(a);
+        memcpy(&cls.t[q], &key[q], 8);
+        d[q] = u[q] - cls.t[q];
+        if (d[q] < -32768 || d[q] > 32767) return;
+        const int e = (int)(cls.t[q] >> 52 & 0x7ff);
+        cls.tol[q] = cls.t[q] == 0 ? 0 : 4095;
+        normal &= cls.t[q] == 0 || (e != 0 && e < 0x7fe);
+      }
+      auto it = classes.find(key);
+      if (it == classes.end()) {
+        if (classes.size() >= 65535 || (classes.size() >= 8192 && 2 * classes.size() > (size_t)k)) return;
+        it = classes.emplace(key, (int)classes.size()).first;
+      }
+      cls.id = id = it->second;
+      if (normal) sn = cls;
     }
-    auto u = [](int64_t v) { return (uint32_t)(uint16_t)v; };
-    row[3 * (size_t)k] = (uint32_t)it->second | u(d[0]) << 16;
-    row[3 * (size_t)k + 1] = u(d[1]) | u(d[2]) << 16;
-    row[3 * (size_t)k + 2] = u(d[3]) | u(d[4]) << 16;
+    auto w = [](int64_t v) { return (uint32_t)(uint16_t)v; };
+    row[3 * (size_t)k] = (uint32_t)id | w(d[0]) << 16;
+    row[3 * (size_t)k + 1] = w(d[1]) | w(d[2]) << 16;
+    row[3 * (size_t)k + 2] = w(d[3]) | w(d[4]) << 16;
   }
   hm.n_class = (int)classes.size();
   hm.tab.resize(5 * (size_t)hm.n_class);
