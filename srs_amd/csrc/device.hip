@@ -1066,12 +1066,16 @@ int make_map(const HostMesh& hm, int tile, HostMap* m) {
 // state layout unless SRS_TUNE_TILE gave one.
 //
 // Layout: blocks of 64, or an element's species side by side where the halos of
-// an average element cost 0.6 cache lines less with it.  us per step, blocks of
-// 64 / 1 (lines): 927,816 elements in Morton order 20.0 / 20.3 (0.17), with 5% of
-// the elements anywhere 25.4 / 22.9 (0.41), with 10% 31.9 / 26.4 (0.65), shuffled
-// within 2,048 27.1 / 28.5 (0.46), within 131,072 58.5 / 53.4 (3.6), all of them
-// 116 / 75 (3.9); 2,952,000 with 5% 77.6 / 78.8, 10% 96.9 / 87.9, all 436 / 290;
-// 172,494 shuffled within 2,048 8.8 / 8.7, all 17.6 / 15.3.
+// an average element cost half a cache line less with it.  us per step, blocks of
+// 64 / 1 (lines): 927,816 elements in Morton order 20.4 / 22.5 (0.17), with 5% of
+// the elements anywhere 25.5 / 25.3 (0.41), 8% 29.2 / 26.8 (0.55), 10% 32.1 / 27.7
+// (0.65), in shuffled runs of 32 41.7 / 34.7 (0.58); 2,952,000 with 5% 76.0 / 83.5
+// (0.41), 8% 87.0 / 87.5 (0.56), 10% 96.2 / 90.1, all 436 / 250, runs of 32 127 /
+// 102; four members of 56,250 with 5% 14.9 / 13.4, 10% 16.8 / 14.0, runs of 32
+// 18.2 / 16.1; eight of 15,360 with 15% 13.6 / 10.9.  One realization of up to
+// 32,768 elements, whose states stay in the L2s, gains later: 15,360 with 15% 5.8 /
+// 6.5 (0.59), 30% 6.6 / 6.5 (1.01), all 7.0 / 6.6; 28,800 with 15% 6.3 / 6.5 (0.73),
+// 30% 7.1 / 6.5 (1.28).
 //
 // Tile: 512 elements share the most neighbours inside a tile (halos of 1.4
 // elements per element in the block order, 0.6 in the Morton order, 2.0 in RCM;
@@ -1113,7 +1117,7 @@ int plan_tiles(srs_ctx* c, std::vector<HostMap>* maps) {
     n += c->meshes[hr.mesh]->n;
   }
   for (const HostMap& m : *maps) qcap = std::max(qcap, m.qcap);
-  c->quad_block = lines > 0.6 * n ? 1 : 64;
+  c->quad_block = lines > (c->reals.size() == 1 && n <= 1 << 15 ? 1.0 : 0.5) * n ? 1 : 64;
   if (c->tile_set || c->tile == 128) return SRS_OK;
   if (c->quad_block == 1) return make(128);
   // a CU's 160 KB in granules of 1280 B, 42 for each of three workgroups; the
